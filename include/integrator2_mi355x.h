@@ -50,7 +50,8 @@ int i2_device_count(int* n);
 /* Host-side evaluation of the inner integral (Psi, Theta) of triangle tri9 at
  * n points, with the device formulas compiled for the CPU: fast = 0 is the
  * reference's expression (thetaPsi, src/evaluators/evaluatorJ3DK.cu:266-313),
- * fast = 1 the division-free form used by the batched kernels.  For checking. */
+ * fast = 1 the form the kernels use at any point, fast = 2 the form they use
+ * for points at least twice K_j's longest edge away from it.  For checking. */
 int i2_host_theta_psi(int fast, const double* pts, int64_t n, const double* tri9, double* out4);
 /* Host-side evaluation of the kernels' FP64 logarithm (fn = 0, of x),
  * two-argument arctangent (fn = 1, atan2(y, x)), square root (fn = 2, of x;

@@ -7,6 +7,10 @@ remainder, so that log(m) = T_j + log1p(m invc_j - 1) to well below one ulp.
 
 i2_atantab.inc: entries k = 0..32: {atan(k/32) hi, lo}.
 
+It also prints the coefficients of atanh_over and atan_over of i2_math.hpp:
+the interpolants of (atanh(sqrt s)/sqrt s - 1)/s on [0, 1/16] and
+(atan(sqrt v)/sqrt v - 1)/v on [0, 0.003] at 8 and 5 Chebyshev nodes.
+
 All values from 60-digit mpmath.  Run from this directory:
     python gen_math_tables.py
 """
@@ -43,3 +47,14 @@ with open("i2_atantab.inc", "w") as f:
     for k in range(33):
         hi, lo = split(mpmath.atan(mpmath.mpf(k) / 32))
         f.write("{%r, %r},\n" % (hi, lo))
+
+
+def interpolant(f, top, n):
+    """Coefficients, ascending, of the degree-(n - 1) interpolant of (f(s) - 1)/s on [0, top]."""
+    nodes = [top / 2 * (1 + mpmath.cos(mpmath.pi * (2 * k + 1) / (2 * n))) for k in range(n)]
+    A = mpmath.matrix([[s ** j for j in range(n)] for s in nodes])
+    return [float(c) for c in mpmath.lu_solve(A, mpmath.matrix([(f(s) - 1) / s for s in nodes]))]
+
+
+print("atanh_over", interpolant(lambda s: mpmath.atanh(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf(1) / 16, 8))
+print("atan_over", interpolant(lambda s: mpmath.atan(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf("0.003"), 5))

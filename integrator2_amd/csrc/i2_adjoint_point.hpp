@@ -15,6 +15,36 @@ namespace i2d {
 
 I2_HD __forceinline__ void axpy(d3& y, double a, d3 x) { y.x += a * x.x; y.y += a * x.y; y.z += a * x.z; }
 
+I2_HD __forceinline__ double l_plus_dtau(double l, d3 d, d3 t) {
+    const d3 c = cross(d, t);
+    return dot(c, c) / (l - dot(d, t));
+}
+// Rare branch of the six l + d.tau terms: terms below 1e-4 l recomputed
+// without cancellation, then the reference's degenerate branch (a point on an
+// edge line of K_j keeps the ratio of distances, evaluatorJ3DK.cu:294-307).
+I2_HD __forceinline__ void fix_terms(const JGeom& J, d3 da, d3 db, d3 dc, double la, double lb, double lc,
+                                     double& n1, double& e1, double& n2, double& e2, double& n3, double& e3,
+                                     bool& f1, bool& f2, bool& f3) {
+    const double s = 1e-4;
+    if (n1 < s * la) n1 = l_plus_dtau(la, da, J.tc);
+    if (e1 < s * lb) e1 = l_plus_dtau(lb, db, J.tc);
+    if (n2 < s * lb) n2 = l_plus_dtau(lb, db, J.ta);
+    if (e2 < s * lc) e2 = l_plus_dtau(lc, dc, J.ta);
+    if (n3 < s * lc) n3 = l_plus_dtau(lc, dc, J.tb);
+    if (e3 < s * la) e3 = l_plus_dtau(la, da, J.tb);
+    const double h = 0.5 * EPS_PSI_THETA2;
+    f1 = fabs(e1) < h * lb; f2 = fabs(e2) < h * lc; f3 = fabs(e3) < h * la;
+    if (f1) { n1 = lb; e1 = la; }
+    if (f2) { n2 = lc; e2 = lb; }
+    if (f3) { n3 = la; e3 = lc; }
+}
+// one test per distance for the rare branch (the per-term tests are repeated
+// inside it rather than kept live through the common path)
+I2_HD __forceinline__ bool terms_need_fix(double la, double lb, double lc, double n1, double e1, double n2, double e2,
+                                          double n3, double e3) {
+    const double s = 1e-4;
+    return fmin(fmin(fmin(n1, e3) - s * la, fmin(e1, n2) - s * lb), fmin(e2, n3) - s * lc) < 0.0;
+}
 // cotangents of the parameters of thetaPsi over K_j: vertices and edge tangents
 struct TPBar { d3 a, b, c, ta, tb, tc; };
 

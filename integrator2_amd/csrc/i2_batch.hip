@@ -118,8 +118,10 @@ __device__ __forceinline__ void load_rule(RuleLDS& s, const Rule& R) {
     i2m::fill_mathtab(s.lt);
 }
 
-// Partial quadrature sum_k w_k f(r_k) of one sub-panel over points k = s, s + step, ...
-template <int TYPE>
+// Partial quadrature sum_k w_k f(r_k) of one sub-panel over points k = s,
+// s + step, ...  Disjoint pairs: the inner integral's terms (FAR:
+// theta_terms_far), converted to (Psi, Theta) once per task by the caller.
+template <int TYPE, bool FAR = false>
 __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int step, d3 a, d3 b, d3 c, const JGeom& J,
                                         const Sing<TYPE>& sg) {
     q4 acc = q4zero();
@@ -127,8 +129,9 @@ __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int s
         d3 p = R.L1[k] * a;
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
-        q4 f = theta_psi_fast(p, J, &R.lt);
-        if (TYPE != I2_NOT_NEIGHBORS) f = f - sg.at(p, &R.lt);
+        q4 f;
+        if (TYPE == I2_NOT_NEIGHBORS) f = FAR ? theta_terms_far(p, J) : theta_terms(p, J, &R.lt);
+        else f = theta_psi_fast(p, J, &R.lt) - sg.at(p, &R.lt);
         acc = acc + R.w[k] * f;
     }
     return acc;
@@ -136,10 +139,10 @@ __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int s
 
 // Quadrature points of a disjoint item's control panel K_i (uniform over the
 // workgroup): the level-0 panel and its four level-1 children, in the order
-// sweep_task sums them, computed once per item instead of once per pair.
-// The rule weight of each point is stored beside it, so that one LDS address
-// serves the point and its weight.
-struct PtsLDS { double x[5 * MAX_POINTS], y[5 * MAX_POINTS], z[5 * MAX_POINTS], w[5 * MAX_POINTS]; };
+// sweep_task sums them, computed once per item instead of once per pair.  Each
+// point and its rule weight share a 32-byte record: two 128-bit LDS reads.
+struct alignas(32) QPoint { double x, y, z, w; };
+struct PtsLDS { QPoint q[5 * MAX_POINTS]; };
 
 // Levels 0 and 1 in one pass with a rule whose point 0 is the centroid: the
 // centroid of K_i is also the centroid of its central level-1 child (child 4),
@@ -161,22 +164,48 @@ __device__ __forceinline__ void load_points(PtsLDS& P, const RuleLDS& R, int npt
         d3 p = R.L1[k] * a;
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
-        P.x[t] = p.x; P.y[t] = p.y; P.z[t] = p.z; P.w[t] = R.w[k];
+        P.q[t] = {p.x, p.y, p.z, R.w[k]};
     }
 }
 
-// Partial quadrature sum over the precomputed points base + k, k = s, s + step, ...,
-// added in that order to acc, of (Psi, Theta / 2): the caller doubles the w
-// component (theta_psi_fast_half)
-__device__ __forceinline__ q4 quad_pts_half(const RuleLDS& R, const PtsLDS& P, int base, int npts, int s, int step,
-                                            const JGeom& J, q4 acc = q4zero()) {
-    for (int k = s; k < npts; k += step) {
-        const d3 p{P.x[base + k], P.y[base + k], P.z[base + k]};
-        acc = acc + P.w[base + k] * theta_psi_fast_half(p, J, &R.lt);
+// Weighted sum of the inner integral's terms over the precomputed points k =
+// k0, k0 + step, ... < k1, added in that order to acc.  FAR: theta_terms_far.
+template <bool FAR>
+__device__ __forceinline__ q4 terms_at(const RuleLDS& R, const QPoint& Q, const JGeom& J) {
+    const d3 p{Q.x, Q.y, Q.z};
+    return Q.w * (FAR ? theta_terms_far(p, J) : theta_terms(p, J, &R.lt));
+}
+template <bool FAR>
+__device__ __forceinline__ q4 quad_pts(const RuleLDS& R, const PtsLDS& P, int k0, int k1, int step, const JGeom& J, q4 acc) {
+    for (int k = k0; k < k1; k += step) {
+        const QPoint Q = P.q[k];
+        const d3 p{Q.x, Q.y, Q.z};
+        const q4 t = FAR ? theta_terms_far(p, J) : theta_terms(p, J, &R.lt);
+        acc = {fma(Q.w, t.x, acc.x), fma(Q.w, t.y, acc.y), fma(Q.w, t.z, acc.z), fma(Q.w, t.w, acc.w)};
     }
     return acc;
 }
-__device__ __forceinline__ q4 double_w(q4 v) { return {v.x, v.y, v.z, 2.0 * v.w}; }
+// Sums of the terms over level 0 (T0) and level 1 (T1) of a pair, lane s of LPP.
+template <bool FAR, int LPP>
+__device__ __forceinline__ void sweep_terms(const RuleLDS& R, const PtsLDS& P, int npts, bool share, bool need0, bool need1, int s,
+                                            const JGeom& J, q4& T0, q4& T1) {
+    int k0 = s, k1 = npts + s;
+    if (share) {
+        // point 0 of child 4 stands for point 0 of level 0 as well (lane 0 takes both)
+        if (s == 0) {
+            T0 = terms_at<FAR>(R, P.q[4 * npts], J);
+            T1 = T0;
+            k0 = LPP;
+        }
+        // children 1 to 3 and child 4's other points around the shared one
+        T0 = quad_pts<FAR>(R, P, k0, npts, LPP, J, T0);
+        T1 = quad_pts<FAR>(R, P, k1, 4 * npts, LPP, J, T1);
+        T1 = quad_pts<FAR>(R, P, 4 * npts + k0, 5 * npts, LPP, J, T1);
+        return;
+    }
+    if (need0) T0 = quad_pts<FAR>(R, P, k0, npts, LPP, J, T0);
+    if (need1) T1 = quad_pts<FAR>(R, P, k1, 5 * npts, LPP, J, T1);
+}
 
 __device__ __forceinline__ q4 shfl_sum(q4 v, int G) {
     for (int m = 1; m < G; m <<= 1) {
@@ -261,7 +290,8 @@ __device__ __forceinline__ void add_row(const MeshDesc& M, int type, int i, q4 r
 // Levels 0 and 1 of one task (lane group of LPP lanes), then the Runge check.
 template <int TYPE, int LPP>
 __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS& R, int m, int i, int j, int64_t z, bool valid,
-                                              int s, const Panel& I, const Panel& J, const PtsLDS* pts = nullptr) {
+                                              int s, const Panel& I, const Panel& J, const PtsLDS* pts = nullptr,
+                                              const Ball* ball = nullptr) {
     Sing<TYPE> sg;
     if (TYPE != I2_NOT_NEIGHBORS && valid) sg.init(I, J);
     const JGeom JG = jgeom(J);
@@ -270,25 +300,19 @@ __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS&
     const bool need1 = A.fixed ? A.last_level == 1 : A.last_level >= 1;
     q4 v0 = q4zero(), v1 = q4zero();
     if constexpr (TYPE == I2_NOT_NEIGHBORS) {
+        // one loop per wavefront: far only if every pair of the wavefront is
+        const bool near = __ballot(valid && !panel_far(*ball, JG)) != 0ull;
         if (valid) {
-            const double a1 = 0.25 * I.area;
-            if (share_centroid(A)) {
-                // point 0 of child 4 stands for point 0 of level 0 (lane 0
-                // takes both); child 4 is summed first, so that the shared
-                // value is dead before children 1-3
-                const int k0 = s == 0 ? LPP : s, c4 = 4 * npts;
-                const q4 fc = s == 0 ? pts->w[c4] * theta_psi_fast_half(d3{pts->x[c4], pts->y[c4], pts->z[c4]}, JG, &R.lt)
-                                     : q4zero();
-                v0 = I.area * double_w(quad_pts_half(R, *pts, 0, npts, k0, LPP, JG, fc));
-                v1 = a1 * double_w(quad_pts_half(R, *pts, c4, npts, k0, LPP, JG, fc));
-                for (int sub = 1; sub <= 3; ++sub)
-                    v1 = v1 + a1 * double_w(quad_pts_half(R, *pts, sub * npts, npts, s, LPP, JG));
+            q4 T0 = q4zero(), T1 = q4zero();
+            if (near) {
+                sweep_terms<false, LPP>(R, *pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
             } else {
-                if (need0) v0 = I.area * double_w(quad_pts_half(R, *pts, 0, npts, s, LPP, JG));
-                if (need1)
-                    for (int sub = 1; sub <= 4; ++sub)
-                        v1 = v1 + a1 * double_w(quad_pts_half(R, *pts, sub * npts, npts, s, LPP, JG));
+                sweep_terms<true, LPP>(R, *pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
+                T0 = far_scale(T0, JG);
+                T1 = far_scale(T1, JG);
             }
+            v0 = I.area * psi_of_terms(T0, JG);
+            v1 = (0.25 * I.area) * psi_of_terms(T1, JG);
         }
     } else if (valid) {
         if (need0) v0 = I.area * quad_part<TYPE>(R, npts, s, LPP, I.a, I.b, I.c, JG, sg);
@@ -343,6 +367,7 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
         const int tiles = (M.nT + P - 1) / P;
         const int i = __builtin_amdgcn_readfirstlane((int)(r / tiles));
         const Panel I = M.panels[i];
+        const Ball ball = panel_ball(I.a, I.b, I.c, A.rule.reach);
         load_points(pts, R, A.rule.n, I);
         __syncthreads();
         for (int round = 0; round < P; round += per_round) {
@@ -352,7 +377,7 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
         const Panel J = M.panels[in_range ? j : i];
         const bool valid = in_range && j != i && shared_count(I, J) == 0;
         const int64_t z = valid ? disjoint_task(M, i, j) : 0;
-        const StepOut o = sweep_task<I2_NOT_NEIGHBORS, LPP>(A, R, m, i, j, z, valid, s, I, J, &pts);
+        const StepOut o = sweep_task<I2_NOT_NEIGHBORS, LPP>(A, R, m, i, j, z, valid, s, I, J, &pts, &ball);
         q4 rp0 = q4zero(), rp1 = q4zero();
         if (o.finished) finish_task<I2_NOT_NEIGHBORS, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
         if (OUT == OUT_ROW_SUMS) {
@@ -434,6 +459,7 @@ __device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, 
         }
     }
     acc = shfl_sum(acc, G);
+    if (TYPE == I2_NOT_NEIGHBORS) acc = psi_of_terms(acc, JG);
     if (!valid || s != 0) return;
     const q4 prev = {e.prev.x, e.prev.y, e.prev.z, e.prev.w};
     StepOut o{false, false, level, acc, acc};

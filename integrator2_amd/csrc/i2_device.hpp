@@ -44,6 +44,7 @@ constexpr int MAX_POINTS = 16;   // largest rule has 13 points
 // src/NumericalIntegrator3d.cu:197-216.
 struct Rule {
     double L1[MAX_POINTS], L2[MAX_POINTS], L3[MAX_POINTS], w[MAX_POINTS];
+    double reach;   // largest sum_k |L_k - 1/3| over the points outside the triangle, at least 1 (see panel_ball)
     double pow2p;   // 2^order, the Runge factor (src/evaluators/evaluator3d.cu:101-106)
     int n;
     int order;
@@ -59,6 +60,19 @@ inline int rule_centroid(const double* L1, const double* L2, int n) {
     for (int k = 0; k < n; ++k)
         if (fabs(L1[k] - 1.0 / 3.0) <= 1e-14 && fabs(L2[k] - 1.0 / 3.0) <= 1e-14) return k;
     return -1;
+}
+
+// How far a rule's points reach from a triangle's centroid, relative to its
+// vertices: 1 where every point lies in the triangle (|p - c| is convex), else
+// the bound |p - c| <= sum_k |L_k - 1/3| |v_k - c|.  At least 1, so that the
+// ball of a panel also holds the points of its sub-panels.
+inline double rule_reach(const double* L1, const double* L2, const double* L3, int n) {
+    double reach = 1.0;
+    for (int k = 0; k < n; ++k) {
+        const double s = fabs(L1[k] - 1.0 / 3.0) + fabs(L2[k] - 1.0 / 3.0) + fabs(L3[k] - 1.0 / 3.0);
+        if (!(L1[k] >= 0.0 && L2[k] >= 0.0 && L3[k] >= 0.0)) reach = s > reach || s != s ? s : reach;
+    }
+    return reach;
 }
 
 // ------------------------------------------------------------ vectors
@@ -144,116 +158,129 @@ I2_HD __forceinline__ q4 theta_psi(d3 p, const d3& A, const d3& B, const d3& C, 
     return r;
 }
 
-// Same (Psi, Theta) without unit vectors, for the fast path.  With
-// d = p - vertex and l = |d|, the reference's l (1 + (d/l).tau) is l + d.tau,
-// and the solid-angle atan2 has both arguments multiplied by la lb lc > 0
-// (Van Oosterom and Strackee, IEEE Trans. Biomed. Eng. 30 (1983) 125-126):
-// identical in exact arithmetic, with 3 square roots, 1 reciprocal, 3 logs
-// and 1 atan2 per point instead of 13 divisions (sqrt, log and atan2 from
-// i2_math.hpp, within 2 ulp; `lt` holds their reduction tables, in LDS on the
-// device).  The degenerate-branch tests |1 + (d/l).tau| < eps become
-// |l + d.tau| < eps l.
+// The kernels' form of the inner integral.  Psi_j(p) is the sum over K_j's
+// edges of tau_e times the line integral of 1/|p - r| along the edge, and with
+// l the distances of p to the edge's ends, S their sum and L the edge length
+// that integral is t = ln((S + L)/(S - L)) = 2 atanh(L/S): the reference's
+// log of (l + d.tau) ratios, without dot products and without their
+// cancellation near the edge's extension (S - L cancels near the edge itself
+// only).  Theta = 2 atan2(y, x) with both arguments scaled by la lb lc > 0 (Van
+// Oosterom and Strackee, IEEE Trans. Biomed. Eng. 30 (1983) 125-126): y =
+// da.((B - A) x (C - A)), x = la lb lc + da.db lc + db.dc la + dc.da lb.  Away
+// from the edges, P = S^2 - L^2 = 2 (la lb + da.db) gives 2 x = P_c lc + P_a la
+// + P_b lb - 4 la lb lc, and every term comes from the three distances and
+// per-panel constants.
 //
-// Near an edge line of K_j (in particular next to a vertex that K_i shares
-// with K_j) l + d.tau cancels: with the point at distance delta from the line
-// it is ~delta^2/(2l), and the sum loses l^2/delta^2 ulps, as the reference's
-// 1 + cos does.  Terms below 1e-4 l are recomputed as |d x tau|^2/(l - d.tau),
-// the same number without cancellation, so these points come out more
-// accurate than the reference formula.  The branch is rare for disjoint pairs
-// and skipped by whole wavefronts.
+// The tangents are constant over K_i, so the quadrature sums the three t and
+// Theta/2 and multiplies by the tangents once per sum (psi_of_terms).
 // K_j for the inner integral: vertices, edge tangents (as in the Panel
 // record), edge lengths La = |C - B|, Lb = |A - C|, Lc = |B - A| and
 // N2 = (B - A) x (C - A) (twice the area times the unit normal)
 struct JGeom { d3 a, b, c, ta, tb, tc; double La, Lb, Lc; d3 N2; };
 I2_HD __forceinline__ JGeom make_jgeom(d3 a, d3 b, d3 c, d3 ta, d3 tb, d3 tc) {
-    return {a, b, c, ta, tb, tc, vlen(c - b), vlen(a - c), vlen(b - a), cross(b - a, c - a)};
+    // 0 * tau: a panel with a zero edge (NaN tangent) stays NaN in every term
+    return {a, b, c, ta, tb, tc, vlen(c - b) + 0.0 * ta.x, vlen(a - c) + 0.0 * tb.x, vlen(b - a) + 0.0 * tc.x,
+            cross(b - a, c - a)};
 }
-I2_HD __forceinline__ double l_plus_dtau(double l, d3 d, d3 t) {
-    const d3 c = cross(d, t);
-    return dot(c, c) / (l - dot(d, t));
+// S - L without cancellation, 2 |u x v|^2 / ((lu lv - u.v)(S + L)), from
+// (S - L)(S + L) = 2 (lu lv + u.v) and (lu lv + u.v)(lu lv - u.v) = |u x v|^2;
+// n/e is the ratio (S + L)/(S - L)
+I2_HD __forceinline__ void edge_ratio(d3 u, d3 v, double lu, double lv, double L, double& n, double& e) {
+    const d3 c = cross(u, v);
+    const double c2 = dot(c, c);
+    e = 2.0 * c2 / (fma(lu, lv, -dot(u, v)) * n);
+    // the reference's degenerate branch: a point on the edge's line keeps the
+    // ratio of distances (evaluatorJ3DK.cu:294-307)
+    if (c2 < EPS_PSI_THETA2 * (L * L) * (lv * lv)) { n = lv; e = lu; }
 }
-// Rare branch of the six l + d.tau terms: terms below 1e-4 l recomputed
-// without cancellation, then the reference's degenerate branch (a point on an
-// edge line of K_j keeps the ratio of distances, evaluatorJ3DK.cu:294-307).
-I2_HD __forceinline__ void fix_terms(const JGeom& J, d3 da, d3 db, d3 dc, double la, double lb, double lc,
-                                     double& n1, double& e1, double& n2, double& e2, double& n3, double& e3,
-                                     bool& f1, bool& f2, bool& f3) {
-    const double s = 1e-4;
-    if (n1 < s * la) n1 = l_plus_dtau(la, da, J.tc);
-    if (e1 < s * lb) e1 = l_plus_dtau(lb, db, J.tc);
-    if (n2 < s * lb) n2 = l_plus_dtau(lb, db, J.ta);
-    if (e2 < s * lc) e2 = l_plus_dtau(lc, dc, J.ta);
-    if (n3 < s * lc) n3 = l_plus_dtau(lc, dc, J.tb);
-    if (e3 < s * la) e3 = l_plus_dtau(la, da, J.tb);
-    const double h = 0.5 * EPS_PSI_THETA2;
-    f1 = fabs(e1) < h * lb; f2 = fabs(e2) < h * lc; f3 = fabs(e3) < h * la;
-    if (f1) { n1 = lb; e1 = la; }
-    if (f2) { n2 = lc; e2 = lb; }
-    if (f3) { n3 = la; e3 = lc; }
-}
-// one test per distance for the rare branch (the per-term tests are repeated
-// inside it rather than kept live through the common path)
-I2_HD __forceinline__ bool terms_need_fix(double la, double lb, double lc, double n1, double e1, double n2, double e2,
-                                          double n3, double e3) {
-    const double s = 1e-4;
-    return fmin(fmin(fmin(n1, e3) - s * la, fmin(e1, n2) - s * lb), fmin(e2, n3) - s * lc) < 0.0;
-}
-// The forward kernels reuse three of the terms' dot products in the solid
-// angle: with db = da - Lc tc (and cyclically), da.db = |da|^2 - Lc da.tc,
-// db.dc = |db|^2 - La db.ta, dc.da = |dc|^2 - Lb dc.tb; and
-// da.(db x dc) = da.((B - A) x (C - A)).  The rounding of tc, Lc and N2 makes
-// these a fixed relative 1e-16 perturbation of x and y, which moves Theta by a
-// relative 1e-16.  The terms themselves keep their own dot products: there a
-// fixed absolute error of ulp(Lc) (from db.tc = da.tc - Lc) is relative to
-// l + d.tau, which can be much smaller than Lc, and it does not average out
-// over the points as rounding noise does.
-//
-// theta_psi_fast_half returns (Psi, Theta / 2): a quadrature sum of Theta / 2
-// doubled once equals the sum of Theta bit for bit (scaling by 2 is exact),
-// which saves the doubling per point.
-I2_HD __forceinline__ q4 theta_psi_fast_half(d3 p, const JGeom& J, const i2m::MathTable* __restrict__ lt) {
+// Terms of one point: line integrals t along A->B, B->C, C->A (the edges of
+// tau_c, tau_a, tau_b) and Theta/2.  For any point; `lt` holds the reduction
+// tables of log and atan2.  One rare branch: an edge closer than about L/30
+// (S - L below S/1024), and atan2 arguments outside the table path's range.
+I2_HD __forceinline__ q4 theta_terms(d3 p, const JGeom& J, const i2m::MathTable* __restrict__ lt) {
     const d3 da = p - J.a, db = p - J.b, dc = p - J.c;
-    const double qa = dot(da, da), qb = dot(db, db), qc = dot(dc, dc);
-    const double la = i2m::sqrt_pos(qa), lb = i2m::sqrt_pos(qb), lc = i2m::sqrt_pos(qc);
-    const double s1 = dot(da, J.tc), s2 = dot(db, J.ta), s3 = dot(dc, J.tb);
-    double n1 = la + s1, e1 = lb + dot(db, J.tc);
-    double n2 = lb + s2, e2 = lc + dot(dc, J.ta);
-    double n3 = lc + s3, e3 = la + dot(da, J.tb);
-    if (__builtin_expect(terms_need_fix(la, lb, lc, n1, e1, n2, e2, n3, e3), 0)) {
-        bool f1, f2, f3;
-        fix_terms(J, da, db, dc, la, lb, lc, n1, e1, n2, e2, n3, e3, f1, f2, f3);
+    const double la = i2m::sqrt_cubic(dot(da, da)), lb = i2m::sqrt_cubic(dot(db, db)), lc = i2m::sqrt_cubic(dot(dc, dc));
+    const double S1 = la + lb, S2 = lb + lc, S3 = lc + la;
+    double n1 = S1 + J.Lc, n2 = S2 + J.La, n3 = S3 + J.Lb;
+    double e1 = S1 - J.Lc, e2 = S2 - J.La, e3 = S3 - J.Lb;
+    const double s = 0x1p-10;
+    if (__builtin_expect(fmin(fmin(fma(-s, S1, e1), fma(-s, S2, e2)), fma(-s, S3, e3)) < 0.0, 0)) {
+        if (e1 < s * S1) edge_ratio(da, db, la, lb, J.Lc, n1, e1);
+        if (e2 < s * S2) edge_ratio(db, dc, lb, lc, J.La, n2, e2);
+        if (e3 < s * S3) edge_ratio(dc, da, lc, la, J.Lb, n3, e3);
     }
     const double e12 = e1 * e2;
-    const double inv = i2m::rcp_pos(e12 * e3);
-    const double a1 = n1 * (e2 * e3) * inv, a2 = n2 * (e1 * e3) * inv, a3 = n3 * e12 * inv;
+    const double inv = i2m::rcp_cubic(e12 * e3);
+    const double i12 = inv * e3;
+    // x from the dot products: beside an edge x and y both vanish, and P there
+    // has the rounding of S^2, several times that of da.db
     const double y = dot(da, J.N2);
-    const double x = la * lb * lc + fma(-J.Lc, s1, qa) * lc + fma(-J.La, s2, qb) * la + fma(-J.Lb, s3, qc) * lb;
-    // The table paths run without branches on every lane, so that the four
-    // evaluations overlap; the rare lanes outside their ranges are redone by
-    // the library below.
-    const bool o1 = i2m::pos_normal(a1), o2 = i2m::pos_normal(a2), o3 = i2m::pos_normal(a3);
-    const bool o4 = i2m::atan2_in_range(y, x);
-    double t1 = i2m::log_tab_any(a1, lt);
-    double t2 = i2m::log_tab_any(a2, lt);
-    double t3 = i2m::log_tab_any(a3, lt);
-    double th = i2m::atan2_any(y, x, lt);
-    if (__builtin_expect(!(o1 & o2 & o3 & o4), 0)) {
-        if (!o1) t1 = i2m::log_slow(a1);
-        if (!o2) t2 = i2m::log_slow(a2);
-        if (!o3) t3 = i2m::log_slow(a3);
-        if (!o4) th = i2m::atan2_slow(y, x);
+    const double x = la * lb * lc + dot(da, db) * lc + dot(db, dc) * la + dot(dc, da) * lb;
+    // a ratio is positive and normal unless it is NaN, which the table path
+    // keeps: no range test is needed
+    const double t1 = i2m::log_tab_any(n1 * (i12 * e2), lt);
+    const double t2 = i2m::log_tab_any(n2 * (i12 * e1), lt);
+    const double t3 = i2m::log_tab_any(n3 * (inv * e12), lt);
+    double h = i2m::atan2_any(y, x, lt);
+    if (__builtin_expect(!i2m::atan2_in_range(y, x), 0)) {
+        // zero, NaN, or lengths near the ends of the exponent range
+        const double sum = fabs(x) + fabs(y), k = sum < 1.0 ? 0x1p600 : 0x1p-600;
+        h = sum == 0.0 ? 0.0 : i2m::atan2_any(y * k, x * k, lt);
+        if (!(sum <= 1.7976931348623157e308)) h = sum - sum;
     }
-    q4 r;
-    r.x = t1 * J.tc.x + t2 * J.ta.x + t3 * J.tb.x;
-    r.y = t1 * J.tc.y + t2 * J.ta.y + t3 * J.tb.y;
-    r.z = t1 * J.tc.z + t2 * J.ta.z + t3 * J.tb.z;
-    r.w = th;
-    return r;
+    return {t1, t2, t3, h};
+}
+// The same for a point and a panel K_j whose every point is at least twice
+// K_j's longest edge away (z = L/S <= 1/4 per edge; the solid angle is at most
+// (sqrt 3/4)/4, so that |tan(Theta/4)| <= 0.0542): polynomials instead of
+// tables, one reciprocal of S1 S2 S3 2x, no branch.  The line integrals come
+// without their factor 2 L (far_scale).  About 105 FP64 instructions against
+// 180 for theta_terms; the reference's formula as the kernels evaluated it
+// before (six dot products, three table logs, table atan2) took 212.
+I2_HD __forceinline__ q4 theta_terms_far(d3 p, const JGeom& J) {
+    const d3 da = p - J.a, db = p - J.b, dc = p - J.c;
+    const double la = i2m::sqrt_cubic(dot(da, da)), lb = i2m::sqrt_cubic(dot(db, db)), lc = i2m::sqrt_cubic(dot(dc, dc));
+    const double q1 = J.Lc * J.Lc, q2 = J.La * J.La, q3 = J.Lb * J.Lb;
+    const double S1 = la + lb, S2 = lb + lc, S3 = lc + la;
+    const double P1 = fma(S1, S1, -q1), P2 = fma(S2, S2, -q2), P3 = fma(S3, S3, -q3);
+    const double x = fma(fma(la * lb, -4.0, P1), lc, fma(P2, la, P3 * lb));   // 2 x
+    const double y = dot(da, 2.0 * J.N2);
+    const double s12 = S1 * S2, s3x = S3 * x;
+    const double inv = i2m::rcp_cubic(s12 * s3x);
+    const double i12 = inv * s3x, i3x = inv * s12;
+    const double r1 = i12 * S2, r2 = i12 * S1, r3 = i3x * x, u = y * (i3x * S3);
+    return {r1 * i2m::atanh_over(q1 * (r1 * r1)), r2 * i2m::atanh_over(q2 * (r2 * r2)), r3 * i2m::atanh_over(q3 * (r3 * r3)),
+            u * i2m::atan_over(u * u)};
+}
+// sums of theta_terms_far to sums of theta_terms
+I2_HD __forceinline__ q4 far_scale(q4 T, const JGeom& J) { return {2.0 * J.Lc * T.x, 2.0 * J.La * T.y, 2.0 * J.Lb * T.z, T.w}; }
+// (Psi, Theta) of a sum of terms
+I2_HD __forceinline__ q4 psi_of_terms(q4 T, const JGeom& J) {
+    return {T.x * J.tc.x + T.y * J.ta.x + T.z * J.tb.x, T.x * J.tc.y + T.y * J.ta.y + T.z * J.tb.y,
+            T.x * J.tc.z + T.y * J.ta.z + T.z * J.tb.z, 2.0 * T.w};
 }
 I2_HD __forceinline__ q4 theta_psi_fast(d3 p, const JGeom& J, const i2m::MathTable* __restrict__ lt) {
-    q4 r = theta_psi_fast_half(p, J, lt);
-    r.w = 2.0 * r.w;
-    return r;
+    return psi_of_terms(theta_terms(p, J, lt), J);
+}
+
+// Bounding ball of a control panel's quadrature points on every refinement
+// level: centroid, and the radius of its vertices times the rule's reach
+struct Ball { d3 c; double r; };
+I2_HD __forceinline__ Ball panel_ball(d3 a, d3 b, d3 c, double reach) {
+    const d3 m = (1.0 / 3.0) * (a + b + c);
+    const d3 u = a - m, v = b - m, w = c - m;
+    return {m, reach * sqrt(fmax(fmax(dot(u, u), dot(v, v)), dot(w, w)))};
+}
+// True where theta_terms_far holds for every quadrature point of the control
+// panel in ball B: K_j lies within 2/3 of its longest edge M of its centroid
+// (a vertex is 2/3 of a median away), so every distance to it is at least
+// 2 M if the centroids are B.r + (2 + 2/3) M apart (1 + 2^-20 covers the
+// rounding of this test).  The scale test keeps S1 S2 S3 2x in range.  NaN
+// panels are not far.
+I2_HD __forceinline__ bool panel_far(const Ball& B, const JGeom& J) {
+    const d3 d = (1.0 / 3.0) * (J.a + J.b + J.c) - B.c;
+    const double M = fmax(fmax(J.La, J.Lb), J.Lc), need = fma(M, 8.0 / 3.0, B.r) * (1.0 + 0x1p-20), d2 = dot(d, d);
+    return d2 >= need * need && M >= 0x1p-150 && d2 <= 0x1p300;
 }
 
 // ------------------------------------------------------------ singular parts

@@ -53,7 +53,9 @@ template <> struct PairCtx<I2_SIMPLE_NEIGHBORS> {
 // own FP64 form loses up to 1e-7 of a value to cancellation where a
 // quadrature point lies near the extension of an edge line of K_j, which
 // moves Runge decisions; both paths therefore take decisions on accurate values.
-template <int TYPE>
+// Disjoint pairs sum the inner integral's terms (FAR: theta_terms_far), which
+// the caller converts to (Psi, Theta) once per task.
+template <int TYPE, bool FAR>
 __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, d3 a, d3 b, d3 c, double area,
                                        const JGeom& J, const PairCtx<TYPE>& ctx) {
     q4 acc = q4zero();
@@ -61,8 +63,9 @@ __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, 
         d3 p = R.L1[k] * a;
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
-        q4 f = theta_psi_fast(p, J, lt);
-        if (TYPE != I2_NOT_NEIGHBORS) f = f - ctx.sing(p, lt);
+        q4 f;
+        if (TYPE == I2_NOT_NEIGHBORS) f = FAR ? theta_terms_far(p, J) : theta_terms(p, J, lt);
+        else f = theta_psi_fast(p, J, lt) - ctx.sing(p, lt);
         acc = acc + R.w[k] * f;
     }
     return area * acc;
@@ -71,7 +74,7 @@ __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, 
 // Level-`level` value of tasks: lanes per task = 1 << lanes_log2; lane `sub`
 // walks sub-panels sub, sub + G, ... < 4^level; butterfly reduction.
 template <int TYPE, bool IMPLICIT>
-__global__ __launch_bounds__(256) void k_level(int64_t nitems, const int32_t* __restrict__ list, TaskSource src,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_NOT_NEIGHBORS ? 3 : 2))) void k_level(int64_t nitems, const int32_t* __restrict__ list, TaskSource src,
                                                const Panel* __restrict__ panels, Rule R, int level, int lanes_log2,
                                                double4* __restrict__ out) {
     __shared__ i2m::MathTable lt;
@@ -96,11 +99,23 @@ __global__ __launch_bounds__(256) void k_level(int64_t nitems, const int32_t* __
         double area = I.area;
         for (int l = 0; l < level; ++l) area *= 0.25;
         const uint32_t nsub = 1u << (2 * level);
-        for (uint32_t c = sub; c < nsub; c += G) {
-            d3 a = I.a, b = I.b, cc = I.c;
-            sub_panel(a, b, cc, level, c);
-            acc = acc + quad_sub<TYPE>(R, &lt, a, b, cc, area, JG, ctx);
+        // disjoint pairs: one loop per wavefront, far only if every pair of it is
+        const bool far = TYPE == I2_NOT_NEIGHBORS && __all(panel_far(panel_ball(I.a, I.b, I.c, R.reach), JG));
+        if (far) {
+            for (uint32_t c = sub; c < nsub; c += G) {
+                d3 a = I.a, b = I.b, cc = I.c;
+                sub_panel(a, b, cc, level, c);
+                acc = acc + quad_sub<TYPE, true>(R, &lt, a, b, cc, area, JG, ctx);
+            }
+            acc = far_scale(acc, JG);
+        } else {
+            for (uint32_t c = sub; c < nsub; c += G) {
+                d3 a = I.a, b = I.b, cc = I.c;
+                sub_panel(a, b, cc, level, c);
+                acc = acc + quad_sub<TYPE, false>(R, &lt, a, b, cc, area, JG, ctx);
+            }
         }
+        if (TYPE == I2_NOT_NEIGHBORS) acc = psi_of_terms(acc, JG);
     }
     for (int m = 1; m < G; m <<= 1) {
         acc.x += __shfl_xor(acc.x, m);
@@ -504,6 +519,7 @@ int i2_integrator_create(i2_integrator** out, const i2_mesh* mesh, const double*
         }
     }
     it->rule.centroid = i2d::rule_centroid(it->rule.L1, it->rule.L2, nPts);
+    it->rule.reach = i2d::rule_reach(it->rule.L1, it->rule.L2, it->rule.L3, nPts);
     it->rule.pad = 0;
     {
         std::lock_guard<std::mutex> lock(g_integrators_mutex);

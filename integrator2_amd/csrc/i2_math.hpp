@@ -76,6 +76,15 @@ I2_HD __forceinline__ double rcp_pos(double x) {
     return fma(y, e, y);
 }
 
+// The same from one cubic step y += y (e + e^2), e = 1 - x y: 2^-24 -> 2^-72,
+// then rounding.  One instruction less than two Newton steps; used by the
+// inner integral, where it runs once per point and panel.
+I2_HD __forceinline__ double rcp_cubic(double x) {
+    const double y = rcp_estimate(x);
+    const double e = fma(-x, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+
 // a / b for |b| in [2^-1000, 2^1000]: one Newton step on 1/b (relative error
 // eps ~ 2^-48), the quotient q = a y, and one residual correction
 // q + (a - b q) y, whose relative error is eps^2 plus rounding
@@ -95,6 +104,17 @@ I2_HD __forceinline__ double sqrt_pos(double s) {
     h = fma(h, r, h);
     const double d = fma(-g, g, s);
     return fma(d, h, g);
+}
+
+// The same from one cubic step: with y ~ 1/sqrt(s), g = s y and e = 1 - g y,
+// sqrt(s) = g (1 - e)^(-1/2) = g + g e (1/2 + 3 e/8 + ...), truncated below
+// 2^-70 and within 1 ulp (g's own rounding enters by half through e).  Five
+// instructions after the estimate instead of seven; used by the inner integral.
+I2_HD __forceinline__ double sqrt_cubic(double s) {
+    const double y = rsq_estimate(s);
+    const double g = s * y;
+    const double e = fma(-g, y, 1.0);
+    return fma(g * e, fma(e, 0.375, 0.5), g);
 }
 
 // a * b + c for a Horner step whose addend c is a constant.  On the device
@@ -225,6 +245,27 @@ I2_HD __forceinline__ double atan2_any(double y, double x, const MathTable* __re
     // r >= 0 here, and atan2 takes the sign of y (for y = -0 as well): one
     // bit operation instead of compares and a branch
     return copysign(r, y);
+}
+
+// atanh(z)/z for z^2 = s in [0, 1/16] (relative error below 2^-54.9) and
+// atan(u)/u for u^2 = v in [0, 0.003] (below 2^-62): 1 + s q(s), q interpolating
+// (f - 1)/s at the Chebyshev nodes of the interval (gen_math_tables.py)
+I2_HD __forceinline__ double atanh_over(double s) {
+    double q = fma_k(s, 0.07395269887839463, 0.06506094123632396);
+    q = fma_k(q, s, 0.07700982152842295);
+    q = fma_k(q, s, 0.09090651861920544);
+    q = fma_k(q, s, 0.11111115233521718);
+    q = fma_k(q, s, 0.1428571425336631);
+    q = fma_k(q, s, 0.2000000000009649);
+    q = fma_k(q, s, 0.33333333333333287);
+    return fma(q, s, 1.0);
+}
+I2_HD __forceinline__ double atan_over(double v) {
+    double q = fma_k(v, -0.09033459667472876, 0.11110960509214748);
+    q = fma_k(q, v, -0.14285714124452448);
+    q = fma_k(q, v, 0.19999999999939544);
+    q = fma_k(q, v, -0.3333333333333333);
+    return fma(q, v, 1.0);
 }
 
 I2_HD __forceinline__ double atan2_fast(double y, double x, const MathTable* __restrict__ tab) {

@@ -290,7 +290,9 @@ int i2_host_theta_psi(int fast, const double* pts, int64_t n, const double* tri9
     const JGeom J = make_jgeom(A, B, C, unit(C - B), unit(A - C), unit(B - A));
     for (int64_t q = 0; q < n; ++q) {
         const d3 p = {pts[3 * q], pts[3 * q + 1], pts[3 * q + 2]};
-        const q4 r = fast ? theta_psi_fast(p, J, &i2m::h_mathtab) : theta_psi(p, J.a, J.b, J.c, J.ta, J.tb, J.tc);
+        const q4 r = fast == 2 ? psi_of_terms(far_scale(theta_terms_far(p, J), J), J)
+                     : fast    ? theta_psi_fast(p, J, &i2m::h_mathtab)
+                               : theta_psi(p, J.a, J.b, J.c, J.ta, J.tb, J.tc);
         out4[4 * q] = r.x; out4[4 * q + 1] = r.y; out4[4 * q + 2] = r.z; out4[4 * q + 3] = r.w;
     }
     return I2_OK;
