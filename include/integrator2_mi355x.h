@@ -250,7 +250,9 @@ int i2_host_loss_weights(uint64_t seed, const int32_t* ij, int64_t n, int nT, do
 /* Host-side reverse mode of one per-point function, for checking: kind 0
  * thetaPsi (params: A, B, C, tau_a, tau_b, tau_c; 18), 1 edge-sharing singular
  * part (JB, JC, tau_a, tau_b, tau_c, 1/|JC-JB|; 16), 2 vertex-sharing singular
- * part (JA, tau_a, tau_b, e, 1/sqrt(S_i); 13).  Returns f(p) and gbar4 . df
+ * part (JA, tau_a, tau_b, e, 1/sqrt(S_i); 13), 3 and 4 the terms of thetaPsi
+ * (line integrals of 1/r along AB, BC, CA and Theta/2) in the general and in
+ * the far form (A, B, C; 9).  Returns f(p) and gbar4 . df
  * with respect to p (pbar3) and to every parameter (parbar). */
 int i2_host_point_adjoint(int kind, const double* p3, const double* params, const double* gbar4, double* f4,
                           double* pbar3, double* parbar);

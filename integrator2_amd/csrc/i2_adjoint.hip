@@ -121,6 +121,9 @@ __device__ __forceinline__ Panel uniform_panel(const Panel& P) {
     U.v2 = __builtin_amdgcn_readfirstlane(P.v2); U.pad = 0;
     return U;
 }
+__device__ __forceinline__ JGeom uniform_jgeom(const JGeom& J) {
+    return {J.a, J.b, J.c, J.ta, J.tb, J.tc, uniform_d(J.La), uniform_d(J.Lb), uniform_d(J.Lc), uniform_d3(J.N2)};
+}
 __device__ __forceinline__ double wsum(double x) {
     for (int m = 1; m < 64; m <<= 1) x += __shfl_xor(x, m);
     return x;
@@ -170,6 +173,58 @@ __device__ __forceinline__ void child_bary(int ch, d3& ba, d3& bb, d3& bc) {
     else if (ch == 2) { ba = mCA; bb = A; bc = mAB; }
     else { ba = mBC; bb = mCA; bc = mAB; }
 }
+// The rule's points on level 0 and on the four level-1 children, barycentric
+// on the original panel, with their weights (32-byte records in LDS)
+struct alignas(32) BaryPoint { double b0, b1, b2, w; };
+__device__ __forceinline__ void load_bary(BaryPoint* P, const RuleSh& R, int npts) {
+    for (int t = threadIdx.x; t < 5 * npts; t += blockDim.x) {
+        const int sub = t / npts, k = t - sub * npts;
+        d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
+        if (sub > 0) child_bary(sub - 1, ba, bb, bc);
+        d3 b = R.L1[k] * ba;
+        b = b + R.L2[k] * bb;
+        b = b + R.L3[k] * bc;
+        P[t] = {b.x, b.y, b.z, R.w[k]};
+    }
+}
+
+// Sums of nine values over the wavefront, in a fixed order: pairs of registers
+// exchange halves and then rows, so that one register ends with four values'
+// sums, one per row of 16 lanes, and each row is summed by rotations.  57
+// instructions and no LDS instead of nine six-step butterflies through LDS.
+__device__ __forceinline__ double swap_add(double a, double b, bool half) {
+    const uint64_t x = __double_as_longlong(a), y = __double_as_longlong(b);
+    uint64_t p, q;
+    if (half) {
+        const auto l = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        p = ((uint64_t)h[0] << 32) | l[0]; q = ((uint64_t)h[1] << 32) | l[1];
+    } else {
+        const auto l = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        p = ((uint64_t)h[0] << 32) | l[0]; q = ((uint64_t)h[1] << 32) | l[1];
+    }
+    return __longlong_as_double((long long)p) + __longlong_as_double((long long)q);
+}
+template <int N> __device__ __forceinline__ double ror_add(double v) {
+    const uint64_t x = __double_as_longlong(v);
+    const unsigned l = __builtin_amdgcn_update_dpp(0, (int)(unsigned)x, 0x120 + N, 0xf, 0xf, false);
+    const unsigned h = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), 0x120 + N, 0xf, 0xf, false);
+    return v + __longlong_as_double((long long)(((uint64_t)h << 32) | l));
+}
+__device__ __forceinline__ double row_sum16(double v) { return ror_add<1>(ror_add<2>(ror_add<4>(ror_add<8>(v)))); }
+// four sums in one register: row 0 a, row 1 b, row 2 c, row 3 d
+__device__ __forceinline__ double sum_rows4(double a, double b, double c, double d) {
+    return row_sum16(swap_add(swap_add(a, c, true), swap_add(b, d, true), false));
+}
+__device__ __forceinline__ double sum_all(double v) { return row_sum16(swap_add(swap_add(v, v, true), swap_add(v, v, true), false)); }
+// the nine cotangents of K_j's vertices, summed over the wavefront into its slot
+__device__ __forceinline__ void store_sum9(double* slot, int lane, d3 a, d3 b, d3 c) {
+    const double s0 = sum_rows4(a.x, a.y, a.z, b.x), s1 = sum_rows4(b.y, b.z, c.x, c.y), s2 = sum_all(c.z);
+    const int row = lane >> 4;
+    if ((lane & 15) == 0) { slot[row] = s0; slot[4 + row] = s1; }
+    if (lane == 0) slot[8] = s2;
+}
 
 // ------------------------------------------------------------ disjoint sweep
 constexpr int ADJ_BLOCK = 256;
@@ -188,52 +243,70 @@ __device__ __forceinline__ DeepOut deep_pair(const AdjArgs& A, const RuleSh& R, 
     const Panel J = uniform_panel(M.panels[j]);
     const Weights W = weights(A.seed, i, j, M.nT);
     const q4 gb = task_cotangent(W, J.n);
-    const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
+    const JGeom JG = uniform_jgeom(make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc));
     const int npts = A.rule.n;
     double fa = I.area;
     for (int l = 0; l < level; ++l) fa *= 0.25;
-    TPBar g = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+    const d3 gP = {gb.x, gb.y, gb.z};
+    const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
+    TermsBar g = terms_bar_zero();
     DeepOut o;
-    o.X0 = {0.0, 0.0, 0.0}; o.X1 = o.X0; o.X2 = o.X0;
-    q4 F = q4zero();
+    o.X0 = {0.0, 0.0, 0.0}; o.X1 = o.X0;
     const int64_t total = (int64_t)npts << (2 * level);
     for (int64_t q = lane; q < total; q += 64) {
         const uint32_t sub = (uint32_t)(q / npts);
         const int k = (int)(q % npts);
-        d3 a = I.a, b = I.b, c = I.c;
-        sub_panel(a, b, c, level, sub);
         d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
         sub_panel(ba, bb, bc, level, sub);
-        d3 p = R.L1[k] * a;
-        p = p + R.L2[k] * b;
-        p = p + R.L3[k] * c;
-        d3 pb;
-        const q4 f = theta_psi_fast_rev(p, JG, &R.lt, (fa * R.w[k]) * gb, &pb, g);
-        F = F + R.w[k] * f;
         const d3 beta = R.L1[k] * ba + R.L2[k] * bb + R.L3[k] * bc;
-        axpy(o.X0, beta.x, pb); axpy(o.X1, beta.y, pb); axpy(o.X2, beta.z, pb);
+        d3 p = beta.x * I.a;
+        p = p + beta.y * I.b;
+        p = p + beta.z * I.c;
+        const d3 pb = theta_terms_rev<false>(p, JG, &R.lt, R.w[k], ct, g);
+        axpy(o.X0, beta.x, pb); axpy(o.X1, beta.y, pb);
     }
-    wsum3(g.a); wsum3(g.b); wsum3(g.c); wsum3(g.ta); wsum3(g.tb); wsum3(g.tc);
-    wsum3(o.X0); wsum3(o.X1); wsum3(o.X2); wsum4(F);
+    wsum3(g.a); wsum3(g.b); wsum3(g.c); wsum3(g.n); wsum3(o.X0); wsum3(o.X1); wsum4(g.T);
+    g.y = wsum(g.y); g.La = wsum(g.La); g.Lb = wsum(g.Lb); g.Lc = wsum(g.Lc);
+    const q4 F = psi_of_terms(g.T, JG);
     const q4 Iv = fa * F;
     o.Sb = dot4(gb, F) * (fa / I.area);
     const d3 psi = {Iv.x, Iv.y, Iv.z};
     const d3 nb = RECIP_4PI * (Iv.w * W.v + cross(W.v, psi));
     const d3 Jr = finalize_plain(Iv, J.n);
     o.loss = W.w * Iv.w + dot(W.v, Jr);
-    o.Ab = g.a; o.Bb = g.b; o.Cb = g.c;
-    panel_chain(J, g.ta, g.tb, g.tc, nb, 0.0, o.Ab, o.Bb, o.Cb);
+    o.X2 = g.a + g.b + g.c;
+    axpy(o.X2, g.y, JG.N2);
+    o.X2 = o.X2 - o.X0 - o.X1;
+    terms_chain(JG, ct, g, fa * gP, nb, i2m::rcp_cubic(JG.La), i2m::rcp_cubic(JG.Lb), i2m::rcp_cubic(JG.Lc),
+                i2m::rcp_cubic(2.0 * J.area), J.n, o.Ab, o.Bb, o.Cb);
     return o;
+}
+
+// Reverse mode over the points k0 <= k < k1 of one pair.
+template <bool FAR>
+__device__ __forceinline__ void points_rev(const RuleSh& R, const BaryPoint* pts, int k0, int k1, const Panel& I, const JGeom& JG,
+                                           const q4& ct, TermsBar& g, d3& X0, d3& X1) {
+    for (int k = k0; k < k1; ++k) {
+        const BaryPoint Q = pts[k];
+        d3 p = Q.b0 * I.a;
+        p = p + Q.b1 * I.b;
+        p = p + Q.b2 * I.c;
+        const d3 pb = theta_terms_rev<FAR>(p, JG, &R.lt, Q.w, ct, g);
+        axpy(X0, Q.b0, pb); axpy(X1, Q.b1, pb);
+    }
 }
 
 // One wavefront per workgroup: an item is a wavefront of 64 control panels i
 // and a tile of panels j.
 __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
     __shared__ RuleSh R;
+    __shared__ BaryPoint pts[5 * MAX_POINTS];
     __shared__ long long item_sh;
     load_rule_sh(R, A.rule);
+    __syncthreads();
     const int lane = threadIdx.x;
     const int npts = A.rule.n;
+    load_bary(pts, R, npts);
     for (;;) {
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -252,8 +325,10 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
         const int i = iw * 64 + lane;
         const bool ivalid = i < M.nT;
         const Panel I = M.panels[ivalid ? i : 0];
+        const Ball ball = panel_ball(I.a, I.b, I.c, A.rule.reach);
         const int K = M.K[I2_NOT_NEIGHBORS];
-        d3 X0 = {0.0, 0.0, 0.0}, X1 = X0, X2 = X0;   // cotangents of K_i's vertices
+        // cotangents of K_i through its points: of vertices a and b, and of the points' sum
+        d3 X0 = {0.0, 0.0, 0.0}, X1 = X0, Xs = X0;
         double Sb = 0.0, loss = 0.0;
         uint32_t deep = 0u;                           // bit j - j0: (i, j) is at reported level >= 2
         const int j0 = jt * JT, j1 = min(M.nT, j0 + JT);
@@ -271,60 +346,41 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
             Weights W = {0.0, {0.0, 0.0, 0.0}};
             if (valid) W = weights(A.seed, i, j, M.nT);
             const q4 gb = task_cotangent(W, J.n);
-            const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
-            TPBar g = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-            q4 F = q4zero();
-            const int nsub = lev == 1 ? 4 : 1;
+            const JGeom JG = uniform_jgeom(make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc));
+            const d3 gP = {gb.x, gb.y, gb.z};
             const double fa = lev == 1 ? 0.25 * I.area : I.area;
-            for (int sub = 0; sub < 4; ++sub) {
-                const bool act = valid && sub < nsub;
-                if (__ballot(act) == 0ull) break;
+            const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
+            const bool near = __ballot(valid && !panel_far(ball, JG)) != 0ull;
+            TermsBar g = terms_bar_zero();
+            for (int lv = 0; lv < 2; ++lv) {          // the pairs at reported level 0, then those at level 1
+                const bool act = valid && lev == lv;
+                if (__ballot(act) == 0ull) continue;
                 if (!act) continue;
-                d3 a = I.a, b = I.b, c = I.c;
-                d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
-                if (lev == 1) {
-                    const d3 mBC = 0.5 * (I.b + I.c), mCA = 0.5 * (I.c + I.a), mAB = 0.5 * (I.a + I.b);
-                    if (sub == 0) { a = mAB; b = I.b; c = mBC; }
-                    else if (sub == 1) { a = mBC; b = I.c; c = mCA; }
-                    else if (sub == 2) { a = mCA; b = I.a; c = mAB; }
-                    else { a = mBC; b = mCA; c = mAB; }
-                    child_bary(sub, ba, bb, bc);
-                }
-                d3 ab = {0.0, 0.0, 0.0}, bbar = ab, cb = ab;   // cotangents of the sub-panel's vertices
-                for (int k = 0; k < npts; ++k) {
-                    d3 p = R.L1[k] * a;
-                    p = p + R.L2[k] * b;
-                    p = p + R.L3[k] * c;
-                    d3 pb;
-                    const q4 f = theta_psi_fast_rev(p, JG, &R.lt, (fa * R.w[k]) * gb, &pb, g);
-                    F = F + R.w[k] * f;
-                    axpy(ab, R.L1[k], pb); axpy(bbar, R.L2[k], pb); axpy(cb, R.L3[k], pb);
-                }
-                // sub-panel vertices are fixed combinations of K_i's vertices
-                axpy(X0, ba.x, ab); axpy(X0, bb.x, bbar); axpy(X0, bc.x, cb);
-                axpy(X1, ba.y, ab); axpy(X1, bb.y, bbar); axpy(X1, bc.y, cb);
-                axpy(X2, ba.z, ab); axpy(X2, bb.z, bbar); axpy(X2, bc.z, cb);
+                const int k0 = lv == 0 ? 0 : npts, k1 = lv == 0 ? npts : 5 * npts;
+                if (near) points_rev<false>(R, pts, k0, k1, I, JG, ct, g, X0, X1);
+                else points_rev<true>(R, pts, k0, k1, I, JG, ct, g, X0, X1);
             }
             d3 nb = {0.0, 0.0, 0.0};
             if (valid) {
+                const q4 F = psi_of_terms(g.T, JG);
                 const q4 Iv = fa * F;
                 Sb += dot4(gb, F) * (fa / I.area);
                 const d3 psi = {Iv.x, Iv.y, Iv.z};
                 nb = RECIP_4PI * (Iv.w * W.v + cross(W.v, psi));
                 const d3 Jr = finalize_plain(Iv, J.n);
                 loss += W.w * Iv.w + dot(W.v, Jr);
+                Xs = Xs + g.a + g.b + g.c;
+                axpy(Xs, g.y, JG.N2);
             }
-            // K_j: summed over the wavefront into its slot
-            wsum3(g.a); wsum3(g.b); wsum3(g.c); wsum3(g.ta); wsum3(g.tb); wsum3(g.tc); wsum3(nb);
-            if (lane == 0) {
-                d3 Ab = g.a, Bb = g.b, Cb = g.c;
-                panel_chain(J, g.ta, g.tb, g.tc, nb, 0.0, Ab, Bb, Cb);
-                double* kslot = kjw + 9 * (int64_t)j;
-                store3(kslot, Ab); store3(kslot + 3, Bb); store3(kslot + 6, Cb);
-            }
+            // K_j: each lane's chain to the vertices, summed over the wavefront into its slot
+            d3 Ab, Bb, Cb;
+            terms_chain(JG, ct, g, fa * gP, nb, i2m::rcp_cubic(JG.La), i2m::rcp_cubic(JG.Lb), i2m::rcp_cubic(JG.Lc),
+                        i2m::rcp_cubic(2.0 * J.area), J.n, Ab, Bb, Cb);
+            store_sum9(kjw + 9 * (int64_t)j, lane, Ab, Bb, Cb);
         }
         A.deep_mask[item * 64 + lane] = deep;   // taken by k_adj_deep
         if (ivalid) {
+            d3 X2 = Xs - X0 - X1;
             if (Sb != 0.0 || dot(X0, X0) + dot(X1, X1) + dot(X2, X2) != 0.0) {
                 const d3 zero = {0.0, 0.0, 0.0};
                 panel_chain(I, zero, zero, zero, zero, Sb, X0, X1, X2);
@@ -1010,6 +1066,17 @@ int i2_host_point_adjoint(int kind, const double* p3, const double* params, cons
         VertexBar g = {z3, z3, z3, z3, 0.0};
         f = sing_vertex_rev(p, c, gb, &pb, g);
         put(0, g.JA); put(3, g.taua); put(6, g.taub); put(9, g.e); parbar[12] = g.invAri;
+    } else if (kind == 3 || kind == 4) {
+        const d3 A = v(0), B = v(3), C = v(6), cr = cross(B - A, C - A);
+        const JGeom J = make_jgeom(A, B, C, unit(C - B), unit(A - C), unit(B - A));
+        TermsBar g = terms_bar_zero();
+        pb = kind == 4 ? theta_terms_rev<true>(p, J, &i2m::h_mathtab, 1.0, gb, g)
+                       : theta_terms_rev<false>(p, J, &i2m::h_mathtab, 1.0, gb, g);
+        f = g.T;
+        g.T = q4zero();
+        d3 ab, bb, cb;
+        terms_chain(J, gb, g, z3, z3, 1.0 / J.La, 1.0 / J.Lb, 1.0 / J.Lc, 1.0 / vlen(cr), unit(cr), ab, bb, cb);
+        put(0, ab); put(3, bb); put(6, cb);
     } else {
         set_error("unknown point function %d", kind);
         return I2_ERR_INVALID;

@@ -127,6 +127,125 @@ I2_HD __forceinline__ q4 theta_psi_fast_rev(d3 p, const JGeom& J, const i2m::Mat
     return r;
 }
 
+// Reverse mode of the terms of the inner integral (theta_terms, or with FAR
+// theta_terms_far times its factors): with P = (S - L)(S + L) per edge,
+//   t = ln((S + L)/(S - L)):  dt = (2 S dL - 2 L dS)/P,
+//   Theta/2 = h = atan2(Y, X), X = 2 x = P_c lc + P_a la + P_b lb - 4 la lb lc
+//   and Y = 2 da.N2:  X^2 + Y^2 = P_c P_a P_b (for unit vectors |1 + a.b + b.c +
+//   c.a|^2 + (a.(b x c))^2 = 2 (1 + a.b)(1 + b.c)(1 + c.a)),
+// so one reciprocal of the three P serves every derivative.  Parameters are
+// the distances through p and the vertices, the edge lengths and N2.
+//
+// Cotangents summed over a pair's points.  a, b, c: sums of (dL/dl)/l d per
+// vertex, whose negatives belong to the vertices; y: sum of 2 dL/dY, times N2
+// another share of vertex a; n: dL/dN2; Lc, La, Lb: half of dL/dL; T: the
+// weighted terms themselves.
+struct TermsBar { d3 a, b, c, n; double y, Lc, La, Lb; q4 T; };
+I2_HD __forceinline__ TermsBar terms_bar_zero() {
+    const d3 z = {0.0, 0.0, 0.0};
+    return {z, z, z, z, 0.0, 0.0, 0.0, 0.0, q4zero()};
+}
+// One point of weight w, with the cotangents ct of the weighted terms; returns
+// the point's cotangent.
+template <bool FAR>
+I2_HD __forceinline__ d3 theta_terms_rev(d3 p, const JGeom& J, const i2m::MathTable* __restrict__ lt, double w, const q4& ct,
+                                         TermsBar& g) {
+    const d3 da = p - J.a, db = p - J.b, dc = p - J.c;
+    double ila, ilb, ilc;
+    const double la = i2m::sqrt_rsqrt(dot(da, da), &ila), lb = i2m::sqrt_rsqrt(dot(db, db), &ilb),
+                 lc = i2m::sqrt_rsqrt(dot(dc, dc), &ilc);
+    const double S1 = la + lb, S2 = lb + lc, S3 = lc + la;
+    const double c1 = w * ct.x, c2 = w * ct.y, c3 = w * ct.z, ch = w * ct.w;
+    const double Y = 2.0 * dot(da, J.N2);
+    double P1, P2, P3, X, t1, t2, t3, h, R, iP1, iP2, iP3;
+    double xa = 0.0, xb = 0.0, xc = 0.0;           // dL/dl of terms in the degenerate branch
+    double m1 = c1, m2 = c2, m3 = c3;
+    if (FAR) {
+        P1 = fma(S1, S1, -(J.Lc * J.Lc)); P2 = fma(S2, S2, -(J.La * J.La)); P3 = fma(S3, S3, -(J.Lb * J.Lb));
+        X = fma(fma(la * lb, -4.0, P1), lc, fma(P2, la, P3 * lb));
+        const double s12 = S1 * S2, s3x = S3 * X;
+        const double inv = i2m::rcp_cubic(s12 * s3x);
+        const double i12 = inv * s3x, i3x = inv * s12;
+        const double z1 = J.Lc * (i12 * S2), z2 = J.La * (i12 * S1), z3 = J.Lb * (i3x * X), u = Y * (i3x * S3);
+        t1 = 2.0 * z1 * i2m::atanh_over(z1 * z1);
+        t2 = 2.0 * z2 * i2m::atanh_over(z2 * z2);
+        t3 = 2.0 * z3 * i2m::atanh_over(z3 * z3);
+        h = u * i2m::atan_over(u * u);
+        const double P12 = P1 * P2;
+        R = i2m::rcp_cubic(P12 * P3);
+        const double R3 = R * P3;
+        iP1 = R3 * P2; iP2 = R3 * P1; iP3 = R * P12;
+    } else {
+        const double n1 = S1 + J.Lc, n2 = S2 + J.La, n3 = S3 + J.Lb;
+        double e1 = S1 - J.Lc, e2 = S2 - J.La, e3 = S3 - J.Lb;
+        double r1 = 0.0, r2 = 0.0, r3 = 0.0;        // ratios of terms in the degenerate branch
+        const double s = 0x1p-10;
+        if (__builtin_expect(fmin(fmin(fma(-s, S1, e1), fma(-s, S2, e2)), fma(-s, S3, e3)) < 0.0, 0)) {
+            if (e1 < s * S1) {
+                if (edge_gap(da, db, la, lb, J.Lc, n1, e1)) { r1 = lb / la; xb += c1 / lb; xa -= c1 / la; m1 = 0.0; }
+            }
+            if (e2 < s * S2) {
+                if (edge_gap(db, dc, lb, lc, J.La, n2, e2)) { r2 = lc / lb; xc += c2 / lc; xb -= c2 / lb; m2 = 0.0; }
+            }
+            if (e3 < s * S3) {
+                if (edge_gap(dc, da, lc, la, J.Lb, n3, e3)) { r3 = la / lc; xa += c3 / la; xc -= c3 / lc; m3 = 0.0; }
+            }
+        }
+        P1 = n1 * e1; P2 = n2 * e2; P3 = n3 * e3;
+        const double P12 = P1 * P2;
+        R = i2m::rcp_cubic(P12 * P3);
+        const double R3 = R * P3;
+        iP1 = R3 * P2; iP2 = R3 * P1; iP3 = R * P12;
+        const double a1 = r1 != 0.0 ? r1 : n1 * n1 * iP1, a2 = r2 != 0.0 ? r2 : n2 * n2 * iP2, a3 = r3 != 0.0 ? r3 : n3 * n3 * iP3;
+        X = 2.0 * (la * lb * lc + dot(da, db) * lc + dot(db, dc) * la + dot(dc, da) * lb);
+        t1 = i2m::log_tab_any(a1, lt); t2 = i2m::log_tab_any(a2, lt); t3 = i2m::log_tab_any(a3, lt);
+        h = atan2_terms(Y, X, lt);
+    }
+    g.T = {fma(w, t1, g.T.x), fma(w, t2, g.T.y), fma(w, t3, g.T.z), fma(w, h, g.T.w)};
+    // ---- reverse
+    m1 *= iP1; m2 *= iP2; m3 *= iP3;
+    const double Rh = R * ch;
+    const double xb_ = -(Y * Rh), yb = 2.0 * (X * Rh);          // dL/dX and 2 dL/dY
+    const double q1 = xb_ * lc, q2 = xb_ * la, q3 = xb_ * lb;   // dL/dP
+    const double u1 = fma(S1, q1, -(J.Lc * m1)), u2 = fma(S2, q2, -(J.La * m2)), u3 = fma(S3, q3, -(J.Lb * m3));   // dL/dS / 2
+    g.Lc = fma(S1, m1, fma(-J.Lc, q1, g.Lc));
+    g.La = fma(S2, m2, fma(-J.La, q2, g.La));
+    g.Lb = fma(S3, m3, fma(-J.Lb, q3, g.Lb));
+    const double va = fma(xb_, fma(lb * lc, -4.0, P2), xa), vb = fma(xb_, fma(lc * la, -4.0, P3), xb),
+                 vc = fma(xb_, fma(la * lb, -4.0, P1), xc);
+    const double sa = fma(2.0, u1 + u3, va) * ila, sb = fma(2.0, u1 + u2, vb) * ilb, sc = fma(2.0, u2 + u3, vc) * ilc;
+    axpy(g.a, sa, da); axpy(g.b, sb, db); axpy(g.c, sc, dc);
+    axpy(g.n, yb, da);
+    g.y += yb;
+    d3 pb = yb * J.N2;
+    axpy(pb, sa, da); axpy(pb, sb, db); axpy(pb, sc, dc);
+    return pb;
+}
+// Cotangents of K_j's vertices from a pair's sums: ct as in theta_terms_rev,
+// nb the cotangent of the unit normal and gP that of the quadrature sum of
+// Psi = T.x tau_c + T.y tau_a + T.z tau_b (ct.x = gP.tau_c, ...).
+I2_HD __forceinline__ void terms_chain(const JGeom& J, const q4& ct, const TermsBar& g, d3 gP, d3 nb, double iLa, double iLb,
+                                       double iLc, double iN, d3 n, d3& Ab, d3& Bb, d3& Cb) {
+    Ab = -g.a; Bb = -g.b; Cb = -g.c;
+    axpy(Ab, -g.y, J.N2);
+    // an edge e = L tau: dL/de = (T gP - (T gP.tau) tau)/L + dL/dL tau
+    auto edge = [&](double T, double c, double Lh, double iL, d3 tau) {
+        const double k = T * iL;
+        d3 e = k * gP;
+        axpy(e, fma(2.0, Lh, -(k * c)), tau);
+        return e;
+    };
+    const d3 ec = edge(g.T.x, ct.x, g.Lc, iLc, J.tc), ea = edge(g.T.y, ct.y, g.La, iLa, J.ta),
+             eb = edge(g.T.z, ct.z, g.Lb, iLb, J.tb);
+    Bb = Bb + ec - ea; Ab = Ab - ec + eb; Cb = Cb + ea - eb;
+    // N2 = (B - A) x (C - A), n = N2/|N2|
+    d3 N = iN * nb;
+    axpy(N, -dot(N, n), n);
+    N = N + g.n;
+    const d3 gu = cross(J.c - J.a, N), gv = cross(N, J.b - J.a);
+    Bb = Bb + gu; Cb = Cb + gv; Ab = Ab - gu - gv;
+}
+
 // d(u / |u|) backwards: cotangent of u from that of the unit vector
 I2_HD __forceinline__ d3 unit_rev(d3 u, d3 ub) {
     const double l = sqrt(dot(u, u));

@@ -182,16 +182,26 @@ I2_HD __forceinline__ JGeom make_jgeom(d3 a, d3 b, d3 c, d3 ta, d3 tb, d3 tc) {
     return {a, b, c, ta, tb, tc, vlen(c - b) + 0.0 * ta.x, vlen(a - c) + 0.0 * tb.x, vlen(b - a) + 0.0 * tc.x,
             cross(b - a, c - a)};
 }
-// S - L without cancellation, 2 |u x v|^2 / ((lu lv - u.v)(S + L)), from
-// (S - L)(S + L) = 2 (lu lv + u.v) and (lu lv + u.v)(lu lv - u.v) = |u x v|^2;
-// n/e is the ratio (S + L)/(S - L)
-I2_HD __forceinline__ void edge_ratio(d3 u, d3 v, double lu, double lv, double L, double& n, double& e) {
+// e = S - L without cancellation, 2 |u x v|^2 / ((lu lv - u.v) n) with n = S +
+// L, from (S - L)(S + L) = 2 (lu lv + u.v) and (lu lv + u.v)(lu lv - u.v) =
+// |u x v|^2.  True in the reference's degenerate branch, a point on the edge's
+// line, which takes lv/lu in place of n/e (evaluatorJ3DK.cu:294-307).
+I2_HD __forceinline__ bool edge_gap(d3 u, d3 v, double lu, double lv, double L, double n, double& e) {
     const d3 c = cross(u, v);
     const double c2 = dot(c, c);
     e = 2.0 * c2 / (fma(lu, lv, -dot(u, v)) * n);
-    // the reference's degenerate branch: a point on the edge's line keeps the
-    // ratio of distances (evaluatorJ3DK.cu:294-307)
-    if (c2 < EPS_PSI_THETA2 * (L * L) * (lv * lv)) { n = lv; e = lu; }
+    return c2 < EPS_PSI_THETA2 * (L * L) * (lv * lv);
+}
+// Theta/2 = atan2(y, x) for any arguments: the table path, then the lanes
+// outside its range (zero, NaN, lengths near the ends of the exponent range)
+I2_HD __forceinline__ double atan2_terms(double y, double x, const i2m::MathTable* __restrict__ lt) {
+    double h = i2m::atan2_any(y, x, lt);
+    if (__builtin_expect(!i2m::atan2_in_range(y, x), 0)) {
+        const double sum = fabs(x) + fabs(y), k = sum < 1.0 ? 0x1p600 : 0x1p-600;
+        h = sum == 0.0 ? 0.0 : i2m::atan2_any(y * k, x * k, lt);
+        if (!(sum <= 1.7976931348623157e308)) h = sum - sum;
+    }
+    return h;
 }
 // Terms of one point: line integrals t along A->B, B->C, C->A (the edges of
 // tau_c, tau_a, tau_b) and Theta/2.  For any point; `lt` holds the reduction
@@ -205,9 +215,9 @@ I2_HD __forceinline__ q4 theta_terms(d3 p, const JGeom& J, const i2m::MathTable*
     double e1 = S1 - J.Lc, e2 = S2 - J.La, e3 = S3 - J.Lb;
     const double s = 0x1p-10;
     if (__builtin_expect(fmin(fmin(fma(-s, S1, e1), fma(-s, S2, e2)), fma(-s, S3, e3)) < 0.0, 0)) {
-        if (e1 < s * S1) edge_ratio(da, db, la, lb, J.Lc, n1, e1);
-        if (e2 < s * S2) edge_ratio(db, dc, lb, lc, J.La, n2, e2);
-        if (e3 < s * S3) edge_ratio(dc, da, lc, la, J.Lb, n3, e3);
+        if (e1 < s * S1 && edge_gap(da, db, la, lb, J.Lc, n1, e1)) { n1 = lb; e1 = la; }
+        if (e2 < s * S2 && edge_gap(db, dc, lb, lc, J.La, n2, e2)) { n2 = lc; e2 = lb; }
+        if (e3 < s * S3 && edge_gap(dc, da, lc, la, J.Lb, n3, e3)) { n3 = la; e3 = lc; }
     }
     const double e12 = e1 * e2;
     const double inv = i2m::rcp_cubic(e12 * e3);
@@ -221,13 +231,7 @@ I2_HD __forceinline__ q4 theta_terms(d3 p, const JGeom& J, const i2m::MathTable*
     const double t1 = i2m::log_tab_any(n1 * (i12 * e2), lt);
     const double t2 = i2m::log_tab_any(n2 * (i12 * e1), lt);
     const double t3 = i2m::log_tab_any(n3 * (inv * e12), lt);
-    double h = i2m::atan2_any(y, x, lt);
-    if (__builtin_expect(!i2m::atan2_in_range(y, x), 0)) {
-        // zero, NaN, or lengths near the ends of the exponent range
-        const double sum = fabs(x) + fabs(y), k = sum < 1.0 ? 0x1p600 : 0x1p-600;
-        h = sum == 0.0 ? 0.0 : i2m::atan2_any(y * k, x * k, lt);
-        if (!(sum <= 1.7976931348623157e308)) h = sum - sum;
-    }
+    const double h = atan2_terms(y, x, lt);
     return {t1, t2, t3, h};
 }
 // The same for a point and a panel K_j whose every point is at least twice

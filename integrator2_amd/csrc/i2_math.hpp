@@ -117,6 +117,16 @@ I2_HD __forceinline__ double sqrt_cubic(double s) {
     return fma(g * e, fma(e, 0.375, 0.5), g);
 }
 
+// sqrt(s) as sqrt_cubic and 1/sqrt(s) from the same estimate (y + y e (1/2 + 3 e/8))
+I2_HD __forceinline__ double sqrt_rsqrt(double s, double* inv) {
+    const double y = rsq_estimate(s);
+    const double g = s * y;
+    const double e = fma(-g, y, 1.0);
+    const double c = fma(e, 0.375, 0.5);
+    *inv = fma(y * e, c, y);
+    return fma(g * e, c, g);
+}
+
 // a * b + c for a Horner step whose addend c is a constant.  On the device
 // this is one three-operand v_fma_f64: left to itself the compiler keeps such
 // constants in VGPRs and emits a copy into the accumulator before each
