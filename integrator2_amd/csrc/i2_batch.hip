@@ -231,7 +231,14 @@ struct StepOut {
 __device__ __forceinline__ void push_deep(const BatchArgs& A, int level, int type, int m, int i, int j, int64_t z, q4 prev) {
     const int qi = level * 3 + type;
     const unsigned long long slot = atomicAdd(&A.counters[1 + qi], 1ull);
-    if (slot >= (unsigned long long)A.qcap[type]) return;   // counted: the host grows the queue and runs again
+    if (slot >= (unsigned long long)A.qcap[type]) {
+        // counted: the host grows the queue and runs again.  No kernel finishes
+        // the task in this run, but the adjoint of the same graph reads its
+        // convergence iteration as a refinement level: it gets a valid one.
+        int8_t* conv = A.meshes[m].conv[type];
+        if (conv) conv[z] = 0;
+        return;
+    }
     QEntry e;
     e.m = m; e.i = i; e.j = j; e.pad = 0; e.z = z; e.pad2 = 0;
     e.prev = make_double4(prev.x, prev.y, prev.z, prev.w);
@@ -823,9 +830,16 @@ int engine_setup(Engine& E, const i2_integrator& it) {
     E.h_row_base.assign(M + 1, 0);
     for (int m = 0; m < M; ++m) E.h_row_base[m + 1] = E.h_row_base[m] + E.h_meshes[m].nT;
     A.total_rows = E.h_row_base[M];
-    // queue segments: levels 2..last, capacity per type (grown after an overflow)
+    // queue segments: levels 2..last, capacity per type (grown after an
+    // overflow, which costs a second run).  Most vertex- and edge-sharing tasks
+    // are refined at tight tolerances and there are few of them: room for all
+    // up to 4 M (256 MB per level), where an eighth overflowed on the first run
+    // of every mesh above some 7,000 panels.
     for (int t = 0; t < 3; ++t)
-        if (A.qcap[t] <= 0) A.qcap[t] = std::max<int64_t>(1, std::min<int64_t>(E.ordered[t], std::max<int64_t>(65536, E.ordered[t] / 8)));
+        if (A.qcap[t] <= 0) {
+            const int64_t least = t == I2_NOT_NEIGHBORS ? 65536 : (int64_t)4 << 20;
+            A.qcap[t] = std::max<int64_t>(1, std::min<int64_t>(E.ordered[t], std::max<int64_t>(least, E.ordered[t] / 8)));
+        }
     E.h_qoff.assign(MAX_LEVELS * 3, 0);
     int64_t qtot = 0;
     for (int L = 2; L <= A.last_level; ++L)
