@@ -241,7 +241,8 @@ int i2_evaluator_set_tuning(i2_evaluator* ev, int pairsPerWorkgroup, int pointsP
  * Refinement levels, the vertex-sharing 2*pi*p wrap and all branches are
  * frozen at the forward pass's choices.  Both integration paths.  The sums
  * have a fixed order: two calls on the same mesh give the same bits.  Device
- * memory: about nT*(nT/32 + nT/64)*72 bytes of partial-cotangent slots. */
+ * memory: about nT*(nT/jt + nT/64)*72 bytes of partial-cotangent slots, with
+ * jt = 32 above 16,384 panels, 16 above some 2,900 and less below. */
 int i2_evaluator_loss_and_grad(i2_evaluator* ev, uint64_t seed, double* loss, double* dLdX);
 /* Device milliseconds of the last adjoint run. */
 int i2_evaluator_adjoint_ms(const i2_evaluator* ev, double* ms);

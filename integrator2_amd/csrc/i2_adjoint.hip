@@ -18,10 +18,9 @@
 //                   stay in registers for the whole tile and those of K_j are
 //                   summed over the wavefront into the slot of (wavefront, j).
 //                   Pairs at reported level >= 2 are marked per lane.
-//   k_adj_deep      the marked pairs, item by item: four wavefronts share an
-//                   item's pairs in a fixed order, one pair at a time each over
-//                   its 13 * 4^L points, and add to the item's own slots in a
-//                   fixed order.
+//   k_adj_deep      the marked pairs, item by item: 16 pairs at a time, 16
+//                   lanes each over their 13 * 4^L points, added to the item's
+//                   own slots in a fixed order.
 //   k_adj_singular  vertex- and edge-sharing pairs: one wavefront per pair;
 //                   reverse mode over the points; the cotangents of the
 //                   per-pair quantities go to a record per pair.
@@ -208,8 +207,8 @@ __device__ __forceinline__ double swap_add(double a, double b, bool half) {
 }
 template <int N> __device__ __forceinline__ double ror_add(double v) {
     const uint64_t x = __double_as_longlong(v);
-    const unsigned l = __builtin_amdgcn_update_dpp(0, (int)(unsigned)x, 0x120 + N, 0xf, 0xf, false);
-    const unsigned h = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), 0x120 + N, 0xf, 0xf, false);
+    const unsigned l = __builtin_amdgcn_mov_dpp((int)(unsigned)x, 0x120 + N, 0xf, 0xf, false);
+    const unsigned h = __builtin_amdgcn_mov_dpp((int)(unsigned)(x >> 32), 0x120 + N, 0xf, 0xf, false);
     return v + __longlong_as_double((long long)(((uint64_t)h << 32) | l));
 }
 __device__ __forceinline__ double row_sum16(double v) { return ror_add<1>(ror_add<2>(ror_add<4>(ror_add<8>(v)))); }
@@ -228,59 +227,8 @@ __device__ __forceinline__ void store_sum9(double* slot, int lane, d3 a, d3 b, d
 
 // ------------------------------------------------------------ disjoint sweep
 constexpr int ADJ_BLOCK = 256;
-
-// One disjoint pair at reported level >= 2, taken by the whole wavefront over
-// its npts * 4^level points.  The results are uniform over the wavefront.
-struct DeepOut {
-    d3 X0, X1, X2;    // cotangents of K_i's vertices through the points (before K_i's panel chain)
-    double Sb;        // cotangent of K_i's area
-    d3 Ab, Bb, Cb;    // cotangents of K_j's vertices (after K_j's panel chain)
-    double loss;      // the pair's term of L
-};
-__device__ __forceinline__ DeepOut deep_pair(const AdjArgs& A, const RuleSh& R, const AdjMesh& M, int i, int j, int level,
-                                             int lane) {
-    const Panel I = uniform_panel(M.panels[i]);
-    const Panel J = uniform_panel(M.panels[j]);
-    const Weights W = weights(A.seed, i, j, M.nT);
-    const q4 gb = task_cotangent(W, J.n);
-    const JGeom JG = uniform_jgeom(make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc));
-    const int npts = A.rule.n;
-    double fa = I.area;
-    for (int l = 0; l < level; ++l) fa *= 0.25;
-    const d3 gP = {gb.x, gb.y, gb.z};
-    const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
-    TermsBar g = terms_bar_zero();
-    DeepOut o;
-    o.X0 = {0.0, 0.0, 0.0}; o.X1 = o.X0;
-    const int64_t total = (int64_t)npts << (2 * level);
-    for (int64_t q = lane; q < total; q += 64) {
-        const uint32_t sub = (uint32_t)(q / npts);
-        const int k = (int)(q % npts);
-        d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
-        sub_panel(ba, bb, bc, level, sub);
-        const d3 beta = R.L1[k] * ba + R.L2[k] * bb + R.L3[k] * bc;
-        d3 p = beta.x * I.a;
-        p = p + beta.y * I.b;
-        p = p + beta.z * I.c;
-        const d3 pb = theta_terms_rev<false>(p, JG, &R.lt, R.w[k], ct, g);
-        axpy(o.X0, beta.x, pb); axpy(o.X1, beta.y, pb);
-    }
-    wsum3(g.a); wsum3(g.b); wsum3(g.c); wsum3(g.n); wsum3(o.X0); wsum3(o.X1); wsum4(g.T);
-    g.y = wsum(g.y); g.La = wsum(g.La); g.Lb = wsum(g.Lb); g.Lc = wsum(g.Lc);
-    const q4 F = psi_of_terms(g.T, JG);
-    const q4 Iv = fa * F;
-    o.Sb = dot4(gb, F) * (fa / I.area);
-    const d3 psi = {Iv.x, Iv.y, Iv.z};
-    const d3 nb = RECIP_4PI * (Iv.w * W.v + cross(W.v, psi));
-    const d3 Jr = finalize_plain(Iv, J.n);
-    o.loss = W.w * Iv.w + dot(W.v, Jr);
-    o.X2 = g.a + g.b + g.c;
-    axpy(o.X2, g.y, JG.N2);
-    o.X2 = o.X2 - o.X0 - o.X1;
-    terms_chain(JG, ct, g, fa * gP, nb, i2m::rcp_cubic(JG.La), i2m::rcp_cubic(JG.Lb), i2m::rcp_cubic(JG.Lc),
-                i2m::rcp_cubic(2.0 * J.area), J.n, o.Ab, o.Bb, o.Cb);
-    return o;
-}
+// panels j per disjoint item at most (one bit of a lane's mask each)
+constexpr int ADJ_TILE = 32;
 
 // Reverse mode over the points k0 <= k < k1 of one pair.
 template <bool FAR>
@@ -319,7 +267,7 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
         const int m = __builtin_amdgcn_readfirstlane(find_base_a(A.item_base, A.nmeshes, item));
         const AdjMesh& M = A.meshes[m];
         const int64_t rr = item - A.item_base[m];
-        const int JT = A.j_tile;
+        const int JT = M.jt;
         const int jtiles = M.jtiles;
         const int iw = (int)(rr / jtiles), jt = (int)(rr % jtiles);
         const int i = iw * 64 + lane;
@@ -378,7 +326,10 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
                         i2m::rcp_cubic(2.0 * J.area), J.n, Ab, Bb, Cb);
             store_sum9(kjw + 9 * (int64_t)j, lane, Ab, Bb, Cb);
         }
-        A.deep_mask[item * 64 + lane] = deep;   // taken by k_adj_deep
+        if (__ballot(deep != 0u) != 0ull) {         // the item is taken by k_adj_deep
+            A.deep_mask[item * 64 + lane] = deep;
+            if (lane == 0) A.deep_items[atomicAdd(&A.counters[1], 1ull)] = item;
+        }
         if (ivalid) {
             d3 X2 = Xs - X0 - X1;
             if (Sb != 0.0 || dot(X0, X0) + dot(X1, X1) + dot(X2, X2) != 0.0) {
@@ -393,66 +344,150 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
     }
 }
 
-// The disjoint pairs at reported level >= 2 that k_adj_disjoint marked, item
-// by item (one workgroup of four wavefronts per item).  The item's pairs are
-// numbered in a fixed order (lanes in order, each lane's j in order) and
-// wavefront w takes pairs w, w + 4, ..., the whole wavefront on one pair at a
-// time over its 13 * 4^L points, into partial sums of its own in LDS.  The
-// first wavefront then adds the four partials in order to the item's slots:
-// each lane's K_i slot, the K_j slot of each j of the tile, the item's loss.
-// Every slot belongs to one item, so each has one writer and a fixed order of
-// additions.
-constexpr int DEEP_NK = 11;   // per lane: X0, X1, X2 (9), Sb, loss
+// The disjoint pairs at reported level >= 2, item by item: the items that hold
+// any, as k_adj_disjoint listed them, claimed by workgroups of 256.  An item's
+// pairs are numbered in a fixed order (lanes in order, each lane's j in order)
+// and taken 16 at a time, 16 lanes per pair: at level 2 each lane has one of
+// the 16 sub-panels (13 points), at level L >= 3 every 16th of 4^L.  The
+// batch's results go to LDS and are added in the pairs' order to the item's
+// sums, which the item's slots receive at the end; every slot belongs to one
+// item, so the order in which items are claimed does not matter.
+//
+// 16 lanes instead of a wavefront per pair: 208 points fill 13 rounds of 16
+// lanes but 3.25 of 64, and what is done once per pair (weights, sums over
+// the lanes, the chain to the vertices) serves four pairs per instruction.
+constexpr int DEEP_NK = 11;             // per pair: X0, X1, X2 (9), Sb, loss
+constexpr int DEEP_REC = DEEP_NK + 9;   // and the cotangents of K_j's vertices
+__device__ __forceinline__ double quad_lane(double v, int q) {
+    const uint64_t x = __double_as_longlong(v);
+    const int lo = (int)(unsigned)x, hi = (int)(unsigned)(x >> 32);
+    unsigned l, h;
+    if (q == 0) { l = __builtin_amdgcn_mov_dpp(lo, 0x00, 0xf, 0xf, false); h = __builtin_amdgcn_mov_dpp(hi, 0x00, 0xf, 0xf, false); }
+    else if (q == 1) { l = __builtin_amdgcn_mov_dpp(lo, 0x55, 0xf, 0xf, false); h = __builtin_amdgcn_mov_dpp(hi, 0x55, 0xf, 0xf, false); }
+    else if (q == 2) { l = __builtin_amdgcn_mov_dpp(lo, 0xaa, 0xf, 0xf, false); h = __builtin_amdgcn_mov_dpp(hi, 0xaa, 0xf, 0xf, false); }
+    else { l = __builtin_amdgcn_mov_dpp(lo, 0xff, 0xf, 0xf, false); h = __builtin_amdgcn_mov_dpp(hi, 0xff, 0xf, 0xf, false); }
+    return __longlong_as_double((long long)(((uint64_t)h << 32) | l));
+}
+__device__ __forceinline__ void row_sum3(d3& v) { v.x = row_sum16(v.x); v.y = row_sum16(v.y); v.z = row_sum16(v.z); }
+// One pair by 16 lanes (lane s of its row); every lane of the row gets the results.
+__device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, const AdjMesh& M, int i, int j, int level, int s,
+                                          double* rec) {
+    const Panel I = M.panels[i];
+    const Panel J = M.panels[j];
+    // one of the pair's four draws per lane of a quad
+    const double draw = normal_draw(A.seed, (uint64_t)i * (uint64_t)M.nT + (uint64_t)j, (uint64_t)(s & 3));
+    const Weights W = {quad_lane(draw, 0), {quad_lane(draw, 1), quad_lane(draw, 2), quad_lane(draw, 3)}};
+    const q4 gb = task_cotangent(W, J.n);
+    const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
+    const int npts = A.rule.n;
+    double fa = I.area;
+    for (int l = 0; l < level; ++l) fa *= 0.25;
+    const d3 gP = {gb.x, gb.y, gb.z};
+    const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
+    TermsBar g = terms_bar_zero();
+    d3 X0 = {0.0, 0.0, 0.0}, X1 = X0;
+    const uint32_t nsub = 1u << (2 * level);
+    for (uint32_t sub = s; sub < nsub; sub += 16) {
+        d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
+        sub_panel(ba, bb, bc, level, sub);
+        for (int k = 0; k < npts; ++k) {
+            const d3 beta = R.L1[k] * ba + R.L2[k] * bb + R.L3[k] * bc;
+            d3 p = beta.x * I.a;
+            p = p + beta.y * I.b;
+            p = p + beta.z * I.c;
+            const d3 pb = theta_terms_rev<false>(p, JG, &R.lt, R.w[k], ct, g);
+            axpy(X0, beta.x, pb); axpy(X1, beta.y, pb);
+        }
+    }
+    row_sum3(g.a); row_sum3(g.b); row_sum3(g.c); row_sum3(g.n); row_sum3(X0); row_sum3(X1);
+    g.T = {row_sum16(g.T.x), row_sum16(g.T.y), row_sum16(g.T.z), row_sum16(g.T.w)};
+    g.y = row_sum16(g.y); g.La = row_sum16(g.La); g.Lb = row_sum16(g.Lb); g.Lc = row_sum16(g.Lc);
+    const q4 F = psi_of_terms(g.T, JG);
+    const q4 Iv = fa * F;
+    const d3 psi = {Iv.x, Iv.y, Iv.z};
+    const d3 nb = RECIP_4PI * (Iv.w * W.v + cross(W.v, psi));
+    const d3 Jr = finalize_plain(Iv, J.n);
+    d3 X2 = g.a + g.b + g.c;
+    axpy(X2, g.y, JG.N2);
+    X2 = X2 - X0 - X1;
+    d3 Ab, Bb, Cb;
+    terms_chain(JG, ct, g, fa * gP, nb, i2m::rcp_cubic(JG.La), i2m::rcp_cubic(JG.Lb), i2m::rcp_cubic(JG.Lc),
+                i2m::rcp_cubic(2.0 * J.area), J.n, Ab, Bb, Cb);
+    if (s == 0) {
+        store3(rec, X0); store3(rec + 3, X1); store3(rec + 6, X2);
+        rec[9] = dot4(gb, F) * (fa / I.area);
+        rec[10] = W.w * Iv.w + dot(W.v, Jr);
+        store3(rec + 11, Ab); store3(rec + 14, Bb); store3(rec + 17, Cb);
+    }
+}
+
 __global__ __launch_bounds__(256) I2_TWO_WAVES void k_adj_deep(AdjArgs A) {
     __shared__ RuleSh R;
-    __shared__ double kip[4][64][DEEP_NK];   // per wavefront and lane i
-    __shared__ double kjp[4][32][9];         // per wavefront and j of the tile
+    __shared__ double kip[64][DEEP_NK];      // the item's sums per lane i
+    __shared__ double kjp[ADJ_TILE][9];      // and per j of the tile
+    __shared__ double rec[16][DEEP_REC];     // the batch's pairs
+    __shared__ uint16_t list[64 * ADJ_TILE]; // the item's pairs, lane * ADJ_TILE + bit
+    __shared__ int npairs;
+    __shared__ long long item_sh;
+    const unsigned long long nitems = A.counters[1];
+    if ((unsigned long long)blockIdx.x >= nitems) return;
     load_rule_sh(R, A.rule);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int64_t item = blockIdx.x; item < A.disjoint_items; item += gridDim.x) {
-        // the same 64 masks in every wavefront: the test is uniform over the workgroup
-        const uint32_t mask = A.deep_mask[item * 64 + lane];
-        if (__ballot(mask != 0u) == 0ull) continue;
+    const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 4;
+    for (;;) {
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned long long pos = atomicAdd(&A.counters[2], 1ull);
+            item_sh = pos < nitems ? A.deep_items[pos] : -1ll;
+        }
+        __syncthreads();
+        const int64_t item = uniform64a(item_sh);
+        if (item < 0) break;
         const int m = __builtin_amdgcn_readfirstlane(find_base_a(A.item_base, A.nmeshes, item));
         const AdjMesh& M = A.meshes[m];
         const int64_t rr = item - A.item_base[m];
         const int iw = (int)(rr / M.jtiles), jt = (int)(rr % M.jtiles);
-        const int i = iw * 64 + lane;
-        const int j0 = jt * A.j_tile;
+        const int j0 = jt * M.jt;
         const int K = M.K[I2_NOT_NEIGHBORS];
-        for (int q = lane; q < 64 * DEEP_NK; q += 64) (&kip[wave][0][0])[q] = 0.0;
-        for (int q = lane; q < 32 * 9; q += 64) (&kjp[wave][0][0])[q] = 0.0;
-        uint32_t deep = mask;
-        for (int k = 0;; ++k) {
-            const uint64_t pend = __ballot(deep != 0u);
-            if (pend == 0ull) break;
-            const int L = (int)__builtin_ctzll(pend);
-            const uint32_t dL = (uint32_t)__builtin_amdgcn_readlane((int)deep, L);
-            const int b = (int)__builtin_ctz(dL);
-            const int id = __builtin_amdgcn_readlane(i, L);
-            if (lane == L) deep &= deep - 1u;
-            if ((k & 3) != wave) continue;
-            const int jd = j0 + b;
-            const int levd = reported_level(A, M.conv[I2_NOT_NEIGHBORS][task_disjoint(M, id, jd)], K);
-            const DeepOut o = deep_pair(A, R, M, id, jd, levd, lane);
-            if (lane == 0) {
-                double* kp = kip[wave][L];
-                kp[0] += o.X0.x; kp[1] += o.X0.y; kp[2] += o.X0.z;
-                kp[3] += o.X1.x; kp[4] += o.X1.y; kp[5] += o.X1.z;
-                kp[6] += o.X2.x; kp[7] += o.X2.y; kp[8] += o.X2.z;
-                kp[9] += o.Sb; kp[10] += o.loss;
-                double* jp = kjp[wave][b];
-                jp[0] += o.Ab.x; jp[1] += o.Ab.y; jp[2] += o.Ab.z;
-                jp[3] += o.Bb.x; jp[4] += o.Bb.y; jp[5] += o.Bb.z;
-                jp[6] += o.Cb.x; jp[7] += o.Cb.y; jp[8] += o.Cb.z;
+        const uint32_t mask = A.deep_mask[item * 64 + lane];   // the same in every wavefront
+        if (tid < 64) {
+            int at = 0;                     // pairs of the lanes before this one
+            const int cnt = __popc(mask);
+            int run = cnt;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int v = __shfl_up(run, d);
+                if (lane >= d) run += v;
             }
+            at = run - cnt;
+            for (uint32_t r = mask; r != 0u; r &= r - 1u) list[at++] = (uint16_t)(lane * ADJ_TILE + __builtin_ctz(r));
+            if (lane == 63) npairs = run;
         }
+        for (int q = tid; q < 64 * DEEP_NK; q += 256) (&kip[0][0])[q] = 0.0;
+        for (int q = tid; q < ADJ_TILE * 9; q += 256) (&kjp[0][0])[q] = 0.0;
         __syncthreads();
-        if (wave == 0) {
-            double v[DEEP_NK];
-            for (int c = 0; c < DEEP_NK; ++c) v[c] = ((kip[0][lane][c] + kip[1][lane][c]) + kip[2][lane][c]) + kip[3][lane][c];
+        const int n = npairs;
+        for (int base = 0; base < n; base += 16) {
+            if (base + grp < n) {
+                const int e = list[base + grp];
+                const int i = iw * 64 + e / ADJ_TILE, j = j0 + e % ADJ_TILE;
+                const int level = reported_level(A, M.conv[I2_NOT_NEIGHBORS][task_disjoint(M, i, j)], K);
+                deep_pair(A, R, M, i, j, level, tid & 15, rec[grp]);
+            }
+            __syncthreads();
+            const int nb = min(16, n - base);
+            for (int q = 0; q < nb; ++q) {   // in the pairs' order
+                const int e = list[base + q];
+                if (tid < 64) {
+                    if (e / ADJ_TILE == tid) for (int c = 0; c < DEEP_NK; ++c) kip[tid][c] += rec[q][c];
+                } else if (tid < 64 + ADJ_TILE) {
+                    if (e % ADJ_TILE == tid - 64) for (int c = 0; c < 9; ++c) kjp[tid - 64][c] += rec[q][DEEP_NK + c];
+                }
+            }
+            __syncthreads();
+        }
+        if (tid < 64) {
             if (mask != 0u) {
+                const int i = iw * 64 + lane;
+                const double* v = kip[lane];
                 d3 X0 = {v[0], v[1], v[2]}, X1 = {v[3], v[4], v[5]}, X2 = {v[6], v[7], v[8]};
                 const Panel I = M.panels[i];
                 const d3 zero = {0.0, 0.0, 0.0};
@@ -460,19 +495,17 @@ __global__ __launch_bounds__(256) I2_TWO_WAVES void k_adj_deep(AdjArgs A) {
                 double* kslot = M.ki + ((int64_t)jt * M.nT + i) * 9;
                 add_to3(kslot, X0); add_to3(kslot + 3, X1); add_to3(kslot + 6, X2);
             }
+            const double loss = wsum(kip[lane][10]);
+            if (lane == 0) A.item_loss[item] += loss;
+        } else if (tid < 128) {
             // the j of the tile that hold a pair of the item (OR of the lanes' masks)
             uint32_t anyj = mask;
             for (int d = 1; d < 64; d <<= 1) anyj |= (uint32_t)__shfl_xor((int)anyj, d);
-            if (lane < 32 && ((anyj >> lane) & 1u)) {
-                double w[9];
-                for (int c = 0; c < 9; ++c) w[c] = ((kjp[0][lane][c] + kjp[1][lane][c]) + kjp[2][lane][c]) + kjp[3][lane][c];
+            if (lane < ADJ_TILE && ((anyj >> lane) & 1u)) {
                 double* kslot = M.kj + ((int64_t)iw * M.nT + j0 + lane) * 9;
-                for (int c = 0; c < 9; ++c) kslot[c] += w[c];
+                for (int c = 0; c < 9; ++c) kslot[c] += kjp[lane][c];
             }
-            const double loss = wsum(v[10]);
-            if (lane == 0) A.item_loss[item] += loss;
         }
-        __syncthreads();
     }
 }
 
@@ -789,6 +822,21 @@ int adjoint_launch(AdjState& S, hipStream_t st) {
     return I2_OK;
 }
 
+// Panels j per disjoint item of a mesh.  2,048 wavefronts are in flight (two per
+// SIMD), so a mesh wants some four rounds of items; smaller tiles cost a K_i
+// slot and the chain of K_i each.  Measured, forward and gradient: 320 panels
+// 4.1 ms with tiles of 32 (50 items), 1.76 ms with 1; 1,280 panels 6.1 ms with
+// 32, 4.0 with 4, 3.8 with 2, 4.05 with 1; 5,120 panels 26.4-27.1 ms with 32 (6.25
+// rounds), 25.0 with 16.  Above 16,384 panels the slots (nT^2/jt * 72 bytes) keep
+// the tile at 32.  From the mesh's size alone, so that a mesh has the same sums
+// in any batch.
+static int adjoint_tile(int nT) {
+    const int64_t niw = (nT + 63) / 64;
+    int jt = nT > 16384 ? ADJ_TILE : ADJ_TILE / 2;
+    while (jt > 1 && niw * ((nT + jt - 1) / jt) < 8192) jt /= 2;
+    return jt;
+}
+
 // Builds the adjoint's descriptors for meshes D (panels, lists, convergence
 // iterations and device K already set): the partial-cotangent slots, dX and
 // loss (one block of 3 nV + 1 doubles per mesh), and the vertex gather's
@@ -801,7 +849,6 @@ int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::ve
     const int M = (int)D.size();
     if ((int)meshes.size() != M) { set_error("adjoint setup: %d descriptors for %d meshes", M, (int)meshes.size()); return I2_ERR_INVALID; }
     AdjArgs& A = S.args;
-    A.j_tile = 32;   // at most 32: k_adj_disjoint marks a lane's deep pairs in a 32-bit word
     S.nV.assign(M, 0);
     for (int m = 0; m < M; ++m) S.nV[m] = meshes[m]->nV;
     S.grad_off.assign(M + 1, 0);
@@ -811,7 +858,9 @@ int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::ve
         pbase(M + 1, 0);
     for (int m = 0; m < M; ++m) {
         const int64_t niw = (D[m].nT + 63) / 64;
-        const int64_t jtiles = (D[m].nT + A.j_tile - 1) / A.j_tile;
+        const int jt = adjoint_tile(D[m].nT);
+        const int64_t jtiles = (D[m].nT + jt - 1) / jt;
+        D[m].jt = jt;
         D[m].jtiles = (int)jtiles;
         D[m].niw = (int)niw;
         item_base[m + 1] = item_base[m] + niw * jtiles;
@@ -938,6 +987,8 @@ int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::ve
     A.loss_part = S.d_loss_part.p;
     I2_TRY(S.d_deep_mask.ensure(64 * A.disjoint_items));
     A.deep_mask = S.d_deep_mask.p;
+    I2_TRY(S.d_deep_items.ensure(A.disjoint_items));
+    A.deep_items = S.d_deep_items.p;
     I2_TRY(S.d_counters.ensure(4));
     A.counters = S.d_counters.p;
     return I2_OK;

@@ -21,7 +21,7 @@ struct AdjMesh {
     int nT;
     int jtiles;                   // tiles of panels j (disjoint items per block of panels i)
     int niw;                      // wavefronts of 64 panels i
-    int pad;
+    int jt;                       // panels j per tile
     // Partial cotangents of the panels' vertices, 9 doubles each (vertex a,
     // b, c; x, y, z): ki[tile][i] from the disjoint item (wavefront of i,
     // tile) as the control panel, kj[iw][j] from the wavefront iw of panels
@@ -56,18 +56,18 @@ struct AdjArgs {
     int quirk;
     i2d::Rule rule;
     uint64_t seed;
-    int j_tile;                   // panels j per disjoint item
-    int pad;
     int64_t disjoint_items;       // items: (mesh, wavefront of 64 panels i, tile of panels j)
     const int64_t* item_base;     // per mesh
     int64_t singular_tasks;       // ordered vertex- and edge-sharing tasks of all meshes
     const int64_t* sing_base;     // [kind * nmeshes + m], kind 0 vertex-, 1 edge-sharing
-    unsigned long long* counters; // [0] disjoint item
+    unsigned long long* counters; // [0] disjoint item, [1] items with pairs at level >= 2, [2] claims of those
     SingRec* sing_rec;            // per singular task (singular_tasks entries)
     double* sing_dl;              // per singular task: dL/d of its 18 vertex coordinates (I's a, b, c, J's a, b, c)
     double* item_loss;            // per disjoint item: its pairs' terms of L
     double* loss_part;            // per mesh: partial sums of L (k_adj_loss_part)
     uint32_t* deep_mask;          // per disjoint item and lane: bit b set if (i, j0 + b) is at reported level >= 2
+                                  // (written for the items in deep_items)
+    int64_t* deep_items;          // the disjoint items that hold such a pair, counters[1] of them
     // the vertex gather: panel sums (9 per panel, mesh m's from pbase[m]);
     // vertices of all meshes (mesh m's from vbase[m]), each with its (panel,
     // corner) incidences (3 p + corner, panels ascending) and its
@@ -99,6 +99,7 @@ struct AdjState {
     DBuf<int64_t> d_pbase, d_vbase, d_inc_start, d_sing_start, d_sing_idx;
     DBuf<int32_t> d_inc;
     DBuf<uint32_t> d_deep_mask;
+    DBuf<int64_t> d_deep_items;
     DBuf<unsigned long long> d_counters;
     DBuf<SingRec> d_sing_rec;
     hipEvent_t e0 = nullptr, e1 = nullptr;
