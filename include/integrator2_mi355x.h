@@ -229,7 +229,9 @@ int i2_evaluator_output_results_to_file(const i2_evaluator* ev, int type, int fo
  * outputs in the same task order. */
 int i2_evaluator_set_path(i2_evaluator* ev, int path);
 /* Launch shape of the batched path: pairs per workgroup and quadrature points
- * per lane (1, 2, 4 or 13 = the whole 13-point rule in one lane). */
+ * per lane (1, 2, 4 or 13 = the whole 13-point rule in one lane).  Until
+ * the first call the shape follows the mesh's size: 64 pairs of one lane each,
+ * fewer pairs and more lanes per pair on small meshes. */
 int i2_evaluator_set_tuning(i2_evaluator* ev, int pairsPerWorkgroup, int pointsPerLane);
 
 /* ---- shape sensitivity (no counterpart in the reference) --------------

@@ -162,29 +162,8 @@ __device__ __forceinline__ void panel_chain(const Panel& P, d3 tab, d3 tbb, d3 t
     Bb = Bb + gu; Cb = Cb + gv; Ab = Ab - gu - gv;
 }
 
-// Barycentric weights (w.r.t. the original panel) of the vertices of level-1 child `ch`:
-// children {m_AB, B, m_BC}, {m_BC, C, m_CA}, {m_CA, A, m_AB}, {m_BC, m_CA, m_AB}
-__device__ __forceinline__ void child_bary(int ch, d3& ba, d3& bb, d3& bc) {
-    const d3 A = {1.0, 0.0, 0.0}, B = {0.0, 1.0, 0.0}, C = {0.0, 0.0, 1.0};
-    const d3 mAB = {0.5, 0.5, 0.0}, mBC = {0.0, 0.5, 0.5}, mCA = {0.5, 0.0, 0.5};
-    if (ch == 0) { ba = mAB; bb = B; bc = mBC; }
-    else if (ch == 1) { ba = mBC; bb = C; bc = mCA; }
-    else if (ch == 2) { ba = mCA; bb = A; bc = mAB; }
-    else { ba = mBC; bb = mCA; bc = mAB; }
-}
-// The rule's points on level 0 and on the four level-1 children, barycentric
-// on the original panel, with their weights (32-byte records in LDS)
-struct alignas(32) BaryPoint { double b0, b1, b2, w; };
 __device__ __forceinline__ void load_bary(BaryPoint* P, const RuleSh& R, int npts) {
-    for (int t = threadIdx.x; t < 5 * npts; t += blockDim.x) {
-        const int sub = t / npts, k = t - sub * npts;
-        d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
-        if (sub > 0) child_bary(sub - 1, ba, bb, bc);
-        d3 b = R.L1[k] * ba;
-        b = b + R.L2[k] * bb;
-        b = b + R.L3[k] * bc;
-        P[t] = {b.x, b.y, b.z, R.w[k]};
-    }
+    for (int t = threadIdx.x; t < 5 * npts; t += blockDim.x) P[t] = bary_point(R.L1, R.L2, R.L3, R.w, npts, t);
 }
 
 // Sums of nine values over the wavefront, in a fixed order: pairs of registers
@@ -236,9 +215,7 @@ __device__ __forceinline__ void points_rev(const RuleSh& R, const BaryPoint* pts
                                            const q4& ct, TermsBar& g, d3& X0, d3& X1) {
     for (int k = k0; k < k1; ++k) {
         const BaryPoint Q = pts[k];
-        d3 p = Q.b0 * I.a;
-        p = p + Q.b1 * I.b;
-        p = p + Q.b2 * I.c;
+        const d3 p = at_bary(Q, I.a, I.b, I.c);
         const d3 pb = theta_terms_rev<FAR>(p, JG, &R.lt, Q.w, ct, g);
         axpy(X0, Q.b0, pb); axpy(X1, Q.b1, pb);
     }

@@ -77,10 +77,10 @@ I2_HD __forceinline__ q4 theta_psi_fast_rev(d3 p, const JGeom& J, const i2m::Mat
     double t3 = i2m::log_tab_any(a3, lt);
     double th = i2m::atan2_any(y, x, lt);
     if (__builtin_expect(!(o1 & o2 & o3 & o4), 0)) {
-        if (!o1) t1 = i2m::log_slow(a1);
-        if (!o2) t2 = i2m::log_slow(a2);
-        if (!o3) t3 = i2m::log_slow(a3);
-        if (!o4) th = i2m::atan2_slow(y, x);
+        if (!o1) t1 = i2m::log_rare(a1, lt);
+        if (!o2) t2 = i2m::log_rare(a2, lt);
+        if (!o3) t3 = i2m::log_rare(a3, lt);
+        if (!o4) th = i2m::atan2_rare(y, x, lt);
     }
     q4 r;
     r.x = t1 * J.tc.x + t2 * J.ta.x + t3 * J.tb.x;

@@ -20,14 +20,12 @@
 //              split its quadrature points.  Vertex- and edge-sharing tasks
 //              come from the mesh's lists, P per item.  Items are claimed from
 //              an atomic counter by persistent workgroups.
-//   k_deep     refinement level L >= 2 of the tasks queued by level L-1:
-//              min(4^L, 64) lanes per task, one sub-panel per lane,
-//              fixed-order butterfly reduction.
+//   k_deep     refinement level L >= 2 of the tasks queued by level L-1: 16 or
+//              64 lanes per task, fixed-order reduction.
 //   k_levels / k_compute_K   K per (mesh, type) from queue membership.
 //   per-pair outputs (value, J) are written by the task's last kernel for
-//   K = maxLevel; k_finalize_disjoint (per row of the disjoint pair list) and
-//   k_finalize_singular correct the types whose K differs by an odd number;
-//   k_finalize_rows   row sums for K's parity.
+//   K = maxLevel; k_finalize_pairs corrects the types whose K differs by an odd
+//   number; k_finalize_rows   row sums for K's parity.
 #include "i2_batch.hpp"
 #include "i2_adjoint.hpp"
 
@@ -294,50 +292,10 @@ __device__ __forceinline__ void add_row(const MeshDesc& M, int type, int i, q4 r
     atomicAdd(a1 + 0, rp1.x); atomicAdd(a1 + 1, rp1.y); atomicAdd(a1 + 2, rp1.z); atomicAdd(a1 + 3, rp1.w);
 }
 
-// Levels 0 and 1 of one task (lane group of LPP lanes), then the Runge check.
-template <int TYPE, int LPP>
-__device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS& R, int m, int i, int j, int64_t z, bool valid,
-                                              int s, const Panel& I, const Panel& J, const PtsLDS* pts = nullptr,
-                                              const Ball* ball = nullptr) {
-    Sing<TYPE> sg;
-    if (TYPE != I2_NOT_NEIGHBORS && valid) sg.init(I, J);
-    const JGeom JG = jgeom(J);
-    const int npts = A.rule.n;
-    const bool need0 = !A.fixed || A.last_level == 0;
-    const bool need1 = A.fixed ? A.last_level == 1 : A.last_level >= 1;
-    q4 v0 = q4zero(), v1 = q4zero();
-    if constexpr (TYPE == I2_NOT_NEIGHBORS) {
-        // one loop per wavefront: far only if every pair of the wavefront is
-        const bool near = __ballot(valid && !panel_far(*ball, JG)) != 0ull;
-        if (valid) {
-            q4 T0 = q4zero(), T1 = q4zero();
-            if (near) {
-                sweep_terms<false, LPP>(R, *pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
-            } else {
-                sweep_terms<true, LPP>(R, *pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
-                T0 = far_scale(T0, JG);
-                T1 = far_scale(T1, JG);
-            }
-            v0 = I.area * psi_of_terms(T0, JG);
-            v1 = (0.25 * I.area) * psi_of_terms(T1, JG);
-        }
-    } else if (valid) {
-        if (need0) v0 = I.area * quad_part<TYPE>(R, npts, s, LPP, I.a, I.b, I.c, JG, sg);
-        if (need1) {
-            const double a1 = 0.25 * I.area;
-            const d3 mBC = 0.5 * (I.b + I.c), mCA = 0.5 * (I.c + I.a), mAB = 0.5 * (I.a + I.b);
-            v1 = v1 + a1 * quad_part<TYPE>(R, npts, s, LPP, mAB, I.b, mBC, JG, sg);
-            v1 = v1 + a1 * quad_part<TYPE>(R, npts, s, LPP, mBC, I.c, mCA, JG, sg);
-            v1 = v1 + a1 * quad_part<TYPE>(R, npts, s, LPP, mCA, I.a, mAB, JG, sg);
-            v1 = v1 + a1 * quad_part<TYPE>(R, npts, s, LPP, mBC, mCA, mAB, JG, sg);
-        }
-    }
-    if (LPP > 1) {
-        v0 = shfl_sum(v0, LPP);
-        v1 = shfl_sum(v1, LPP);
-    }
+// The Runge check of a task after its levels 0 and 1 (v0, v1).
+template <int TYPE>
+__device__ __forceinline__ StepOut sweep_check(const BatchArgs& A, int m, int i, int j, int64_t z, q4 v0, q4 v1) {
     StepOut o{false, false, 0, v0, v0};
-    if (!valid || s != 0) return o;
     if (A.fixed) {
         if (A.last_level <= 1) { o.finished = true; o.c = A.last_level; o.cur = o.prev = (A.last_level == 0 ? v0 : v1); }
         else { push_deep(A, A.last_level, TYPE, m, i, j, z, v1); o.pushed = true; }
@@ -348,6 +306,37 @@ __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS&
     if (!(crit > A.tol) || A.last_level == 1) { o.finished = true; o.c = 1; o.cur = v1; o.prev = A.quirk ? v0 : v1; o.unconv = crit > A.tol; }
     else { push_deep(A, 2, TYPE, m, i, j, z, v1); o.pushed = true; }
     return o;
+}
+
+// Levels 0 and 1 of one disjoint task (lane group of LPP lanes), then the Runge check.
+template <int LPP>
+__device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS& R, int m, int i, int j, int64_t z, bool valid,
+                                              int s, const Panel& I, const Panel& J, const PtsLDS& pts, const Ball& ball) {
+    const JGeom JG = jgeom(J);
+    const int npts = A.rule.n;
+    const bool need0 = !A.fixed || A.last_level == 0;
+    const bool need1 = A.fixed ? A.last_level == 1 : A.last_level >= 1;
+    q4 v0 = q4zero(), v1 = q4zero();
+    // one loop per wavefront: far only if every pair of the wavefront is
+    const bool near = __ballot(valid && !panel_far(ball, JG)) != 0ull;
+    if (valid) {
+        q4 T0 = q4zero(), T1 = q4zero();
+        if (near) {
+            sweep_terms<false, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
+        } else {
+            sweep_terms<true, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
+            T0 = far_scale(T0, JG);
+            T1 = far_scale(T1, JG);
+        }
+        v0 = I.area * psi_of_terms(T0, JG);
+        v1 = (0.25 * I.area) * psi_of_terms(T1, JG);
+    }
+    if (LPP > 1) {
+        v0 = shfl_sum(v0, LPP);
+        v1 = shfl_sum(v1, LPP);
+    }
+    if (!valid || s != 0) return StepOut{false, false, 0, v0, v0};
+    return sweep_check<I2_NOT_NEIGHBORS>(A, m, i, j, z, v0, v1);
 }
 
 // Disjoint pairs, levels 0 and 1: item = (mesh, control panel i, P consecutive j),
@@ -384,7 +373,7 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
         const Panel J = M.panels[in_range ? j : i];
         const bool valid = in_range && j != i && shared_count(I, J) == 0;
         const int64_t z = valid ? disjoint_task(M, i, j) : 0;
-        const StepOut o = sweep_task<I2_NOT_NEIGHBORS, LPP>(A, R, m, i, j, z, valid, s, I, J, &pts, &ball);
+        const StepOut o = sweep_task<LPP>(A, R, m, i, j, z, valid, s, I, J, pts, ball);
         q4 rp0 = q4zero(), rp1 = q4zero();
         if (o.finished) finish_task<I2_NOT_NEIGHBORS, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
         if (OUT == OUT_ROW_SUMS) {
@@ -399,55 +388,75 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
     }
 }
 
-// Vertex- and edge-sharing tasks, levels 0 and 1: one task per lane, 256 per item.
-template <int OUT>
+// Vertex- and edge-sharing tasks, levels 0 and 1: G lanes per task, which
+// split the 5 npts points of both levels.  What is done once per task (the
+// singular part's context with its atan2, the panel records) is repeated by the
+// group, some 1,000 instructions against 450 per point.  Bounds: with one
+// lane per task the 65 points in series took 110-170 us whatever the mesh
+// (320 panels: 59 wavefronts on 1,024 SIMDs).
+template <int TYPE, int OUT, int G>
+__device__ __forceinline__ void singular_sweep_task(const BatchArgs& A, const RuleLDS& R, const BaryPoint* pts, int m, int64_t z, int i,
+                                                    int j, int s) {
+    const MeshDesc& M = A.meshes[m];
+    const Panel I = M.panels[i];
+    const Panel J = M.panels[j];
+    Sing<TYPE> sg;
+    sg.init(I, J);
+    const JGeom JG = jgeom(J);
+    const int npts = A.rule.n;
+    const bool need0 = !A.fixed || A.last_level == 0;
+    const bool need1 = A.fixed ? A.last_level == 1 : A.last_level >= 1;
+    const int k0 = need0 ? 0 : npts, k1 = need1 ? 5 * npts : npts;
+    q4 v0 = q4zero(), v1 = q4zero();
+    for (int k = k0 + s; k < k1; k += G) {
+        const BaryPoint Q = pts[k];
+        const d3 p = at_bary(Q, I.a, I.b, I.c);
+        const q4 f = theta_psi_fast(p, JG, &R.lt) - sg.at(p, &R.lt);
+        const double w0 = k < npts ? Q.w : 0.0, w1 = k < npts ? 0.0 : Q.w;
+        v0 = v0 + w0 * f;
+        v1 = v1 + w1 * f;
+    }
+    v0 = I.area * shfl_sum(v0, G);
+    v1 = (0.25 * I.area) * shfl_sum(v1, G);
+    if (s != 0) return;
+    const StepOut o = sweep_check<TYPE>(A, m, i, j, z, v0, v1);
+    if (o.finished) {
+        q4 rp0, rp1;
+        finish_task<TYPE, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
+        if (OUT == OUT_ROW_SUMS) add_row(M, TYPE, i, rp0, rp1);
+    }
+}
+template <int OUT, int G>
 __global__ __launch_bounds__(256) I2_TWO_WAVES void k_sweep_singular(BatchArgs A) {
     __shared__ RuleLDS R;
-    __shared__ long long item_sh;
+    __shared__ BaryPoint pts[5 * MAX_POINTS];
     load_rule(R, A.rule);
-    const int P = blockDim.x;
-    for (;;) {
-        __syncthreads();
-        if (threadIdx.x == 0) item_sh = (long long)atomicAdd(&A.counters[1 + MAX_LEVELS * 3], 1ull);
-        __syncthreads();
-        const int64_t item = uniform64(item_sh);
-        if (item >= A.singular_items) break;
-        const int b = __builtin_amdgcn_readfirstlane(find_base(A.sing_base, 2 * A.nmeshes, item));
+    __syncthreads();
+    for (int t = threadIdx.x; t < 5 * A.rule.n; t += blockDim.x) pts[t] = bary_point(R.L1, R.L2, R.L3, R.w, A.rule.n, t);
+    __syncthreads();
+    const int s = threadIdx.x % G;
+    const int64_t total = A.singular_items * 256, step = (int64_t)gridDim.x * (blockDim.x / G);
+    for (int64_t g = (int64_t)blockIdx.x * (blockDim.x / G) + threadIdx.x / G; g < total; g += step) {
+        const int b = find_base(A.sing_base, 2 * A.nmeshes, g >> 8);
         const int type = b / A.nmeshes == 0 ? I2_SIMPLE_NEIGHBORS : I2_ATTACHED_NEIGHBORS;
         const int m = b % A.nmeshes;
         const MeshDesc& M = A.meshes[m];
         const int64_t n = M.npairs[type];
-        const int64_t z = (item - A.sing_base[b]) * P + threadIdx.x;
-        const bool valid = z < 2 * n;
-        int i = 0, j = 0;
-        if (valid) {
-            const int32_t* L = M.lists[type];
-            const int64_t k = z < n ? z : z - n;
-            i = L[3 * k]; j = L[3 * k + 1];
-            if (z >= n) { const int t = i; i = j; j = t; }
-        }
-        const Panel I = M.panels[i];
-        const Panel J = M.panels[j];
-        q4 rp0 = q4zero(), rp1 = q4zero();
-        if (type == I2_SIMPLE_NEIGHBORS) {
-            const StepOut o = sweep_task<I2_SIMPLE_NEIGHBORS, 1>(A, R, m, i, j, z, valid, 0, I, J);
-            if (o.finished) {
-                finish_task<I2_SIMPLE_NEIGHBORS, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
-                if (OUT == OUT_ROW_SUMS) add_row(M, type, i, rp0, rp1);
-            }
-        } else {
-            const StepOut o = sweep_task<I2_ATTACHED_NEIGHBORS, 1>(A, R, m, i, j, z, valid, 0, I, J);
-            if (o.finished) {
-                finish_task<I2_ATTACHED_NEIGHBORS, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
-                if (OUT == OUT_ROW_SUMS) add_row(M, type, i, rp0, rp1);
-            }
-        }
+        const int64_t z = (g >> 8) * 256 - A.sing_base[b] * 256 + (g & 255);
+        if (z >= 2 * n) continue;
+        const int64_t k = z < n ? z : z - n;
+        int i = M.lists[type][3 * k], j = M.lists[type][3 * k + 1];
+        if (z >= n) { const int t = i; i = j; j = t; }
+        if (type == I2_SIMPLE_NEIGHBORS) singular_sweep_task<I2_SIMPLE_NEIGHBORS, OUT, G>(A, R, pts, m, z, i, j, s);
+        else singular_sweep_task<I2_ATTACHED_NEIGHBORS, OUT, G>(A, R, pts, m, z, i, j, s);
     }
 }
 
 // Refinement level >= 2 of one queued task.
+// G lanes, Q of them per sub-panel.
 template <int TYPE, int OUT>
-__device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, int level, int G, int s, const QEntry& e, bool valid) {
+__device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, int level, int G, int Q, int s, const QEntry& e,
+                                          bool valid) {
     const MeshDesc& M = A.meshes[e.m];
     const Panel I = M.panels[e.i];
     const Panel J = M.panels[e.j];
@@ -459,10 +468,10 @@ __device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, 
         double area = I.area;
         for (int l = 0; l < level; ++l) area *= 0.25;
         const uint32_t nsub = 1u << (2 * level);
-        for (uint32_t c = s; c < nsub; c += G) {
+        for (uint32_t c = s / Q; c < nsub; c += G / Q) {
             d3 a = I.a, b = I.b, cc = I.c;
             sub_panel(a, b, cc, level, c);
-            acc = acc + area * quad_part<TYPE>(R, A.rule.n, 0, 1, a, b, cc, JG, sg);
+            acc = acc + area * quad_part<TYPE>(R, A.rule.n, s % Q, Q, a, b, cc, JG, sg);
         }
     }
     acc = shfl_sum(acc, G);
@@ -484,27 +493,38 @@ __device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, 
     }
 }
 
-// Refinement level L >= 2 of the queued tasks of the types in [t0, t1].
+// Refinement level L >= 2 of the queued tasks of the types in [t0, t1]: a
+// wavefront per task from level 3 (a sub-panel per lane at level 3), at level 2
+// 16 lanes per task, one sub-panel each, or a wavefront with four lanes per
+// sub-panel where 16 lanes each would leave SIMDs empty (4 rounds of points
+// instead of 13 in series, at 81 % of the lanes).  A workgroup without a task
+// ends before it loads the tables.
 template <int OUT, int T0, int T1>
 __global__ __launch_bounds__(256) I2_TWO_WAVES void k_deep(BatchArgs A, int level) {
     __shared__ RuleLDS R;
-    load_rule(R, A.rule);
-    __syncthreads();
-    const int G = level >= 3 ? 64 : 16;                 // lanes per task
-    const int per_block = blockDim.x / G;
-    const int slot = threadIdx.x / G, s = threadIdx.x % G;
+    bool loaded = false;
     for (int type = T0; type <= T1; ++type) {
         const int qi = level * 3 + type;
         const unsigned long long cnt = min(A.counters[1 + qi], (unsigned long long)A.qcap[type]);
+        const bool wide = level >= 3 || cnt <= 8192;
+        const int G = wide ? 64 : 16, Q = level == 2 && wide ? 4 : 1;
+        const int per_block = blockDim.x / G;
+        if ((unsigned long long)blockIdx.x * per_block >= cnt) continue;   // uniform
+        if (!loaded) {
+            load_rule(R, A.rule);
+            __syncthreads();
+            loaded = true;
+        }
+        const int slot = threadIdx.x / G, s = threadIdx.x % G;
         const QEntry* q = A.queue + A.qoff[qi];
         for (unsigned long long base = (unsigned long long)blockIdx.x * per_block; base < cnt;
              base += (unsigned long long)gridDim.x * per_block) {
             const unsigned long long t = base + slot;
             const bool valid = t < cnt;
             QEntry e = q[valid ? t : base];
-            if (type == I2_NOT_NEIGHBORS) deep_task<I2_NOT_NEIGHBORS, OUT>(A, R, level, G, s, e, valid);
-            else if (type == I2_SIMPLE_NEIGHBORS) deep_task<I2_SIMPLE_NEIGHBORS, OUT>(A, R, level, G, s, e, valid);
-            else deep_task<I2_ATTACHED_NEIGHBORS, OUT>(A, R, level, G, s, e, valid);
+            if (type == I2_NOT_NEIGHBORS) deep_task<I2_NOT_NEIGHBORS, OUT>(A, R, level, G, Q, s, e, valid);
+            else if (type == I2_SIMPLE_NEIGHBORS) deep_task<I2_SIMPLE_NEIGHBORS, OUT>(A, R, level, G, Q, s, e, valid);
+            else deep_task<I2_ATTACHED_NEIGHBORS, OUT>(A, R, level, G, Q, s, e, valid);
         }
     }
 }
@@ -543,6 +563,7 @@ __global__ __launch_bounds__(256) void k_levels(BatchArgs A) {
 
 // K per (mesh, type): 0 when maxLevel = 0 (automatic) or no task; else the
 // deepest level any of its tasks reached (at least 1).  Fixed mode: the level.
+// With one mesh the queue counts say which levels were reached.
 __global__ void k_compute_K(BatchArgs A) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= 3 * A.nmeshes) return;
@@ -552,8 +573,11 @@ __global__ void k_compute_K(BatchArgs A) {
     if (A.fixed) K = A.last_level;
     else if (any && A.last_level >= 1) {
         K = 1;
-        for (int L = 2; L <= A.last_level; ++L)
-            if ((A.levelmask[(L * 3 + type) * MASK_WORDS + (m >> 6)] >> (m & 63)) & 1ull) K = L;
+        for (int L = 2; L <= A.last_level; ++L) {
+            const bool reached = A.nmeshes == 1 ? A.counters[1 + L * 3 + type] != 0ull
+                                                : (A.levelmask[(L * 3 + type) * MASK_WORDS + (m >> 6)] >> (m & 63)) & 1ull;
+            if (reached) K = L;
+        }
     }
     A.K[g] = K;
 }
@@ -577,29 +601,6 @@ __device__ __forceinline__ void finalize_task(const BatchArgs& A, const MeshDesc
     o[0] = r.x; o[1] = r.y; o[2] = r.z;
 }
 
-// Disjoint tasks, one row i of the lexicographic pair list per workgroup
-// pass: the lanes walk its pairs (i, j), j > i, and finalize (i, j) and its
-// reversed task (j, i), with j from i's sorted neighbour list (no search).
-__global__ __launch_bounds__(256) void k_finalize_disjoint(BatchArgs A) {
-    for (int64_t r = blockIdx.x; r < A.total_rows; r += gridDim.x) {
-        const int m = find_base(A.row_base, A.nmeshes, r);
-        if (!needs_correction(A, m, I2_NOT_NEIGHBORS)) continue;
-        const MeshDesc& M = A.meshes[m];
-        const int ii = (int)(r - A.row_base[m]);
-        const int64_t k0 = M.row_start[ii], cnt = M.row_start[ii + 1] - k0;
-        const int64_t n = M.npairs[I2_NOT_NEIGHBORS];
-        const int64_t q0 = M.nbr_start[ii], q1 = M.nbr_start[ii + 1];
-        for (int64_t t = threadIdx.x; t < cnt; t += blockDim.x) {
-            int64_t jj = ii + 1 + t;
-            for (int64_t q = q0; q < q1; ++q) {
-                if (M.nbr[q] <= jj) ++jj; else break;
-            }
-            finalize_task(A, M, m, I2_NOT_NEIGHBORS, k0 + t, ii, (int)jj);
-            finalize_task(A, M, m, I2_NOT_NEIGHBORS, n + k0 + t, (int)jj, ii);
-        }
-    }
-}
-
 // The closed-form singular integral of every vertex- and edge-sharing task, one
 // task per lane (the task's last kernel adds it to the level value; a refinement
 // kernel would otherwise evaluate it on one lane of each lane group).
@@ -621,8 +622,13 @@ __global__ __launch_bounds__(256) void k_singular_closed(BatchArgs A) {
     }
 }
 
-// Vertex- and edge-sharing tasks, enumerated as the singular sweep's items.
-__global__ __launch_bounds__(256) void k_finalize_singular(BatchArgs A) {
+// All tasks whose type needs the correction.  Vertex- and edge-sharing tasks
+// are enumerated as the singular sweep's; disjoint ones by rows i of the
+// lexicographic pair list, one per workgroup pass: the lanes walk its pairs
+// (i, j), j > i, and finalize (i, j) and its reversed task (j, i), with j from
+// i's sorted neighbour list (no search).
+__global__ __launch_bounds__(256) void k_finalize_pairs(BatchArgs A) {
+    if (!A.quirk) return;
     const int64_t total = A.singular_items * 256;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += (int64_t)gridDim.x * blockDim.x) {
         const int64_t item = g >> 8;
@@ -639,28 +645,64 @@ __global__ __launch_bounds__(256) void k_finalize_singular(BatchArgs A) {
         if (z >= n) { const int t = i; i = j; j = t; }
         finalize_task(A, M, m, type, z, i, j);
     }
+    for (int64_t r = blockIdx.x; r < A.total_rows; r += gridDim.x) {
+        const int m = find_base(A.row_base, A.nmeshes, r);
+        if (!needs_correction(A, m, I2_NOT_NEIGHBORS)) {
+            r += (A.row_base[m + 1] - 1 - r) / gridDim.x * gridDim.x;   // on to the next mesh
+            continue;
+        }
+        const MeshDesc& M = A.meshes[m];
+        const int ii = (int)(r - A.row_base[m]);
+        const int64_t k0 = M.row_start[ii], cnt = M.row_start[ii + 1] - k0;
+        const int64_t n = M.npairs[I2_NOT_NEIGHBORS];
+        const int64_t q0 = M.nbr_start[ii], q1 = M.nbr_start[ii + 1];
+        for (int64_t t = threadIdx.x; t < cnt; t += blockDim.x) {
+            int64_t jj = ii + 1 + t;
+            for (int64_t q = q0; q < q1; ++q) {
+                if (M.nbr[q] <= jj) ++jj; else break;
+            }
+            finalize_task(A, M, m, I2_NOT_NEIGHBORS, k0 + t, ii, (int)jj);
+            finalize_task(A, M, m, I2_NOT_NEIGHBORS, n + k0 + t, (int)jj, ii);
+        }
+    }
 }
 
-// Row sums for K's parity, summed over the three types: (sum_j J, sum_j Theta).
-__global__ void k_finalize_rows(BatchArgs A, int m) {
+// Row sums for K's parity, summed over the three types: (sum_j J, sum_j
+// Theta), the rows of all meshes.
+__global__ void k_finalize_rows(BatchArgs A) {
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= A.total_rows) return;
+    const int m = find_base(A.row_base, A.nmeshes, r);
     const MeshDesc& M = A.meshes[m];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= M.nT) return;
-    double r[4] = {0, 0, 0, 0};
+    const int i = (int)(r - A.row_base[m]);
+    double v[4] = {0, 0, 0, 0};
     for (int type = 0; type < 3; ++type) {
         const int par = A.K[3 * m + type] & 1;
         const double* acc = M.rowacc + (((size_t)type * 2 + par) * M.nT + i) * 4;
-        for (int c = 0; c < 4; ++c) r[c] += acc[c];
+        for (int c = 0; c < 4; ++c) v[c] += acc[c];
     }
-    for (int c = 0; c < 4; ++c) M.rowout[4 * (size_t)i + c] = r[c];
+    for (int c = 0; c < 4; ++c) M.rowout[4 * (size_t)i + c] = v[c];
 }
 
-// Zero-fill kernels (graph-safe replacement of hipMemsetAsync).
-__global__ void k_zero_u64(unsigned long long* p, int64_t n) {
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) p[q] = 0ull;
-}
-__global__ void k_zero_f64(double* p, int64_t n) {
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) p[q] = 0.0;
+// The start of a run: counters, level masks and, per row of every mesh, the row
+// sums or the unconverged flags (by a kernel: a memset recorded in a graph can
+// give wrong results on later replays).
+__global__ __launch_bounds__(256) void k_begin(BatchArgs A) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t q = t; q < N_COUNTERS; q += step) A.counters[q] = 0ull;
+    for (int64_t q = t; q < MAX_LEVELS * 3 * MASK_WORDS; q += step) A.levelmask[q] = 0ull;
+    for (int64_t r = t; r < A.total_rows; r += step) {
+        const int m = find_base(A.row_base, A.nmeshes, r);
+        const MeshDesc& M = A.meshes[m];
+        const int64_t i = r - A.row_base[m];
+        if (M.rowacc)
+            for (int c = 0; c < 6; ++c) {
+                double* a = M.rowacc + ((size_t)c * M.nT + i) * 4;
+                a[0] = 0.0; a[1] = 0.0; a[2] = 0.0; a[3] = 0.0;
+            }
+        for (int type = 0; type < 3; ++type)
+            if (M.unconv[type]) M.unconv[type][i] = 0;
+    }
 }
 
 // ------------------------------------------------------------ host engine
@@ -701,8 +743,15 @@ static int launch_sweep(const Engine& E, hipStream_t st) {
     I2_TRY(check_launch("k_sweep_disjoint"));
     if (E.prof1) I2_HIP(hipEventRecord(E.prof1, st));
     if (E.args.singular_items > 0) {
-        if (E.out == OUT_PER_PAIR) hipLaunchKernelGGL((k_sweep_singular<OUT_PER_PAIR>), dim3(E.deep_grid), dim3(256), 0, st, E.args);
-        else hipLaunchKernelGGL((k_sweep_singular<OUT_ROW_SUMS>), dim3(E.deep_grid), dim3(256), 0, st, E.args);
+        // 16 lanes per task until that is about two rounds of the wavefronts the
+        // chip holds (two per SIMD), then 4
+        const bool few = E.args.singular_items <= 64;
+        const int64_t blocks = E.args.singular_items * (few ? 16 : 4);
+        const dim3 grid((unsigned)std::min<int64_t>(blocks, E.deep_grid));
+#define I2_SING(O, G) hipLaunchKernelGGL((k_sweep_singular<O, G>), grid, dim3(256), 0, st, E.args)
+        if (E.out == OUT_PER_PAIR) { if (few) I2_SING(OUT_PER_PAIR, 16); else I2_SING(OUT_PER_PAIR, 4); }
+        else { if (few) I2_SING(OUT_ROW_SUMS, 16); else I2_SING(OUT_ROW_SUMS, 4); }
+#undef I2_SING
         I2_TRY(check_launch("k_sweep_singular"));
     }
     return I2_OK;
@@ -734,10 +783,9 @@ static int compute_grids(Engine& E) {
 
 int batch_enqueue(Engine& E, hipStream_t st) {
     const BatchArgs& A = E.args;
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(256), 0, st, E.d_counters.p, (int64_t)E.d_counters.n);
-    I2_TRY(check_launch("k_zero_u64"));
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(256), 0, st, E.d_levelmask.p, (int64_t)E.d_levelmask.n);
-    I2_TRY(check_launch("k_zero_u64"));
+    const unsigned row_blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>((A.total_rows + 255) / 256, E.fin_grid));
+    hipLaunchKernelGGL(k_begin, dim3(row_blocks), dim3(256), 0, st, A);
+    I2_TRY(check_launch("k_begin"));
     if (A.singular_items > 0) {
         hipLaunchKernelGGL(k_singular_closed, dim3(E.deep_grid), dim3(256), 0, st, A);
         I2_TRY(check_launch("k_singular_closed"));
@@ -757,27 +805,33 @@ int batch_enqueue(Engine& E, hipStream_t st) {
         }
         I2_TRY(check_launch("k_deep"));
     }
-    if (A.last_level >= 2) {
+    if (A.last_level >= 2 && A.nmeshes > 1) {
         hipLaunchKernelGGL(k_levels, dim3(E.levels_grid), dim3(256), 0, st, A);
         I2_TRY(check_launch("k_levels"));
     }
     hipLaunchKernelGGL(k_compute_K, dim3((3 * A.nmeshes + 255) / 256), dim3(256), 0, st, A);
     I2_TRY(check_launch("k_compute_K"));
     if (E.out == OUT_PER_PAIR) {
-        hipLaunchKernelGGL(k_finalize_disjoint, dim3(E.fin_grid), dim3(256), 0, st, A);
-        I2_TRY(check_launch("k_finalize_disjoint"));
-        if (A.singular_items > 0) {
-            hipLaunchKernelGGL(k_finalize_singular, dim3(E.deep_grid), dim3(256), 0, st, A);
-            I2_TRY(check_launch("k_finalize_singular"));
+        if (A.quirk) {
+            const int64_t most = std::max<int64_t>({A.total_rows, A.singular_items, 1});
+            hipLaunchKernelGGL(k_finalize_pairs, dim3((unsigned)std::min<int64_t>(most, E.fin_grid)), dim3(256), 0, st, A);
+            I2_TRY(check_launch("k_finalize_pairs"));
         }
     } else {
-        for (int m = 0; m < A.nmeshes; ++m) {
-            const int nT = (int)E.nT[m];
-            hipLaunchKernelGGL(k_finalize_rows, dim3((nT + 255) / 256), dim3(256), 0, st, A, m);
-            I2_TRY(check_launch("k_finalize_rows"));
-        }
+        hipLaunchKernelGGL(k_finalize_rows, dim3((unsigned)((A.total_rows + 255) / 256)), dim3(256), 0, st, A);
+        I2_TRY(check_launch("k_finalize_rows"));
     }
     return I2_OK;
+}
+
+// Launch shape for a caller who has set none: one lane per pair where that
+// makes enough wavefronts (3,072 in flight, three per SIMD), else several
+// lanes per pair.
+void engine_auto_shape(Engine& E) {
+    int64_t waves = 0;
+    for (const MeshDesc& D : E.h_meshes) waves += (int64_t)D.nT * ((D.nT + 63) / 64);
+    E.ppl = waves >= 6144 ? 13 : (waves >= 768 ? 4 : 1);
+    E.pairs_per_wg = 64 / lanes_for_points_per_lane(E.ppl);
 }
 
 int engine_setup(Engine& E, const i2_integrator& it) {
@@ -851,9 +905,8 @@ int engine_setup(Engine& E, const i2_integrator& it) {
     I2_TRY(E.d_sing_base.ensure(2 * M + 1));
     I2_TRY(E.d_pair_base.ensure(3 * M + 1));
     I2_TRY(E.d_row_base.ensure(M + 1));
-    I2_TRY(E.d_counters.ensure(2 + MAX_LEVELS * 3));
+    I2_TRY(E.d_counters.ensure(N_COUNTERS + (3 * M + 1) / 2));
     I2_TRY(E.d_levelmask.ensure(MAX_LEVELS * 3 * MASK_WORDS));
-    I2_TRY(E.d_K.ensure(3 * M));
     I2_HIP(hipMemcpy(E.d_qoff.p, E.h_qoff.data(), sizeof(int64_t) * E.h_qoff.size(), hipMemcpyHostToDevice));
     I2_HIP(hipMemcpy(E.d_meshes.p, E.h_meshes.data(), sizeof(MeshDesc) * M, hipMemcpyHostToDevice));
     I2_HIP(hipMemcpy(E.d_item_base.p, E.h_item_base.data(), sizeof(int64_t) * (M + 1), hipMemcpyHostToDevice));
@@ -869,21 +922,28 @@ int engine_setup(Engine& E, const i2_integrator& it) {
     A.queue = E.d_queue.p;
     A.qoff = E.d_qoff.p;
     A.levelmask = E.d_levelmask.p;
-    A.K = E.d_K.p;
+    A.K = reinterpret_cast<int*>(E.d_counters.p + N_COUNTERS);   // behind the counters: one copy brings both to the host
     return I2_OK;
 }
 
-int engine_check_queues(Engine& E, hipStream_t st, bool* overflow, std::vector<unsigned long long>* counts) {
-    std::vector<unsigned long long> c(2 + MAX_LEVELS * 3);
-    I2_HIP(hipMemcpyAsync(c.data(), E.d_counters.p, sizeof(unsigned long long) * c.size(), hipMemcpyDeviceToHost, st));
+int engine_check_queues(Engine& E, hipStream_t st, bool* overflow, std::vector<unsigned long long>* counts, std::vector<int>* K) {
+    const size_t nK = 3 * E.h_meshes.size(), bytes = sizeof(unsigned long long) * N_COUNTERS + sizeof(int) * nK;
+    if (!E.h_sync) {
+        const size_t most = sizeof(unsigned long long) * N_COUNTERS + sizeof(int) * 3 * MAX_BATCH_MESHES;
+        I2_HIP(hipHostMalloc((void**)&E.h_sync, most, hipHostMallocDefault));
+    }
+    I2_HIP(hipMemcpyAsync(E.h_sync, E.d_counters.p, bytes, hipMemcpyDeviceToHost, st));
     I2_HIP(hipStreamSynchronize(st));
+    const unsigned long long* c = E.h_sync;
     *overflow = false;
     int64_t need[3] = {0, 0, 0};
     for (int L = 2; L <= E.args.last_level; ++L)
         for (int t = 0; t < 3; ++t) need[t] = std::max<int64_t>(need[t], (int64_t)c[1 + L * 3 + t]);
     for (int t = 0; t < 3; ++t)
         if (need[t] > E.args.qcap[t]) { *overflow = true; E.args.qcap[t] = need[t] + need[t] / 4 + 1; }
-    if (counts) *counts = c;
+    counts->assign(c, c + N_COUNTERS);
+    const int* k = reinterpret_cast<const int*>(c + N_COUNTERS);
+    K->assign(k, k + nK);
     return I2_OK;
 }
 
@@ -899,6 +959,7 @@ struct i2_batch {
     bool have_cfg = false;
     int out = i2::OUT_PER_PAIR;
     int P = 64, ppl = 13;
+    bool tuned = false;                  // the caller set the launch shape
     i2::Engine E;
     bool dirty = true;
     hipGraph_t graph = nullptr;
@@ -983,7 +1044,8 @@ static int batch_prepare(i2_batch* b) {
                 D.fin[t] = o.fin[t].p; D.prev[t] = o.prev[t].p; D.conv[t] = o.conv[t].p; D.res[t] = o.res[t].p;
             }
             I2_TRY(o.unconv.ensure((3 * mesh->nT + 7) / 8));
-            for (int t = 0; t < 3; ++t) D.unconv[t] = reinterpret_cast<uint8_t*>(o.unconv.p) + t * mesh->nT;
+            if (!b->cfg.fixed)
+                for (int t = 0; t < 3; ++t) D.unconv[t] = reinterpret_cast<uint8_t*>(o.unconv.p) + t * mesh->nT;
         } else {
             I2_TRY(o.rowacc.ensure(24 * mesh->nT));
             I2_TRY(o.rowout.ensure(4 * mesh->nT));
@@ -997,6 +1059,7 @@ static int batch_prepare(i2_batch* b) {
         }
         E.h_meshes[m] = D;
     }
+    if (!b->tuned) engine_auto_shape(E);
     I2_TRY(engine_setup(E, b->cfg));
     for (const i2_mesh* mesh : b->meshes) b->generations.push_back(mesh->generation);
     if (!b->adjoint) return I2_OK;
@@ -1009,22 +1072,12 @@ static int batch_prepare(i2_batch* b) {
         }
     }
     std::vector<AdjMesh> AD(M);
-    for (int m = 0; m < M; ++m) AD[m] = adjoint_mesh(b->meshes[m], E.h_meshes[m].conv, E.d_K.p + 3 * m);
+    for (int m = 0; m < M; ++m) AD[m] = adjoint_mesh(b->meshes[m], E.h_meshes[m].conv, E.args.K + 3 * m);
     return adjoint_setup(*b->adj, b->device, AD, b->meshes, &b->cfg, b->adj_seed);
 }
 
 static int batch_enqueue_all(i2_batch* b) {
     Engine& E = b->E;
-    if (E.out == OUT_PER_PAIR && !b->cfg.fixed)
-        for (auto& o : b->outs) {
-            hipLaunchKernelGGL(k_zero_u64, dim3(64), dim3(256), 0, b->stream, o.unconv.p, (int64_t)o.unconv.n);
-            I2_TRY(check_launch("k_zero_u64"));
-        }
-    if (E.out == OUT_ROW_SUMS)
-        for (auto& o : b->outs) {
-            hipLaunchKernelGGL(k_zero_f64, dim3(1024), dim3(256), 0, b->stream, o.rowacc.p, (int64_t)o.rowacc.n);
-            I2_TRY(check_launch("k_zero_f64"));
-        }
     I2_TRY(batch_enqueue(E, b->stream));
     if (b->adjoint) I2_TRY(adjoint_launch(*b->adj, b->stream));
     return I2_OK;
@@ -1069,7 +1122,7 @@ static int batch_run(i2_batch* b, double* ms) {
         }
         I2_HIP(hipEventRecord(b->e1, b->stream));
         bool overflow = false;
-        I2_TRY(engine_check_queues(b->E, b->stream, &overflow, &b->counts));
+        I2_TRY(engine_check_queues(b->E, b->stream, &overflow, &b->counts, &b->K));
         if (!overflow) {
             float f = 0.f;
             I2_HIP(hipEventElapsedTime(&f, b->e0, b->e1));
@@ -1079,8 +1132,6 @@ static int batch_run(i2_batch* b, double* ms) {
                 I2_HIP(hipEventElapsedTime(&g, b->E.prof0, b->E.prof1));
                 b->sweep_ms = g;
             }
-            b->K.resize(3 * b->meshes.size());
-            I2_HIP(hipMemcpy(b->K.data(), b->E.d_K.p, sizeof(int) * b->K.size(), hipMemcpyDeviceToHost));
             b->ran = true;
             return I2_OK;
         }
@@ -1114,7 +1165,12 @@ int engine_run_evaluator(i2_evaluator* ev) {
         b->have_cfg = true;
         b->dirty = true;
     }
-    if (b->P != ev->fast_P || b->ppl != ev->fast_ppl) { b->P = ev->fast_P; b->ppl = ev->fast_ppl; b->dirty = true; }
+    if (b->P != ev->fast_P || b->ppl != ev->fast_ppl || b->tuned != ev->fast_tuned) {
+        b->P = ev->fast_P;
+        b->ppl = ev->fast_ppl;
+        b->tuned = ev->fast_tuned;
+        b->dirty = true;
+    }
     b->out = OUT_PER_PAIR;
     b->profile = ev->profile;
     double ms = 0.0;
@@ -1150,6 +1206,7 @@ void engine_release_evaluator(i2_evaluator* ev) {
     drop_graph(b);
     if (b->E.prof0) (void)hipEventDestroy(b->E.prof0);
     if (b->E.prof1) (void)hipEventDestroy(b->E.prof1);
+    if (b->E.h_sync) (void)hipHostFree(b->E.h_sync);
     if (b->e0) (void)hipEventDestroy(b->e0);
     if (b->e1) (void)hipEventDestroy(b->e1);
     b->stream = nullptr;   // owned by the evaluator
@@ -1194,6 +1251,7 @@ void i2_batch_destroy(i2_batch* b) {
         adjoint_release(b->adj);
         if (b->E.prof0) (void)hipEventDestroy(b->E.prof0);
         if (b->E.prof1) (void)hipEventDestroy(b->E.prof1);
+        if (b->E.h_sync) (void)hipHostFree(b->E.h_sync);
         if (b->e0) (void)hipEventDestroy(b->e0);
         if (b->e1) (void)hipEventDestroy(b->e1);
         if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -1240,6 +1298,7 @@ int i2_batch_set_tuning(i2_batch* b, int pairsPerWorkgroup, int pointsPerLane) {
     if (pointsPerLane != 1 && pointsPerLane != 2 && pointsPerLane != 4 && pointsPerLane != 13) { set_error("points per lane must be 1, 2, 4 or 13"); return I2_ERR_INVALID; }
     b->P = pairsPerWorkgroup;
     b->ppl = pointsPerLane;
+    b->tuned = true;
     b->dirty = true;
     return I2_OK;
 }

@@ -46,6 +46,8 @@ static_assert(sizeof(QEntry) == 64, "queue entries are 64 bytes");
 constexpr int MAX_BATCH_MESHES = 256;
 constexpr int MASK_WORDS = MAX_BATCH_MESHES / 64;
 
+constexpr int N_COUNTERS = 2 + MAX_LEVELS * 3;
+
 struct BatchArgs {
     const MeshDesc* meshes;
     int nmeshes;
@@ -66,8 +68,7 @@ struct BatchArgs {
     const int64_t* pair_base;
     const int64_t* row_base;
     int64_t total_rows;
-    // counters: [0] disjoint item counter, [1 + level*3 + type] queue counts,
-    // [1 + MAX_LEVELS*3] singular item counter
+    // counters: [0] disjoint item counter, [1 + level*3 + type] queue counts
     unsigned long long* counters;
     QEntry* queue;                // segment (level, type) at qoff[level*3 + type], capacity qcap[type]
     const int64_t* qoff;
@@ -94,7 +95,7 @@ struct Engine {
     DBuf<unsigned long long> d_counters;
     DBuf<QEntry> d_queue;
     DBuf<unsigned long long> d_levelmask;
-    DBuf<int> d_K;
+    unsigned long long* h_sync = nullptr;   // pinned: counters and K of a run
     int64_t total_tasks = 0;
     // profiling: events around the disjoint sweep (non-captured runs only)
     hipEvent_t prof0 = nullptr, prof1 = nullptr;
@@ -106,10 +107,10 @@ int batch_enqueue(Engine& E, hipStream_t stream);
 // Builds device descriptors and work queues for the meshes in E.h_meshes
 // (outputs already set) with the rule and error control of `it`.
 int engine_setup(Engine& E, const i2_integrator& it);
-// After a run: queue counts per (level, type); returns I2_ERR_RANGE-free
-// status and sets *overflow when a queue segment was too small (the queues are
-// then grown and the caller must run again).
-int engine_check_queues(Engine& E, hipStream_t stream, bool* overflow, std::vector<unsigned long long>* counts);
+// After a run: queue counts per (level, type) and K per (mesh, type); returns
+// I2_ERR_RANGE-free status and sets *overflow when a queue segment was too
+// small (the queues are then grown and the caller must run again).
+int engine_check_queues(Engine& E, hipStream_t stream, bool* overflow, std::vector<unsigned long long>* counts, std::vector<int>* K);
 // Runs an evaluator's mesh through the batched kernels (per-pair outputs).
 int engine_run_evaluator(i2_evaluator* ev);
 void engine_release_evaluator(i2_evaluator* ev);

@@ -192,15 +192,10 @@ I2_HD __forceinline__ bool edge_gap(d3 u, d3 v, double lu, double lv, double L, 
     e = 2.0 * c2 / (fma(lu, lv, -dot(u, v)) * n);
     return c2 < EPS_PSI_THETA2 * (L * L) * (lv * lv);
 }
-// Theta/2 = atan2(y, x) for any arguments: the table path, then the lanes
-// outside its range (zero, NaN, lengths near the ends of the exponent range)
+// atan2(y, x) for any arguments: the table path, then the lanes outside its range
 I2_HD __forceinline__ double atan2_terms(double y, double x, const i2m::MathTable* __restrict__ lt) {
     double h = i2m::atan2_any(y, x, lt);
-    if (__builtin_expect(!i2m::atan2_in_range(y, x), 0)) {
-        const double sum = fabs(x) + fabs(y), k = sum < 1.0 ? 0x1p600 : 0x1p-600;
-        h = sum == 0.0 ? 0.0 : i2m::atan2_any(y * k, x * k, lt);
-        if (!(sum <= 1.7976931348623157e308)) h = sum - sum;
-    }
+    if (__builtin_expect(!i2m::atan2_in_range(y, x), 0)) h = i2m::atan2_rare(y, x, lt);
     return h;
 }
 // Terms of one point: line integrals t along A->B, B->C, C->A (the edges of
@@ -356,11 +351,11 @@ I2_HD __forceinline__ q4 sing_edge_fast(d3 p, const EdgeCtx& c, const i2m::MathT
     double g1 = i2m::atan2_any(y1, x1, lt);
     double g2 = i2m::atan2_any(y2, x2, lt);
     if (__builtin_expect(!(o1 & o2 & o3 & o4 & o5), 0)) {
-        if (!o1) l1 = i2m::log_slow(a1);
-        if (!o2) l2 = i2m::log_slow(a2);
-        if (!o3) l3 = i2m::log_slow(a3);
-        if (!o4) g1 = i2m::atan2_slow(y1, x1);
-        if (!o5) g2 = i2m::atan2_slow(y2, x2);
+        if (!o1) l1 = i2m::log_rare(a1, lt);
+        if (!o2) l2 = i2m::log_rare(a2, lt);
+        if (!o3) l3 = i2m::log_rare(a3, lt);
+        if (!o4) g1 = i2m::atan2_rare(y1, x1, lt);
+        if (!o5) g2 = i2m::atan2_rare(y2, x2, lt);
     }
     q4 r;
     r.x = l1 * c.tauc.x - l2 * c.taub.x - l3 * c.taua.x;
@@ -443,10 +438,10 @@ I2_HD __forceinline__ q4 sing_vertex_fast(d3 p, const VertexCtx& c, const i2m::M
     double g1 = i2m::atan2_any(y1, x1, lt);
     double g2 = i2m::atan2_any(y2, x2, lt);
     if (__builtin_expect(!(o1 & o2 & o3 & o4), 0)) {
-        if (!o1) la = i2m::log_slow(a1);
-        if (!o2) lb = i2m::log_slow(a2);
-        if (!o3) g1 = i2m::atan2_slow(y1, x1);
-        if (!o4) g2 = i2m::atan2_slow(y2, x2);
+        if (!o1) la = i2m::log_rare(a1, lt);
+        if (!o2) lb = i2m::log_rare(a2, lt);
+        if (!o3) g1 = i2m::atan2_rare(y1, x1, lt);
+        if (!o4) g2 = i2m::atan2_rare(y2, x2, lt);
     }
     q4 r;
     r.x = -(la * c.taua.x + lb * c.taub.x);
@@ -458,7 +453,13 @@ I2_HD __forceinline__ q4 sing_vertex_fast(d3 p, const VertexCtx& c, const i2m::M
 
 // ------------------------------------------------------------ topology of a pair
 I2_HD __forceinline__ int vid(const Panel& P, int k) { return k == 0 ? P.v0 : (k == 1 ? P.v1 : P.v2); }
-I2_HD __forceinline__ d3 vtx(const Panel& P, int k) { return k == 0 ? P.a : (k == 1 ? P.b : P.c); }
+// a, b or c by a run-time index, as selects between values: passed by value,
+// because a conditional between members of a record selects an address, and
+// the whole record then lives in scratch memory
+I2_HD __forceinline__ d3 pick(d3 a, d3 b, d3 c, int k) {
+    return {k == 0 ? +a.x : (k == 1 ? +b.x : +c.x), k == 0 ? +a.y : (k == 1 ? +b.y : +c.y), k == 0 ? +a.z : (k == 1 ? +b.z : +c.z)};
+}
+I2_HD __forceinline__ d3 vtx(const Panel& P, int k) { return pick(P.a, P.b, P.c, k); }
 // number of shared vertex indices (src/Mesh3d.cu:111-122)
 I2_HD __forceinline__ int shared_count(const Panel& I, const Panel& J) {
     int c = 0;
@@ -717,6 +718,35 @@ I2_HD __forceinline__ void sub_panel(d3& a, d3& b, d3& c, int level, uint32_t pa
         else if (ch == 2) { b = a; a = mCA; c = mAB; }
         else { a = mBC; b = mCA; c = mAB; }
     }
+}
+
+// A rule's point on a sub-panel, barycentric on the original panel, with its
+// weight: 32-byte records that the kernels keep in LDS for levels 0 and 1
+// (the rule's points on the panel, then on its four level-1 children).
+struct alignas(32) BaryPoint { double b0, b1, b2, w; };
+// vertices of level-1 child `ch` in those coordinates (sub_panel's children)
+I2_HD __forceinline__ void child_bary(int ch, d3& ba, d3& bb, d3& bc) {
+    const d3 A = {1.0, 0.0, 0.0}, B = {0.0, 1.0, 0.0}, C = {0.0, 0.0, 1.0};
+    const d3 mAB = {0.5, 0.5, 0.0}, mBC = {0.0, 0.5, 0.5}, mCA = {0.5, 0.0, 0.5};
+    if (ch == 0) { ba = mAB; bb = B; bc = mBC; }
+    else if (ch == 1) { ba = mBC; bb = C; bc = mCA; }
+    else if (ch == 2) { ba = mCA; bb = A; bc = mAB; }
+    else { ba = mBC; bb = mCA; bc = mAB; }
+}
+// record t of the 5 npts of a rule given as barycentric arrays and weights
+I2_HD __forceinline__ BaryPoint bary_point(const double* L1, const double* L2, const double* L3, const double* w, int npts, int t) {
+    const int sub = t / npts, k = t - sub * npts;
+    d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
+    if (sub > 0) child_bary(sub - 1, ba, bb, bc);
+    d3 b = L1[k] * ba;
+    b = b + L2[k] * bb;
+    b = b + L3[k] * bc;
+    return {b.x, b.y, b.z, w[k]};
+}
+I2_HD __forceinline__ d3 at_bary(const BaryPoint& Q, d3 a, d3 b, d3 c) {
+    d3 p = Q.b0 * a;
+    p = p + Q.b1 * b;
+    return p + Q.b2 * c;
 }
 
 }  // namespace i2d

@@ -670,6 +670,7 @@ int i2_evaluator_set_tuning(i2_evaluator* ev, int pairsPerWorkgroup, int pointsP
     }
     ev->fast_P = pairsPerWorkgroup;
     ev->fast_ppl = pointsPerLane;
+    ev->fast_tuned = true;
     return I2_OK;
 }
 

@@ -215,6 +215,16 @@ I2_HD __forceinline__ double log_tab_any(double x, const MathTable* __restrict__
     return fma(dk, LN2_HI, tab->thi[j]) + (fma(dk, LN2_LO, tab->tlo[j]) + p);
 }
 
+// log of an argument that is not positive normal: -inf at 0, NaN below,
+// infinity and NaN themselves, subnormals scaled into the table's range.  Inline,
+// so that the quadrature kernels make no calls (a call reserves the callee's
+// registers and a stack frame in every kernel that contains it).
+I2_HD __forceinline__ double log_rare(double x, const MathTable* __restrict__ tab) {
+    const double t = log_tab_any(x * 0x1p54, tab) - 54.0 * 0.69314718055994530942;
+    const double big = x + x;                                  // infinity or NaN
+    return x > 0.0 ? (x <= 1.7976931348623157e308 ? t : big) : (x == 0.0 ? -HUGE_VAL : (x - x) / 0.0);
+}
+
 I2_HD __forceinline__ double log_tab(double x, const MathTable* __restrict__ tab) {
     if (!pos_normal(x)) return log_slow(x);
     return log_tab_any(x, tab);
@@ -276,6 +286,17 @@ I2_HD __forceinline__ double atan_over(double v) {
     q = fma_k(q, v, 0.19999999999939544);
     q = fma_k(q, v, -0.3333333333333333);
     return fma(q, v, 1.0);
+}
+
+// atan2 outside atan2_in_range: (0, 0) by the signs, magnitudes near the ends
+// of the exponent range scaled into the table path's, NaN for infinite and
+// NaN arguments (no panel has them without NaN elsewhere)
+I2_HD __forceinline__ double atan2_rare(double y, double x, const MathTable* __restrict__ tab) {
+    const double sum = fabs(x) + fabs(y), k = sum < 1.0 ? 0x1p600 : 0x1p-600;
+    double h = atan2_any(y * k, x * k, tab);
+    if (sum == 0.0) h = copysign(copysign(1.0, x) < 0.0 ? PI_HI : 0.0, y);
+    if (!(sum <= 1.7976931348623157e308)) h = sum - sum;
+    return h;
 }
 
 I2_HD __forceinline__ double atan2_fast(double y, double x, const MathTable* __restrict__ tab) {
