@@ -308,6 +308,17 @@ __device__ __forceinline__ StepOut sweep_check(const BatchArgs& A, int m, int i,
     return o;
 }
 
+// A row's sums of the wavefront's lanes (or the whole smaller workgroup's), one
+// set of atomics; the lanes' shares are cleared.
+__device__ __forceinline__ void flush_row(const MeshDesc& M, int type, int i, q4& acc0, q4& acc1) {
+    const int W = blockDim.x < 64 ? (int)blockDim.x : 64;
+    acc0 = shfl_sum(acc0, W);
+    acc1 = shfl_sum(acc1, W);
+    if ((threadIdx.x & (W - 1)) == 0) add_row(M, type, i, acc0, acc1);
+    acc0 = q4zero();
+    acc1 = q4zero();
+}
+
 // Levels 0 and 1 of one disjoint task (lane group of LPP lanes), then the Runge check.
 template <int LPP>
 __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS& R, int m, int i, int j, int64_t z, bool valid,
@@ -340,51 +351,64 @@ __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS&
 }
 
 // Disjoint pairs, levels 0 and 1: item = (mesh, control panel i, P consecutive j),
-// processed in rounds of blockDim/LPP pairs.
+// processed in rounds of blockDim/LPP pairs.  A workgroup claims A.sweep_chunk
+// consecutive items at a time (the first by its number, without an atomic):
+// claims of single items queue on one address, 129 against 92 us for 320
+// panels at 4 lanes per pair and 3 % for 5,120 at one.  Consecutive items
+// mostly share the control panel, whose points and row sums are then kept from
+// one to the next.
 template <int OUT, int LPP>
 __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs A) {
     __shared__ struct { PtsLDS pts; RuleLDS R; } S;
     RuleLDS& R = S.R;
     PtsLDS& pts = S.pts;
-    __shared__ long long item_sh;
+    __shared__ long long chunk_sh;
     load_rule(R, A.rule);
     const int P = A.pairs_per_item;
     const int per_round = blockDim.x / LPP;
     const int p0 = threadIdx.x / LPP, s = threadIdx.x % LPP;
-    for (;;) {
-        __syncthreads();
-        if (threadIdx.x == 0) item_sh = (long long)atomicAdd(&A.counters[0], 1ull);
-        __syncthreads();
-        const int64_t item = uniform64(item_sh);
-        if (item >= A.disjoint_items) break;
-        const int m = __builtin_amdgcn_readfirstlane(find_base(A.item_base, A.nmeshes, item));
-        const MeshDesc& M = A.meshes[m];
-        const int64_t r = item - A.item_base[m];
-        const int tiles = (M.nT + P - 1) / P;
-        const int i = __builtin_amdgcn_readfirstlane((int)(r / tiles));
-        const Panel I = M.panels[i];
-        const Ball ball = panel_ball(I.a, I.b, I.c, A.rule.reach);
-        load_points(pts, R, A.rule.n, I);
-        __syncthreads();
-        for (int round = 0; round < P; round += per_round) {
-        const int p = round + p0;
-        const int j = (int)(r % tiles) * P + p;
-        const bool in_range = p < P && j < M.nT;
-        const Panel J = M.panels[in_range ? j : i];
-        const bool valid = in_range && j != i && shared_count(I, J) == 0;
-        const int64_t z = valid ? disjoint_task(M, i, j) : 0;
-        const StepOut o = sweep_task<LPP>(A, R, m, i, j, z, valid, s, I, J, pts, ball);
-        q4 rp0 = q4zero(), rp1 = q4zero();
-        if (o.finished) finish_task<I2_NOT_NEIGHBORS, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
-        if (OUT == OUT_ROW_SUMS) {
-            // i is uniform: reduce over the wavefront (or the whole smaller
-            // workgroup), one set of atomics per wavefront
-            const int W = blockDim.x < 64 ? (int)blockDim.x : 64;
-            rp0 = shfl_sum(rp0, W);
-            rp1 = shfl_sum(rp1, W);
-            if ((threadIdx.x & (W - 1)) == 0) add_row(M, I2_NOT_NEIGHBORS, i, rp0, rp1);
+    const int64_t chunks = (A.disjoint_items + A.sweep_chunk - 1) / A.sweep_chunk;
+    for (int64_t chunk = blockIdx.x; chunk < chunks;) {
+        const int64_t first = chunk * A.sweep_chunk, last = min(first + A.sweep_chunk, A.disjoint_items);
+        int m = __builtin_amdgcn_readfirstlane(find_base(A.item_base, A.nmeshes, first));
+        int i = -1, i_mesh = -1;
+        q4 acc0 = q4zero(), acc1 = q4zero();   // this lane's share of row i's sums, for both parities of K
+        for (int64_t item = first; item < last; ++item) {
+            while (m + 1 < A.nmeshes && item >= A.item_base[m + 1]) ++m;
+            const MeshDesc& M = A.meshes[m];
+            const int64_t r = item - A.item_base[m];
+            const int tiles = (M.nT + P - 1) / P;
+            const int row = __builtin_amdgcn_readfirstlane((int)(r / tiles));
+            const int tile = (int)(r - (int64_t)row * tiles);
+            const Panel I = M.panels[row];
+            if (row != i || m != i_mesh) {
+                if (OUT == OUT_ROW_SUMS && i >= 0) flush_row(A.meshes[i_mesh], I2_NOT_NEIGHBORS, i, acc0, acc1);
+                i = row;
+                i_mesh = m;
+                __syncthreads();
+                load_points(pts, R, A.rule.n, I);
+                __syncthreads();
+            }
+            const Ball ball = panel_ball(I.a, I.b, I.c, A.rule.reach);
+            for (int round = 0; round < P; round += per_round) {
+                const int p = round + p0;
+                const int j = tile * P + p;
+                const bool in_range = p < P && j < M.nT;
+                const Panel J = M.panels[in_range ? j : i];
+                const bool valid = in_range && j != i && shared_count(I, J) == 0;
+                const int64_t z = valid ? disjoint_task(M, i, j) : 0;
+                const StepOut o = sweep_task<LPP>(A, R, m, i, j, z, valid, s, I, J, pts, ball);
+                q4 rp0 = q4zero(), rp1 = q4zero();
+                if (o.finished) finish_task<I2_NOT_NEIGHBORS, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
+                if (OUT == OUT_ROW_SUMS) { acc0 = acc0 + rp0; acc1 = acc1 + rp1; }
+            }
         }
-        }
+        if (OUT == OUT_ROW_SUMS) flush_row(A.meshes[i_mesh], I2_NOT_NEIGHBORS, i, acc0, acc1);
+        if (chunks <= (int64_t)gridDim.x) break;
+        __syncthreads();
+        if (threadIdx.x == 0) chunk_sh = (long long)gridDim.x + (long long)atomicAdd(&A.counters[0], 1ull);
+        __syncthreads();
+        chunk = uniform64(chunk_sh);
     }
 }
 
@@ -824,13 +848,15 @@ int batch_enqueue(Engine& E, hipStream_t st) {
     return I2_OK;
 }
 
-// Launch shape for a caller who has set none: one lane per pair where that
-// makes enough wavefronts (3,072 in flight, three per SIMD), else several
-// lanes per pair.
+// Launch shape for a caller who has set none: one lane per pair, or four while
+// that leaves most SIMDs without a wavefront (1,024 SIMDs).  Row sums by shape,
+// one / four lanes: 80 panels (160 wavefronts) 220 / 196 us, 320 panels (1,600)
+// 295 / 312, 1,280 panels 840 / 1,090; eight and sixteen lanes are slower than
+// four on all three.
 void engine_auto_shape(Engine& E) {
     int64_t waves = 0;
     for (const MeshDesc& D : E.h_meshes) waves += (int64_t)D.nT * ((D.nT + 63) / 64);
-    E.ppl = waves >= 6144 ? 13 : (waves >= 768 ? 4 : 1);
+    E.ppl = waves >= 512 ? 13 : 4;
     E.pairs_per_wg = 64 / lanes_for_points_per_lane(E.ppl);
 }
 
@@ -861,6 +887,10 @@ int engine_setup(Engine& E, const i2_integrator& it) {
     }
     E.h_item_base[M] = acc;
     A.disjoint_items = acc;
+    // items per claim: some 32 claims per workgroup, at most 64 items each;
+    // without claims where every workgroup has a few items at most
+    A.sweep_chunk = acc <= 4 * (int64_t)E.sweep_grid ? std::max<int64_t>(1, (acc + E.sweep_grid - 1) / E.sweep_grid)
+                                                     : std::max<int64_t>(1, std::min<int64_t>(64, acc / (32 * (int64_t)E.sweep_grid)));
     acc = 0;
     for (int kind = 0; kind < 2; ++kind)
         for (int m = 0; m < M; ++m) {

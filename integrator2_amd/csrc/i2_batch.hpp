@@ -62,13 +62,14 @@ struct BatchArgs {
     const int64_t* item_base;
     const int64_t* sing_base;
     int64_t disjoint_items;
+    int64_t sweep_chunk;          // consecutive disjoint items per claim
     int64_t singular_items;
     // per-pair finalize ranges: pair_base[3 * m + type]; disjoint rows of all
     // meshes: row_base[m] (nmeshes + 1)
     const int64_t* pair_base;
     const int64_t* row_base;
     int64_t total_rows;
-    // counters: [0] disjoint item counter, [1 + level*3 + type] queue counts
+    // counters: [0] disjoint chunk counter, [1 + level*3 + type] queue counts
     unsigned long long* counters;
     QEntry* queue;                // segment (level, type) at qoff[level*3 + type], capacity qcap[type]
     const int64_t* qoff;
