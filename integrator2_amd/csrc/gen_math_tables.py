@@ -58,3 +58,5 @@ def interpolant(f, top, n):
 
 print("atanh_over", interpolant(lambda s: mpmath.atanh(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf(1) / 16, 8))
 print("atan_over", interpolant(lambda s: mpmath.atan(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf("0.003"), 5))
+print("atanh_over, distant", interpolant(lambda s: mpmath.atanh(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf(1) / 144, 5))
+print("atan_over, distant", interpolant(lambda s: mpmath.atan(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf("3.7e-5"), 3))

@@ -162,8 +162,12 @@ __device__ __forceinline__ void panel_chain(const Panel& P, d3 tab, d3 tbb, d3 t
     Bb = Bb + gu; Cb = Cb + gv; Ab = Ab - gu - gv;
 }
 
-__device__ __forceinline__ void load_bary(BaryPoint* P, const RuleSh& R, int npts) {
-    for (int t = threadIdx.x; t < 5 * npts; t += blockDim.x) P[t] = bary_point(R.L1, R.L2, R.L3, R.w, npts, t);
+__device__ __forceinline__ void load_bary(BaryPoint* P, FarPoint* F, const RuleSh& R, int npts) {
+    for (int t = threadIdx.x; t < 5 * npts; t += blockDim.x) {
+        const BaryPoint Q = bary_point(R.L1, R.L2, R.L3, R.w, npts, t);
+        P[t] = Q;
+        F[t] = far_point(Q.b0 - 1.0 / 3.0, Q.b1 - 1.0 / 3.0, Q.w);
+    }
 }
 
 // Sums of nine values over the wavefront, in a fixed order: pairs of registers
@@ -209,16 +213,23 @@ constexpr int ADJ_BLOCK = 256;
 // panels j per disjoint item at most (one bit of a lane's mask each)
 constexpr int ADJ_TILE = 32;
 
-// Reverse mode over the points k0 <= k < k1 of one pair.
-template <bool FAR>
+// Reverse mode over the points k0 <= k < k1 of one pair: the general form, and
+// the far one's scalar sums.
 __device__ __forceinline__ void points_rev(const RuleSh& R, const BaryPoint* pts, int k0, int k1, const Panel& I, const JGeom& JG,
                                            const q4& ct, TermsBar& g, d3& X0, d3& X1) {
     for (int k = k0; k < k1; ++k) {
         const BaryPoint Q = pts[k];
         const d3 p = at_bary(Q, I.a, I.b, I.c);
-        const d3 pb = theta_terms_rev<FAR>(p, JG, &R.lt, Q.w, ct, g);
+        const d3 pb = theta_terms_rev(p, JG, &R.lt, Q.w, ct, g);
         axpy(X0, Q.b0, pb); axpy(X1, Q.b1, pb);
     }
+}
+template <bool DISTANT>
+__device__ __forceinline__ void points_far_rev(const FarPoint* pts, int npts, bool act0, bool act1, const FarFrame& F,
+                                               const FarGeom& G, const JGeom& JG, const q4& ct, FarBar& f) {
+    // the pairs at reported level 0, then those at level 1
+    if (act0) for (int k = 0; k < npts; ++k) theta_terms_far_rev<DISTANT>(pts[k], F, G, JG, ct, f);
+    if (act1) for (int k = npts; k < 5 * npts; ++k) theta_terms_far_rev<DISTANT>(pts[k], F, G, JG, ct, f);
 }
 
 // One wavefront per workgroup: an item is a wavefront of 64 control panels i
@@ -226,12 +237,13 @@ __device__ __forceinline__ void points_rev(const RuleSh& R, const BaryPoint* pts
 __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
     __shared__ RuleSh R;
     __shared__ BaryPoint pts[5 * MAX_POINTS];
+    __shared__ FarPoint fpts[5 * MAX_POINTS];
     __shared__ long long item_sh;
     load_rule_sh(R, A.rule);
     __syncthreads();
     const int lane = threadIdx.x;
     const int npts = A.rule.n;
-    load_bary(pts, R, npts);
+    load_bary(pts, fpts, R, npts);
     for (;;) {
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -275,15 +287,24 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
             const d3 gP = {gb.x, gb.y, gb.z};
             const double fa = lev == 1 ? 0.25 * I.area : I.area;
             const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
-            const bool near = __ballot(valid && !panel_far(ball, JG)) != 0ull;
+            const int form = wave_form(valid, ball, JG);
             TermsBar g = terms_bar_zero();
-            for (int lv = 0; lv < 2; ++lv) {          // the pairs at reported level 0, then those at level 1
-                const bool act = valid && lev == lv;
-                if (__ballot(act) == 0ull) continue;
-                if (!act) continue;
-                const int k0 = lv == 0 ? 0 : npts, k1 = lv == 0 ? npts : 5 * npts;
-                if (near) points_rev<false>(R, pts, k0, k1, I, JG, ct, g, X0, X1);
-                else points_rev<true>(R, pts, k0, k1, I, JG, ct, g, X0, X1);
+            if (form == 0) {
+                for (int lv = 0; lv < 2; ++lv) {      // the pairs at reported level 0, then those at level 1
+                    const bool act = valid && lev == lv;
+                    if (__ballot(act) == 0ull) continue;
+                    if (!act) continue;
+                    points_rev(R, pts, lv == 0 ? 0 : npts, lv == 0 ? npts : 5 * npts, I, JG, ct, g, X0, X1);
+                }
+            } else {
+                const FarFrame F = far_frame(I.a, I.b, I.c);
+                FarBar f = far_bar_zero();
+                {
+                    const FarGeom G = far_geom(F, JG);
+                    if (form == 1) points_far_rev<false>(fpts, npts, valid && lev == 0, valid && lev == 1, F, G, JG, ct, f);
+                    else points_far_rev<true>(fpts, npts, valid && lev == 0, valid && lev == 1, F, G, JG, ct, f);
+                }
+                far_bar_expand(f, F, JG, g, X0, X1);
             }
             d3 nb = {0.0, 0.0, 0.0};
             if (valid) {
@@ -372,7 +393,7 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
             d3 p = beta.x * I.a;
             p = p + beta.y * I.b;
             p = p + beta.z * I.c;
-            const d3 pb = theta_terms_rev<false>(p, JG, &R.lt, R.w[k], ct, g);
+            const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
             axpy(X0, beta.x, pb); axpy(X1, beta.y, pb);
         }
     }
@@ -1094,12 +1115,25 @@ int i2_host_point_adjoint(int kind, const double* p3, const double* params, cons
         VertexBar g = {z3, z3, z3, z3, 0.0};
         f = sing_vertex_rev(p, c, gb, &pb, g);
         put(0, g.JA); put(3, g.taua); put(6, g.taub); put(9, g.e); parbar[12] = g.invAri;
-    } else if (kind == 3 || kind == 4) {
+    } else if (kind >= 3 && kind <= 5) {
         const d3 A = v(0), B = v(3), C = v(6), cr = cross(B - A, C - A);
         const JGeom J = make_jgeom(A, B, C, unit(C - B), unit(A - C), unit(B - A));
         TermsBar g = terms_bar_zero();
-        pb = kind == 4 ? theta_terms_rev<true>(p, J, &i2m::h_mathtab, 1.0, gb, g)
-                       : theta_terms_rev<false>(p, J, &i2m::h_mathtab, 1.0, gb, g);
+        if (kind == 3) {
+            pb = theta_terms_rev(p, J, &i2m::h_mathtab, 1.0, gb, g);
+        } else {   // p as a point of a control panel of K_j's size and shape
+            const FarPoint Q = far_point(0.3, -0.2, 1.0);
+            const d3 o = p - ((Q.b0 + 1.0 / 3.0) * A + (Q.b1 + 1.0 / 3.0) * B + (1.0 / 3.0 - Q.b0 - Q.b1) * C);
+            const FarFrame F = far_frame(A + o, B + o, C + o);
+            const FarGeom G = far_geom(F, J);
+            FarBar fb = far_bar_zero();
+            if (kind == 4) theta_terms_far_rev<false>(Q, F, G, J, gb, fb);
+            else theta_terms_far_rev<true>(Q, F, G, J, gb, fb);
+            d3 X0 = z3, X1 = z3;
+            far_bar_expand(fb, F, J, g, X0, X1);
+            pb = g.a + g.b + g.c;
+            axpy(pb, g.y, J.N2);
+        }
         f = g.T;
         g.T = q4zero();
         d3 ab, bb, cb;

@@ -127,8 +127,8 @@ I2_HD __forceinline__ q4 theta_psi_fast_rev(d3 p, const JGeom& J, const i2m::Mat
     return r;
 }
 
-// Reverse mode of the terms of the inner integral (theta_terms, or with FAR
-// theta_terms_far times its factors): with P = (S - L)(S + L) per edge,
+// Reverse mode of the terms of the inner integral (theta_terms): with P = (S -
+// L)(S + L) per edge,
 //   t = ln((S + L)/(S - L)):  dt = (2 S dL - 2 L dS)/P,
 //   Theta/2 = h = atan2(Y, X), X = 2 x = P_c lc + P_a la + P_b lb - 4 la lb lc
 //   and Y = 2 da.N2:  X^2 + Y^2 = P_c P_a P_b (for unit vectors |1 + a.b + b.c +
@@ -147,7 +147,6 @@ I2_HD __forceinline__ TermsBar terms_bar_zero() {
 }
 // One point of weight w, with the cotangents ct of the weighted terms; returns
 // the point's cotangent.
-template <bool FAR>
 I2_HD __forceinline__ d3 theta_terms_rev(d3 p, const JGeom& J, const i2m::MathTable* __restrict__ lt, double w, const q4& ct,
                                          TermsBar& g) {
     const d3 da = p - J.a, db = p - J.b, dc = p - J.c;
@@ -157,69 +156,117 @@ I2_HD __forceinline__ d3 theta_terms_rev(d3 p, const JGeom& J, const i2m::MathTa
     const double S1 = la + lb, S2 = lb + lc, S3 = lc + la;
     const double c1 = w * ct.x, c2 = w * ct.y, c3 = w * ct.z, ch = w * ct.w;
     const double Y = 2.0 * dot(da, J.N2);
-    double P1, P2, P3, X, t1, t2, t3, h, R, iP1, iP2, iP3;
     double xa = 0.0, xb = 0.0, xc = 0.0;           // dL/dl of terms in the degenerate branch
     double m1 = c1, m2 = c2, m3 = c3;
-    if (FAR) {
-        P1 = fma(S1, S1, -(J.Lc * J.Lc)); P2 = fma(S2, S2, -(J.La * J.La)); P3 = fma(S3, S3, -(J.Lb * J.Lb));
-        X = fma(fma(la * lb, -4.0, P1), lc, fma(P2, la, P3 * lb));
-        const double s12 = S1 * S2, s3x = S3 * X;
-        const double inv = i2m::rcp_cubic(s12 * s3x);
-        const double i12 = inv * s3x, i3x = inv * s12;
-        const double z1 = J.Lc * (i12 * S2), z2 = J.La * (i12 * S1), z3 = J.Lb * (i3x * X), u = Y * (i3x * S3);
-        t1 = 2.0 * z1 * i2m::atanh_over(z1 * z1);
-        t2 = 2.0 * z2 * i2m::atanh_over(z2 * z2);
-        t3 = 2.0 * z3 * i2m::atanh_over(z3 * z3);
-        h = u * i2m::atan_over(u * u);
-        const double P12 = P1 * P2;
-        R = i2m::rcp_cubic(P12 * P3);
-        const double R3 = R * P3;
-        iP1 = R3 * P2; iP2 = R3 * P1; iP3 = R * P12;
-    } else {
-        const double n1 = S1 + J.Lc, n2 = S2 + J.La, n3 = S3 + J.Lb;
-        double e1 = S1 - J.Lc, e2 = S2 - J.La, e3 = S3 - J.Lb;
-        double r1 = 0.0, r2 = 0.0, r3 = 0.0;        // ratios of terms in the degenerate branch
-        const double s = 0x1p-10;
-        if (__builtin_expect(fmin(fmin(fma(-s, S1, e1), fma(-s, S2, e2)), fma(-s, S3, e3)) < 0.0, 0)) {
-            if (e1 < s * S1) {
-                if (edge_gap(da, db, la, lb, J.Lc, n1, e1)) { r1 = lb / la; xb += c1 / lb; xa -= c1 / la; m1 = 0.0; }
-            }
-            if (e2 < s * S2) {
-                if (edge_gap(db, dc, lb, lc, J.La, n2, e2)) { r2 = lc / lb; xc += c2 / lc; xb -= c2 / lb; m2 = 0.0; }
-            }
-            if (e3 < s * S3) {
-                if (edge_gap(dc, da, lc, la, J.Lb, n3, e3)) { r3 = la / lc; xa += c3 / la; xc -= c3 / lc; m3 = 0.0; }
-            }
+    const double n1 = S1 + J.Lc, n2 = S2 + J.La, n3 = S3 + J.Lb;
+    double e1 = S1 - J.Lc, e2 = S2 - J.La, e3 = S3 - J.Lb;
+    double r1 = 0.0, r2 = 0.0, r3 = 0.0;            // ratios of terms in the degenerate branch
+    const double s = 0x1p-10;
+    if (__builtin_expect(fmin(fmin(fma(-s, S1, e1), fma(-s, S2, e2)), fma(-s, S3, e3)) < 0.0, 0)) {
+        if (e1 < s * S1) {
+            if (edge_gap(da, db, la, lb, J.Lc, n1, e1)) { r1 = lb / la; xb += c1 / lb; xa -= c1 / la; m1 = 0.0; }
         }
-        P1 = n1 * e1; P2 = n2 * e2; P3 = n3 * e3;
-        const double P12 = P1 * P2;
-        R = i2m::rcp_cubic(P12 * P3);
-        const double R3 = R * P3;
-        iP1 = R3 * P2; iP2 = R3 * P1; iP3 = R * P12;
-        const double a1 = r1 != 0.0 ? r1 : n1 * n1 * iP1, a2 = r2 != 0.0 ? r2 : n2 * n2 * iP2, a3 = r3 != 0.0 ? r3 : n3 * n3 * iP3;
-        X = 2.0 * (la * lb * lc + dot(da, db) * lc + dot(db, dc) * la + dot(dc, da) * lb);
-        t1 = i2m::log_tab_any(a1, lt); t2 = i2m::log_tab_any(a2, lt); t3 = i2m::log_tab_any(a3, lt);
-        h = atan2_terms(Y, X, lt);
+        if (e2 < s * S2) {
+            if (edge_gap(db, dc, lb, lc, J.La, n2, e2)) { r2 = lc / lb; xc += c2 / lc; xb -= c2 / lb; m2 = 0.0; }
+        }
+        if (e3 < s * S3) {
+            if (edge_gap(dc, da, lc, la, J.Lb, n3, e3)) { r3 = la / lc; xa += c3 / la; xc -= c3 / lc; m3 = 0.0; }
+        }
     }
+    const double P1 = n1 * e1, P2 = n2 * e2, P3 = n3 * e3;
+    const double P12 = P1 * P2;
+    const double R = i2m::rcp_cubic(P12 * P3);
+    const double R3 = R * P3;
+    const double iP1 = R3 * P2, iP2 = R3 * P1, iP3 = R * P12;
+    const double a1 = r1 != 0.0 ? r1 : n1 * n1 * iP1, a2 = r2 != 0.0 ? r2 : n2 * n2 * iP2, a3 = r3 != 0.0 ? r3 : n3 * n3 * iP3;
+    const double X = 2.0 * (la * lb * lc + dot(da, db) * lc + dot(db, dc) * la + dot(dc, da) * lb);
+    const double t1 = i2m::log_tab_any(a1, lt), t2 = i2m::log_tab_any(a2, lt), t3 = i2m::log_tab_any(a3, lt);
+    const double h = atan2_terms(Y, X, lt);
     g.T = {fma(w, t1, g.T.x), fma(w, t2, g.T.y), fma(w, t3, g.T.z), fma(w, h, g.T.w)};
-    // ---- reverse
+    // ---- reverse; dX/dl_a = P_a + 2 l_a (l_b + l_c)
     m1 *= iP1; m2 *= iP2; m3 *= iP3;
     const double Rh = R * ch;
     const double xb_ = -(Y * Rh), yb = 2.0 * (X * Rh);          // dL/dX and 2 dL/dY
-    const double q1 = xb_ * lc, q2 = xb_ * la, q3 = xb_ * lb;   // dL/dP
-    const double u1 = fma(S1, q1, -(J.Lc * m1)), u2 = fma(S2, q2, -(J.La * m2)), u3 = fma(S3, q3, -(J.Lb * m3));   // dL/dS / 2
-    g.Lc = fma(S1, m1, fma(-J.Lc, q1, g.Lc));
-    g.La = fma(S2, m2, fma(-J.La, q2, g.La));
-    g.Lb = fma(S3, m3, fma(-J.Lb, q3, g.Lb));
-    const double va = fma(xb_, fma(lb * lc, -4.0, P2), xa), vb = fma(xb_, fma(lc * la, -4.0, P3), xb),
-                 vc = fma(xb_, fma(la * lb, -4.0, P1), xc);
-    const double sa = fma(2.0, u1 + u3, va) * ila, sb = fma(2.0, u1 + u2, vb) * ilb, sc = fma(2.0, u2 + u3, vc) * ilc;
+    g.Lc = fma(S1, m1, fma(-J.Lc, xb_ * lc, g.Lc));
+    g.La = fma(S2, m2, fma(-J.La, xb_ * la, g.La));
+    g.Lb = fma(S3, m3, fma(-J.Lb, xb_ * lb, g.Lb));
+    const double E1 = 2.0 * J.Lc * m1, E2 = 2.0 * J.La * m2, E3 = 2.0 * J.Lb * m3;
+    const double sa = (fma(xb_, fma(la + la, S2, P2), xa) - (E1 + E3)) * ila,
+                 sb = (fma(xb_, fma(lb + lb, S3, P3), xb) - (E1 + E2)) * ilb,
+                 sc = (fma(xb_, fma(lc + lc, S1, P1), xc) - (E2 + E3)) * ilc;
     axpy(g.a, sa, da); axpy(g.b, sb, db); axpy(g.c, sc, dc);
     axpy(g.n, yb, da);
     g.y += yb;
     d3 pb = yb * J.N2;
     axpy(pb, sa, da); axpy(pb, sb, db); axpy(pb, sc, dc);
     return pb;
+}
+// The same for theta_terms_far.  With da = (m - a) + b0 U + b1 V every vector
+// sum over the points follows from sums of scalars: of sa = (dL/dl_a)/l_a, sb,
+// sc and y = 2 dL/dY, alone and times b0 and b1, and of s = sa + sb + sc times
+// b0^2, b0 b1 and b1^2.  Twenty-two sums and no vector per point: 156 FP64
+// instructions (DISTANT; 170 at 2 longest edges), where summing the vectors
+// took 217 and theta_terms_rev takes 310.
+struct FarBar { double a, b, c, y, a0, b0, c0, y0, a1, b1, c1, y1, s00, s01, s11, Lc, La, Lb; q4 T; };
+I2_HD __forceinline__ FarBar far_bar_zero() {
+    return {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, q4zero()};
+}
+template <bool DISTANT>
+I2_HD __forceinline__ void theta_terms_far_rev(const FarPoint& Q, const FarFrame& F, const FarGeom& G, const JGeom& J, const q4& ct,
+                                               FarBar& g) {
+    const double pp = far_pp(F, Q);
+    double ila, ilb, ilc;
+    const double la = i2m::sqrt_rsqrt(fma(Q.b0, G.ua, fma(Q.b1, G.va, G.ka + pp)), &ila),
+                 lb = i2m::sqrt_rsqrt(fma(Q.b0, G.ub, fma(Q.b1, G.vb, G.kb + pp)), &ilb),
+                 lc = i2m::sqrt_rsqrt(fma(Q.b0, G.uc, fma(Q.b1, G.vc, G.kc + pp)), &ilc);
+    const double Y = fma(Q.b0, G.uy, fma(Q.b1, G.vy, G.ky));
+    const double S1 = la + lb, S2 = lb + lc, S3 = lc + la;
+    const double s12 = S1 * S2, s123 = s12 * S3;
+    const double X = fma(-G.q3, lb, fma(-G.q2, la, fma(-G.q1, lc, s123)));
+    const double inv = i2m::rcp_cubic(s123 * X);
+    const double i = inv * X, iX = inv * s123, i3 = i * S3;
+    const double r1 = i3 * S2, r2 = i3 * S1, r3 = i * s12, u = Y * iX, v = u * u;
+    const double w = Q.w;
+    g.T = {fma(w, r1 * i2m::atanh_over<DISTANT>(G.q1 * (r1 * r1)), g.T.x), fma(w, r2 * i2m::atanh_over<DISTANT>(G.q2 * (r2 * r2)), g.T.y),
+           fma(w, r3 * i2m::atanh_over<DISTANT>(G.q3 * (r3 * r3)), g.T.z), fma(w, u * i2m::atan_over<DISTANT>(v), g.T.w)};
+    // ---- reverse
+    const double P1 = fma(S1, S1, -G.q1), P2 = fma(S2, S2, -G.q2), P3 = fma(S3, S3, -G.q3), P12 = P1 * P2;
+    // 1/(P1 P2 P3) = 1/(X^2 + Y^2) = (1/X)^2/(1 + v), v <= 3.7e-5 where DISTANT
+    const double R = DISTANT ? (iX * iX) * fma(fma(1.0 - v, v, -1.0), v, 1.0) : i2m::rcp_cubic(P12 * P3);
+    const double R3 = R * P3;
+    const double m1 = (w * ct.x) * (R3 * P2), m2 = (w * ct.y) * (R3 * P1), m3 = (w * ct.z) * (R * P12);
+    const double Rh = R * (w * ct.w);
+    const double xb = -(Y * Rh), yb = 2.0 * (X * Rh);           // dL/dX and 2 dL/dY
+    g.Lc = fma(S1, m1, fma(-J.Lc, xb * lc, g.Lc));
+    g.La = fma(S2, m2, fma(-J.La, xb * la, g.La));
+    g.Lb = fma(S3, m3, fma(-J.Lb, xb * lb, g.Lb));
+    const double E1 = 2.0 * J.Lc * m1, E2 = 2.0 * J.La * m2, E3 = 2.0 * J.Lb * m3;
+    const double sa = fma(xb, fma(la + la, S2, P2), -(E1 + E3)) * ila, sb = fma(xb, fma(lb + lb, S3, P3), -(E1 + E2)) * ilb,
+                 sc = fma(xb, fma(lc + lc, S1, P1), -(E2 + E3)) * ilc;
+    g.a += sa; g.b += sb; g.c += sc; g.y += yb;
+    g.a0 = fma(Q.b0, sa, g.a0); g.b0 = fma(Q.b0, sb, g.b0); g.c0 = fma(Q.b0, sc, g.c0); g.y0 = fma(Q.b0, yb, g.y0);
+    g.a1 = fma(Q.b1, sa, g.a1); g.b1 = fma(Q.b1, sb, g.b1); g.c1 = fma(Q.b1, sc, g.c1); g.y1 = fma(Q.b1, yb, g.y1);
+    const double t = sa + sb + sc;
+    g.s00 = fma(Q.b00, t, g.s00); g.s01 = fma(Q.b01, t, g.s01); g.s11 = fma(Q.b11, t, g.s11);
+}
+// The vector sums: g as theta_terms_rev leaves it, and added to X0 and X1 the
+// points' cotangents times their first two barycentric coordinates.
+I2_HD __forceinline__ void far_bar_expand(const FarBar& f, const FarFrame& F, const JGeom& J, TermsBar& g, d3& X0, d3& X1) {
+    const d3 a = F.m - J.a, b = F.m - J.b, c = F.m - J.c;
+    g.a = f.a * a; axpy(g.a, f.a0, F.U); axpy(g.a, f.a1, F.V);
+    g.b = f.b * b; axpy(g.b, f.b0, F.U); axpy(g.b, f.b1, F.V);
+    g.c = f.c * c; axpy(g.c, f.c0, F.U); axpy(g.c, f.c1, F.V);
+    g.n = f.y * a; axpy(g.n, f.y0, F.U); axpy(g.n, f.y1, F.V);
+    g.y = f.y; g.Lc = f.Lc; g.La = f.La; g.Lb = f.Lb;
+    g.T = far_scale(f.T, J);
+    d3 Xs = g.a + g.b + g.c;
+    axpy(Xs, f.y, J.N2);
+    auto along = [&](d3& X, double sa, double sb, double sc, double sy, double su, double sv) {
+        axpy(X, 1.0 / 3.0, Xs);
+        axpy(X, sy, J.N2); axpy(X, sa, a); axpy(X, sb, b); axpy(X, sc, c); axpy(X, su, F.U); axpy(X, sv, F.V);
+    };
+    along(X0, f.a0, f.b0, f.c0, f.y0, f.s00, f.s01);
+    along(X1, f.a1, f.b1, f.c1, f.y1, f.s01, f.s11);
 }
 // Cotangents of K_j's vertices from a pair's sums: ct as in theta_terms_rev,
 // nb the cotangent of the unit normal and gP that of the quadrature sum of

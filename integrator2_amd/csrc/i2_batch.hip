@@ -117,9 +117,9 @@ __device__ __forceinline__ void load_rule(RuleLDS& s, const Rule& R) {
 }
 
 // Partial quadrature sum_k w_k f(r_k) of one sub-panel over points k = s,
-// s + step, ...  Disjoint pairs: the inner integral's terms (FAR:
-// theta_terms_far), converted to (Psi, Theta) once per task by the caller.
-template <int TYPE, bool FAR = false>
+// s + step, ...  Disjoint pairs: the inner integral's terms, converted to (Psi,
+// Theta) once per task by the caller.
+template <int TYPE>
 __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int step, d3 a, d3 b, d3 c, const JGeom& J,
                                         const Sing<TYPE>& sg) {
     q4 acc = q4zero();
@@ -128,7 +128,7 @@ __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int s
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
         q4 f;
-        if (TYPE == I2_NOT_NEIGHBORS) f = FAR ? theta_terms_far(p, J) : theta_terms(p, J, &R.lt);
+        if (TYPE == I2_NOT_NEIGHBORS) f = theta_terms(p, J, &R.lt);
         else f = theta_psi_fast(p, J, &R.lt) - sg.at(p, &R.lt);
         acc = acc + R.w[k] * f;
     }
@@ -138,9 +138,10 @@ __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int s
 // Quadrature points of a disjoint item's control panel K_i (uniform over the
 // workgroup): the level-0 panel and its four level-1 children, in the order
 // sweep_task sums them, computed once per item instead of once per pair.  Each
-// point and its rule weight share a 32-byte record: two 128-bit LDS reads.
+// point and its rule weight share a 32-byte record, two 128-bit LDS reads: the
+// place for the general form, or |b0 U + b1 V|^2 and (b0, b1) for the far one.
 struct alignas(32) QPoint { double x, y, z, w; };
-struct PtsLDS { QPoint q[5 * MAX_POINTS]; };
+struct PtsLDS { QPoint q[5 * MAX_POINTS], f[5 * MAX_POINTS]; };
 
 // Levels 0 and 1 in one pass with a rule whose point 0 is the centroid: the
 // centroid of K_i is also the centroid of its central level-1 child (child 4),
@@ -163,46 +164,59 @@ __device__ __forceinline__ void load_points(PtsLDS& P, const RuleLDS& R, int npt
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
         P.q[t] = {p.x, p.y, p.z, R.w[k]};
+        const BaryPoint Q = bary_point(R.L1, R.L2, R.L3, R.w, npts, t);
+        const FarPoint F = far_point(Q.b0 - 1.0 / 3.0, Q.b1 - 1.0 / 3.0, Q.w);
+        P.f[t] = {far_pp(far_frame(I.a, I.b, I.c), F), F.b0, F.b1, F.w};
     }
 }
 
 // Weighted sum of the inner integral's terms over the precomputed points k =
-// k0, k0 + step, ... < k1, added in that order to acc.  FAR: theta_terms_far.
-template <bool FAR>
-__device__ __forceinline__ q4 terms_at(const RuleLDS& R, const QPoint& Q, const JGeom& J) {
-    const d3 p{Q.x, Q.y, Q.z};
-    return Q.w * (FAR ? theta_terms_far(p, J) : theta_terms(p, J, &R.lt));
-}
-template <bool FAR>
-__device__ __forceinline__ q4 quad_pts(const RuleLDS& R, const PtsLDS& P, int k0, int k1, int step, const JGeom& J, q4 acc) {
-    for (int k = k0; k < k1; k += step) {
+// k0, k0 + step, ... < k1, added in that order to acc.  FORM as in wave_form.
+template <int FORM> struct FormGeom { const FarGeom G; };
+template <> struct FormGeom<0> { const JGeom& G; };
+template <int FORM>
+__device__ __forceinline__ q4 terms_at(const RuleLDS& R, const PtsLDS& P, int k, const FormGeom<FORM>& J, double& w) {
+    if constexpr (FORM == 0) {
         const QPoint Q = P.q[k];
-        const d3 p{Q.x, Q.y, Q.z};
-        const q4 t = FAR ? theta_terms_far(p, J) : theta_terms(p, J, &R.lt);
-        acc = {fma(Q.w, t.x, acc.x), fma(Q.w, t.y, acc.y), fma(Q.w, t.z, acc.z), fma(Q.w, t.w, acc.w)};
+        w = Q.w;
+        return theta_terms(d3{Q.x, Q.y, Q.z}, J.G, &R.lt);
+    } else {
+        const QPoint Q = P.f[k];
+        w = Q.w;
+        return theta_terms_far<FORM == 2>(Q.y, Q.z, Q.x, J.G);
+    }
+}
+template <int FORM>
+__device__ __forceinline__ q4 quad_pts(const RuleLDS& R, const PtsLDS& P, int k0, int k1, int step, const FormGeom<FORM>& J, q4 acc) {
+    for (int k = k0; k < k1; k += step) {
+        double w;
+        const q4 t = terms_at<FORM>(R, P, k, J, w);
+        acc = {fma(w, t.x, acc.x), fma(w, t.y, acc.y), fma(w, t.z, acc.z), fma(w, t.w, acc.w)};
     }
     return acc;
 }
 // Sums of the terms over level 0 (T0) and level 1 (T1) of a pair, lane s of LPP.
-template <bool FAR, int LPP>
+template <int FORM, int LPP>
 __device__ __forceinline__ void sweep_terms(const RuleLDS& R, const PtsLDS& P, int npts, bool share, bool need0, bool need1, int s,
-                                            const JGeom& J, q4& T0, q4& T1) {
+                                            const FormGeom<FORM>& J, q4& T0, q4& T1) {
     int k0 = s, k1 = npts + s;
     if (share) {
         // point 0 of child 4 stands for point 0 of level 0 as well (lane 0 takes both)
         if (s == 0) {
-            T0 = terms_at<FAR>(R, P.q[4 * npts], J);
+            double w;
+            T0 = terms_at<FORM>(R, P, 4 * npts, J, w);
+            T0 = w * T0;
             T1 = T0;
             k0 = LPP;
         }
         // children 1 to 3 and child 4's other points around the shared one
-        T0 = quad_pts<FAR>(R, P, k0, npts, LPP, J, T0);
-        T1 = quad_pts<FAR>(R, P, k1, 4 * npts, LPP, J, T1);
-        T1 = quad_pts<FAR>(R, P, 4 * npts + k0, 5 * npts, LPP, J, T1);
+        T0 = quad_pts<FORM>(R, P, k0, npts, LPP, J, T0);
+        T1 = quad_pts<FORM>(R, P, k1, 4 * npts, LPP, J, T1);
+        T1 = quad_pts<FORM>(R, P, 4 * npts + k0, 5 * npts, LPP, J, T1);
         return;
     }
-    if (need0) T0 = quad_pts<FAR>(R, P, k0, npts, LPP, J, T0);
-    if (need1) T1 = quad_pts<FAR>(R, P, k1, 5 * npts, LPP, J, T1);
+    if (need0) T0 = quad_pts<FORM>(R, P, k0, npts, LPP, J, T0);
+    if (need1) T1 = quad_pts<FORM>(R, P, k1, 5 * npts, LPP, J, T1);
 }
 
 __device__ __forceinline__ q4 shfl_sum(q4 v, int G) {
@@ -328,14 +342,16 @@ __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS&
     const bool need0 = !A.fixed || A.last_level == 0;
     const bool need1 = A.fixed ? A.last_level == 1 : A.last_level >= 1;
     q4 v0 = q4zero(), v1 = q4zero();
-    // one loop per wavefront: far only if every pair of the wavefront is
-    const bool near = __ballot(valid && !panel_far(ball, JG)) != 0ull;
+    // one loop per wavefront, in the form that holds for all its pairs
+    const int form = wave_form(valid, ball, JG);
     if (valid) {
         q4 T0 = q4zero(), T1 = q4zero();
-        if (near) {
-            sweep_terms<false, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
+        if (form == 0) {
+            sweep_terms<0, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, FormGeom<0>{JG}, T0, T1);
         } else {
-            sweep_terms<true, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, JG, T0, T1);
+            const FarGeom G = far_geom(far_frame(I.a, I.b, I.c), JG);
+            if (form == 1) sweep_terms<1, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, FormGeom<1>{G}, T0, T1);
+            else sweep_terms<2, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, FormGeom<2>{G}, T0, T1);
             T0 = far_scale(T0, JG);
             T1 = far_scale(T1, JG);
         }

@@ -53,9 +53,9 @@ template <> struct PairCtx<I2_SIMPLE_NEIGHBORS> {
 // own FP64 form loses up to 1e-7 of a value to cancellation where a
 // quadrature point lies near the extension of an edge line of K_j, which
 // moves Runge decisions; both paths therefore take decisions on accurate values.
-// Disjoint pairs sum the inner integral's terms (FAR: theta_terms_far), which
-// the caller converts to (Psi, Theta) once per task.
-template <int TYPE, bool FAR>
+// Disjoint pairs sum the inner integral's terms, which the caller converts to
+// (Psi, Theta) once per task.
+template <int TYPE>
 __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, d3 a, d3 b, d3 c, double area,
                                        const JGeom& J, const PairCtx<TYPE>& ctx) {
     q4 acc = q4zero();
@@ -64,11 +64,30 @@ __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, 
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
         q4 f;
-        if (TYPE == I2_NOT_NEIGHBORS) f = FAR ? theta_terms_far(p, J) : theta_terms(p, J, lt);
+        if (TYPE == I2_NOT_NEIGHBORS) f = theta_terms(p, J, lt);
         else f = theta_psi_fast(p, J, lt) - ctx.sing(p, lt);
         acc = acc + R.w[k] * f;
     }
     return area * acc;
+}
+
+// The same sum of a disjoint pair's far terms over the sub-panels sub, sub + G,
+// ... of `level`, in barycentric coordinates of K_i less 1/3.
+template <bool DISTANT>
+__device__ __forceinline__ q4 quad_far(const Rule& R, int level, int sub, int G, const FarFrame& F, const FarGeom& J) {
+    q4 acc = q4zero();
+    const double h = 1.0 / 3.0;
+    for (uint32_t c = sub; c < (1u << (2 * level)); c += G) {
+        d3 a = {1.0 - h, -h, 0.0}, b = {-h, 1.0 - h, 0.0}, o = {-h, -h, 0.0};
+        sub_panel(a, b, o, level, c);
+        for (int k = 0; k < R.n; ++k) {
+            const double l1 = R.L1[k], l2 = R.L2[k], l3 = R.L3[k], w = R.w[k];
+            const FarPoint Q = far_point(l1 * a.x + l2 * b.x + l3 * o.x, l1 * a.y + l2 * b.y + l3 * o.y, w);
+            const q4 t = theta_terms_far<DISTANT>(Q.b0, Q.b1, far_pp(F, Q), J);
+            acc = {fma(w, t.x, acc.x), fma(w, t.y, acc.y), fma(w, t.z, acc.z), fma(w, t.w, acc.w)};
+        }
+    }
+    return acc;
 }
 
 // Level-`level` value of tasks: lanes per task = 1 << lanes_log2; lane `sub`
@@ -99,20 +118,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_
         double area = I.area;
         for (int l = 0; l < level; ++l) area *= 0.25;
         const uint32_t nsub = 1u << (2 * level);
-        // disjoint pairs: one loop per wavefront, far only if every pair of it is
-        const bool far = TYPE == I2_NOT_NEIGHBORS && __all(panel_far(panel_ball(I.a, I.b, I.c, R.reach), JG));
-        if (far) {
-            for (uint32_t c = sub; c < nsub; c += G) {
-                d3 a = I.a, b = I.b, cc = I.c;
-                sub_panel(a, b, cc, level, c);
-                acc = acc + quad_sub<TYPE, true>(R, &lt, a, b, cc, area, JG, ctx);
-            }
-            acc = far_scale(acc, JG);
+        // disjoint pairs: one loop per wavefront, in the form that holds for all its pairs
+        const int form = TYPE == I2_NOT_NEIGHBORS ? wave_form(true, panel_ball(I.a, I.b, I.c, R.reach), JG) : 0;
+        if (form != 0) {
+            const FarFrame F = far_frame(I.a, I.b, I.c);
+            const FarGeom FG = far_geom(F, JG);
+            acc = area * far_scale(form == 1 ? quad_far<false>(R, level, sub, G, F, FG) : quad_far<true>(R, level, sub, G, F, FG), JG);
         } else {
             for (uint32_t c = sub; c < nsub; c += G) {
                 d3 a = I.a, b = I.b, cc = I.c;
                 sub_panel(a, b, cc, level, c);
-                acc = acc + quad_sub<TYPE, false>(R, &lt, a, b, cc, area, JG, ctx);
+                acc = acc + quad_sub<TYPE>(R, &lt, a, b, cc, area, JG, ctx);
             }
         }
         if (TYPE == I2_NOT_NEIGHBORS) acc = psi_of_terms(acc, JG);

@@ -269,8 +269,17 @@ I2_HD __forceinline__ double atan2_any(double y, double x, const MathTable* __re
 
 // atanh(z)/z for z^2 = s in [0, 1/16] (relative error below 2^-54.9) and
 // atan(u)/u for u^2 = v in [0, 0.003] (below 2^-62): 1 + s q(s), q interpolating
-// (f - 1)/s at the Chebyshev nodes of the interval (gen_math_tables.py)
+// (f - 1)/s at the Chebyshev nodes of the interval (gen_math_tables.py).  DISTANT:
+// the same on s in [0, 1/144] (below 2^-55.6) and v in [0, 3.7e-5] (below 2^-67)
+template <bool DISTANT>
 I2_HD __forceinline__ double atanh_over(double s) {
+    if (DISTANT) {
+        double q = fma_k(s, 0.09225773056807902, 0.11110289065026226);
+        q = fma_k(q, s, 0.14285716327371326);
+        q = fma_k(q, s, 0.19999999998226609);
+        q = fma_k(q, s, 0.3333333333333358);
+        return fma(q, s, 1.0);
+    }
     double q = fma_k(s, 0.07395269887839463, 0.06506094123632396);
     q = fma_k(q, s, 0.07700982152842295);
     q = fma_k(q, s, 0.09090651861920544);
@@ -280,7 +289,12 @@ I2_HD __forceinline__ double atanh_over(double s) {
     q = fma_k(q, s, 0.33333333333333287);
     return fma(q, s, 1.0);
 }
+template <bool DISTANT>
 I2_HD __forceinline__ double atan_over(double v) {
+    if (DISTANT) {
+        const double q = fma_k(fma_k(v, -0.14285097640048655, 0.19999999991444123), v, -0.33333333333333315);
+        return fma(q, v, 1.0);
+    }
     double q = fma_k(v, -0.09033459667472876, 0.11110960509214748);
     q = fma_k(q, v, -0.14285714124452448);
     q = fma_k(q, v, 0.19999999999939544);

@@ -290,9 +290,17 @@ int i2_host_theta_psi(int fast, const double* pts, int64_t n, const double* tri9
     const JGeom J = make_jgeom(A, B, C, unit(C - B), unit(A - C), unit(B - A));
     for (int64_t q = 0; q < n; ++q) {
         const d3 p = {pts[3 * q], pts[3 * q + 1], pts[3 * q + 2]};
-        const q4 r = fast == 2 ? psi_of_terms(far_scale(theta_terms_far(p, J), J), J)
-                     : fast    ? theta_psi_fast(p, J, &i2m::h_mathtab)
-                               : theta_psi(p, J.a, J.b, J.c, J.ta, J.tb, J.tc);
+        q4 r;
+        if (fast == 2 || fast == 3) {   // p as a point of a control panel of K_j's size and shape
+            const double b0 = 0.3, b1 = -0.2;
+            const d3 o = p - ((b0 + 1.0 / 3.0) * J.a + (b1 + 1.0 / 3.0) * J.b + (1.0 / 3.0 - b0 - b1) * J.c);
+            const FarFrame F = far_frame(J.a + o, J.b + o, J.c + o);
+            const FarGeom G = far_geom(F, J);
+            const double pp = far_pp(F, far_point(b0, b1, 0.0));
+            r = psi_of_terms(far_scale(fast == 3 ? theta_terms_far<true>(b0, b1, pp, G) : theta_terms_far<false>(b0, b1, pp, G), J), J);
+        } else {
+            r = fast ? theta_psi_fast(p, J, &i2m::h_mathtab) : theta_psi(p, J.a, J.b, J.c, J.ta, J.tb, J.tc);
+        }
         out4[4 * q] = r.x; out4[4 * q + 1] = r.y; out4[4 * q + 2] = r.z; out4[4 * q + 3] = r.w;
     }
     return I2_OK;

@@ -146,6 +146,40 @@ def test_reverse_mode_of_the_terms(i2, shape, far):
         assert np.abs(np.concatenate([pb, par]) - ref).max() <= 2.0 ** -44 * 8 * np.abs(g).sum() / d
 
 
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("scale", [1e-20, 1.0, 1e20])
+def test_distant_form(i2, shape, scale):
+    """From six longest edges on, with the bounds of test_far_form."""
+    rng = np.random.default_rng(11)
+    T = _panel(shape, rng, scale)
+    M = max(np.linalg.norm(T[k] - T[k - 1]) for k in range(3))
+    u = rng.normal(size=(30, 3))
+    u /= np.linalg.norm(u, axis=1, keepdims=True)
+    pts = T.mean(axis=0) + (M * np.repeat([20 / 3 * (1 + 1e-6), 30.0, 1e4], 10))[:, None] * u
+    for p, g in zip(pts, _form(i2, 3, pts, T)):
+        psi, theta, t, dth = _exact(p, T)
+        assert np.abs(g[:3] - psi).max() <= 8 * 2 * EPS * t
+        assert abs(g[3] - theta) <= dth + 8 * 2 * EPS * abs(theta)
+
+
+@pytest.mark.parametrize("shape", ["equilateral", "right"])
+def test_reverse_mode_distant_against_far(i2, shape):
+    """The two polynomial forms' gradients, each within the far form's bound of
+    the exact ones (test_reverse_mode_of_the_terms), from six longest edges on."""
+    rng = np.random.default_rng(12)
+    T = np.ascontiguousarray(_panel(shape, rng))
+    P = ctypes.c_void_p
+    for r in (6.7 * 1.05, 12.0, 300.0):
+        u = rng.normal(size=3)
+        p, g = np.ascontiguousarray(T.mean(axis=0) + r * u / np.linalg.norm(u)), rng.normal(size=4)
+        out = []
+        for kind in (4, 5):
+            f, pb, par = np.zeros(4), np.zeros(3), np.zeros(9)
+            assert i2.lib().i2_host_point_adjoint(ctypes.c_int(kind), *(a.ctypes.data_as(P) for a in (p, T, g, f, pb, par))) == 0
+            out.append(np.concatenate([f, pb, par]))
+        assert np.abs(out[0] - out[1]).max() <= 2 * 2.0 ** -44 * 8 * np.abs(g).sum() / (r / 2)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("path", [0, 1])
 def test_rule_with_points_outside_the_triangle(gpu, oracle_mod, path):
