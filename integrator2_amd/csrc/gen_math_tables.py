@@ -60,3 +60,5 @@ print("atanh_over", interpolant(lambda s: mpmath.atanh(mpmath.sqrt(s)) / mpmath.
 print("atan_over", interpolant(lambda s: mpmath.atan(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf("0.003"), 5))
 print("atanh_over, distant", interpolant(lambda s: mpmath.atanh(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf(1) / 144, 5))
 print("atan_over, distant", interpolant(lambda s: mpmath.atan(mpmath.sqrt(s)) / mpmath.sqrt(s), mpmath.mpf("3.7e-5"), 3))
+print("cos_turns, c", interpolant(lambda s: mpmath.cos(2 * mpmath.pi * mpmath.sqrt(s)), mpmath.mpf(1) / 64, 7))
+print("cos_turns, s", interpolant(lambda s: 1 + mpmath.sqrt(s) * mpmath.sin(2 * mpmath.pi * mpmath.sqrt(s)), mpmath.mpf(1) / 64, 7))

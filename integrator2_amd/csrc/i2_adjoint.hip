@@ -55,18 +55,21 @@ I2_HD __forceinline__ uint64_t mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 // N(0,1) by Box-Muller from two 53-bit uniforms in (0, 1) of the splitmix64
-// hash of (seed, pair id, stream); streams 0 (w) and 1..3 (v)
-I2_HD __forceinline__ double normal_draw(uint64_t seed, uint64_t pid, uint64_t stream) {
+// hash of (seed, pair id, stream); streams 0 (w) and 1..3 (v).  Table log and
+// polynomial cosine: four draws of the libraries' functions were an eighth of
+// k_adj_disjoint's instructions.  The bound keeps the root's estimate finite where u1
+// rounds to 1.
+I2_HD __forceinline__ double normal_draw(uint64_t seed, uint64_t pid, uint64_t stream, const i2m::MathTable* __restrict__ lt) {
     const uint64_t base = mix64(seed ^ mix64(pid * 4ull + stream));
     const double u1 = ((double)(mix64(base ^ 0x1ull) >> 11) + 0.5) * (1.0 / 9007199254740992.0);
     const double u2 = ((double)(mix64(base ^ 0x2ull) >> 11) + 0.5) * (1.0 / 9007199254740992.0);
-    return sqrt(-2.0 * log(u1)) * cos(TWO_PI * u2);
+    return i2m::sqrt_pos(fmax(-2.0 * i2m::log_tab_any(u1, lt), 0x1p-900)) * i2m::cos_turns(u2);
 }
 
 struct Weights { double w; d3 v; };
-__device__ __forceinline__ Weights weights(uint64_t seed, int i, int j, int nT) {
+__device__ __forceinline__ Weights weights(uint64_t seed, int i, int j, int nT, const i2m::MathTable* __restrict__ lt) {
     const uint64_t pid = (uint64_t)i * (uint64_t)nT + (uint64_t)j;
-    return {normal_draw(seed, pid, 0), {normal_draw(seed, pid, 1), normal_draw(seed, pid, 2), normal_draw(seed, pid, 3)}};
+    return {normal_draw(seed, pid, 0, lt), {normal_draw(seed, pid, 1, lt), normal_draw(seed, pid, 2, lt), normal_draw(seed, pid, 3, lt)}};
 }
 // cotangent of a pair's (Psi, Theta): dL/dPsi = n_j x v / (4 pi), dL/dTheta = w + v . n_j / (4 pi)
 __device__ __forceinline__ q4 task_cotangent(const Weights& W, d3 nJ) {
@@ -269,19 +272,47 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
         double Sb = 0.0, loss = 0.0;
         uint32_t deep = 0u;                           // bit j - j0: (i, j) is at reported level >= 2
         const int j0 = jt * JT, j1 = min(M.nT, j0 + JT);
+        // two bits per j, read before the points' loop so that the loads overlap:
+        // reported level 0 or 1, 2: that of k_adj_deep, 3: not a pair
+        uint64_t levels = ~0ull;
+        {
+            const int ii = ivalid ? i : 0;
+            // pairs (i, j > i) stand in row i's order, without the neighbours
+            const int64_t n0 = M.nbr_start[ii], n1 = M.nbr_start[ii + 1], row = M.row_start[ii];
+            int64_t q = n0;
+            while (q < n1 && M.nbr[q] < j0) ++q;
+            int next = q < n1 ? M.nbr[q] : INT32_MAX;
+            const int8_t* conv = M.conv[I2_NOT_NEIGHBORS];
+#pragma unroll 4
+            for (int j = j0; j < j1; ++j) {
+                int64_t z = row + (j - ii - 1) - (q - n0);
+                bool nb = next == j;
+                if (nb) { ++q; next = q < n1 ? M.nbr[q] : INT32_MAX; }
+                if (__ballot(ii > j) != 0ull) {         // pairs (j < i): row j's order, the same list for all lanes
+                    int below = 0;
+                    bool nbj = false;
+                    for (int64_t r = M.nbr_start[j]; r < M.nbr_start[j + 1]; ++r) {
+                        const int x = M.nbr[r];
+                        below += x < ii;
+                        nbj |= x == ii;
+                    }
+                    if (ii > j) { z = M.npairs[I2_NOT_NEIGHBORS] + M.row_start[j] + (ii - j - 1) - below; nb = nbj; }
+                }
+                if (ivalid && j != ii && !nb) {
+                    const int lev = reported_level(A, conv[z], K);
+                    levels &= ~((uint64_t)(3 - min(lev, 2)) << (2 * (j - j0)));
+                }
+            }
+        }
         double* const kjw = M.kj + (int64_t)iw * M.nT * 9;   // this wavefront's K_j slots
         for (int j = j0; j < j1; ++j) {
             const Panel J = uniform_panel(M.panels[j]);   // j is uniform: K_j lives in scalar registers
-            bool valid = ivalid && j != i && shared_count(I, J) == 0;
-            int lev = 0;
-            if (valid) {
-                const int64_t z = task_disjoint(M, i, j);
-                lev = reported_level(A, M.conv[I2_NOT_NEIGHBORS][z], K);
-                if (lev >= 2) { deep |= 1u << (j - j0); valid = false; }
-            }
+            const int lev = (int)(levels >> (2 * (j - j0))) & 3;
+            const bool valid = lev < 2;
+            if (lev == 2) deep |= 1u << (j - j0);
             if (__ballot(valid) == 0ull) continue;   // the slot keeps the zeros of k_adj_zero
             Weights W = {0.0, {0.0, 0.0, 0.0}};
-            if (valid) W = weights(A.seed, i, j, M.nT);
+            if (valid) W = weights(A.seed, i, j, M.nT, &R.lt);
             const q4 gb = task_cotangent(W, J.n);
             const JGeom JG = uniform_jgeom(make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc));
             const d3 gP = {gb.x, gb.y, gb.z};
@@ -373,7 +404,7 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
     const Panel I = M.panels[i];
     const Panel J = M.panels[j];
     // one of the pair's four draws per lane of a quad
-    const double draw = normal_draw(A.seed, (uint64_t)i * (uint64_t)M.nT + (uint64_t)j, (uint64_t)(s & 3));
+    const double draw = normal_draw(A.seed, (uint64_t)i * (uint64_t)M.nT + (uint64_t)j, (uint64_t)(s & 3), &R.lt);
     const Weights W = {quad_lane(draw, 0), {quad_lane(draw, 1), quad_lane(draw, 2), quad_lane(draw, 3)}};
     const q4 gb = task_cotangent(W, J.n);
     const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
@@ -537,7 +568,7 @@ __device__ __forceinline__ void singular_task(const AdjArgs& A, const RuleSh& R,
                                               int level, int lane) {
     const Panel I = uniform_panel(M.panels[i]);   // one wavefront per pair
     const Panel J = uniform_panel(M.panels[j]);
-    const Weights W = weights(A.seed, i, j, M.nT);
+    const Weights W = weights(A.seed, i, j, M.nT, &R.lt);
     const q4 gb = task_cotangent(W, J.n);
     const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
     int s1, s2;
@@ -1085,7 +1116,7 @@ int i2_host_loss_weights(uint64_t seed, const int32_t* ij, int64_t n, int nT, do
     if (!ij || !out4 || n < 0 || nT <= 0) { set_error("invalid argument"); return I2_ERR_INVALID; }
     for (int64_t q = 0; q < n; ++q) {
         const uint64_t pid = (uint64_t)ij[2 * q] * (uint64_t)nT + (uint64_t)ij[2 * q + 1];
-        for (int s = 0; s < 4; ++s) out4[4 * q + s] = normal_draw(seed, pid, (uint64_t)s);
+        for (int s = 0; s < 4; ++s) out4[4 * q + s] = normal_draw(seed, pid, (uint64_t)s, &i2m::h_mathtab);
     }
     return I2_OK;
 }
