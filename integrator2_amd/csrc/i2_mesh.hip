@@ -61,20 +61,24 @@ __global__ void k_panel_table(int64_t nT, const double* __restrict__ xyz, const 
 // workgroup: each thread scans a contiguous chunk.
 template <class T>
 __global__ __launch_bounds__(1024) void k_scan_counts(int64_t n, const T* __restrict__ cnt, int64_t* __restrict__ out) {
-    __shared__ int64_t part[1024];
+    __shared__ int64_t part[16];
     const int64_t chunk = (n + blockDim.x - 1) / blockDim.x;
     const int64_t b = threadIdx.x * chunk, e = b + chunk < n ? b + chunk : n;
     int64_t s = 0;
     for (int64_t q = b; q < e; ++q) s += (int64_t)cnt[q];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int64_t run = 0;
-        for (unsigned t = 0; t < blockDim.x; ++t) { const int64_t v = part[t]; part[t] = run; run += v; }
-        out[n] = run;
+    const int lane = threadIdx.x & 63;
+    int64_t run = s;                       // inclusive over the wavefront
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t v = (int64_t)__shfl_up((long long)run, d);
+        if (lane >= d) run += v;
     }
+    if (lane == 63) part[threadIdx.x >> 6] = run;
     __syncthreads();
-    int64_t run = part[threadIdx.x];
+    int64_t before = 0;                    // the wavefronts before this one
+    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) before += part[w];
+    run += before;
+    if (threadIdx.x == blockDim.x - 1) out[n] = run;
+    run -= s;
     for (int64_t q = b; q < e; ++q) { out[q] = run; run += (int64_t)cnt[q]; }
 }
 
