@@ -18,12 +18,13 @@
 //                   stay in registers for the whole tile and those of K_j are
 //                   summed over the wavefront into the slot of (wavefront, j).
 //                   Pairs at reported level >= 2 are marked per lane.
-//   k_adj_deep      the marked pairs, item by item: 16 pairs at a time, 16
-//                   lanes each over their 13 * 4^L points, added to the item's
-//                   own slots in a fixed order.
-//   k_adj_singular  vertex- and edge-sharing pairs: one wavefront per pair;
-//                   reverse mode over the points; the cotangents of the
-//                   per-pair quantities go to a record per pair.
+//   k_adj_deep      the marked pairs, from a list, 16 or 64 lanes each over
+//                   their 13 * 4^L points, to a record per pair.
+//   k_adj_deep_sum  those records, added to their item's slots in a fixed order.
+//   k_adj_singular  vertex- and edge-sharing pairs: 16 lanes per pair, or a
+//                   wavefront per pair above reported level 2; reverse mode
+//                   over the points; the cotangents of the per-pair quantities
+//                   go to a record per pair.
 //   k_adj_singular_dual  the per-pair chain of every record: forward-mode
 //                   dual numbers along the 18 vertex coordinates of the pair
 //                   (one per lane, 3.5 pairs per wavefront) through the
@@ -283,7 +284,6 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
             while (q < n1 && M.nbr[q] < j0) ++q;
             int next = q < n1 ? M.nbr[q] : INT32_MAX;
             const int8_t* conv = M.conv[I2_NOT_NEIGHBORS];
-#pragma unroll 4
             for (int j = j0; j < j1; ++j) {
                 int64_t z = row + (j - ii - 1) - (q - n0);
                 bool nb = next == j;
@@ -355,9 +355,30 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
                         i2m::rcp_cubic(2.0 * J.area), J.n, Ab, Bb, Cb);
             store_sum9(kjw + 9 * (int64_t)j, lane, Ab, Bb, Cb);
         }
-        if (__ballot(deep != 0u) != 0ull) {         // the item is taken by k_adj_deep
+        if (__ballot(deep != 0u) != 0ull) {         // the item's marked pairs, lanes in order
+            const int cnt = __popc(deep);
+            int run = cnt;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int v = __shfl_up(run, d);
+                if (lane >= d) run += v;
+            }
+            const int n = __builtin_amdgcn_readlane(run, 63);
+            unsigned long long base = 0ull;
+            if (lane == 0) base = atomicAdd(&A.counters[2], (unsigned long long)n);
+            base = (unsigned long long)uniform64a((int64_t)base);
+            DeepItem* d = A.deep_items;
             A.deep_mask[item * 64 + lane] = deep;
-            if (lane == 0) A.deep_items[atomicAdd(&A.counters[1], 1ull)] = item;
+            if (lane == 0) d[atomicAdd(&A.counters[1], 1ull)] = {item, (int64_t)base, n};
+            if (base + n <= (unsigned long long)A.deep_cap) {
+                int64_t at = (int64_t)base + run - cnt;
+                for (uint32_t r = deep; r != 0u; r &= r - 1u) {
+                    const int b = (int)__builtin_ctz(r);
+                    const int level = reported_level(A, M.conv[I2_NOT_NEIGHBORS][task_disjoint(M, i, j0 + b)], K);
+                    A.deep_pairs[at++] = {item, (int16_t)(lane * ADJ_TILE + b), (int16_t)level};
+                }
+            } else {                                // the list's last entries, which hold no item
+                for (int64_t q = (int64_t)base + lane; q < A.deep_cap; q += 64) A.deep_pairs[q] = {-1, 0, 0};
+            }
         }
         if (ivalid) {
             d3 X2 = Xs - X0 - X1;
@@ -373,18 +394,18 @@ __global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_disjoint(AdjArgs A) {
     }
 }
 
-// The disjoint pairs at reported level >= 2, item by item: the items that hold
-// any, as k_adj_disjoint listed them, claimed by workgroups of 256.  An item's
-// pairs are numbered in a fixed order (lanes in order, each lane's j in order)
-// and taken 16 at a time, 16 lanes per pair: at level 2 each lane has one of
-// the 16 sub-panels (13 points), at level L >= 3 every 16th of 4^L.  The
-// batch's results go to LDS and are added in the pairs' order to the item's
-// sums, which the item's slots receive at the end; every slot belongs to one
-// item, so the order in which items are claimed does not matter.
+// The disjoint pairs at reported level >= 2, as k_adj_disjoint listed them: a
+// wavefront takes its pair if it is above level 2 (832 points in 13 rounds), and
+// every fourth one the pairs at level 2 among its four, 16 lanes each (208
+// points are 13 rounds of 16 lanes, and what is done once per pair serves four
+// pairs per instruction), and leaves a pair's cotangents in its record.  k_adj_deep_sum
+// adds an item's records to the item's slots, lanes and then each lane's j in
+// order, so the order in which items are listed does not matter.  Pairs beyond
+// the list's end are done there as well, in the same way, one after another.
 //
-// 16 lanes instead of a wavefront per pair: 208 points fill 13 rounds of 16
-// lanes but 3.25 of 64, and what is done once per pair (weights, sums over
-// the lanes, the chain to the vertices) serves four pairs per instruction.
+// With an item as the unit of work the longest item (over a hundred pairs on a
+// thin torus) set the time, at 20 % of the issue slots: 1.15 ms on two tori of
+// 3,072 panels against 0.80 as a list, and 0.41 against 0.13 ms on 5,120 panels.
 constexpr int DEEP_NK = 11;             // per pair: X0, X1, X2 (9), Sb, loss
 constexpr int DEEP_REC = DEEP_NK + 9;   // and the cotangents of K_j's vertices
 __device__ __forceinline__ double quad_lane(double v, int q) {
@@ -397,8 +418,10 @@ __device__ __forceinline__ double quad_lane(double v, int q) {
     else { l = __builtin_amdgcn_mov_dpp(lo, 0xff, 0xf, 0xf, false); h = __builtin_amdgcn_mov_dpp(hi, 0xff, 0xf, 0xf, false); }
     return __longlong_as_double((long long)(((uint64_t)h << 32) | l));
 }
-__device__ __forceinline__ void row_sum3(d3& v) { v.x = row_sum16(v.x); v.y = row_sum16(v.y); v.z = row_sum16(v.z); }
-// One pair by 16 lanes (lane s of its row); every lane of the row gets the results.
+// One pair by G lanes: 16 (a row of the wavefront) or 64.
+template <int G> __device__ __forceinline__ double group_sum(double v) { return G == 16 ? row_sum16(v) : sum_all(v); }
+template <int G> __device__ __forceinline__ void group_sum3(d3& v) { v = {group_sum<G>(v.x), group_sum<G>(v.y), group_sum<G>(v.z)}; }
+template <int G>
 __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, const AdjMesh& M, int i, int j, int level, int s,
                                           double* rec) {
     const Panel I = M.panels[i];
@@ -415,22 +438,18 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
     const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
     TermsBar g = terms_bar_zero();
     d3 X0 = {0.0, 0.0, 0.0}, X1 = X0;
-    const uint32_t nsub = 1u << (2 * level);
-    for (uint32_t sub = s; sub < nsub; sub += 16) {
-        d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
-        sub_panel(ba, bb, bc, level, sub);
-        for (int k = 0; k < npts; ++k) {
-            const d3 beta = R.L1[k] * ba + R.L2[k] * bb + R.L3[k] * bc;
-            d3 p = beta.x * I.a;
-            p = p + beta.y * I.b;
-            p = p + beta.z * I.c;
-            const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
-            axpy(X0, beta.x, pb); axpy(X1, beta.y, pb);
-        }
+    const uint32_t total = (uint32_t)npts << (2 * level);
+    const uint32_t magic = (uint32_t)((0x100000000ull + npts - 1) / npts);   // q / npts for q <= 2^28
+    for (uint32_t q = s; q < total; q += G) {
+        const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+        const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
+        const d3 p = beta.x * I.a + beta.y * I.b + beta.z * I.c;
+        const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
+        axpy(X0, beta.x, pb); axpy(X1, beta.y, pb);
     }
-    row_sum3(g.a); row_sum3(g.b); row_sum3(g.c); row_sum3(g.n); row_sum3(X0); row_sum3(X1);
-    g.T = {row_sum16(g.T.x), row_sum16(g.T.y), row_sum16(g.T.z), row_sum16(g.T.w)};
-    g.y = row_sum16(g.y); g.La = row_sum16(g.La); g.Lb = row_sum16(g.Lb); g.Lc = row_sum16(g.Lc);
+    group_sum3<G>(g.a); group_sum3<G>(g.b); group_sum3<G>(g.c); group_sum3<G>(g.n); group_sum3<G>(X0); group_sum3<G>(X1);
+    g.T = {group_sum<G>(g.T.x), group_sum<G>(g.T.y), group_sum<G>(g.T.z), group_sum<G>(g.T.w)};
+    g.y = group_sum<G>(g.y); g.La = group_sum<G>(g.La); g.Lb = group_sum<G>(g.Lb); g.Lc = group_sum<G>(g.Lc);
     const q4 F = psi_of_terms(g.T, JG);
     const q4 Iv = fa * F;
     const d3 psi = {Iv.x, Iv.y, Iv.z};
@@ -450,90 +469,131 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
     }
 }
 
+// the tile's first j and wavefront of control panels of an item of mesh M
+__device__ __forceinline__ void item_at(const AdjArgs& A, const AdjMesh& M, int m, int64_t item, int* iw, int* jt) {
+    const int64_t rr = item - A.item_base[m];
+    *iw = (int)(rr / M.jtiles);
+    *jt = (int)(rr % M.jtiles);
+}
 __global__ __launch_bounds__(256) I2_TWO_WAVES void k_adj_deep(AdjArgs A) {
     __shared__ RuleSh R;
-    __shared__ double kip[64][DEEP_NK];      // the item's sums per lane i
-    __shared__ double kjp[ADJ_TILE][9];      // and per j of the tile
-    __shared__ double rec[16][DEEP_REC];     // the batch's pairs
-    __shared__ uint16_t list[64 * ADJ_TILE]; // the item's pairs, lane * ADJ_TILE + bit
-    __shared__ int npairs;
-    __shared__ long long item_sh;
-    const unsigned long long nitems = A.counters[1];
-    if ((unsigned long long)blockIdx.x >= nitems) return;
+    const int64_t n = min((int64_t)A.counters[2], A.deep_cap);
+    // one quarter of the grid for each of four consecutive pairs: a workgroup's
+    // wavefronts then have the same kind of work, and the first quarter, which
+    // takes the pairs at level 2, covers all XCDs
+    const int quarter = gridDim.x / 4, r = blockIdx.x / quarter;
+    int64_t four = 16 * (int64_t)(blockIdx.x % quarter);
+    if (four >= n) return;
     load_rule_sh(R, A.rule);
-    const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 4;
-    for (;;) {
-        __syncthreads();
-        if (tid == 0) {
-            const unsigned long long pos = atomicAdd(&A.counters[2], 1ull);
-            item_sh = pos < nitems ? A.deep_items[pos] : -1ll;
-        }
-        __syncthreads();
-        const int64_t item = uniform64a(item_sh);
-        if (item < 0) break;
-        const int m = __builtin_amdgcn_readfirstlane(find_base_a(A.item_base, A.nmeshes, item));
+    __syncthreads();
+    const int lane = threadIdx.x & 63, row = lane >> 4;
+    for (four += 4 * (threadIdx.x >> 6); four < n; four += 16 * (int64_t)quarter) {
+        // four pairs, one per row; this wavefront's own is number r
+        const int64_t q = four + row;
+        const DeepPair e = A.deep_pairs[min(q, n - 1)];
+        const bool here = q < n && e.item >= 0;   // an item that did not fit has no entries
+        const int level = here ? e.level : 0;
+        if (__ballot(r == 0 ? level != 0 : level > 2) == 0ull) continue;
+        const int64_t item = here ? e.item : 0;
+        const int m = find_base_a(A.item_base, A.nmeshes, item);
         const AdjMesh& M = A.meshes[m];
-        const int64_t rr = item - A.item_base[m];
-        const int iw = (int)(rr / M.jtiles), jt = (int)(rr % M.jtiles);
+        int iw, jt;
+        item_at(A, M, m, item, &iw, &jt);
+        const int i = iw * 64 + e.at / ADJ_TILE, j = jt * M.jt + e.at % ADJ_TILE;
+        if (r == 0 && here && level == 2) deep_pair<16>(A, R, M, i, j, level, lane & 15, A.deep_rec + q * DEEP_REC);
+        const int from = 16 * r, wl = __builtin_amdgcn_readlane(level, from);
+        if (wl > 2)
+            deep_pair<64>(A, R, A.meshes[__builtin_amdgcn_readlane(m, from)], __builtin_amdgcn_readlane(i, from),
+                          __builtin_amdgcn_readlane(j, from), wl, lane, A.deep_rec + (four + r) * DEEP_REC);
+    }
+}
+
+// One wavefront per listed item: lane l adds the records of its pairs (panel
+// i) to K_i's slot, lane b those of panel j0 + b to K_j's.
+__global__ __launch_bounds__(64) I2_TWO_WAVES void k_adj_deep_sum(AdjArgs A) {
+    __shared__ RuleSh R;
+    __shared__ double rec[4][DEEP_REC];
+    __shared__ uint16_t list[64 * ADJ_TILE];   // an unlisted item's pairs
+    __shared__ uint32_t masks[64];
+    __shared__ int starts[64];
+    const int64_t nitems = (int64_t)A.counters[1];
+    const int lane = threadIdx.x;
+    bool loaded = false;
+    for (int64_t x = blockIdx.x; x < nitems; x += gridDim.x) {
+        const DeepItem D = A.deep_items[x];
+        const int m = __builtin_amdgcn_readfirstlane(find_base_a(A.item_base, A.nmeshes, D.item));
+        const AdjMesh& M = A.meshes[m];
+        int iw, jt;
+        item_at(A, M, m, D.item, &iw, &jt);
         const int j0 = jt * M.jt;
-        const int K = M.K[I2_NOT_NEIGHBORS];
-        const uint32_t mask = A.deep_mask[item * 64 + lane];   // the same in every wavefront
-        if (tid < 64) {
-            int at = 0;                     // pairs of the lanes before this one
-            const int cnt = __popc(mask);
-            int run = cnt;
-            for (int d = 1; d < 64; d <<= 1) {
-                const int v = __shfl_up(run, d);
-                if (lane >= d) run += v;
-            }
-            at = run - cnt;
-            for (uint32_t r = mask; r != 0u; r &= r - 1u) list[at++] = (uint16_t)(lane * ADJ_TILE + __builtin_ctz(r));
-            if (lane == 63) npairs = run;
+        const uint32_t mask = A.deep_mask[D.item * 64 + lane];
+        const int cnt = __popc(mask);
+        int at = cnt;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(at, d);
+            if (lane >= d) at += v;
         }
-        for (int q = tid; q < 64 * DEEP_NK; q += 256) (&kip[0][0])[q] = 0.0;
-        for (int q = tid; q < ADJ_TILE * 9; q += 256) (&kjp[0][0])[q] = 0.0;
+        at -= cnt;
         __syncthreads();
-        const int n = npairs;
-        for (int base = 0; base < n; base += 16) {
-            if (base + grp < n) {
-                const int e = list[base + grp];
-                const int i = iw * 64 + e / ADJ_TILE, j = j0 + e % ADJ_TILE;
-                const int level = reported_level(A, M.conv[I2_NOT_NEIGHBORS][task_disjoint(M, i, j)], K);
-                deep_pair(A, R, M, i, j, level, tid & 15, rec[grp]);
-            }
-            __syncthreads();
-            const int nb = min(16, n - base);
-            for (int q = 0; q < nb; ++q) {   // in the pairs' order
-                const int e = list[base + q];
-                if (tid < 64) {
-                    if (e / ADJ_TILE == tid) for (int c = 0; c < DEEP_NK; ++c) kip[tid][c] += rec[q][c];
-                } else if (tid < 64 + ADJ_TILE) {
-                    if (e % ADJ_TILE == tid - 64) for (int c = 0; c < 9; ++c) kjp[tid - 64][c] += rec[q][DEEP_NK + c];
+        masks[lane] = mask;
+        starts[lane] = at;
+        __syncthreads();
+        double ki[DEEP_NK] = {}, kj[9] = {};
+        if (D.base + D.n <= A.deep_cap) {
+            const double* rec0 = A.deep_rec + D.base * DEEP_REC;
+            for (int q = 0; q < cnt; ++q)
+                for (int c = 0; c < DEEP_NK; ++c) ki[c] += rec0[(int64_t)(at + q) * DEEP_REC + c];
+            for (uint64_t some = __ballot(mask != 0u); some != 0ull; some &= some - 1ull) {
+                const int l = (int)__builtin_ctzll(some);
+                const uint32_t lm = masks[l];
+                if (lane < ADJ_TILE && ((lm >> lane) & 1u)) {
+                    const double* r = rec0 + (int64_t)(starts[l] + __popc(lm & ((1u << lane) - 1u))) * DEEP_REC + DEEP_NK;
+                    for (int c = 0; c < 9; ++c) kj[c] += r[c];
                 }
             }
+        } else {
+            if (!loaded) { load_rule_sh(R, A.rule); loaded = true; }
+            const int K = M.K[I2_NOT_NEIGHBORS];
+            int k = at;
+            for (uint32_t r = mask; r != 0u; r &= r - 1u) list[k++] = (uint16_t)(lane * ADJ_TILE + __builtin_ctz(r));
             __syncthreads();
+            for (int first = 0; first < D.n; first += 4) {
+                const int row = lane >> 4, q = first + row;
+                const int e = list[min(q, D.n - 1)];
+                const int i = iw * 64 + e / ADJ_TILE, j = j0 + e % ADJ_TILE;
+                const int level = q < D.n ? reported_level(A, M.conv[I2_NOT_NEIGHBORS][task_disjoint(M, i, j)], K) : 0;
+                if (level == 2) deep_pair<16>(A, R, M, i, j, level, lane & 15, rec[row]);
+                for (int r = 0; r < 4; ++r) {
+                    const int wl = __builtin_amdgcn_readlane(level, 16 * r);
+                    if (wl > 2)
+                        deep_pair<64>(A, R, M, __builtin_amdgcn_readlane(i, 16 * r), __builtin_amdgcn_readlane(j, 16 * r), wl, lane, rec[r]);
+                }
+                __syncthreads();
+                for (int r = 0; r < 4 && first + r < D.n; ++r) {
+                    const int f = list[first + r];
+                    if (lane == f / ADJ_TILE) for (int c = 0; c < DEEP_NK; ++c) ki[c] += rec[r][c];
+                    if (lane == f % ADJ_TILE) for (int c = 0; c < 9; ++c) kj[c] += rec[r][DEEP_NK + c];
+                }
+                __syncthreads();
+            }
         }
-        if (tid < 64) {
-            if (mask != 0u) {
-                const int i = iw * 64 + lane;
-                const double* v = kip[lane];
-                d3 X0 = {v[0], v[1], v[2]}, X1 = {v[3], v[4], v[5]}, X2 = {v[6], v[7], v[8]};
-                const Panel I = M.panels[i];
-                const d3 zero = {0.0, 0.0, 0.0};
-                panel_chain(I, zero, zero, zero, zero, v[9], X0, X1, X2);
-                double* kslot = M.ki + ((int64_t)jt * M.nT + i) * 9;
-                add_to3(kslot, X0); add_to3(kslot + 3, X1); add_to3(kslot + 6, X2);
-            }
-            const double loss = wsum(kip[lane][10]);
-            if (lane == 0) A.item_loss[item] += loss;
-        } else if (tid < 128) {
-            // the j of the tile that hold a pair of the item (OR of the lanes' masks)
-            uint32_t anyj = mask;
-            for (int d = 1; d < 64; d <<= 1) anyj |= (uint32_t)__shfl_xor((int)anyj, d);
-            if (lane < ADJ_TILE && ((anyj >> lane) & 1u)) {
-                double* kslot = M.kj + ((int64_t)iw * M.nT + j0 + lane) * 9;
-                for (int c = 0; c < 9; ++c) kslot[c] += kjp[lane][c];
-            }
+        if (mask != 0u) {
+            const int i = iw * 64 + lane;
+            d3 X0 = {ki[0], ki[1], ki[2]}, X1 = {ki[3], ki[4], ki[5]}, X2 = {ki[6], ki[7], ki[8]};
+            const Panel I = M.panels[i];
+            const d3 zero = {0.0, 0.0, 0.0};
+            panel_chain(I, zero, zero, zero, zero, ki[9], X0, X1, X2);
+            double* kslot = M.ki + ((int64_t)jt * M.nT + i) * 9;
+            add_to3(kslot, X0); add_to3(kslot + 3, X1); add_to3(kslot + 6, X2);
+        }
+        const double loss = wsum(ki[10]);
+        if (lane == 0) A.item_loss[D.item] += loss;
+        // the j of the tile that hold a pair of the item (OR of the lanes' masks)
+        uint32_t anyj = mask;
+        for (int d = 1; d < 64; d <<= 1) anyj |= (uint32_t)__shfl_xor((int)anyj, d);
+        if (lane < ADJ_TILE && ((anyj >> lane) & 1u)) {
+            double* kslot = M.kj + ((int64_t)iw * M.nT + j0 + lane) * 9;
+            for (int c = 0; c < 9; ++c) kslot[c] += kj[c];
         }
     }
 }
@@ -555,22 +615,57 @@ __device__ __forceinline__ double dd(d3 bar, D3 x) { return bar.x * x.x.d + bar.
 template <class T>
 __device__ __forceinline__ T pick3(int s, const T& a, const T& b, const T& c) { return s == 0 ? a : (s == 1 ? b : c); }
 
-struct SingBars {
-    TPBar g;          // thetaPsi parameters (K_j vertices, tangents)
-    EdgeBar ge;       // edge-sharing context
-    VertexBar gv;     // vertex-sharing context
-    d3 X[3];          // K_i vertices (through the quadrature points)
-    q4 F;             // sum_k w_k f
-};
-
-template <int TYPE>
+// One singular task by G lanes (16: a row of the wavefront, four tasks at a
+// time; 64).  Two loops over the points, the inner integral's and then the
+// singular part's, so that one set of sums and of geometry is live at a time:
+// with both in one loop the kernel held 512 registers, one wavefront per SIMD.
+// Points are found from their number alone (sub_point): vertices of sub-panels
+// kept over the rule's points made it spill.
+// What belongs to the whole pair (closed-form integral, normals, areas) follows
+// in k_adj_singular_dual, which has the closed form's value beside its
+// derivatives.
+template <int TYPE, int G>
 __device__ __forceinline__ void singular_task(const AdjArgs& A, const RuleSh& R, const AdjMesh& M, int64_t t, int i, int j,
-                                              int level, int lane) {
-    const Panel I = uniform_panel(M.panels[i]);   // one wavefront per pair
-    const Panel J = uniform_panel(M.panels[j]);
-    const Weights W = weights(A.seed, i, j, M.nT, &R.lt);
-    const q4 gb = task_cotangent(W, J.n);
-    const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
+                                              int level, int s) {
+    const Panel I = M.panels[i];
+    const int npts = A.rule.n;
+    const uint32_t total = (uint32_t)npts << (2 * level);
+    const uint32_t magic = (uint32_t)((0x100000000ull + npts - 1) / npts);   // q / npts for q <= 2^28
+    double fa = I.area;
+    for (int l = 0; l < level; ++l) fa *= 0.25;
+    // one of the pair's four draws per lane of a quad
+    const double draw = normal_draw(A.seed, (uint64_t)i * (uint64_t)M.nT + (uint64_t)j, (uint64_t)(s & 3), &R.lt);
+    const Weights W = {quad_lane(draw, 0), {quad_lane(draw, 1), quad_lane(draw, 2), quad_lane(draw, 3)}};
+    SingRec& r = A.sing_rec[t];
+    q4 gb, F;
+    d3 X0 = {0.0, 0.0, 0.0}, X1 = X0, X2;
+    {
+        const Panel J = M.panels[j];
+        gb = task_cotangent(W, J.n);
+        const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
+        const d3 gP = {gb.x, gb.y, gb.z};
+        const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
+        TermsBar g = terms_bar_zero();
+        for (uint32_t q = s; q < total; q += G) {
+            const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+            const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
+            const d3 p = beta.x * I.a + beta.y * I.b + beta.z * I.c;
+            const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
+            axpy(X0, beta.x, pb); axpy(X1, beta.y, pb);
+        }
+        group_sum3<G>(g.a); group_sum3<G>(g.b); group_sum3<G>(g.c); group_sum3<G>(g.n); group_sum3<G>(X0); group_sum3<G>(X1);
+        g.T = {group_sum<G>(g.T.x), group_sum<G>(g.T.y), group_sum<G>(g.T.z), group_sum<G>(g.T.w)};
+        g.y = group_sum<G>(g.y); g.La = group_sum<G>(g.La); g.Lb = group_sum<G>(g.Lb); g.Lc = group_sum<G>(g.Lc);
+        F = psi_of_terms(g.T, JG);
+        X2 = g.a + g.b + g.c;
+        axpy(X2, g.y, JG.N2);
+        X2 = X2 - X0 - X1;
+        d3 Ab, Bb, Cb;
+        terms_chain(JG, ct, g, fa * gP, d3{0.0, 0.0, 0.0}, i2m::rcp_cubic(JG.La), i2m::rcp_cubic(JG.Lb), i2m::rcp_cubic(JG.Lc),
+                    i2m::rcp_cubic(2.0 * J.area), J.n, Ab, Bb, Cb);
+        if (s == 0) { r.g[0] = Ab; r.g[1] = Bb; r.g[2] = Cb; }
+    }
+    const Panel J = M.panels[j];
     int s1, s2;
     EdgeCtx ec;
     VertexCtx vc;
@@ -581,87 +676,65 @@ __device__ __forceinline__ void singular_task(const AdjArgs& A, const RuleSh& R,
         shifts_vertex(I, J, &s1, &s2);
         vc = vertex_ctx(vtx(J, s2), vtx(J, (s2 + 1) % 3), vtx(J, (s2 + 2) % 3), I.n, J.n, I.area);
     }
-    double fa = I.area;
-    for (int l = 0; l < level; ++l) fa *= 0.25;
     const d3 z3 = {0.0, 0.0, 0.0};
-    SingBars B;
-    B.g = {z3, z3, z3, z3, z3, z3};
-    B.ge = {z3, z3, z3, z3, z3, 0.0};
-    B.gv = {z3, z3, z3, z3, 0.0};
-    B.X[0] = B.X[1] = B.X[2] = z3;
-    B.F = q4zero();
-    const int npts = A.rule.n;
-    const int64_t total = (int64_t)npts << (2 * level);
-    for (int64_t q = lane; q < total; q += 64) {
-        const uint32_t sub = (uint32_t)(q / npts);
-        const int k = (int)(q % npts);
+    EdgeBar ge = {z3, z3, z3, z3, z3, 0.0};
+    VertexBar gv = {z3, z3, z3, z3, 0.0};
+    q4 Fs = q4zero();
+    d3 Y0 = z3, Y1 = z3;
+    for (uint32_t q = s; q < total; q += G) {
+        const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+        // these derivatives amplify the point's rounding: it comes from the
+        // sub-panel's vertices, as in the quadrature
         d3 a = I.a, b = I.b, c = I.c;
         sub_panel(a, b, c, level, sub);
-        d3 ba = {1.0, 0.0, 0.0}, bb = {0.0, 1.0, 0.0}, bc = {0.0, 0.0, 1.0};
-        sub_panel(ba, bb, bc, level, sub);
         d3 p = R.L1[k] * a;
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
-        const q4 gp = (fa * R.w[k]) * gb;
-        const q4 gm = (-1.0) * gp;
-        d3 pb, ps;
-        q4 f = theta_psi_fast_rev(p, JG, &R.lt, gp, &pb, B.g);
-        if (TYPE == I2_ATTACHED_NEIGHBORS) f = f - sing_edge_rev(p, ec, gm, &ps, B.ge);
-        else f = f - sing_vertex_rev(p, vc, gm, &ps, B.gv);
-        pb = pb + ps;
-        B.F = B.F + R.w[k] * f;
-        const d3 beta = R.L1[k] * ba + R.L2[k] * bb + R.L3[k] * bc;
-        axpy(B.X[0], beta.x, pb); axpy(B.X[1], beta.y, pb); axpy(B.X[2], beta.z, pb);
+        const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
+        const q4 gm = -(fa * R.w[k]) * gb;
+        d3 ps;
+        const q4 f = TYPE == I2_ATTACHED_NEIGHBORS ? sing_edge_rev(p, ec, &R.lt, gm, &ps, ge) : sing_vertex_rev(p, vc, &R.lt, gm, &ps, gv);
+        Fs = Fs + R.w[k] * f;
+        axpy(Y0, beta.x, ps); axpy(Y1, beta.y, ps);
     }
-    wsum3(B.g.a); wsum3(B.g.b); wsum3(B.g.c); wsum3(B.g.ta); wsum3(B.g.tb); wsum3(B.g.tc);
-    wsum3(B.X[0]); wsum3(B.X[1]); wsum3(B.X[2]); wsum4(B.F);
+    group_sum3<G>(Y0); group_sum3<G>(Y1);
+    Fs = {group_sum<G>(Fs.x), group_sum<G>(Fs.y), group_sum<G>(Fs.z), group_sum<G>(Fs.w)};
+    d3 Y2;
     if (TYPE == I2_ATTACHED_NEIGHBORS) {
-        wsum3(B.ge.JB); wsum3(B.ge.JC); wsum3(B.ge.taua); wsum3(B.ge.taub); wsum3(B.ge.tauc); B.ge.ilvc = wsum(B.ge.ilvc);
+        group_sum3<G>(ge.JB); group_sum3<G>(ge.JC); group_sum3<G>(ge.taua); group_sum3<G>(ge.taub); group_sum3<G>(ge.tauc);
+        ge.ilvc = group_sum<G>(ge.ilvc) / ec.ilvc;
+        Y2 = -(ge.JB + ge.JC) - Y0 - Y1;      // the points' cotangents are minus the vertices'
     } else {
-        wsum3(B.gv.JA); wsum3(B.gv.taua); wsum3(B.gv.taub); wsum3(B.gv.e); B.gv.invAri = wsum(B.gv.invAri);
+        group_sum3<G>(gv.JA); group_sum3<G>(gv.taua); group_sum3<G>(gv.taub); group_sum3<G>(gv.e);
+        gv.invAri = group_sum<G>(gv.invAri) / vc.invAri;
+        Y2 = -gv.JA - Y0 - Y1;
     }
-    // whole-pair values (uniform over the wavefront)
-    q4 sing;
-    if (TYPE == I2_ATTACHED_NEIGHBORS)
-        sing = integrate_sing_edge(vtx(I, s1), vtx(I, (s1 + 1) % 3), vtx(I, (s1 + 2) % 3),
-                                   vtx(J, s2), vtx(J, (s2 + 1) % 3), vtx(J, (s2 + 2) % 3), I.n, J.n, I.area);
-    else
-        sing = integrate_sing_vertex(vtx(I, s1), vtx(I, (s1 + 1) % 3), vtx(I, (s1 + 2) % 3),
-                                     vtx(J, s2), vtx(J, (s2 + 1) % 3), vtx(J, (s2 + 2) % 3), I.n, J.n, I.area);
-    const q4 Iv = fa * B.F + sing;
-    const int pw = TYPE == I2_SIMPLE_NEIGHBORS ? wrap_count(Iv.w, I.area) : 0;
-    const d3 Jr = TYPE == I2_SIMPLE_NEIGHBORS ? finalize_vertex_p(Iv, J.n, I.area, pw) : finalize_plain(Iv, J.n);
-    const d3 psi = {Iv.x, Iv.y, Iv.z};
-    const double thetaw = Iv.w + 2.0 * pw * (TWO_PI * I.area);
-    const d3 nb = RECIP_4PI * (thetaw * W.v + cross(W.v, psi));
-    const double Sb = dot4(gb, B.F) * (fa / I.area) + (TYPE == I2_SIMPLE_NEIGHBORS ? pw * dot(W.v, J.n) : 0.0);
-    // the per-task chain runs in k_adj_singular_dual, one coordinate per lane
-    if (lane == 0) {
-        SingRec& r = A.sing_rec[t];
+    if (s == 0) {
         r.i = i; r.j = j; r.s1 = s1; r.s2 = s2;
-        r.g[0] = B.g.a; r.g[1] = B.g.b; r.g[2] = B.g.c; r.g[3] = B.g.ta; r.g[4] = B.g.tb; r.g[5] = B.g.tc;
         if (TYPE == I2_ATTACHED_NEIGHBORS) {
-            r.cb[0] = B.ge.JB; r.cb[1] = B.ge.JC; r.cb[2] = B.ge.taua; r.cb[3] = B.ge.taub; r.cb[4] = B.ge.tauc;
-            r.cs = B.ge.ilvc;
+            r.cb[0] = ge.JB; r.cb[1] = ge.JC; r.cb[2] = ge.taua; r.cb[3] = ge.taub; r.cb[4] = ge.tauc;
+            r.cs = ge.ilvc;
         } else {
-            r.cb[0] = B.gv.JA; r.cb[1] = B.gv.taua; r.cb[2] = B.gv.taub; r.cb[3] = B.gv.e; r.cb[4] = {0.0, 0.0, 0.0};
-            r.cs = B.gv.invAri;
+            r.cb[0] = gv.JA; r.cb[1] = gv.taua; r.cb[2] = gv.taub; r.cb[3] = gv.e; r.cb[4] = z3;
+            r.cs = gv.invAri;
         }
-        r.X[0] = B.X[0]; r.X[1] = B.X[1]; r.X[2] = B.X[2];
-        r.nb = nb;
-        r.Sb = Sb;
+        r.X[0] = X0 + Y0; r.X[1] = X1 + Y1; r.X[2] = X2 + Y2;
+        r.F = F - Fs;
+        r.fa = fa;
         r.gb = gb;
-        r.loss = W.w * Iv.w + dot(W.v, Jr);
+        r.w = W.w;
+        r.v = W.v;
     }
 }
 
 // Forward mode along coordinate d = 3 * slot + axis (slots 0..2 = K_i's,
 // 3..5 = K_j's vertices) of a singular task's per-task chain: panel normals,
 // area and tangents, the singular context and the closed-form singular
-// integral, weighted by the cotangents the point loop left in the record.
-// Returns the task's whole dL/d(coordinate d).
+// integral, weighted by the cotangents the point loop left in the record and
+// those of the pair's values, which the closed form's value completes.  Returns
+// the task's whole dL/d(coordinate d), and in `loss` the task's term of L.
 template <int TYPE>
-__device__ __forceinline__ double singular_chain(const AdjMesh& M, const SingRec& r, int d) {
+__device__ __forceinline__ double singular_chain(const AdjMesh& M, const SingRec& r, int d, double* loss) {
     const Panel I = M.panels[r.i];
     const Panel J = M.panels[r.j];
     const int s1 = r.s1, s2 = r.s2;
@@ -671,13 +744,11 @@ __device__ __forceinline__ double singular_chain(const AdjMesh& M, const SingRec
     const D3 cri = cross(ib - ia, ic - ia), crj = cross(jb - ja, jc - ja);
     const D3 nI = unit(cri), nJ = unit(crj);
     const Dual SI = vlen(cri) * Dual(0.5);
-    const D3 ta = unit(jc - jb), tb = unit(ja - jc), tc = unit(jb - ja);
     const D3 i0 = pick3(s1, ia, ib, ic), i1 = pick3((s1 + 1) % 3, ia, ib, ic), i2v = pick3((s1 + 2) % 3, ia, ib, ic);
     const D3 j0 = pick3(s2, ja, jb, jc), j1 = pick3((s2 + 1) % 3, ja, jb, jc), j2 = pick3((s2 + 2) % 3, ja, jb, jc);
     double dl = 0.0;
     const d3 gx = pick3(slot % 3, slot < 3 ? r.X[0] : r.g[0], slot < 3 ? r.X[1] : r.g[1], slot < 3 ? r.X[2] : r.g[2]);
     dl += (axis == 0 ? gx.x : (axis == 1 ? gx.y : gx.z));
-    dl += dd(r.g[3], ta) + dd(r.g[4], tb) + dd(r.g[5], tc) + dd(r.nb, nJ) + r.Sb * SI.d;
     Q4 sd;
     if (TYPE == I2_ATTACHED_NEIGHBORS) {
         const EdgeCtxT<Dual> c = edge_ctx(j0, j1, j2);
@@ -691,16 +762,36 @@ __device__ __forceinline__ double singular_chain(const AdjMesh& M, const SingRec
     }
     const q4 gb = r.gb;
     dl += gb.x * sd.x.d + gb.y * sd.y.d + gb.z * sd.z.d + gb.w * sd.w.d;
+    const q4 Iv = r.fa * r.F + q4{sd.x.v, sd.y.v, sd.z.v, sd.w.v};
+    const int pw = TYPE == I2_SIMPLE_NEIGHBORS ? wrap_count(Iv.w, I.area) : 0;
+    const d3 Jr = TYPE == I2_SIMPLE_NEIGHBORS ? finalize_vertex_p(Iv, J.n, I.area, pw) : finalize_plain(Iv, J.n);
+    const d3 psi = {Iv.x, Iv.y, Iv.z};
+    const double thetaw = Iv.w + 2.0 * pw * (TWO_PI * I.area);
+    const d3 nb = RECIP_4PI * (thetaw * r.v + cross(r.v, psi));
+    const double Sb = dot4(gb, r.F) * (r.fa / I.area) + (TYPE == I2_SIMPLE_NEIGHBORS ? pw * dot(r.v, J.n) : 0.0);
+    dl += dd(nb, nJ) + Sb * SI.d;
+    *loss = r.w * Iv.w + dot(r.v, Jr);
     return dl;
 }
 
-__global__ __launch_bounds__(ADJ_BLOCK) void k_adj_singular(AdjArgs A) {
+// The singular tasks in three launches, by their reported level: STEP 0 takes
+// those at levels 0 and 1, 16 lanes each (52 points of the 13-point rule in
+// four rounds), and lists the others, the list's start for level 2 and its end
+// for the rest; STEP 1 takes level 2, 16 lanes each (208 points in 13 rounds),
+// STEP 2 the rest, a wavefront each (832 points in 13 rounds).  Every task has
+// a record of its own, so the lists' order does not matter.
+template <int STEP>
+__global__ __launch_bounds__(ADJ_BLOCK) I2_TWO_WAVES void k_adj_singular(AdjArgs A) {
     __shared__ RuleSh R;
+    constexpr int G = STEP == 2 ? 64 : 16;
+    const int64_t groups = (int64_t)gridDim.x * (ADJ_BLOCK / G), g0 = (int64_t)blockIdx.x * (ADJ_BLOCK / G);
+    const int64_t count = STEP == 0 ? A.singular_tasks : (int64_t)A.counters[2 + STEP];
+    if (g0 >= count) return;
     load_rule_sh(R, A.rule);
     __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int waves = ADJ_BLOCK / 64;
-    for (int64_t t = (int64_t)blockIdx.x * waves + threadIdx.x / 64; t < A.singular_tasks; t += (int64_t)gridDim.x * waves) {
+    const int s = threadIdx.x & (G - 1);
+    for (int64_t e = g0 + threadIdx.x / G; e < count; e += groups) {
+        const int64_t t = STEP == 0 ? e : A.sing_deep[STEP == 1 ? e : A.singular_tasks - 1 - e];
         const int b = find_base_a(A.sing_base, 2 * A.nmeshes, t);
         const int type = b / A.nmeshes == 0 ? I2_SIMPLE_NEIGHBORS : I2_ATTACHED_NEIGHBORS;
         const AdjMesh& M = A.meshes[b % A.nmeshes];
@@ -709,10 +800,17 @@ __global__ __launch_bounds__(ADJ_BLOCK) void k_adj_singular(AdjArgs A) {
         const int32_t* L = M.lists[type];
         const int64_t k = z < n ? z : z - n;
         int i = L[3 * k], j = L[3 * k + 1];
-        if (z >= n) { const int s = i; i = j; j = s; }
+        if (z >= n) { const int x = i; i = j; j = x; }
         const int level = reported_level(A, M.conv[type][z], M.K[type]);
-        if (type == I2_ATTACHED_NEIGHBORS) singular_task<I2_ATTACHED_NEIGHBORS>(A, R, M, t, i, j, level, lane);
-        else singular_task<I2_SIMPLE_NEIGHBORS>(A, R, M, t, i, j, level, lane);
+        if (STEP == 0 && level >= 2) {
+            if (s == 0) {
+                if (level == 2) A.sing_deep[atomicAdd(&A.counters[3], 1ull)] = t;
+                else A.sing_deep[A.singular_tasks - 1 - (int64_t)atomicAdd(&A.counters[4], 1ull)] = t;
+            }
+            continue;
+        }
+        if (type == I2_ATTACHED_NEIGHBORS) singular_task<I2_ATTACHED_NEIGHBORS, G>(A, R, M, t, i, j, level, s);
+        else singular_task<I2_SIMPLE_NEIGHBORS, G>(A, R, M, t, i, j, level, s);
     }
 }
 
@@ -726,29 +824,46 @@ __global__ __launch_bounds__(ADJ_BLOCK) void k_adj_singular_dual(AdjArgs A) {
         const int b = find_base_a(A.sing_base, 2 * A.nmeshes, t);
         const AdjMesh& M = A.meshes[b % A.nmeshes];
         const SingRec& r = A.sing_rec[t];
-        A.sing_dl[g] = (b / A.nmeshes == 0) ? singular_chain<I2_SIMPLE_NEIGHBORS>(M, r, d)
-                                            : singular_chain<I2_ATTACHED_NEIGHBORS>(M, r, d);
+        double loss;
+        A.sing_dl[g] = (b / A.nmeshes == 0) ? singular_chain<I2_SIMPLE_NEIGHBORS>(M, r, d, &loss)
+                                            : singular_chain<I2_ATTACHED_NEIGHBORS>(M, r, d, &loss);
+        if (d == 0) A.sing_rec[t].loss = loss;
     }
 }
 
-// The slots of each panel vertex coordinate, one thread per (panel, 9
-// coordinates): its tiles as the control panel, then its wavefronts of
-// control panels as the influencing panel.
-__global__ void k_adj_panel_sum(AdjArgs A) {
+// The slots of each panel vertex coordinate: its tiles as the control panel,
+// then its wavefronts of control panels as the influencing panel.  A workgroup
+// takes 16 consecutive (panel, coordinate)s, 16 threads each: thread s adds
+// slots s, s + 16, ..., and a fixed tree adds the threads.  The slots are read
+// once and lines of 16 values at a time; one thread per coordinate left 325
+// loads in series, 82 us for 320 panels.
+__global__ __launch_bounds__(256) void k_adj_panel_sum(AdjArgs A) {
+    __shared__ double part[16][17];
     const int64_t total = 9 * A.npanels;
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t gp = q / 9;
-        const int comp = (int)(q - 9 * gp);
-        const int m = find_base_a(A.pbase, A.nmeshes, gp);
-        const AdjMesh& M = A.meshes[m];
-        const int64_t p = gp - A.pbase[m];
+    const int c = threadIdx.x & 15, s = threadIdx.x >> 4;
+    for (int64_t q0 = 16 * (int64_t)blockIdx.x; q0 < total; q0 += 16 * (int64_t)gridDim.x) {
+        const int64_t q = q0 + c;
         double acc = 0.0;
-        const int64_t stride = 9 * (int64_t)M.nT;
-        const double* ki = M.ki + 9 * p + comp;
-        for (int t = 0; t < M.jtiles; ++t) acc += ki[stride * t];
-        const double* kj = M.kj + 9 * p + comp;
-        for (int t = 0; t < M.niw; ++t) acc += kj[stride * t];
-        A.psum[q] = acc;
+        if (q < total) {
+            const int64_t gp = q / 9;
+            const int comp = (int)(q - 9 * gp);
+            const int m = find_base_a(A.pbase, A.nmeshes, gp);
+            const AdjMesh& M = A.meshes[m];
+            const int64_t p = gp - A.pbase[m];
+            const int64_t stride = 9 * (int64_t)M.nT;
+            const double* ki = M.ki + 9 * p + comp;
+            for (int t = s; t < M.jtiles; t += 16) acc += ki[stride * t];
+            const double* kj = M.kj + 9 * p + comp;
+            for (int t = s; t < M.niw; t += 16) acc += kj[stride * t];
+        }
+        __syncthreads();
+        part[s][c] = acc;
+        __syncthreads();
+        for (int h = 8; h > 0; h >>= 1) {
+            if (s < h) part[s][c] += part[s + h][c];
+            __syncthreads();
+        }
+        if (s == 0 && q < total) A.psum[q] = part[0][c];
     }
 }
 
@@ -822,20 +937,25 @@ __global__ void k_adj_zero(unsigned long long* c, int nc, double* kj, int64_t nk
 
 // ------------------------------------------------------------ host side
 int adjoint_launch(AdjState& S, hipStream_t st) {
-    hipLaunchKernelGGL(k_adj_zero, dim3(4 * S.grid), dim3(256), 0, st, S.d_counters.p, 4, S.d_kj.p, S.kj_total);
+    hipLaunchKernelGGL(k_adj_zero, dim3(4 * S.grid), dim3(256), 0, st, S.d_counters.p, N_ADJ_COUNTERS, S.d_kj.p, S.kj_total);
     I2_TRY(check_launch("k_adj_zero"));
     hipLaunchKernelGGL(k_adj_disjoint, dim3(4 * S.grid), dim3(64), 0, st, S.args);
     I2_TRY(check_launch("k_adj_disjoint"));
-    hipLaunchKernelGGL(k_adj_deep, dim3(S.grid), dim3(256), 0, st, S.args);
+    hipLaunchKernelGGL(k_adj_deep, dim3(16 * S.grid), dim3(256), 0, st, S.args);
     I2_TRY(check_launch("k_adj_deep"));
+    hipLaunchKernelGGL(k_adj_deep_sum, dim3(4 * S.grid), dim3(64), 0, st, S.args);
+    I2_TRY(check_launch("k_adj_deep_sum"));
     if (S.args.singular_tasks > 0) {
-        hipLaunchKernelGGL(k_adj_singular, dim3(S.grid), dim3(ADJ_BLOCK), 0, st, S.args);
+        const int64_t blocks = std::min<int64_t>((S.args.singular_tasks + 15) / 16, 4 * (int64_t)S.grid);
+        hipLaunchKernelGGL(k_adj_singular<0>, dim3((unsigned)blocks), dim3(ADJ_BLOCK), 0, st, S.args);
+        hipLaunchKernelGGL(k_adj_singular<1>, dim3((unsigned)blocks), dim3(ADJ_BLOCK), 0, st, S.args);
+        hipLaunchKernelGGL(k_adj_singular<2>, dim3((unsigned)std::min<int64_t>(4 * blocks, 4 * (int64_t)S.grid)), dim3(ADJ_BLOCK), 0, st, S.args);
         I2_TRY(check_launch("k_adj_singular"));
         hipLaunchKernelGGL(k_adj_singular_dual, dim3(S.grid), dim3(ADJ_BLOCK), 0, st, S.args);
         I2_TRY(check_launch("k_adj_singular_dual"));
     }
     if (S.args.npanels > 0) {
-        const int64_t blocks = std::min<int64_t>((9 * S.args.npanels + 255) / 256, 16 * (int64_t)S.grid);
+        const int64_t blocks = std::min<int64_t>((9 * S.args.npanels + 15) / 16, 16 * (int64_t)S.grid);
         hipLaunchKernelGGL(k_adj_panel_sum, dim3((unsigned)blocks), dim3(256), 0, st, S.args);
         I2_TRY(check_launch("k_adj_panel_sum"));
     }
@@ -1008,6 +1128,8 @@ int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::ve
     A.sing_base = S.d_sing_base.p;
     I2_TRY(S.d_sing_rec.ensure(A.singular_tasks));
     A.sing_rec = S.d_sing_rec.p;
+    I2_TRY(S.d_sing_deep.ensure(A.singular_tasks));
+    A.sing_deep = S.d_sing_deep.p;
     I2_TRY(S.d_sing_dl.ensure(18 * A.singular_tasks));
     A.sing_dl = S.d_sing_dl.p;
     I2_TRY(S.d_item_loss.ensure(A.disjoint_items));
@@ -1018,7 +1140,16 @@ int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::ve
     A.deep_mask = S.d_deep_mask.p;
     I2_TRY(S.d_deep_items.ensure(A.disjoint_items));
     A.deep_items = S.d_deep_items.p;
-    I2_TRY(S.d_counters.ensure(4));
+    // room for every pair of small meshes, 1/64 of the pairs of larger ones (0.6 %
+    // are refined on 1,280 panels, 0.03 % on 5,120), at most 2^20 pairs (168 MB)
+    int64_t pairs = 0;
+    for (int m = 0; m < M; ++m) pairs += 2 * D[m].npairs[I2_NOT_NEIGHBORS];
+    A.deep_cap = std::min<int64_t>(std::min(pairs, std::max<int64_t>(65536, pairs / 64)), (int64_t)1 << 20);
+    I2_TRY(S.d_deep_pairs.ensure(A.deep_cap));
+    I2_TRY(S.d_deep_rec.ensure(DEEP_REC * A.deep_cap));
+    A.deep_pairs = S.d_deep_pairs.p;
+    A.deep_rec = S.d_deep_rec.p;
+    I2_TRY(S.d_counters.ensure(N_ADJ_COUNTERS));
     A.counters = S.d_counters.p;
     return I2_OK;
 }
@@ -1139,12 +1270,14 @@ int i2_host_point_adjoint(int kind, const double* p3, const double* params, cons
     } else if (kind == 1) {
         const EdgeCtx c = {v(0), v(3), v(6), v(9), v(12), params[15]};
         EdgeBar g = {z3, z3, z3, z3, z3, 0.0};
-        f = sing_edge_rev(p, c, gb, &pb, g);
+        f = sing_edge_rev(p, c, &i2m::h_mathtab, gb, &pb, g);
+        g.ilvc /= c.ilvc;
         put(0, g.JB); put(3, g.JC); put(6, g.taua); put(9, g.taub); put(12, g.tauc); parbar[15] = g.ilvc;
     } else if (kind == 2) {
         const VertexCtx c = {v(0), v(3), v(6), v(9), params[12]};
         VertexBar g = {z3, z3, z3, z3, 0.0};
-        f = sing_vertex_rev(p, c, gb, &pb, g);
+        f = sing_vertex_rev(p, c, &i2m::h_mathtab, gb, &pb, g);
+        g.invAri /= c.invAri;
         put(0, g.JA); put(3, g.taua); put(6, g.taub); put(9, g.e); parbar[12] = g.invAri;
     } else if (kind >= 3 && kind <= 5) {
         const d3 A = v(0), B = v(3), C = v(6), cr = cross(B - A, C - A);

@@ -38,15 +38,24 @@ struct AdjMesh {
 // coordinate per lane, in a kernel of its own).
 struct SingRec {
     int i, j, s1, s2;
-    i2d::d3 g[6];       // thetaPsi: K_j vertices a, b, c and tangents ta, tb, tc
+    i2d::d3 g[3];       // inner integral: K_j vertices a, b, c
     i2d::d3 cb[5];      // singular context: JB, JC, tau_a, tau_b, tau_c (edge) or JA, tau_a, tau_b, e (vertex)
     double cs;          // 1/|JC - JB| (edge) or 1/sqrt(S_i) (vertex)
     i2d::d3 X[3];       // K_i vertices through the quadrature points
-    i2d::d3 nb;         // unit normal of K_j
-    double Sb;          // area of K_i
+    i2d::q4 F;          // quadrature sum of the regular part
+    double fa;          // area of a sub-panel of K_i at the task's level
     i2d::q4 gb;         // the task's (Psi, Theta) cotangent
+    double w;           // its weights
+    i2d::d3 v;
     double loss;        // the task's term of L
 };
+
+// a disjoint item with pairs at reported level >= 2: its pairs are entries base
+// to base + n - 1 of the pair list; and such a pair: lane * 32 + bit of its item
+// (up to 2,047) and its level
+struct DeepItem { int64_t item, base; int n; };
+struct DeepPair { int64_t item; int16_t at, level; };
+constexpr int N_ADJ_COUNTERS = 5;
 
 struct AdjArgs {
     const AdjMesh* meshes;
@@ -60,14 +69,18 @@ struct AdjArgs {
     const int64_t* item_base;     // per mesh
     int64_t singular_tasks;       // ordered vertex- and edge-sharing tasks of all meshes
     const int64_t* sing_base;     // [kind * nmeshes + m], kind 0 vertex-, 1 edge-sharing
-    unsigned long long* counters; // [0] disjoint item, [1] items with pairs at level >= 2, [2] claims of those
+    unsigned long long* counters; // [0] disjoint item, [1] items with pairs at level >= 2, [2] those pairs, [3] singular tasks at level 2, [4] above
     SingRec* sing_rec;            // per singular task (singular_tasks entries)
+    int64_t* sing_deep;           // the singular tasks at level 2 from its start, those above from its end (singular_tasks entries)
     double* sing_dl;              // per singular task: dL/d of its 18 vertex coordinates (I's a, b, c, J's a, b, c)
     double* item_loss;            // per disjoint item: its pairs' terms of L
     double* loss_part;            // per mesh: partial sums of L (k_adj_loss_part)
     uint32_t* deep_mask;          // per disjoint item and lane: bit b set if (i, j0 + b) is at reported level >= 2
                                   // (written for the items in deep_items)
-    int64_t* deep_items;          // the disjoint items that hold such a pair, counters[1] of them
+    DeepItem* deep_items;         // the disjoint items that hold such a pair, counters[1] of them
+    DeepPair* deep_pairs;         // their pairs, counters[2] of them, as far as deep_cap entries hold an item's
+    double* deep_rec;             // per entry: the pair's cotangents
+    int64_t deep_cap;
     // the vertex gather: panel sums (9 per panel, mesh m's from pbase[m]);
     // vertices of all meshes (mesh m's from vbase[m]), each with its (panel,
     // corner) incidences (3 p + corner, panels ascending) and its
@@ -99,9 +112,12 @@ struct AdjState {
     DBuf<int64_t> d_pbase, d_vbase, d_inc_start, d_sing_start, d_sing_idx;
     DBuf<int32_t> d_inc;
     DBuf<uint32_t> d_deep_mask;
-    DBuf<int64_t> d_deep_items;
+    DBuf<DeepItem> d_deep_items;
+    DBuf<DeepPair> d_deep_pairs;
+    DBuf<double> d_deep_rec;
     DBuf<unsigned long long> d_counters;
     DBuf<SingRec> d_sing_rec;
+    DBuf<int64_t> d_sing_deep;
     hipEvent_t e0 = nullptr, e1 = nullptr;
 };
 

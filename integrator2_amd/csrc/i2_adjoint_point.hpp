@@ -301,39 +301,50 @@ I2_HD __forceinline__ d3 unit_rev(d3 u, d3 ub) {
 }
 
 // cotangents of the edge-sharing context
+// (ilvc, and VertexBar's invAri: times that constant, d/d log)
 struct EdgeBar { d3 JB, JC, taua, taub, tauc; double ilvc; };
 
-I2_HD __forceinline__ q4 sing_edge_rev(d3 p, const EdgeCtx& c, q4 gb, d3* pbar, EdgeBar& g) {
+// log and atan2 from the tables; reciprocals of quantities that are not small
+// differences by rcp_pos.  The unit vectors and the differences 1 -+ t.(v/l)
+// keep sing_edge's and sing_vertex's operations: their rounding is what these
+// derivatives amplify.
+I2_HD __forceinline__ double log_terms(double x, const i2m::MathTable* __restrict__ lt) {
+    double t = i2m::log_tab_any(x, lt);
+    if (__builtin_expect(!i2m::pos_normal(x), 0)) t = i2m::log_rare(x, lt);
+    return t;
+}
+I2_HD __forceinline__ q4 sing_edge_rev(d3 p, const EdgeCtx& c, const i2m::MathTable* __restrict__ lt, q4 gb, d3* pbar, EdgeBar& g) {
     // ---- forward, as sing_edge
     const d3 pa = p - c.JB, pb = p - c.JC;
     const double lva = vlen(pa), lvb = vlen(pb);
     const d3 va = divs(pa, lva), vb = divs(pb, lvb);
     const double P1 = dot(c.tauc, c.tauc - vb), Q1 = dot(c.tauc, c.tauc - va);
     const double P2 = dot(c.taub, c.taub + va), P3 = dot(c.taua, c.taua - vb);
-    const double l1 = log((lvb * P1) / (lva * Q1));
-    const double l2 = log(lva * P2 * c.ilvc);
-    const double l3 = log(lvb * P3 * c.ilvc);
+    const double l1 = log_terms((lvb * P1) / (lva * Q1), lt);
+    const double l2 = log_terms(lva * P2 * c.ilvc, lt);
+    const double l3 = log_terms(lvb * P3 * c.ilvc, lt);
     q4 r;
     r.x = l1 * c.tauc.x - l2 * c.taub.x - l3 * c.taua.x;
     r.y = l1 * c.tauc.y - l2 * c.taub.y - l3 * c.taua.y;
     r.z = l1 * c.tauc.z - l2 * c.taub.z - l3 * c.taua.z;
     const double y1 = dot(cross(va, c.taub), c.tauc), x1 = dot(c.taub - c.tauc, c.taub + va);
     const double y2 = dot(cross(vb, c.taua), c.tauc), x2 = dot(c.taua - c.tauc, c.taua - vb);
-    r.w = 2.0 * (atan2(y1, x1) - atan2(y2, x2));
+    r.w = 2.0 * (atan2_terms(y1, x1, lt) - atan2_terms(y2, x2, lt));
     // ---- reverse
+    const double ila = i2m::rcp_pos(lva), ilb = i2m::rcp_pos(lvb);
     const d3 gP = {gb.x, gb.y, gb.z};
     const double l1b = dot(gP, c.tauc), l2b = -dot(gP, c.taub), l3b = -dot(gP, c.taua);
     axpy(g.tauc, l1, gP); axpy(g.taub, -l2, gP); axpy(g.taua, -l3, gP);
-    double lvab = -l1b / lva + l2b / lva, lvbb = l1b / lvb + l3b / lvb;
+    const double lvab = (l2b - l1b) * ila, lvbb = (l1b + l3b) * ilb;
     const double P1b = l1b / P1, Q1b = -l1b / Q1, P2b = l2b / P2, P3b = l3b / P3;
-    g.ilvc += (l2b + l3b) / c.ilvc;
+    g.ilvc += l2b + l3b;
     d3 vab = {0.0, 0.0, 0.0}, vbb = vab;
     axpy(g.tauc, P1b, 2.0 * c.tauc - vb); axpy(vbb, -P1b, c.tauc);
     axpy(g.tauc, Q1b, 2.0 * c.tauc - va); axpy(vab, -Q1b, c.tauc);
     axpy(g.taub, P2b, 2.0 * c.taub + va); axpy(vab, P2b, c.taub);
     axpy(g.taua, P3b, 2.0 * c.taua - vb); axpy(vbb, -P3b, c.taua);
     const double th1b = 2.0 * gb.w, th2b = -2.0 * gb.w;
-    const double q1 = 1.0 / (x1 * x1 + y1 * y1), q2 = 1.0 / (x2 * x2 + y2 * y2);
+    const double q1 = i2m::rcp_pos(x1 * x1 + y1 * y1), q2 = i2m::rcp_pos(x2 * x2 + y2 * y2);
     const double y1b = th1b * x1 * q1, x1b = -th1b * y1 * q1;
     const double y2b = th2b * x2 * q2, x2b = -th2b * y2 * q2;
     axpy(vab, y1b, cross(c.taub, c.tauc)); axpy(g.taub, y1b, cross(c.tauc, va)); axpy(g.tauc, y1b, cross(va, c.taub));
@@ -341,8 +352,8 @@ I2_HD __forceinline__ q4 sing_edge_rev(d3 p, const EdgeCtx& c, q4 gb, d3* pbar, 
     axpy(vbb, y2b, cross(c.taua, c.tauc)); axpy(g.taua, y2b, cross(c.tauc, vb)); axpy(g.tauc, y2b, cross(vb, c.taua));
     axpy(g.taua, x2b, (c.taua - vb) + (c.taua - c.tauc)); axpy(g.tauc, -x2b, c.taua - vb); axpy(vbb, -x2b, c.taua - c.tauc);
     // va = pa / |pa|, vb = pb / |pb|
-    d3 pab = (1.0 / lva) * (vab - dot(vab, va) * va);
-    d3 pbb = (1.0 / lvb) * (vbb - dot(vbb, vb) * vb);
+    d3 pab = ila * (vab - dot(vab, va) * va);
+    d3 pbb = ilb * (vbb - dot(vbb, vb) * vb);
     axpy(pab, lvab, va);
     axpy(pbb, lvbb, vb);
     *pbar = pab + pbb;
@@ -354,40 +365,41 @@ I2_HD __forceinline__ q4 sing_edge_rev(d3 p, const EdgeCtx& c, q4 gb, d3* pbar, 
 // cotangents of the vertex-sharing context
 struct VertexBar { d3 JA, taua, taub, e; double invAri; };
 
-I2_HD __forceinline__ q4 sing_vertex_rev(d3 p, const VertexCtx& c, q4 gb, d3* pbar, VertexBar& g) {
+I2_HD __forceinline__ q4 sing_vertex_rev(d3 p, const VertexCtx& c, const i2m::MathTable* __restrict__ lt, q4 gb, d3* pbar, VertexBar& g) {
     // ---- forward, as sing_vertex
     const d3 pc = p - c.JA;
     const double lvc = vlen(pc);
     const d3 o = divs(pc, lvc);
     const double A1 = 1.0 + dot(c.taua, o), B1 = 1.0 - dot(c.taub, o);
-    const double la = log((lvc * A1) * c.invAri);
-    const double lb = log((lvc * B1) * c.invAri);
+    const double la = log_terms((lvc * A1) * c.invAri, lt);
+    const double lb = log_terms((lvc * B1) * c.invAri, lt);
     q4 r;
     r.x = -(la * c.taua.x + lb * c.taub.x);
     r.y = -(la * c.taua.y + lb * c.taub.y);
     r.z = -(la * c.taua.z + lb * c.taub.z);
     const double y1 = dot(cross(o, c.taua), c.e), x1 = dot(c.e - o, c.e - c.taua);
     const double y2 = dot(cross(o, c.taub), c.e), x2 = dot(c.e - o, c.e + c.taub);
-    r.w = 2.0 * (atan2(y1, x1) + atan2(y2, x2));
+    r.w = 2.0 * (atan2_terms(y1, x1, lt) + atan2_terms(y2, x2, lt));
     // ---- reverse
+    const double ilc = i2m::rcp_pos(lvc);
     const d3 gP = {gb.x, gb.y, gb.z};
     const double lab = -dot(gP, c.taua), lbb = -dot(gP, c.taub);
     axpy(g.taua, -la, gP); axpy(g.taub, -lb, gP);
-    const double lvcb = (lab + lbb) / lvc;
-    g.invAri += (lab + lbb) / c.invAri;
+    const double lvcb = (lab + lbb) * ilc;
+    g.invAri += lab + lbb;
     const double A1b = lab / A1, B1b = lbb / B1;
     d3 ob = {0.0, 0.0, 0.0};
     axpy(g.taua, A1b, o); axpy(ob, A1b, c.taua);
     axpy(g.taub, -B1b, o); axpy(ob, -B1b, c.taub);
     const double thb = 2.0 * gb.w;
-    const double q1 = 1.0 / (x1 * x1 + y1 * y1), q2 = 1.0 / (x2 * x2 + y2 * y2);
+    const double q1 = i2m::rcp_pos(x1 * x1 + y1 * y1), q2 = i2m::rcp_pos(x2 * x2 + y2 * y2);
     const double y1b = thb * x1 * q1, x1b = -thb * y1 * q1;
     const double y2b = thb * x2 * q2, x2b = -thb * y2 * q2;
     axpy(ob, y1b, cross(c.taua, c.e)); axpy(g.taua, y1b, cross(c.e, o)); axpy(g.e, y1b, cross(o, c.taua));
     axpy(g.e, x1b, (c.e - c.taua) + (c.e - o)); axpy(ob, -x1b, c.e - c.taua); axpy(g.taua, -x1b, c.e - o);
     axpy(ob, y2b, cross(c.taub, c.e)); axpy(g.taub, y2b, cross(c.e, o)); axpy(g.e, y2b, cross(o, c.taub));
     axpy(g.e, x2b, (c.e + c.taub) + (c.e - o)); axpy(ob, -x2b, c.e + c.taub); axpy(g.taub, x2b, c.e - o);
-    d3 pcb = (1.0 / lvc) * (ob - dot(ob, o) * o);
+    d3 pcb = ilc * (ob - dot(ob, o) * o);
     axpy(pcb, lvcb, o);
     *pbar = pcb;
     g.JA = g.JA - pcb;

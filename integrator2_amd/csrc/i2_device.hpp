@@ -761,6 +761,20 @@ I2_HD __forceinline__ void sub_panel(d3& a, d3& b, d3& c, int level, uint32_t pa
     }
 }
 
+// Barycentric coordinates on the original panel of the point with coordinates
+// b on sub-panel `path`: the splits undone from the last to the first (child 0
+// {m_AB, B, m_BC} takes (x, y, z) to (x/2, (1 + y)/2, z/2), and so on).
+I2_HD __forceinline__ d3 sub_point(d3 b, int level, uint32_t path) {
+    for (int l = 0; l < level; ++l, path >>= 2) {
+        const int ch = path & 3;
+        const double x = 0.5 * b.x, y = fma(0.5, b.y, 0.5), z = 0.5 * b.z;
+        b.x = ch == 0 ? x : (ch == 1 ? z : (ch == 2 ? y : 0.5 - x));
+        b.y = ch == 0 ? y : (ch == 1 ? x : (ch == 2 ? z : 1.0 - y));
+        b.z = ch == 0 ? z : (ch == 1 ? y : (ch == 2 ? x : 0.5 - z));
+    }
+    return b;
+}
+
 // A rule's point on a sub-panel, barycentric on the original panel, with its
 // weight: 32-byte records that the kernels keep in LDS for levels 0 and 1
 // (the rule's points on the panel, then on its four level-1 children).
