@@ -54,12 +54,12 @@ template <> struct PairCtx<I2_SIMPLE_NEIGHBORS> {
 // quadrature point lies near the extension of an edge line of K_j, which
 // moves Runge decisions; both paths therefore take decisions on accurate values.
 // Disjoint pairs sum the inner integral's terms, which the caller converts to
-// (Psi, Theta) once per task.
+// (Psi, Theta) once per task.  Points k0, k0 + step, ...
 template <int TYPE>
 __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, d3 a, d3 b, d3 c, double area,
-                                       const JGeom& J, const PairCtx<TYPE>& ctx) {
+                                       const JGeom& J, const PairCtx<TYPE>& ctx, int k0, int step) {
     q4 acc = q4zero();
-    for (int k = 0; k < R.n; ++k) {
+    for (int k = k0; k < R.n; k += step) {
         d3 p = R.L1[k] * a;
         p = p + R.L2[k] * b;
         p = p + R.L3[k] * c;
@@ -74,13 +74,14 @@ __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, 
 // The same sum of a disjoint pair's far terms over the sub-panels sub, sub + G,
 // ... of `level`, in barycentric coordinates of K_i less 1/3.
 template <bool DISTANT>
-__device__ __forceinline__ q4 quad_far(const Rule& R, int level, int sub, int G, const FarFrame& F, const FarGeom& J) {
+__device__ __forceinline__ q4 quad_far(const Rule& R, int level, int sub, int G, int k0, int step, const FarFrame& F,
+                                       const FarGeom& J) {
     q4 acc = q4zero();
     const double h = 1.0 / 3.0;
     for (uint32_t c = sub; c < (1u << (2 * level)); c += G) {
         d3 a = {1.0 - h, -h, 0.0}, b = {-h, 1.0 - h, 0.0}, o = {-h, -h, 0.0};
         sub_panel(a, b, o, level, c);
-        for (int k = 0; k < R.n; ++k) {
+        for (int k = k0; k < R.n; k += step) {
             const double l1 = R.L1[k], l2 = R.L2[k], l3 = R.L3[k], w = R.w[k];
             const FarPoint Q = far_point(l1 * a.x + l2 * b.x + l3 * o.x, l1 * a.y + l2 * b.y + l3 * o.y, w);
             const q4 t = theta_terms_far<DISTANT>(Q.b0, Q.b1, far_pp(F, Q), J);
@@ -90,19 +91,20 @@ __device__ __forceinline__ q4 quad_far(const Rule& R, int level, int sub, int G,
     return acc;
 }
 
-// Level-`level` value of tasks: lanes per task = 1 << lanes_log2; lane `sub`
-// walks sub-panels sub, sub + G, ... < 4^level; butterfly reduction.
+// Level-`level` value of tasks: lanes per task = 1 << lanes_log2, of which
+// 1 << per_log2 share a sub-panel's points; the groups walk the sub-panels
+// < 4^level; butterfly reduction.
 template <int TYPE, bool IMPLICIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_NOT_NEIGHBORS ? 3 : 2))) void k_level(int64_t nitems, const int32_t* __restrict__ list, TaskSource src,
-                                               const Panel* __restrict__ panels, Rule R, int level, int lanes_log2,
+                                               const Panel* __restrict__ panels, Rule R, int level, int lanes_log2, int per_log2,
                                                double4* __restrict__ out) {
     __shared__ i2m::MathTable lt;
     i2m::fill_mathtab(lt);
     __syncthreads();
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int G = 1 << lanes_log2;
+    const int lanes = 1 << lanes_log2, step = 1 << per_log2, G = lanes >> per_log2;
     const int64_t slot = gid >> lanes_log2;
-    const int sub = (int)(gid & (G - 1));
+    const int sub = (int)(gid & (lanes - 1)) >> per_log2, k0 = (int)(gid & (step - 1));
     const bool active = slot < nitems;
     q4 acc = q4zero();
     int64_t z = 0;
@@ -123,17 +125,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_
         if (form != 0) {
             const FarFrame F = far_frame(I.a, I.b, I.c);
             const FarGeom FG = far_geom(F, JG);
-            acc = area * far_scale(form == 1 ? quad_far<false>(R, level, sub, G, F, FG) : quad_far<true>(R, level, sub, G, F, FG), JG);
+            acc = area * far_scale(form == 1 ? quad_far<false>(R, level, sub, G, k0, step, F, FG)
+                                               : quad_far<true>(R, level, sub, G, k0, step, F, FG), JG);
         } else {
             for (uint32_t c = sub; c < nsub; c += G) {
                 d3 a = I.a, b = I.b, cc = I.c;
                 sub_panel(a, b, cc, level, c);
-                acc = acc + quad_sub<TYPE>(R, &lt, a, b, cc, area, JG, ctx);
+                acc = acc + quad_sub<TYPE>(R, &lt, a, b, cc, area, JG, ctx, k0, step);
             }
         }
         if (TYPE == I2_NOT_NEIGHBORS) acc = psi_of_terms(acc, JG);
     }
-    for (int m = 1; m < G; m <<= 1) {
+    for (int m = 1; m < lanes; m <<= 1) {
         acc.x += __shfl_xor(acc.x, m);
         acc.y += __shfl_xor(acc.y, m);
         acc.z += __shfl_xor(acc.z, m);
@@ -219,17 +222,26 @@ __global__ void k_symmetry(int64_t n, const double* __restrict__ r, double* __re
 }
 
 // ------------------------------------------------------------ host orchestration
+constexpr int64_t LANES_FULL = 524288;   // eight wavefronts per SIMD
 static unsigned blocks_for(int64_t threads, int bs) { return (unsigned)((threads + bs - 1) / bs); }
 
-static int lanes_log2_for(int level) {
-    if (level <= 1) return 0;
-    return std::min(2 * level, 6);   // 16 lanes at level 2, a wavefront from level 3
+// Lanes per task of k_level: one for levels 0 and 1, 16 at level 2, a wavefront
+// from level 3; more while the launch leaves most of the chip without work, down
+// to one point per lane.  A lane repeats the pair's geometry, so few lanes are
+// better once the chip is full.  Plain run of 80 panels 375 us with the fewest
+// lanes, 249, 228 and 254 with the line at 2, 8 and 32 wavefronts per SIMD.
+static int lanes_log2_for(int level, int64_t items) {
+    int ll = level <= 1 ? 0 : std::min(2 * level, 6);
+    const int most = std::min(2 * level + 4, 6);
+    while (ll + 2 <= most && (items << (ll + 2)) <= LANES_FULL) ll += 2;
+    return ll;
 }
+static int per_log2_for(int level, int lanes_log2) { return std::max(0, lanes_log2 - 2 * level); }
 
 template <int TYPE, bool IMPLICIT>
 static int launch_level(i2_evaluator* ev, int64_t nitems, const int32_t* list, const TaskSource& src, int level, double4* out) {
     if (nitems == 0) return I2_OK;
-    const int ll = lanes_log2_for(level);
+    const int ll = lanes_log2_for(level, nitems);
     const int64_t threads = nitems << ll;
     LaunchRecord rec{TYPE, level, nitems, nullptr, nullptr};
     if (ev->profile) {
@@ -238,7 +250,7 @@ static int launch_level(i2_evaluator* ev, int64_t nitems, const int32_t* list, c
         I2_HIP(hipEventRecord(rec.e0, ev->stream));
     }
     hipLaunchKernelGGL((k_level<TYPE, IMPLICIT>), dim3(blocks_for(threads, 256)), dim3(256), 0, ev->stream, nitems, list, src,
-                       ev->mesh->d_panels.p, ev->integ->rule, level, ll, out);
+                       ev->mesh->d_panels.p, ev->integ->rule, level, ll, per_log2_for(level, ll), out);
     I2_TRY(check_launch("k_level"));
     if (ev->profile) {
         I2_HIP(hipEventRecord(rec.e1, ev->stream));
@@ -255,64 +267,153 @@ static void clear_launches(i2_evaluator* ev) {
     ev->launches.clear();
 }
 
-template <int TYPE, bool IMPLICIT>
-static int run_type(i2_evaluator* ev, TypeState& ts, const TaskSource& src) {
+static int launch_level_of(i2_evaluator* ev, int type, bool implicit, int64_t nitems, const int32_t* list, const TaskSource& src,
+                           int level, double4* out) {
+    if (type == I2_SIMPLE_NEIGHBORS) return launch_level<I2_SIMPLE_NEIGHBORS, false>(ev, nitems, list, src, level, out);
+    if (type == I2_ATTACHED_NEIGHBORS) return launch_level<I2_ATTACHED_NEIGHBORS, false>(ev, nitems, list, src, level, out);
+    return implicit ? launch_level<I2_NOT_NEIGHBORS, true>(ev, nitems, list, src, level, out)
+                    : launch_level<I2_NOT_NEIGHBORS, false>(ev, nitems, list, src, level, out);
+}
+static int launch_finalize(i2_evaluator* ev, int type, TypeState& ts, const TaskSource& src) {
+    const dim3 grid(blocks_for(ts.n, 256)), block(256);
+    const Panel* panels = ev->mesh->d_panels.p;
+    double4* ints = ts.buf[ts.final_buf].p;
+#define I2_FINALIZE(T, I) hipLaunchKernelGGL((k_finalize<T, I>), grid, block, 0, ev->stream, ts.n, src, panels, ints, ts.results.p)
+    if (type == I2_SIMPLE_NEIGHBORS) I2_FINALIZE(I2_SIMPLE_NEIGHBORS, false);
+    else if (type == I2_ATTACHED_NEIGHBORS) I2_FINALIZE(I2_ATTACHED_NEIGHBORS, false);
+    else if (ts.implicit) I2_FINALIZE(I2_NOT_NEIGHBORS, true);
+    else I2_FINALIZE(I2_NOT_NEIGHBORS, false);
+#undef I2_FINALIZE
+    return check_launch("k_finalize");
+}
+
+// The counters of all levels and the types' flags of unconverged control panels
+__global__ void k_begin_run(unsigned long long* counters, int nc, uint8_t* f0, uint8_t* f1, uint8_t* f2, int nT) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < nc) counters[q] = 0ull;
+    if (q < nT) {
+        if (f0) f0[q] = 0;
+        if (f1) f1[q] = 0;
+        if (f2) f2[q] = 0;
+    }
+}
+
+// Device time of the launches between marks on the evaluator's stream, by type
+struct RunMarks {
+    i2_evaluator* ev;
+    size_t used = 0;
+    std::vector<int> type;           // of the stretch that ends at the mark, -1: none
+    int mark(int t) {
+        if (used == ev->marks.size()) {
+            hipEvent_t e;
+            I2_HIP(hipEventCreate(&e));
+            ev->marks.push_back(e);
+        }
+        I2_HIP(hipEventRecord(ev->marks[used++], ev->stream));
+        type.push_back(t);
+        return I2_OK;
+    }
+    int times() {
+        for (int t = 0; t < 3; ++t) ev->type[t].ms = 0.0;
+        for (size_t q = 1; q < used; ++q) {
+            if (type[q] < 0) continue;
+            float ms = 0.f;
+            I2_HIP(hipEventElapsedTime(&ms, ev->marks[q - 1], ev->marks[q]));
+            ev->type[type[q]].ms += ms;
+        }
+        return I2_OK;
+    }
+};
+
+// The three types' levels in step: level 0 and 1 of each, then one level after
+// the other for the types with tasks left, with one wait per level for the
+// three counts.  A type at a time cost a wait per level and type and a clearing
+// copy per level: a plain run of 80 panels 228 us against 186 in step, of 390
+// 180 and 155.
+static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
     const i2_integrator& it = *ev->integ;
-    const int64_t n = ts.n;
-    ts.K = 0; ts.final_buf = 0; ts.refined_tasks = 0; ts.ms = 0.0;
-    if (n == 0) return I2_OK;
-    if (n > (int64_t)INT32_MAX) { set_error("%lld tasks of one type exceed the plain path's 32-bit task lists", (long long)n); return I2_ERR_RANGE; }
-    I2_TRY(ts.buf[0].ensure(n));
-    I2_TRY(ts.buf[1].ensure(n));
-    I2_TRY(ts.results.ensure(3 * n));
-    I2_TRY(ts.conv.ensure(n));
-    I2_HIP(hipEventRecord(ev->ev0, ev->stream));
-    if (it.fixed) {
-        I2_HIP(hipMemsetAsync(ts.conv.p, it.fixed_level, (size_t)n, ev->stream));
-        I2_TRY((launch_level<TYPE, IMPLICIT>(ev, n, nullptr, src, it.fixed_level, ts.buf[0].p)));
-        ts.refined_tasks = n << (2 * it.fixed_level);
-        ts.K = it.fixed_level;
-        ts.final_buf = 0;
-    } else {
+    const int nT = (int)ev->mesh->nT;
+    RunMarks marks{ev};
+    for (int t = 0; t < 3; ++t) {
+        TypeState& ts = ev->type[t];
+        const int64_t n = ts.n;
+        ts.K = 0; ts.final_buf = 0; ts.refined_tasks = 0; ts.ms = 0.0;
+        if (n == 0) continue;
+        if (n > (int64_t)INT32_MAX) { set_error("%lld tasks of one type exceed the plain path's 32-bit task lists", (long long)n); return I2_ERR_RANGE; }
+        I2_TRY(ts.buf[0].ensure(n));
+        I2_TRY(ts.buf[1].ensure(n));
+        I2_TRY(ts.results.ensure(3 * n));
+        I2_TRY(ts.conv.ensure(n));
+        if (it.fixed) continue;
         I2_TRY(ts.rest[0].ensure(n));
         I2_TRY(ts.rest[1].ensure(n));
-        I2_TRY(ts.unconv.ensure(src.nT));
-        I2_HIP(hipMemsetAsync(ts.conv.p, 0, (size_t)n, ev->stream));
-        I2_HIP(hipMemsetAsync(ts.unconv.p, 0, (size_t)src.nT, ev->stream));
-        I2_TRY((launch_level<TYPE, IMPLICIT>(ev, n, nullptr, src, 0, ts.buf[0].p)));
-        ts.refined_tasks = n;
-        int64_t remaining = n;
-        int iter = 0, cur_rest = 0;
-        while (remaining > 0 && iter < it.max_level) {
-            ++iter;
-            const int32_t* list = (iter == 1) ? nullptr : ts.rest[cur_rest].p;
-            double4* cur = ts.buf[iter % 2].p;
-            double4* prev = ts.buf[(iter - 1) % 2].p;
-            I2_TRY((launch_level<TYPE, IMPLICIT>(ev, remaining, list, src, iter, cur)));
-            ts.refined_tasks += remaining << (2 * iter);
-            I2_HIP(hipMemsetAsync(ev->d_counter.p, 0, sizeof(unsigned long long), ev->stream));
-            hipLaunchKernelGGL(k_compare, dim3(blocks_for(remaining, 256)), dim3(256), 0, ev->stream, remaining, list, cur, prev,
-                               it.rule.pow2p, it.tol, it.quirk ? 0 : 1, iter, ts.conv.p, ts.rest[1 - cur_rest].p, ev->d_counter.p);
-            I2_TRY(check_launch("k_compare"));
-            I2_HIP(hipMemcpyAsync(ev->h_counter, ev->d_counter.p, sizeof(unsigned long long), hipMemcpyDeviceToHost, ev->stream));
-            I2_HIP(hipStreamSynchronize(ev->stream));
-            remaining = (int64_t)*ev->h_counter;
-            cur_rest = 1 - cur_rest;
-        }
-        ts.K = iter;
-        ts.final_buf = iter % 2;
-        if (remaining > 0)   // still unconverged after the comparison at maxLevel (all tasks when maxLevel = 0)
-            I2_TRY(mark_unconverged(ev, IMPLICIT, src, remaining, iter == 0 ? nullptr : ts.rest[cur_rest].p, ts.unconv.p));
+        I2_TRY(ts.unconv.ensure(nT));
     }
-    hipLaunchKernelGGL((k_finalize<TYPE, IMPLICIT>), dim3(blocks_for(n, 256)), dim3(256), 0, ev->stream, n, src,
-                       ev->mesh->d_panels.p, ts.buf[ts.final_buf].p, ts.results.p);
-    I2_TRY(check_launch("k_finalize"));
-    I2_HIP(hipEventRecord(ev->ev1, ev->stream));
-    I2_HIP(hipEventSynchronize(ev->ev1));
-    float ms = 0.f;
-    I2_HIP(hipEventElapsedTime(&ms, ev->ev0, ev->ev1));
-    ts.ms = ms;
-    return I2_OK;
+    I2_TRY(marks.mark(-1));
+    if (it.fixed) {
+        for (int t = 0; t < 3; ++t) {
+            TypeState& ts = ev->type[t];
+            if (ts.n == 0) continue;
+            I2_HIP(hipMemsetAsync(ts.conv.p, it.fixed_level, (size_t)ts.n, ev->stream));
+            I2_TRY(launch_level_of(ev, t, ts.implicit, ts.n, nullptr, src[t], it.fixed_level, ts.buf[0].p));
+            ts.refined_tasks = ts.n << (2 * it.fixed_level);
+            ts.K = it.fixed_level;
+            I2_TRY(launch_finalize(ev, t, ts, src[t]));
+            I2_TRY(marks.mark(t));
+        }
+    } else {
+        const int nc = 3 * (it.max_level + 1);
+        I2_TRY(ev->d_counter.ensure(nc));
+        uint8_t* flags[3];
+        for (int t = 0; t < 3; ++t) flags[t] = ev->type[t].n > 0 ? ev->type[t].unconv.p : nullptr;
+        hipLaunchKernelGGL(k_begin_run, dim3(blocks_for(std::max(nc, nT), 256)), dim3(256), 0, ev->stream, ev->d_counter.p, nc,
+                           flags[0], flags[1], flags[2], nT);
+        I2_TRY(check_launch("k_begin_run"));
+        int64_t remaining[3];
+        int cur_rest[3] = {0, 0, 0};
+        for (int t = 0; t < 3; ++t) remaining[t] = ev->type[t].n;
+        for (int iter = 0; iter <= it.max_level && (remaining[0] > 0 || remaining[1] > 0 || remaining[2] > 0); ++iter) {
+            if (iter > 1) I2_TRY(marks.mark(-1));
+            for (int t = 0; t < 3; ++t) {
+                TypeState& ts = ev->type[t];
+                const int64_t n = remaining[t];
+                if (n == 0) continue;
+                const int32_t* list = iter <= 1 ? nullptr : ts.rest[cur_rest[t]].p;
+                double4* cur = ts.buf[iter % 2].p;
+                I2_TRY(launch_level_of(ev, t, ts.implicit, n, list, src[t], iter, cur));
+                ts.refined_tasks += n << (2 * iter);
+                ts.K = iter;
+                ts.final_buf = iter % 2;
+                if (iter > 0) {
+                    hipLaunchKernelGGL(k_compare, dim3(blocks_for(n, 256)), dim3(256), 0, ev->stream, n, list, cur, ts.buf[1 - iter % 2].p,
+                                       it.rule.pow2p, it.tol, it.quirk ? 0 : 1, iter, ts.conv.p, ts.rest[1 - cur_rest[t]].p,
+                                       ev->d_counter.p + 3 * iter + t);
+                    I2_TRY(check_launch("k_compare"));
+                } else if (it.max_level == 0) {
+                    I2_HIP(hipMemsetAsync(ts.conv.p, 0, (size_t)n, ev->stream));
+                }
+                I2_TRY(marks.mark(t));
+            }
+            if (iter == 0) continue;
+            I2_HIP(hipMemcpyAsync(ev->h_counter, ev->d_counter.p + 3 * iter, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, ev->stream));
+            I2_HIP(hipStreamSynchronize(ev->stream));
+            for (int t = 0; t < 3; ++t) {
+                if (remaining[t] > 0) cur_rest[t] = 1 - cur_rest[t];
+                remaining[t] = (int64_t)ev->h_counter[t];
+            }
+        }
+        I2_TRY(marks.mark(-1));
+        for (int t = 0; t < 3; ++t) {
+            TypeState& ts = ev->type[t];
+            if (ts.n == 0) continue;
+            if (remaining[t] > 0)   // still unconverged after the comparison at maxLevel (all tasks when maxLevel = 0)
+                I2_TRY(mark_unconverged(ev, ts.implicit, src[t], remaining[t], it.max_level == 0 ? nullptr : ts.rest[cur_rest[t]].p, ts.unconv.p));
+            I2_TRY(launch_finalize(ev, t, ts, src[t]));
+            I2_TRY(marks.mark(t));
+        }
+    }
+    I2_HIP(hipStreamSynchronize(ev->stream));
+    return marks.times();
 }
 
 TaskSource task_source(const i2_evaluator* ev, int type) {
@@ -347,19 +448,12 @@ int evaluator_run(i2_evaluator* ev, bool all_pairs, bool check) {
     ev->ran = false;
     ev->all_pairs = all_pairs;
     clear_launches(ev);
-    // types in the reference's order: vertex-sharing, edge-sharing, disjoint (evaluator3d.cu:173-186)
+    // the reference runs the types one after another (evaluator3d.cu:173-186)
+    const TaskSource src[3] = {task_source(ev, 0), task_source(ev, 1), task_source(ev, 2)};
+    for (int t = 0; t < 3; ++t) ev->type[t].has_errors = ev->type[t].refinements_ready = false;
+    I2_TRY(run_types(ev, src));
     for (int t = 0; t < 3; ++t) {
         TypeState& ts = ev->type[t];
-        const TaskSource src = task_source(ev, t);
-        ts.has_errors = false;
-        ts.refinements_ready = false;
-        if (ts.implicit) {
-            I2_TRY((run_type<I2_NOT_NEIGHBORS, true>(ev, ts, src)));
-        } else {
-            if (t == I2_SIMPLE_NEIGHBORS) I2_TRY((run_type<I2_SIMPLE_NEIGHBORS, false>(ev, ts, src)));
-            else if (t == I2_ATTACHED_NEIGHBORS) I2_TRY((run_type<I2_ATTACHED_NEIGHBORS, false>(ev, ts, src)));
-            else I2_TRY((run_type<I2_NOT_NEIGHBORS, false>(ev, ts, src)));
-        }
         if (check && all_pairs && ts.n > 0) {
             I2_TRY(ts.errors.ensure(ts.n));
             const int64_t half = ts.n / 2;
@@ -368,7 +462,7 @@ int evaluator_run(i2_evaluator* ev, bool all_pairs, bool check) {
             ts.has_errors = true;
         }
     }
-    I2_HIP(hipStreamSynchronize(ev->stream));
+    if (check && all_pairs) I2_HIP(hipStreamSynchronize(ev->stream));
     ev->ran = true;
     ev->ran_path = 0;
     ev->run_generation = m->generation;
@@ -465,9 +559,9 @@ static int run_tasks_noalloc(i2_evaluator* ev, const int32_t* d_tasks3, int64_t 
     int32_t* rest[2] = {reinterpret_cast<int32_t*>(S + NOALLOC_REST0), reinterpret_cast<int32_t*>(S + NOALLOC_REST1)};
     unsigned long long* counter = reinterpret_cast<unsigned long long*>(S + NOALLOC_COUNTERS);
     auto level = [&](int64_t items, const int32_t* list, int L, double4* out) {
-        const int ll = lanes_log2_for(L);
+        const int ll = lanes_log2_for(L, items);
         hipLaunchKernelGGL((k_level<TYPE, false>), dim3(blocks_for(items << ll, 256)), dim3(256), 0, st, items, list, src,
-                           panels, it.rule, L, ll, out);
+                           panels, it.rule, L, ll, per_log2_for(L, ll), out);
         return check_launch("k_level");
     };
     int K = 0, final_buf = 0;
@@ -582,8 +676,7 @@ int i2_evaluator_create(i2_evaluator** out, const i2_mesh* m, i2_integrator* it)
     ev->mesh = m;
     ev->integ = it;
     if (hipStreamCreateWithFlags(&ev->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&ev->ev0) != hipSuccess || hipEventCreate(&ev->ev1) != hipSuccess ||
-        hipHostMalloc((void**)&ev->h_counter, sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&ev->h_counter, 3 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         set_error("failed to create evaluator stream/events");
         i2_evaluator_destroy(ev);
@@ -613,8 +706,7 @@ void i2_evaluator_destroy(i2_evaluator* ev) {
         adjoint_release(ev->adj);
         ev->d_counter.reset();
         if (ev->h_counter) (void)hipHostFree(ev->h_counter);
-        if (ev->ev0) (void)hipEventDestroy(ev->ev0);
-        if (ev->ev1) (void)hipEventDestroy(ev->ev1);
+        for (hipEvent_t e : ev->marks) (void)hipEventDestroy(e);
         if (ev->stream) (void)hipStreamDestroy(ev->stream);
     }
     delete ev;

@@ -220,8 +220,8 @@ struct i2_evaluator {
     uint64_t all_pairs_generation = 0;
     i2::TypeState type[3];
     i2::DBuf<unsigned long long> d_counter;
-    unsigned long long* h_counter = nullptr;   // pinned
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    unsigned long long* h_counter = nullptr;   // pinned, one per type
+    std::vector<hipEvent_t> marks;              // of the plain path's timing
     i2::AdjState* adj = nullptr;   // adjoint buffers (created by the first loss-and-gradient call)
 };
 
