@@ -492,6 +492,117 @@ static int set_tasks(i2_evaluator* ev, int t, const std::vector<int32_t>& h) {
     return I2_OK;
 }
 
+// ------------------------------------------------------------ results to the host
+// Pinned staging memory, two slots per buffer: up to STAGING_KEPT buffers stay
+// allocated while any evaluator lives (a buffer's allocation costs 60-300 us);
+// a call takes one for itself, so calls of several threads do not meet.
+constexpr size_t STAGING_SLOT = (size_t)1 << 20;
+constexpr int STAGING_KEPT = 4;
+static std::mutex g_staging_mutex;
+static unsigned char* g_staging[STAGING_KEPT];
+static int g_staging_count = 0;
+static int64_t g_evaluators = 0;
+
+struct Staging {
+    unsigned char* p = nullptr;
+    int take() {
+        {
+            std::lock_guard<std::mutex> lock(g_staging_mutex);
+            if (g_staging_count > 0) p = g_staging[--g_staging_count];
+        }
+        if (!p) I2_HIP(hipHostMalloc((void**)&p, 2 * STAGING_SLOT, hipHostMallocPortable));
+        return I2_OK;
+    }
+    ~Staging() {
+        if (!p) return;
+        {
+            std::lock_guard<std::mutex> lock(g_staging_mutex);
+            if (g_evaluators > 0 && g_staging_count < STAGING_KEPT) { g_staging[g_staging_count++] = p; return; }
+        }
+        (void)hipHostFree(p);
+    }
+};
+static void evaluator_count(int64_t d) {
+    std::lock_guard<std::mutex> lock(g_staging_mutex);
+    g_evaluators += d;
+    if (g_evaluators == 0) while (g_staging_count > 0) (void)hipHostFree(g_staging[--g_staging_count]);
+}
+
+// A type's outputs of tasks z0 .. z0 + n - 1 into a staging slot, one array after
+// the other: integrals, results, errors, tasks, convergence iterations (those
+// asked for).  The device writes host memory, lines in order.  One launch instead
+// of a copy per array (10-20 us each, whatever its size).
+struct PackArgs {
+    TaskSource src;
+    bool implicit, tasks;
+    const uint64_t *ints, *res, *err;
+    const int8_t* conv;
+};
+__global__ __launch_bounds__(256) void k_pack(PackArgs P, int64_t z0, int64_t n, unsigned char* out) {
+    __shared__ int32_t t3[3 * 256];
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+    uint64_t* o = reinterpret_cast<uint64_t*>(out);
+    if (P.ints) { for (int64_t q = t; q < 4 * n; q += step) o[q] = P.ints[4 * z0 + q]; o += 4 * n; }
+    if (P.res) { for (int64_t q = t; q < 3 * n; q += step) o[q] = P.res[3 * z0 + q]; o += 3 * n; }
+    if (P.err) { for (int64_t q = t; q < n; q += step) o[q] = P.err[z0 + q]; o += n; }
+    int32_t* o4 = reinterpret_cast<int32_t*>(o);
+    if (P.tasks) {
+        for (int64_t base = 256 * (int64_t)blockIdx.x; base < n; base += step) {
+            const int64_t z = z0 + base + threadIdx.x;
+            if (base + threadIdx.x < n) {
+                int i, j;
+                if (P.implicit) task_ij<true>(P.src, z, &i, &j);
+                else task_ij<false>(P.src, z, &i, &j);
+                t3[3 * threadIdx.x] = i; t3[3 * threadIdx.x + 1] = j;
+                t3[3 * threadIdx.x + 2] = P.implicit ? (int32_t)z : P.src.ij3[3 * z + 2];
+            }
+            __syncthreads();
+            const int64_t m = 3 * (n - base < 256 ? n - base : 256);
+            for (int64_t q = threadIdx.x; q < m; q += 256) o4[3 * base + q] = t3[q];
+            __syncthreads();
+        }
+        o4 += 3 * n;
+    }
+    if (P.conv) { int8_t* o1 = reinterpret_cast<int8_t*>(o4); for (int64_t q = t; q < n; q += step) o1[q] = P.conv[z0 + q]; }
+}
+
+static int read_back(hipStream_t st, const PackArgs& P, int64_t n, double* ints, double* res, double* err, int32_t* tasks, int8_t* conv) {
+    const int64_t each = 32 * (ints != nullptr) + 24 * (res != nullptr) + 8 * (err != nullptr) + 12 * (tasks != nullptr) + (conv != nullptr);
+    if (each == 0) return I2_OK;
+    Staging S;
+    I2_TRY(S.take());
+    const int64_t most = (int64_t)STAGING_SLOT / each, chunks = (n + most - 1) / most;
+    struct Events {
+        hipEvent_t e[2] = {nullptr, nullptr};
+        ~Events() { for (hipEvent_t x : e) if (x) (void)hipEventDestroy(x); }
+    } E;
+    if (chunks > 1) for (hipEvent_t& e : E.e) I2_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    auto launch = [&](int64_t c) -> int {
+        const int64_t z0 = c * most, m = std::min(most, n - z0);
+        hipLaunchKernelGGL(k_pack, dim3((unsigned)std::min<int64_t>((m + 255) / 256, 256)), dim3(256), 0, st, P, z0, m,
+                           S.p + (c & 1) * STAGING_SLOT);
+        I2_TRY(check_launch("k_pack"));
+        if (chunks > 1) I2_HIP(hipEventRecord(E.e[c & 1], st));
+        return I2_OK;
+    };
+    int status = launch(0);
+    for (int64_t c = 0; c < chunks && status == I2_OK; ++c) {
+        if (c + 1 < chunks) status = launch(c + 1);       // fills the other slot meanwhile
+        if (status != I2_OK) break;
+        I2_HIP(chunks > 1 ? hipEventSynchronize(E.e[c & 1]) : hipStreamSynchronize(st));
+        const int64_t z0 = c * most, m = std::min(most, n - z0);
+        const unsigned char* p = S.p + (c & 1) * STAGING_SLOT;
+        auto take = [&](auto* dst, int64_t per) {
+            if (!dst) return;
+            memcpy(dst + per * z0, p, sizeof(*dst) * (size_t)(per * m));
+            p += sizeof(*dst) * (size_t)(per * m);
+        };
+        take(ints, 4); take(res, 3); take(err, 1); take(tasks, 3); take(conv, 1);
+    }
+    if (status != I2_OK) (void)hipStreamSynchronize(st);  // before the slots are given back
+    return status;
+}
+
 // ------------------------------------------------------------ allocation-free runPairs of one type
 // Device scratch of i2_evaluator_run_tasks_noalloc: one level buffer (the
 // caller's integrals are the other), the two lists of unconverged tasks, and
@@ -543,7 +654,25 @@ __global__ void k_check_tasks(int64_t n, const int32_t* __restrict__ tasks, int 
     if (shared_count(panels[i], panels[j]) != expect) atomicMin(bad, key + 1ull);
 }
 
-// run_type for an explicit device list, with the caller's integrals as level
+// The same for lists just uploaded, whose third entries are set as well.  The
+// triangles' numbers are compared as the reference's lists define the types.
+__global__ void k_take_tasks(int64_t n, int32_t* __restrict__ tasks, int64_t nT, const int32_t* __restrict__ tri, int expect,
+                             unsigned long long* bad) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    const int64_t i = tasks[3 * q], j = tasks[3 * q + 1];
+    tasks[3 * q + 2] = (int32_t)q;
+    const unsigned long long key = 2ull * (unsigned long long)(q + 1);
+    if (i < 0 || j < 0 || i >= nT || j >= nT) { atomicMin(bad, key); return; }
+    int cnt = 0;
+    for (int x = 0; x < 3; ++x) {
+        const int32_t a = tri[3 * i + x];
+        cnt += a == tri[3 * j] || a == tri[3 * j + 1] || a == tri[3 * j + 2];
+    }
+    if (cnt != expect) atomicMin(bad, key + 1ull);
+}
+
+// run_types for one type's explicit device list, with the caller's integrals as level
 // buffer 0 and the scratch as level buffer 1: the same launches in the same
 // order, so the same values, levels and K.
 template <int TYPE>
@@ -673,6 +802,7 @@ int i2_evaluator_create(i2_evaluator** out, const i2_mesh* m, i2_integrator* it)
     DeviceGuard g(m->device);
     if (!g.ok) return I2_ERR_HIP;
     i2_evaluator* ev = new i2_evaluator;
+    evaluator_count(1);
     ev->mesh = m;
     ev->integ = it;
     if (hipStreamCreateWithFlags(&ev->stream, hipStreamNonBlocking) != hipSuccess ||
@@ -693,7 +823,7 @@ void i2_evaluator_destroy(i2_evaluator* ev) {
         DeviceGuard g(ev->mesh->device);
         if (ev->stream) (void)hipStreamSynchronize(ev->stream);
         for (auto& ts : ev->type) {
-            ts.tasks.reset(); ts.buf[0].reset(); ts.buf[1].reset(); ts.results.reset(); ts.errors.reset();
+            ts.tasks.reset(); ts.new_tasks.reset(); ts.buf[0].reset(); ts.buf[1].reset(); ts.results.reset(); ts.errors.reset();
             ts.conv.reset(); ts.rest[0].reset(); ts.rest[1].reset();
             ts.unconv.reset(); ts.refinements.reset(); ts.task_list.reset();
         }
@@ -709,6 +839,7 @@ void i2_evaluator_destroy(i2_evaluator* ev) {
         for (hipEvent_t e : ev->marks) (void)hipEventDestroy(e);
         if (ev->stream) (void)hipStreamDestroy(ev->stream);
     }
+    evaluator_count(-1);
     delete ev;
 }
 
@@ -795,27 +926,47 @@ int i2_evaluator_run_pairs(i2_evaluator* ev, const int32_t* simple3, int64_t nSi
     const int64_t ns[3] = {nSimple, nAttached, nNot};
     DeviceGuard g(m->device);
     if (!g.ok) return I2_ERR_HIP;
-    // every list is checked before any is installed, so that a rejected call
-    // leaves the previous run's tasks and outputs as they were
-    std::vector<int32_t> h[3];
+    // Every list is checked before any is installed, so that a rejected call
+    // leaves the previous run's tasks and outputs as they were.  The lists are
+    // checked where they are used: host passes over 161,000 tasks and a copy of
+    // them took 300 us.
+    I2_TRY(ev->d_counter.ensure(3));
+    I2_HIP(hipMemsetAsync(ev->d_counter.p, 0xff, 3 * sizeof(unsigned long long), ev->stream));
     for (int t = 0; t < 3; ++t) {
-        h[t].assign(lists[t] ? lists[t] : (const int32_t*)nullptr, lists[t] ? lists[t] + 3 * ns[t] : (const int32_t*)nullptr);
-        for (int64_t q = 0; q < ns[t]; ++q) {
-            const int32_t i = h[t][3 * q], j = h[t][3 * q + 1];
-            if (i < 0 || j < 0 || i >= m->nT || j >= m->nT) { set_error("task %lld of type %d references a cell outside [0, %lld)", (long long)q, t, (long long)m->nT); return I2_ERR_INVALID; }
-            // the integrand of each type is only valid for pairs of that type
-            const int32_t* a = &m->h_tri[3 * (int64_t)i];
-            const int32_t* b = &m->h_tri[3 * (int64_t)j];
-            int cnt = 0;
-            for (int x = 0; x < 3; ++x) if (a[x] == b[0] || a[x] == b[1] || a[x] == b[2]) ++cnt;
-            const int expect = (t == I2_SIMPLE_NEIGHBORS) ? 1 : (t == I2_ATTACHED_NEIGHBORS ? 2 : 0);
-            if (cnt != expect) { set_error("task %lld (%d, %d) shares %d vertices but was given as type %d", (long long)q, i, j, cnt, t); return I2_ERR_TOPOLOGY; }
-            h[t][3 * q + 2] = (int32_t)q;
-        }
+        if (ns[t] == 0) continue;
+        I2_TRY(ev->type[t].new_tasks.ensure(3 * ns[t]));
+        I2_HIP(hipMemcpyAsync(ev->type[t].new_tasks.p, lists[t], sizeof(int32_t) * 3 * (size_t)ns[t], hipMemcpyHostToDevice, ev->stream));
+        // the integrand of each type is only valid for pairs of that type
+        const int expect = (t == I2_SIMPLE_NEIGHBORS) ? 1 : (t == I2_ATTACHED_NEIGHBORS ? 2 : 0);
+        hipLaunchKernelGGL(k_take_tasks, dim3(blocks_for(ns[t], 256)), dim3(256), 0, ev->stream, ns[t], ev->type[t].new_tasks.p,
+                           m->nT, m->d_tri.p, expect, ev->d_counter.p + t);
+        I2_TRY(check_launch("k_take_tasks"));
+    }
+    I2_HIP(hipMemcpyAsync(ev->h_counter, ev->d_counter.p, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, ev->stream));
+    I2_HIP(hipStreamSynchronize(ev->stream));
+    for (int t = 0; t < 3; ++t) {
+        const unsigned long long key = ev->h_counter[t];
+        if (key == ~0ull) continue;
+        const int64_t q = (int64_t)(key / 2) - 1;
+        const int32_t i = lists[t][3 * q], j = lists[t][3 * q + 1];
+        if (key % 2 == 0) { set_error("task %lld of type %d references a cell outside [0, %lld)", (long long)q, t, (long long)m->nT); return I2_ERR_INVALID; }
+        const int32_t* a = &m->h_tri[3 * (int64_t)i];
+        const int32_t* b = &m->h_tri[3 * (int64_t)j];
+        int cnt = 0;
+        for (int x = 0; x < 3; ++x) if (a[x] == b[0] || a[x] == b[1] || a[x] == b[2]) ++cnt;
+        set_error("task %lld (%d, %d) shares %d vertices but was given as type %d", (long long)q, i, j, cnt, t);
+        return I2_ERR_TOPOLOGY;
     }
     ev->ran = false;
     ev->all_pairs_lists = false;
-    for (int t = 0; t < 3; ++t) I2_TRY(set_tasks(ev, t, h[t]));
+    for (int t = 0; t < 3; ++t) {
+        TypeState& ts = ev->type[t];
+        ts.implicit = false;
+        ts.task_list_ready = false;
+        ts.n = ns[t];
+        std::swap(ts.tasks, ts.new_tasks);
+        I2_TRY(ts.tasks.ensure(3 * ns[t]));
+    }
     ev->tasks_generation = m->generation;
     return evaluator_run(ev, false, false);
 }
@@ -880,33 +1031,21 @@ int i2_evaluator_get_results(const i2_evaluator* ev, int type, int32_t* tasks3, 
     const i2_mesh* m = ev->mesh;
     DeviceGuard g(m->device);
     if (!g.ok) return I2_ERR_HIP;
-    const int64_t n = ts.n;
-    if (n == 0) return I2_OK;
-    if (tasks3) {
-        if (ts.implicit) {
-            const int64_t h = n / 2;
-            std::vector<int32_t> l(3 * h);
-            I2_TRY(i2_mesh_copy_neighbors(m, I2_NOT_NEIGHBORS, l.data()));
-            for (int64_t q = 0; q < h; ++q) {
-                tasks3[3 * q] = l[3 * q]; tasks3[3 * q + 1] = l[3 * q + 1]; tasks3[3 * q + 2] = (int32_t)q;
-                tasks3[3 * (h + q)] = l[3 * q + 1]; tasks3[3 * (h + q) + 1] = l[3 * q]; tasks3[3 * (h + q) + 2] = (int32_t)(h + q);
-            }
-        } else {
-            I2_HIP(hipMemcpy(tasks3, ts.tasks.p, sizeof(int32_t) * 3 * n, hipMemcpyDeviceToHost));
-        }
-    }
+    if (ts.n == 0) return I2_OK;
+    if (errors && !ts.has_errors) { set_error("symmetry errors were not computed (runAllPairs with checkCorrectness)"); return I2_ERR_STATE; }
     const double4* d_ints = ts.buf[ts.final_buf].p;
     const double* d_res = ts.results.p;
     const int8_t* d_conv = ts.conv.p;
     if (ev->ran_path == 1) engine_evaluator_outputs(ev, type, &d_ints, &d_res, &d_conv);
-    if (integrals4) I2_HIP(hipMemcpy(integrals4, d_ints, sizeof(double4) * n, hipMemcpyDeviceToHost));
-    if (results3) I2_HIP(hipMemcpy(results3, d_res, sizeof(double) * 3 * n, hipMemcpyDeviceToHost));
-    if (errors) {
-        if (!ts.has_errors) { set_error("symmetry errors were not computed (runAllPairs with checkCorrectness)"); return I2_ERR_STATE; }
-        I2_HIP(hipMemcpy(errors, ts.errors.p, sizeof(double) * n, hipMemcpyDeviceToHost));
-    }
-    if (convLevel) I2_HIP(hipMemcpy(convLevel, d_conv, (size_t)n, hipMemcpyDeviceToHost));
-    return I2_OK;
+    PackArgs P{};
+    P.src = task_source(ev, type);
+    P.implicit = ts.implicit;
+    if (integrals4) P.ints = reinterpret_cast<const uint64_t*>(d_ints);
+    if (results3) P.res = reinterpret_cast<const uint64_t*>(d_res);
+    if (errors) P.err = reinterpret_cast<const uint64_t*>(ts.errors.p);
+    if (convLevel) P.conv = d_conv;
+    P.tasks = tasks3 != nullptr;
+    return read_back(ev->stream, P, ts.n, integrals4, results3, errors, tasks3, convLevel);
 }
 
 int i2_evaluator_refinement_iterations(const i2_evaluator* ev, int type, int* K) {

@@ -171,6 +171,7 @@ struct TypeState {
     int64_t n = 0;                 // ordered tasks
     bool implicit = false;         // disjoint all-pairs: tasks decoded on the fly
     DBuf<int32_t> tasks;           // explicit (i, j, k)
+    DBuf<int32_t> new_tasks;       // runPairs: the next ones, until they are checked
     DBuf<double4> buf[2];          // level values, level k written to buf[k % 2]
     DBuf<double> results;          // J (double3 AoS)
     DBuf<double> errors;           // symmetry error
