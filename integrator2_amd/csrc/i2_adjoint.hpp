@@ -15,6 +15,12 @@ struct AdjMesh {
     const int64_t* nbr_start;
     const int32_t* nbr;
     const int32_t* lists[2];      // vertex- and edge-sharing (i, j, k), i < j
+    const int64_t* off[2];        // where panel i's pairs start in them
+    const int64_t* back_start;    // panel j's pairs with earlier panels: 2 k + kind, or -1
+    const int64_t* back;
+    const int32_t* tri;           // panels' vertices
+    const int64_t* inc_start;     // vertices' panels, ascending
+    const int32_t* inc;
     int64_t npairs[3];
     const int8_t* conv[3];        // per ordered task, reference task order
     const int* K;                 // refinement iterations per type
@@ -81,21 +87,14 @@ struct AdjArgs {
     DeepPair* deep_pairs;         // their pairs, counters[2] of them, as far as deep_cap entries hold an item's
     double* deep_rec;             // per entry: the pair's cotangents
     int64_t deep_cap;
-    // the vertex gather: panel sums (9 per panel, mesh m's from pbase[m]);
-    // vertices of all meshes (mesh m's from vbase[m]), each with its (panel,
-    // corner) incidences (3 p + corner, panels ascending) and its
-    // singular-task coordinates (18 t + 3 slot, tasks ascending)
+    // the vertex gather: panel sums (9 per panel, mesh m's from pbase[m]),
+    // vertices of all meshes (mesh m's from vbase[m])
     double* psum;
     const int64_t* pbase;
     int64_t npanels;
     int64_t nvtx;
     const int64_t* vbase;
-    const int64_t* inc_start;
-    const int32_t* inc;
-    const int64_t* sing_start;
-    const int64_t* sing_idx;
 };
-
 struct AdjState {
     AdjArgs args{};
     int grid = 0;
@@ -103,14 +102,11 @@ struct AdjState {
     std::vector<int64_t> grad_off; // per mesh: dL/dX (3 nV) then L, in d_grad
     double ms = 0.0;              // device time of the last adjoint run
     int64_t kj_total = 0;         // doubles of K_j slots, all meshes
-    DBuf<AdjMesh> d_mesh;
     DBuf<int> d_K;
     DBuf<double> d_grad;          // dL/dX (3 nV) and L
     DBuf<double> d_ki, d_kj;      // partial panel cotangents (all meshes)
     DBuf<double> d_item_loss, d_sing_dl, d_psum, d_loss_part;
-    DBuf<int64_t> d_item_base, d_sing_base;
-    DBuf<int64_t> d_pbase, d_vbase, d_inc_start, d_sing_start, d_sing_idx;
-    DBuf<int32_t> d_inc;
+    DBuf<int64_t> d_base;         // the base tables of AdjArgs, then the mesh descriptors
     DBuf<uint32_t> d_deep_mask;
     DBuf<DeepItem> d_deep_items;
     DBuf<DeepPair> d_deep_pairs;

@@ -470,26 +470,27 @@ int evaluator_run(i2_evaluator* ev, bool all_pairs, bool check) {
     return I2_OK;
 }
 
-// Builds the ordered task list [(i,j,k)] ++ [(j,i,n+k)] of Evaluator3D::runAllPairs
-// (evaluator3d.cu:22-31, 156-169) on the host.
-static std::vector<int32_t> with_reversed(const std::vector<int32_t>& l) {
-    const size_t n = l.size() / 3;
-    std::vector<int32_t> out(6 * n);
-    for (size_t q = 0; q < n; ++q) {
-        out[3 * q] = l[3 * q]; out[3 * q + 1] = l[3 * q + 1]; out[3 * q + 2] = (int32_t)q;
-        out[3 * (n + q)] = l[3 * q + 1]; out[3 * (n + q) + 1] = l[3 * q]; out[3 * (n + q) + 2] = (int32_t)(n + q);
-    }
-    return out;
+// The ordered task list [(i,j,k)] ++ [(j,i,n+k)] of Evaluator3D::runAllPairs
+// (evaluator3d.cu:22-31, 156-169) from the mesh's list.
+__global__ void k_ordered_tasks(int64_t n, const int32_t* __restrict__ list, int32_t* __restrict__ tasks) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    const int32_t i = list[3 * q], j = list[3 * q + 1];
+    int32_t *a = tasks + 3 * q, *b = tasks + 3 * (n + q);
+    a[0] = i; a[1] = j; a[2] = (int32_t)q;
+    b[0] = j; b[1] = i; b[2] = (int32_t)(n + q);
 }
 
-static int set_tasks(i2_evaluator* ev, int t, const std::vector<int32_t>& h) {
+static int set_ordered_tasks(i2_evaluator* ev, int t, const DBuf<int32_t>& list) {
     TypeState& ts = ev->type[t];
+    const int64_t n = ev->mesh->pairs[t];
     ts.implicit = false;
     ts.task_list_ready = false;
-    ts.n = (int64_t)h.size() / 3;
+    ts.n = 2 * n;
     I2_TRY(ts.tasks.ensure(3 * ts.n));
-    if (ts.n) I2_HIP(hipMemcpy(ts.tasks.p, h.data(), sizeof(int32_t) * h.size(), hipMemcpyHostToDevice));
-    return I2_OK;
+    if (n == 0) return I2_OK;
+    hipLaunchKernelGGL(k_ordered_tasks, dim3(blocks_for(n, 256)), dim3(256), 0, ev->stream, n, list.p, ts.tasks.p);
+    return check_launch("k_ordered_tasks");
 }
 
 // ------------------------------------------------------------ results to the host
@@ -851,10 +852,10 @@ int i2_evaluator_run_all_pairs(i2_evaluator* ev, int checkCorrectness) {
     if (!g.ok) return I2_ERR_HIP;
     ev->ran = false;
     if (!ev->all_pairs_lists || ev->all_pairs_generation != m->generation) {
-        // the ordered lists depend only on the mesh: uploaded once per prepared mesh
+        // the ordered lists depend only on the mesh: written once per prepared mesh
         ev->all_pairs_lists = false;
-        I2_TRY(set_tasks(ev, I2_SIMPLE_NEIGHBORS, with_reversed(m->h_simple)));
-        I2_TRY(set_tasks(ev, I2_ATTACHED_NEIGHBORS, with_reversed(m->h_attached)));
+        I2_TRY(set_ordered_tasks(ev, I2_SIMPLE_NEIGHBORS, m->d_simple));
+        I2_TRY(set_ordered_tasks(ev, I2_ATTACHED_NEIGHBORS, m->d_attached));
         TypeState& d = ev->type[I2_NOT_NEIGHBORS];
         d.implicit = true;
         d.task_list_ready = false;

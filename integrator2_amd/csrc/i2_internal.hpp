@@ -88,22 +88,30 @@ struct i2_mesh {
     int64_t nV = 0, nT = 0;
     std::vector<double> h_xyz;          // host copy of vertices (AoS)
     std::vector<int32_t> h_tri;         // host copy of cells (AoS, 0-based)
-    // neighbour lists (i<j, k) for vertex- and edge-sharing pairs, lexicographic
-    std::vector<int32_t> h_simple, h_attached;
     int64_t pairs[3] = {0, 0, 0};
-    // per-cell sorted neighbour indices j > i (CSR) and disjoint-pair row offsets:
-    // the k-th disjoint (i<j) pair in lexicographic order is found from these
-    std::vector<int64_t> h_nbr_start, h_row_start;
-    std::vector<int32_t> h_nbr;
     // device arrays
     i2::DBuf<double> d_xyz;             // vertices (double3 AoS)
     i2::DBuf<int32_t> d_tri;            // cells (int3 AoS)
     i2::DBuf<double> d_normals;         // double3 AoS
     i2::DBuf<double> d_measures;
     i2::DBuf<i2d::Panel> d_panels;      // kernel-side panel records
+    // neighbour lists (i<j, k) for vertex- and edge-sharing pairs, lexicographic,
+    // and where cell i's pairs start in them
     i2::DBuf<int32_t> d_simple, d_attached;
+    i2::DBuf<int64_t> d_off[2];
+    // per-cell sorted neighbour indices j > i (CSR) and disjoint-pair row offsets:
+    // the k-th disjoint (i<j) pair in lexicographic order is found from these
     i2::DBuf<int64_t> d_nbr_start, d_row_start;
     i2::DBuf<int32_t> d_nbr;
+    // cell j's vertex- and edge-sharing pairs (i, j) with earlier cells (CSR):
+    // 2 k or 2 k + 1 for pair k of the one list or the other, or -1
+    i2::DBuf<int64_t> d_back_start, d_back;
+    // per-vertex cells, ascending (CSR; a cell is listed once per corner)
+    i2::DBuf<int64_t> d_inc_start;
+    i2::DBuf<int32_t> d_inc;
+    // counts of the classification, kept for the next one
+    i2::DBuf<int32_t> d_degree, d_counts;
+    i2::DBuf<int64_t> d_totals;
     // disjoint (i < j, k) list, written out on request (the kernels decode it on the fly)
     mutable i2::DBuf<int32_t> d_not_list;
     mutable uint64_t not_list_generation = 0;

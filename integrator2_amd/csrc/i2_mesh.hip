@@ -59,13 +59,13 @@ __global__ void k_panel_table(int64_t nT, const double* __restrict__ xyz, const 
 
 // Exclusive prefix sum of n counts into out[0..n] (out[n] = total), one
 // workgroup: each thread scans a contiguous chunk.
-template <class T>
-__global__ __launch_bounds__(1024) void k_scan_counts(int64_t n, const T* __restrict__ cnt, int64_t* __restrict__ out) {
+template <class F>
+__device__ __forceinline__ void scan_counts(int64_t n, F count, int64_t* __restrict__ out, int64_t* total) {
     __shared__ int64_t part[16];
     const int64_t chunk = (n + blockDim.x - 1) / blockDim.x;
     const int64_t b = threadIdx.x * chunk, e = b + chunk < n ? b + chunk : n;
     int64_t s = 0;
-    for (int64_t q = b; q < e; ++q) s += (int64_t)cnt[q];
+    for (int64_t q = b; q < e; ++q) s += count(q);
     const int lane = threadIdx.x & 63;
     int64_t run = s;                       // inclusive over the wavefront
     for (int d = 1; d < 64; d <<= 1) {
@@ -77,9 +77,30 @@ __global__ __launch_bounds__(1024) void k_scan_counts(int64_t n, const T* __rest
     int64_t before = 0;                    // the wavefronts before this one
     for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) before += part[w];
     run += before;
-    if (threadIdx.x == blockDim.x - 1) out[n] = run;
+    if (threadIdx.x == blockDim.x - 1) { out[n] = run; if (total) *total = run; }
     run -= s;
-    for (int64_t q = b; q < e; ++q) { out[q] = run; run += (int64_t)cnt[q]; }
+    for (int64_t q = b; q < e; ++q) { out[q] = run; run += count(q); }
+}
+__global__ __launch_bounds__(1024) void k_scan_degrees(int64_t n, const int32_t* __restrict__ cnt, int64_t* __restrict__ out) {
+    scan_counts(n, [&](int64_t q) { return (int64_t)cnt[q]; }, out, nullptr);
+}
+// The offsets of the classification's lists, a workgroup each: vertex-sharing,
+// edge-sharing and all sharing cells j > i and all sharing cells j < i from
+// their counts (nT each), and the disjoint pairs of row i, the nT - 1 - i cells
+// j > i less those sharing.
+struct RowOffsets { int64_t* p[5]; };
+__global__ __launch_bounds__(1024) void k_scan_rows(int64_t nT, const int32_t* __restrict__ counts, RowOffsets off, int64_t* totals) {
+    const int w = blockIdx.x;
+    if (w < 4) {
+        const int32_t* c = counts + w * nT;
+        scan_counts(nT, [&](int64_t q) { return (int64_t)c[q]; }, off.p[w], totals + w);
+    } else {
+        const int32_t* n = counts + 2 * nT;
+        scan_counts(nT, [&](int64_t q) { return (nT - 1 - q) - (int64_t)n[q]; }, off.p[w], totals + w);
+    }
+}
+__global__ void k_clear(int64_t n, int32_t* __restrict__ p) {
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) p[q] = 0;
 }
 
 __global__ void k_vertex_degree(int64_t nslots, const int32_t* __restrict__ tri, int32_t* __restrict__ deg) {
@@ -108,46 +129,72 @@ __global__ void k_sort_incidence(int64_t nV, const int64_t* __restrict__ start, 
     }
 }
 
+// A vertex's cells from position q on, the next one held in a register
 struct SlotList {
     const int32_t* p;
     int64_t q, e;
-    // first entry > i
+    int32_t head;
+    __device__ void open(const int32_t* inc, int64_t b, int64_t end) { p = inc; q = b; e = end; read(); }
+    __device__ void read() { head = q < e ? p[q] : INT32_MAX; }
+    // to the first entry > i
     __device__ void seek(int32_t i) {
         int64_t lo = q, hi = e;
         while (lo < hi) { const int64_t mid = (lo + hi) >> 1; if (p[mid] <= i) lo = mid + 1; else hi = mid; }
         q = lo;
+        read();
     }
-    __device__ int32_t head() const { return q < e ? p[q] : INT32_MAX; }
     // advances past every copy of j (a cell with a repeated vertex is listed twice)
     __device__ int take(int32_t j) {
-        if (q >= e || p[q] != j) return 0;
-        while (q < e && p[q] == j) ++q;
+        if (head != j) return 0;
+        do { ++q; read(); } while (head == j && q < e);
         return 1;
     }
 };
 
-// WRITE = false: per cell i, the numbers of vertex-sharing, edge-sharing and
-// all sharing cells j > i.  WRITE = true: the lists at the scanned offsets.
-template <bool WRITE>
-__global__ void k_classify(int64_t nT, const int32_t* __restrict__ tri, const int64_t* __restrict__ start,
-                           const int32_t* __restrict__ inc, int32_t* __restrict__ n_simple, int32_t* __restrict__ n_attached,
-                           int32_t* __restrict__ n_shared, const int64_t* __restrict__ off_simple,
-                           const int64_t* __restrict__ off_attached, const int64_t* __restrict__ off_shared,
-                           int32_t* __restrict__ simple, int32_t* __restrict__ attached, int32_t* __restrict__ nbr) {
-    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < nT; c += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t i = (int32_t)c;
-        SlotList L[3];
+// The three slots' cells of cell c, merged; each cell once.
+struct SlotMerge {
+    SlotList L[3];
+    __device__ SlotMerge(int64_t c, const int32_t* tri, const int64_t* start, const int32_t* inc) {
         for (int k = 0; k < 3; ++k) {
             const int32_t v = tri[3 * c + k];
-            L[k].p = inc; L[k].q = start[v]; L[k].e = start[v + 1];
-            L[k].seek(i);
+            L[k].open(inc, start[v], start[v + 1]);
         }
+    }
+    __device__ int32_t head() const { return min(L[0].head, min(L[1].head, L[2].head)); }
+    __device__ int take(int32_t j) { return L[0].take(j) + L[1].take(j) + L[2].take(j); }
+    // the number of cells before `end`, which are passed
+    __device__ int32_t skip(int32_t end) {
+        int32_t n = 0;
+        for (int32_t j = head(); j < end; j = head()) { take(j); ++n; }
+        return n;
+    }
+};
+
+// WRITE = false: per cell i, the numbers of vertex-sharing, edge-sharing and
+// all sharing cells j > i, and of all sharing cells j < i.  WRITE = true: the
+// lists at the scanned offsets; the lists of earlier cells are cleared.
+template <bool WRITE>
+__global__ void k_classify(int64_t nT, const int32_t* __restrict__ tri, const int64_t* __restrict__ start,
+                           const int32_t* __restrict__ inc, int32_t* __restrict__ counts, const int64_t* __restrict__ off_simple,
+                           const int64_t* __restrict__ off_attached, const int64_t* __restrict__ off_shared,
+                           const int64_t* __restrict__ off_back, int32_t* __restrict__ simple, int32_t* __restrict__ attached,
+                           int32_t* __restrict__ nbr, int64_t* __restrict__ back) {
+    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < nT; c += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t i = (int32_t)c;
+        SlotMerge S(c, tri, start, inc);
         int64_t ws = WRITE ? off_simple[c] : 0, wa = WRITE ? off_attached[c] : 0, wn = WRITE ? off_shared[c] : 0;
-        int32_t cs = 0, ca = 0, cn = 0;
+        int32_t cs = 0, ca = 0, cn = 0, cb = 0;
+        if (WRITE) {
+            for (auto& l : S.L) l.seek(i);
+            for (int64_t q = off_back[c]; q < off_back[c + 1]; ++q) back[q] = -1;
+        } else {
+            cb = S.skip(i);
+            S.take(i);
+        }
         for (;;) {
-            const int32_t j = min(L[0].head(), min(L[1].head(), L[2].head()));
+            const int32_t j = S.head();
             if (j == INT32_MAX) break;
-            const int m = L[0].take(j) + L[1].take(j) + L[2].take(j);
+            const int m = S.take(j);
             ++cn;
             if (m == 1) ++cs;
             if (m == 2) ++ca;
@@ -157,14 +204,25 @@ __global__ void k_classify(int64_t nT, const int32_t* __restrict__ tri, const in
                 if (m == 2) { attached[3 * wa] = i; attached[3 * wa + 1] = j; attached[3 * wa + 2] = (int32_t)wa; ++wa; }
             }
         }
-        if (!WRITE) { n_simple[c] = cs; n_attached[c] = ca; n_shared[c] = cn; }
+        if (!WRITE) { counts[c] = cs; counts[nT + c] = ca; counts[2 * nT + c] = cn; counts[3 * nT + c] = cb; }
     }
 }
 
-// Disjoint pairs of row i: the nT - 1 - i cells j > i less those sharing a vertex.
-__global__ void k_disjoint_row_counts(int64_t nT, const int32_t* __restrict__ n_shared, int64_t* __restrict__ row) {
-    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < nT; c += (int64_t)gridDim.x * blockDim.x)
-        row[c] = (nT - 1 - c) - (int64_t)n_shared[c];
+// The pairs of each cell with earlier cells, in the earlier cells' order: a pair
+// (i, j), number k of its list, stands where i does among the cells before j
+// that share a vertex with it, as 2 k (vertex-sharing) or 2 k + 1 (edge-sharing).
+// Entries of cells that share all three stay -1.
+__global__ void k_back_pairs(int64_t n0, int64_t n1, const int32_t* __restrict__ simple, const int32_t* __restrict__ attached,
+                             const int32_t* __restrict__ tri, const int64_t* __restrict__ start, const int32_t* __restrict__ inc,
+                             const int64_t* __restrict__ off_back, int64_t* __restrict__ back) {
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n0 + n1; q += (int64_t)gridDim.x * blockDim.x) {
+        const int kind = q >= n0;
+        const int64_t k = kind ? q - n0 : q;
+        const int32_t* L = (kind ? attached : simple) + 3 * k;
+        const int32_t i = L[0], j = L[1];
+        SlotMerge S(j, tri, start, inc);
+        back[off_back[j] + S.skip(i)] = 2 * k + kind;
+    }
 }
 
 static unsigned grid_of(int64_t n) {
@@ -172,46 +230,31 @@ static unsigned grid_of(int64_t n) {
     return (unsigned)(b < 1 ? 1 : (b > 65536 ? 65536 : b));
 }
 
-template <class T>
-static int download(std::vector<T>& h, const DBuf<T>& d, int64_t n, hipStream_t s) {
-    h.resize((size_t)n);
-    if (n) I2_HIP(hipMemcpyAsync(h.data(), d.p, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, s));
-    return I2_OK;
-}
-
 static int classify(i2_mesh* m) {
     const int64_t nT = m->nT, nV = m->nV, nslots = 3 * nT;
     hipStream_t st = m->stream;
-    DBuf<int32_t> deg, cursor, inc, ns, na, nn;
-    DBuf<int64_t> start, off_s, off_a, rows;
-    I2_TRY(deg.ensure(nV)); I2_TRY(cursor.ensure(nV)); I2_TRY(inc.ensure(nslots));
-    I2_TRY(start.ensure(nV + 1));
-    I2_TRY(ns.ensure(nT)); I2_TRY(na.ensure(nT)); I2_TRY(nn.ensure(nT));
-    I2_TRY(off_s.ensure(nT + 1)); I2_TRY(off_a.ensure(nT + 1)); I2_TRY(rows.ensure(nT));
-    I2_TRY(m->d_nbr_start.ensure(nT + 1)); I2_TRY(m->d_row_start.ensure(nT + 1));
-    I2_HIP(hipMemsetAsync(deg.p, 0, sizeof(int32_t) * nV, st));
-    I2_HIP(hipMemsetAsync(cursor.p, 0, sizeof(int32_t) * nV, st));
-    hipLaunchKernelGGL(k_vertex_degree, dim3(grid_of(nslots)), dim3(256), 0, st, nslots, m->d_tri.p, deg.p);
+    I2_TRY(m->d_degree.ensure(2 * nV)); I2_TRY(m->d_inc.ensure(nslots)); I2_TRY(m->d_inc_start.ensure(nV + 1));
+    I2_TRY(m->d_counts.ensure(4 * nT)); I2_TRY(m->d_totals.ensure(5));
+    for (DBuf<int64_t>* o : {&m->d_off[0], &m->d_off[1], &m->d_nbr_start, &m->d_back_start, &m->d_row_start}) I2_TRY(o->ensure(nT + 1));
+    int32_t *deg = m->d_degree.p, *cursor = deg + nV;
+    const int64_t* start = m->d_inc_start.p;
+    hipLaunchKernelGGL(k_clear, dim3(grid_of(2 * nV)), dim3(256), 0, st, 2 * nV, deg);
+    hipLaunchKernelGGL(k_vertex_degree, dim3(grid_of(nslots)), dim3(256), 0, st, nslots, m->d_tri.p, deg);
     I2_TRY(check_launch("k_vertex_degree"));
-    hipLaunchKernelGGL(k_scan_counts<int32_t>, dim3(1), dim3(1024), 0, st, nV, deg.p, start.p);
-    I2_TRY(check_launch("k_scan_counts"));
-    hipLaunchKernelGGL(k_fill_incidence, dim3(grid_of(nslots)), dim3(256), 0, st, nslots, m->d_tri.p, start.p, cursor.p, inc.p);
+    hipLaunchKernelGGL(k_scan_degrees, dim3(1), dim3(1024), 0, st, nV, deg, m->d_inc_start.p);
+    I2_TRY(check_launch("k_scan_degrees"));
+    hipLaunchKernelGGL(k_fill_incidence, dim3(grid_of(nslots)), dim3(256), 0, st, nslots, m->d_tri.p, start, cursor, m->d_inc.p);
     I2_TRY(check_launch("k_fill_incidence"));
-    hipLaunchKernelGGL(k_sort_incidence, dim3(grid_of(nV)), dim3(256), 0, st, nV, start.p, inc.p);
+    hipLaunchKernelGGL(k_sort_incidence, dim3(grid_of(nV)), dim3(256), 0, st, nV, start, m->d_inc.p);
     I2_TRY(check_launch("k_sort_incidence"));
-    hipLaunchKernelGGL(k_classify<false>, dim3(grid_of(nT)), dim3(256), 0, st, nT, m->d_tri.p, start.p, inc.p, ns.p, na.p, nn.p,
-                       nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(k_classify<false>, dim3(grid_of(nT)), dim3(256), 0, st, nT, m->d_tri.p, start, m->d_inc.p,
+                       m->d_counts.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
     I2_TRY(check_launch("k_classify"));
-    hipLaunchKernelGGL(k_scan_counts<int32_t>, dim3(1), dim3(1024), 0, st, nT, ns.p, off_s.p);
-    hipLaunchKernelGGL(k_scan_counts<int32_t>, dim3(1), dim3(1024), 0, st, nT, na.p, off_a.p);
-    hipLaunchKernelGGL(k_scan_counts<int32_t>, dim3(1), dim3(1024), 0, st, nT, nn.p, m->d_nbr_start.p);
-    hipLaunchKernelGGL(k_disjoint_row_counts, dim3(grid_of(nT)), dim3(256), 0, st, nT, nn.p, rows.p);
-    hipLaunchKernelGGL(k_scan_counts<int64_t>, dim3(1), dim3(1024), 0, st, nT, rows.p, m->d_row_start.p);
-    I2_TRY(check_launch("k_scan_counts"));
-    int64_t tot[3];
-    I2_HIP(hipMemcpyAsync(&tot[0], off_s.p + nT, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    I2_HIP(hipMemcpyAsync(&tot[1], off_a.p + nT, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    I2_HIP(hipMemcpyAsync(&tot[2], m->d_nbr_start.p + nT, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    const RowOffsets off{{m->d_off[0].p, m->d_off[1].p, m->d_nbr_start.p, m->d_back_start.p, m->d_row_start.p}};
+    hipLaunchKernelGGL(k_scan_rows, dim3(5), dim3(1024), 0, st, nT, m->d_counts.p, off, m->d_totals.p);
+    I2_TRY(check_launch("k_scan_rows"));
+    int64_t tot[5];
+    I2_HIP(hipMemcpyAsync(tot, m->d_totals.p, sizeof tot, hipMemcpyDeviceToHost, st));
     I2_HIP(hipStreamSynchronize(st));
     if (tot[0] > (int64_t)INT32_MAX || tot[1] > (int64_t)INT32_MAX) {
         set_error("%lld vertex-sharing / %lld edge-sharing pairs exceed the 32-bit pair numbers", (long long)tot[0], (long long)tot[1]);
@@ -220,19 +263,18 @@ static int classify(i2_mesh* m) {
     I2_TRY(m->d_simple.ensure(3 * tot[0]));
     I2_TRY(m->d_attached.ensure(3 * tot[1]));
     I2_TRY(m->d_nbr.ensure(tot[2]));
-    hipLaunchKernelGGL(k_classify<true>, dim3(grid_of(nT)), dim3(256), 0, st, nT, m->d_tri.p, start.p, inc.p, nullptr, nullptr, nullptr,
-                       off_s.p, off_a.p, m->d_nbr_start.p, m->d_simple.p, m->d_attached.p, m->d_nbr.p);
+    I2_TRY(m->d_back.ensure(tot[3]));
+    hipLaunchKernelGGL(k_classify<true>, dim3(grid_of(nT)), dim3(256), 0, st, nT, m->d_tri.p, start, m->d_inc.p, nullptr,
+                       off.p[0], off.p[1], off.p[2], off.p[3], m->d_simple.p, m->d_attached.p, m->d_nbr.p, m->d_back.p);
     I2_TRY(check_launch("k_classify"));
-    // host copies for the host-side task lists and getters
-    I2_TRY(download(m->h_simple, m->d_simple, 3 * tot[0], st));
-    I2_TRY(download(m->h_attached, m->d_attached, 3 * tot[1], st));
-    I2_TRY(download(m->h_nbr_start, m->d_nbr_start, nT + 1, st));
-    I2_TRY(download(m->h_row_start, m->d_row_start, nT + 1, st));
-    I2_TRY(download(m->h_nbr, m->d_nbr, tot[2], st));
-    I2_HIP(hipStreamSynchronize(st));
+    if (tot[0] + tot[1] > 0) {
+        hipLaunchKernelGGL(k_back_pairs, dim3(grid_of(tot[0] + tot[1])), dim3(256), 0, st, tot[0], tot[1], m->d_simple.p,
+                           m->d_attached.p, m->d_tri.p, start, m->d_inc.p, off.p[3], m->d_back.p);
+        I2_TRY(check_launch("k_back_pairs"));
+    }
     m->pairs[I2_SIMPLE_NEIGHBORS] = tot[0];
     m->pairs[I2_ATTACHED_NEIGHBORS] = tot[1];
-    m->pairs[I2_NOT_NEIGHBORS] = m->h_row_start[nT];
+    m->pairs[I2_NOT_NEIGHBORS] = tot[4];
     return I2_OK;
 }
 
@@ -456,6 +498,7 @@ void i2_mesh_destroy(i2_mesh* m) {
         (void)hipStreamSynchronize(m->stream);
         m->d_xyz.reset(); m->d_tri.reset(); m->d_normals.reset(); m->d_measures.reset(); m->d_panels.reset();
         m->d_simple.reset(); m->d_attached.reset(); m->d_nbr_start.reset(); m->d_row_start.reset(); m->d_nbr.reset(); m->d_not_list.reset();
+        m->d_off[0].reset(); m->d_off[1].reset(); m->d_back_start.reset(); m->d_back.reset(); m->d_inc_start.reset(); m->d_inc.reset(); m->d_degree.reset(); m->d_counts.reset(); m->d_totals.reset();
         (void)hipStreamDestroy(m->stream);
     }
     delete m;
@@ -551,15 +594,21 @@ int i2_mesh_copy_measures(const i2_mesh* m, double* s) {
 int i2_mesh_copy_neighbors(const i2_mesh* m, int type, int32_t* ijk) {
     if (!m || !ijk) { set_error("null argument"); return I2_ERR_INVALID; }
     if (!m->prepared) { set_error("mesh not prepared"); return I2_ERR_STATE; }
-    if (type == I2_SIMPLE_NEIGHBORS) { std::copy(m->h_simple.begin(), m->h_simple.end(), ijk); return I2_OK; }
-    if (type == I2_ATTACHED_NEIGHBORS) { std::copy(m->h_attached.begin(), m->h_attached.end(), ijk); return I2_OK; }
+    if (type == I2_SIMPLE_NEIGHBORS || type == I2_ATTACHED_NEIGHBORS) {
+        const DBuf<int32_t>& d = type == I2_SIMPLE_NEIGHBORS ? m->d_simple : m->d_attached;
+        return m->pairs[type] ? copy_d2h(d.p, ijk, sizeof(int32_t) * 3 * m->pairs[type], m->device) : I2_OK;
+    }
     if (type != I2_NOT_NEIGHBORS) { set_error("bad neighbour type %d", type); return I2_ERR_INVALID; }
+    std::vector<int64_t> start((size_t)m->nT + 1);
+    I2_TRY(copy_d2h(m->d_nbr_start.p, start.data(), sizeof(int64_t) * (m->nT + 1), m->device));
+    std::vector<int32_t> nbr((size_t)start[m->nT]);
+    if (!nbr.empty()) I2_TRY(copy_d2h(m->d_nbr.p, nbr.data(), sizeof(int32_t) * nbr.size(), m->device));
     int64_t k = 0;
     for (int64_t i = 0; i < m->nT; ++i) {
-        int64_t q = m->h_nbr_start[i];
-        const int64_t qe = m->h_nbr_start[i + 1];
+        int64_t q = start[i];
+        const int64_t qe = start[i + 1];
         for (int64_t j = i + 1; j < m->nT; ++j) {
-            if (q < qe && m->h_nbr[q] == j) { ++q; continue; }
+            if (q < qe && nbr[q] == j) { ++q; continue; }
             ijk[3 * k] = (int32_t)i; ijk[3 * k + 1] = (int32_t)j; ijk[3 * k + 2] = (int32_t)k;
             ++k;
         }
