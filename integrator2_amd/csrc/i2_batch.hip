@@ -138,10 +138,10 @@ __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int s
 // Quadrature points of a disjoint item's control panel K_i (uniform over the
 // workgroup): the level-0 panel and its four level-1 children, in the order
 // sweep_task sums them, computed once per item instead of once per pair.  Each
-// point and its rule weight share a 32-byte record, two 128-bit LDS reads: the
-// place for the general form, or |b0 U + b1 V|^2 and (b0, b1) for the far one.
-struct alignas(32) QPoint { double x, y, z, w; };
-struct PtsLDS { QPoint q[5 * MAX_POINTS], f[5 * MAX_POINTS]; };
+// point is a 32-byte record, two 128-bit LDS reads: |b0 U + b1 V|^2, (b0, b1)
+// and the rule weight.
+struct alignas(32) QPoint { double pp, b0, b1, w; };
+struct PtsLDS { QPoint f[5 * MAX_POINTS]; };
 
 // Levels 0 and 1 in one pass with a rule whose point 0 is the centroid: the
 // centroid of K_i is also the centroid of its central level-1 child (child 4),
@@ -151,72 +151,116 @@ __device__ __forceinline__ bool share_centroid(const BatchArgs& A) {
     return A.rule.centroid == 0 && !A.fixed && A.last_level >= 1;
 }
 
-__device__ __forceinline__ void load_points(PtsLDS& P, const RuleLDS& R, int npts, const Panel& I) {
-    const d3 mBC = 0.5 * (I.b + I.c), mCA = 0.5 * (I.c + I.a), mAB = 0.5 * (I.a + I.b);
+__device__ __forceinline__ void load_points(PtsLDS& P, const RuleLDS& R, int npts, const FarFrame& F) {
     for (int t = threadIdx.x; t < 5 * npts; t += blockDim.x) {
-        const int sub = t / npts, k = t - sub * npts;
-        d3 a = I.a, b = I.b, c = I.c;
-        if (sub == 1) { a = mAB; c = mBC; }
-        else if (sub == 2) { a = mBC; b = I.c; c = mCA; }
-        else if (sub == 3) { a = mCA; b = I.a; c = mAB; }
-        else if (sub == 4) { a = mBC; b = mCA; c = mAB; }
-        d3 p = R.L1[k] * a;
-        p = p + R.L2[k] * b;
-        p = p + R.L3[k] * c;
-        P.q[t] = {p.x, p.y, p.z, R.w[k]};
         const BaryPoint Q = bary_point(R.L1, R.L2, R.L3, R.w, npts, t);
-        const FarPoint F = far_point(Q.b0 - 1.0 / 3.0, Q.b1 - 1.0 / 3.0, Q.w);
-        P.f[t] = {far_pp(far_frame(I.a, I.b, I.c), F), F.b0, F.b1, F.w};
+        const FarPoint x = far_point(Q.b0 - 1.0 / 3.0, Q.b1 - 1.0 / 3.0, Q.w);
+        P.f[t] = {far_pp(F, x), x.b0, x.b1, x.w};
     }
 }
 
-// Weighted sum of the inner integral's terms over the precomputed points k =
-// k0, k0 + step, ... < k1, added in that order to acc.  FORM as in wave_form.
-template <int FORM> struct FormGeom { const FarGeom G; };
-template <> struct FormGeom<0> { const JGeom& G; };
-template <int FORM>
-__device__ __forceinline__ q4 terms_at(const RuleLDS& R, const PtsLDS& P, int k, const FormGeom<FORM>& J, double& w) {
-    if constexpr (FORM == 0) {
-        const QPoint Q = P.q[k];
-        w = Q.w;
-        return theta_terms(d3{Q.x, Q.y, Q.z}, J.G, &R.lt);
-    } else {
-        const QPoint Q = P.f[k];
-        w = Q.w;
-        return theta_terms_far<FORM == 2>(Q.y, Q.z, Q.x, J.G);
+// The ways a wavefront evaluates the terms (forms of wave_form).  General: at
+// the point itself.  Far: from the panel's own distance polynomials.  Shared:
+// as far, with the distances of a tile's vertices computed once per vertex
+// instead of once per panel corner.  sum() adds w times the terms of points k =
+// k0, k0 + step, ... < k1 to acc, in that order.
+struct GeneralTerms {
+    const RuleLDS& R;
+    const PtsLDS& P;
+    const FarFrame& F;
+    const JGeom& J;
+    __device__ __forceinline__ q4 sum(int k0, int k1, int step, q4 acc) const {
+        for (int k = k0; k < k1; k += step) {
+            const QPoint Q = P.f[k];
+            const q4 t = theta_terms(F.m + Q.b0 * F.U + Q.b1 * F.V, J, &R.lt);
+            acc = {fma(Q.w, t.x, acc.x), fma(Q.w, t.y, acc.y), fma(Q.w, t.z, acc.z), fma(Q.w, t.w, acc.w)};
+        }
+        return acc;
     }
-}
-template <int FORM>
-__device__ __forceinline__ q4 quad_pts(const RuleLDS& R, const PtsLDS& P, int k0, int k1, int step, const FormGeom<FORM>& J, q4 acc) {
-    for (int k = k0; k < k1; k += step) {
-        double w;
-        const q4 t = terms_at<FORM>(R, P, k, J, w);
-        acc = {fma(w, t.x, acc.x), fma(w, t.y, acc.y), fma(w, t.z, acc.z), fma(w, t.w, acc.w)};
+};
+template <bool DISTANT>
+struct FarTerms {
+    const PtsLDS& P;
+    const FarGeom& G;
+    __device__ __forceinline__ q4 sum(int k0, int k1, int step, q4 acc) const {
+        for (int k = k0; k < k1; k += step) {
+            const QPoint Q = P.f[k];
+            const q4 t = theta_terms_far<DISTANT>(Q.b0, Q.b1, Q.pp, G);
+            acc = {fma(Q.w, t.x, acc.x), fma(Q.w, t.y, acc.y), fma(Q.w, t.z, acc.z), fma(Q.w, t.w, acc.w)};
+        }
+        return acc;
     }
-    return acc;
-}
+};
+// 64 consecutive panels of a mesh in a local order have some 45 to 66 vertices
+// against 192 corners.  Four points at a time, lane v writes the distance of
+// vertex v (and v + 64) to the wavefront's table in LDS, and each panel reads
+// its three: 65 FP64 instructions per evaluation instead of 83, and three LDS
+// reads.  One wavefront's LDS operations complete in order, so that no barrier
+// is needed between the writes and the reads.  Rows of 5,120 panels 6.75 -> 6.28
+// ms, at 84 % of the issue slots instead of 94; the chip's clock follows the
+// load (1.82 and 1.89 GHz), and two or three wavefronts per SIMD give the same.
+constexpr int TILE_POINTS = 4;
+template <bool DISTANT>
+struct SharedTerms {
+    const PtsLDS& P;
+    const FarGeom& G;
+    double* table;           // TILE_POINTS x TILE_VERTS
+    VertexPoly v0, v1;       // this lane's vertices
+    bool two;                // more than 64 of them (uniform)
+    uint32_t corners;
+    // N points from k on
+    template <int N>
+    __device__ __forceinline__ q4 points(int k, q4 acc) const {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int p = 0; p < N; ++p) {
+            const QPoint Q = P.f[k + p];
+            table[p * TILE_VERTS + lane] = vertex_distance(v0, Q.b0, Q.b1, Q.pp);
+        }
+        if (two && lane < TILE_VERTS - 64) {
+#pragma unroll
+            for (int p = 0; p < N; ++p) {
+                const QPoint Q = P.f[k + p];
+                table[p * TILE_VERTS + 64 + lane] = vertex_distance(v1, Q.b0, Q.b1, Q.pp);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        const double *a = table + (corners & 255u), *b = table + ((corners >> 8) & 255u), *c = table + (corners >> 16);
+#pragma unroll
+        for (int p = 0; p < N; ++p) {
+            const QPoint Q = P.f[k + p];
+            const q4 t = theta_terms_of<DISTANT>(a[p * TILE_VERTS], b[p * TILE_VERTS], c[p * TILE_VERTS], Q.b0, Q.b1, G);
+            acc = {fma(Q.w, t.x, acc.x), fma(Q.w, t.y, acc.y), fma(Q.w, t.z, acc.z), fma(Q.w, t.w, acc.w)};
+        }
+        __builtin_amdgcn_wave_barrier();
+        return acc;
+    }
+    __device__ __forceinline__ q4 sum(int k0, int k1, int, q4 acc) const {
+        int k = k0;
+        for (; k + TILE_POINTS <= k1; k += TILE_POINTS) acc = points<TILE_POINTS>(k, acc);
+        for (; k < k1; ++k) acc = points<1>(k, acc);
+        return acc;
+    }
+};
 // Sums of the terms over level 0 (T0) and level 1 (T1) of a pair, lane s of LPP.
-template <int FORM, int LPP>
-__device__ __forceinline__ void sweep_terms(const RuleLDS& R, const PtsLDS& P, int npts, bool share, bool need0, bool need1, int s,
-                                            const FormGeom<FORM>& J, q4& T0, q4& T1) {
+template <int LPP, class Terms>
+__device__ __forceinline__ void sweep_terms(const Terms& E, int npts, bool share, bool need0, bool need1, int s, q4& T0, q4& T1) {
     int k0 = s, k1 = npts + s;
     if (share) {
         // point 0 of child 4 stands for point 0 of level 0 as well (lane 0 takes both)
         if (s == 0) {
-            double w;
-            T0 = terms_at<FORM>(R, P, 4 * npts, J, w);
-            T0 = w * T0;
+            T0 = E.sum(4 * npts, 4 * npts + 1, 1, q4zero());
             T1 = T0;
             k0 = LPP;
         }
         // children 1 to 3 and child 4's other points around the shared one
-        T0 = quad_pts<FORM>(R, P, k0, npts, LPP, J, T0);
-        T1 = quad_pts<FORM>(R, P, k1, 4 * npts, LPP, J, T1);
-        T1 = quad_pts<FORM>(R, P, 4 * npts + k0, 5 * npts, LPP, J, T1);
+        T0 = E.sum(k0, npts, LPP, T0);
+        T1 = E.sum(k1, 4 * npts, LPP, T1);
+        T1 = E.sum(4 * npts + k0, 5 * npts, LPP, T1);
         return;
     }
-    if (need0) T0 = quad_pts<FORM>(R, P, k0, npts, LPP, J, T0);
-    if (need1) T1 = quad_pts<FORM>(R, P, k1, 5 * npts, LPP, J, T1);
+    if (need0) T0 = E.sum(k0, npts, LPP, T0);
+    if (need1) T1 = E.sum(k1, 5 * npts, LPP, T1);
 }
 
 __device__ __forceinline__ q4 shfl_sum(q4 v, int G) {
@@ -333,10 +377,32 @@ __device__ __forceinline__ void flush_row(const MeshDesc& M, int type, int i, q4
     acc1 = q4zero();
 }
 
-// Levels 0 and 1 of one disjoint task (lane group of LPP lanes), then the Runge check.
+// The sums of a wavefront's pairs by the tile's shared distances; all 64 lanes
+// take part.
+template <bool DISTANT>
+__device__ __forceinline__ void shared_sums(const BatchArgs& A, const PtsLDS& pts, const MeshDesc& M, int tile, uint32_t corners,
+                                            double* table, const FarFrame& F, const JGeom& JG, bool need0, bool need1, q4& T0,
+                                            q4& T1) {
+    const int32_t* list = M.tile_list + (int64_t)tile * TILE_LIST;
+    const int lane = threadIdx.x & 63, n = list[0];
+    auto vertex = [&](int k) {
+        const double* x = M.xyz + 3 * (int64_t)list[1 + (k < n ? k : 0)];
+        return vertex_poly(F, d3{x[0], x[1], x[2]});
+    };
+    const FarGeom G = far_geom(F, JG);
+    const SharedTerms<DISTANT> E{pts, G, table, vertex(lane), vertex(lane + 64), n > 64, corners};
+    sweep_terms<1>(E, A.rule.n, share_centroid(A), need0, need1, 0, T0, T1);
+    T0 = far_scale(T0, JG);
+    T1 = far_scale(T1, JG);
+}
+
+// Levels 0 and 1 of one disjoint task (lane group of LPP lanes), then the Runge
+// check.  table: of the wavefront, whose pairs are with tile `tile` of the mesh
+// (null: their panels are not one tile).
 template <int LPP>
-__device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS& R, int m, int i, int j, int64_t z, bool valid,
-                                              int s, const Panel& I, const Panel& J, const PtsLDS& pts, const Ball& ball) {
+__device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS& R, const MeshDesc& M, int m, int i, int j, int64_t z,
+                                              bool valid, int s, const Panel& I, const Panel& J, const PtsLDS& pts, const Ball& ball,
+                                              const FarFrame& F, double* table, int tile) {
     const JGeom JG = jgeom(J);
     const int npts = A.rule.n;
     const bool need0 = !A.fixed || A.last_level == 0;
@@ -344,17 +410,23 @@ __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS&
     q4 v0 = q4zero(), v1 = q4zero();
     // one loop per wavefront, in the form that holds for all its pairs
     const int form = wave_form(valid, ball, JG);
-    if (valid) {
-        q4 T0 = q4zero(), T1 = q4zero();
+    q4 T0 = q4zero(), T1 = q4zero();
+    if (LPP == 1 && form != 0 && table && M.tile_list[(int64_t)tile * TILE_LIST] > 0) {
+        const uint32_t corners = M.corners[min(j, M.nT - 1)];
+        if (form == 1) shared_sums<false>(A, pts, M, tile, corners, table, F, JG, need0, need1, T0, T1);
+        else shared_sums<true>(A, pts, M, tile, corners, table, F, JG, need0, need1, T0, T1);
+    } else if (valid) {
         if (form == 0) {
-            sweep_terms<0, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, FormGeom<0>{JG}, T0, T1);
+            sweep_terms<LPP>(GeneralTerms{R, pts, F, JG}, npts, share_centroid(A), need0, need1, s, T0, T1);
         } else {
-            const FarGeom G = far_geom(far_frame(I.a, I.b, I.c), JG);
-            if (form == 1) sweep_terms<1, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, FormGeom<1>{G}, T0, T1);
-            else sweep_terms<2, LPP>(R, pts, npts, share_centroid(A), need0, need1, s, FormGeom<2>{G}, T0, T1);
+            const FarGeom G = far_geom(F, JG);
+            if (form == 1) sweep_terms<LPP>(FarTerms<false>{pts, G}, npts, share_centroid(A), need0, need1, s, T0, T1);
+            else sweep_terms<LPP>(FarTerms<true>{pts, G}, npts, share_centroid(A), need0, need1, s, T0, T1);
             T0 = far_scale(T0, JG);
             T1 = far_scale(T1, JG);
         }
+    }
+    if (valid) {
         v0 = I.area * psi_of_terms(T0, JG);
         v1 = (0.25 * I.area) * psi_of_terms(T1, JG);
     }
@@ -379,8 +451,10 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
     RuleLDS& R = S.R;
     PtsLDS& pts = S.pts;
     __shared__ long long chunk_sh;
+    extern __shared__ double wave_tables[];   // one table per wavefront, where each has a tile (tile_table_bytes)
     load_rule(R, A.rule);
     const int P = A.pairs_per_item;
+    double* const tables = LPP == 1 && P % 64 == 0 ? wave_tables : nullptr;
     const int per_round = blockDim.x / LPP;
     const int p0 = threadIdx.x / LPP, s = threadIdx.x % LPP;
     const int64_t chunks = (A.disjoint_items + A.sweep_chunk - 1) / A.sweep_chunk;
@@ -402,10 +476,11 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
                 i = row;
                 i_mesh = m;
                 __syncthreads();
-                load_points(pts, R, A.rule.n, I);
+                load_points(pts, R, A.rule.n, far_frame(I.a, I.b, I.c));
                 __syncthreads();
             }
             const Ball ball = panel_ball(I.a, I.b, I.c, A.rule.reach);
+            const FarFrame F = far_frame(I.a, I.b, I.c);
             for (int round = 0; round < P; round += per_round) {
                 const int p = round + p0;
                 const int j = tile * P + p;
@@ -413,7 +488,10 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
                 const Panel J = M.panels[in_range ? j : i];
                 const bool valid = in_range && j != i && shared_count(I, J) == 0;
                 const int64_t z = valid ? disjoint_task(M, i, j) : 0;
-                const StepOut o = sweep_task<LPP>(A, R, m, i, j, z, valid, s, I, J, pts, ball);
+                const int tile64 = __builtin_amdgcn_readfirstlane((tile * P + p) >> 6);
+                const StepOut o = sweep_task<LPP>(A, R, M, m, i, j, z, valid, s, I, J, pts, ball, F,
+                                                  tables && 64 * tile64 < M.nT ? tables + (threadIdx.x >> 6) * TILE_POINTS * TILE_VERTS : nullptr,
+                                                  tile64);
                 q4 rp0 = q4zero(), rp1 = q4zero();
                 if (o.finished) finish_task<I2_NOT_NEIGHBORS, OUT>(A, M, z, i, j, o, I, J, &rp0, &rp1);
                 if (OUT == OUT_ROW_SUMS) { acc0 = acc0 + rp0; acc1 = acc1 + rp1; }
@@ -758,12 +836,17 @@ int lanes_for_points_per_lane(int ppl) {
 // workgroup of the disjoint sweep: P pairs of LPP lanes, at most 256 lanes
 static int sweep_block(int P, int lpp) { return std::min(256, P * lpp); }
 
+// dynamic LDS: a table per wavefront if the wavefronts' pairs are tiles of 64
+static size_t tile_table_bytes(int P, int lpp) {
+    return lpp == 1 && P % 64 == 0 ? sizeof(double) * TILE_POINTS * TILE_VERTS * (size_t)(sweep_block(P, lpp) / 64) : 0;
+}
+
 template <int OUT, int LPP>
 static int sweep_grid_for(int P, int* grid) {
     int dev = 0, cus = 0, per = 0;
     I2_HIP(hipGetDevice(&dev));
     I2_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    I2_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_sweep_disjoint<OUT, LPP>, sweep_block(P, LPP), 0));
+    I2_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_sweep_disjoint<OUT, LPP>, sweep_block(P, LPP), tile_table_bytes(P, LPP)));
     *grid = std::max(1, cus * std::max(1, per));
     return I2_OK;
 }
@@ -771,7 +854,7 @@ static int sweep_grid_for(int P, int* grid) {
 static int launch_sweep(const Engine& E, hipStream_t st) {
     const int lpp = lanes_for_points_per_lane(E.ppl);
     const dim3 blk(sweep_block(E.pairs_per_wg, lpp)), grd(E.sweep_grid);
-#define I2_SWEEP(O, L) hipLaunchKernelGGL((k_sweep_disjoint<O, L>), grd, blk, 0, st, E.args)
+#define I2_SWEEP(O, L) hipLaunchKernelGGL((k_sweep_disjoint<O, L>), grd, blk, tile_table_bytes(E.pairs_per_wg, L), st, E.args)
     if (E.out == OUT_PER_PAIR) {
         if (lpp == 1) I2_SWEEP(OUT_PER_PAIR, 1); else if (lpp == 4) I2_SWEEP(OUT_PER_PAIR, 4);
         else if (lpp == 8) I2_SWEEP(OUT_PER_PAIR, 8); else I2_SWEEP(OUT_PER_PAIR, 16);
@@ -868,12 +951,14 @@ int batch_enqueue(Engine& E, hipStream_t st) {
 // that leaves most SIMDs without a wavefront (1,024 SIMDs).  Row sums by shape,
 // one / four lanes: 80 panels (160 wavefronts) 220 / 196 us, 320 panels (1,600)
 // 295 / 312, 1,280 panels 840 / 1,090; eight and sixteen lanes are slower than
-// four on all three.
+// four on all three.  Where there are many wavefronts, two share a control
+// panel's points: 6,144 panels of a torus 8.14 -> 8.01 ms, 5,120 of a sphere
+// 5.46 -> 5.40, with 3,000 (141,000 wavefronts) equal.
 void engine_auto_shape(Engine& E) {
     int64_t waves = 0;
     for (const MeshDesc& D : E.h_meshes) waves += (int64_t)D.nT * ((D.nT + 63) / 64);
     E.ppl = waves >= 512 ? 13 : 4;
-    E.pairs_per_wg = 64 / lanes_for_points_per_lane(E.ppl);
+    E.pairs_per_wg = waves >= 65536 ? 128 : 64 / lanes_for_points_per_lane(E.ppl);
 }
 
 int engine_setup(Engine& E, const i2_integrator& it) {
@@ -1021,6 +1106,8 @@ struct i2_batch {
         i2::DBuf<double> rowacc, rowout;
     };
     std::vector<Out> outs;
+    i2::DBuf<int32_t> tile_lists;              // MeshDesc::tile_list of all meshes
+    i2::DBuf<uint32_t> corners;
     std::vector<int> K;
     std::vector<unsigned long long> counts;
     bool ran = false;
@@ -1062,6 +1149,36 @@ static bool batch_current(const i2_batch* b) {
     for (size_t m = 0; m < b->meshes.size(); ++m)
         if (!b->meshes[m]->prepared || b->meshes[m]->generation != b->generations[m]) return false;
     return true;
+}
+
+// The vertex list of a tile of 64 panels, a wavefront each: corners in order
+// (all panels' first corners, then the second and third), each vertex at its
+// first corner.
+__global__ __launch_bounds__(64) void k_tile_vertices(int nT, const int32_t* __restrict__ tri, int32_t* __restrict__ lists,
+                                                      uint32_t* __restrict__ corners) {
+    __shared__ int32_t id[192], rank[192];
+    const int lane = threadIdx.x, j = 64 * blockIdx.x + lane;
+    const bool in = j < nT;
+    for (int c = 0; c < 3; ++c) id[64 * c + lane] = in ? tri[3 * (int64_t)j + c] : -1 - lane - 64 * c;
+    __syncthreads();
+    int32_t* list = lists + (int64_t)blockIdx.x * TILE_LIST;
+    int first[3], n = 0;
+    for (int c = 0; c < 3; ++c) {
+        const int own = 64 * c + lane, x = id[own];
+        int f = own;
+        for (int k = own - 1; k >= 0; --k) if (id[k] == x) f = k;
+        first[c] = f;
+        const unsigned long long fresh = __ballot(in && f == own);
+        if (in && f == own) {
+            const int r = n + __popcll(fresh & ((1ull << lane) - 1ull));
+            rank[own] = r;
+            if (r < TILE_VERTS) list[1 + r] = x;
+        }
+        n += __popcll(fresh);
+    }
+    __syncthreads();
+    if (lane == 0) list[0] = n <= TILE_VERTS ? n : 0;
+    if (in) corners[j] = (uint32_t)rank[first[0]] | (uint32_t)rank[first[1]] << 8 | (uint32_t)rank[first[2]] << 16;
 }
 
 static int batch_prepare(i2_batch* b) {
@@ -1106,6 +1223,25 @@ static int batch_prepare(i2_batch* b) {
         E.h_meshes[m] = D;
     }
     if (!b->tuned) engine_auto_shape(E);
+    int64_t tiles = 0, panels = 0;
+    for (const i2_mesh* mesh : b->meshes) { tiles += (mesh->nT + 63) / 64; panels += mesh->nT; }
+    I2_TRY(b->tile_lists.ensure(TILE_LIST * tiles));
+    I2_TRY(b->corners.ensure(panels));
+    tiles = panels = 0;
+    for (int m = 0; m < M; ++m) {
+        const i2_mesh* mesh = b->meshes[m];
+        const int64_t n = (mesh->nT + 63) / 64;
+        MeshDesc& D = E.h_meshes[m];
+        int32_t* lists = b->tile_lists.p + TILE_LIST * tiles;
+        uint32_t* corners = b->corners.p + panels;
+        hipLaunchKernelGGL(k_tile_vertices, dim3((unsigned)n), dim3(64), 0, b->stream, D.nT, mesh->d_tri.p, lists, corners);
+        I2_TRY(check_launch("k_tile_vertices"));
+        D.xyz = mesh->d_xyz.p;
+        D.tile_list = lists;
+        D.corners = corners;
+        tiles += n;
+        panels += mesh->nT;
+    }
     I2_TRY(engine_setup(E, b->cfg));
     for (const i2_mesh* mesh : b->meshes) b->generations.push_back(mesh->generation);
     if (!b->adjoint) return I2_OK;

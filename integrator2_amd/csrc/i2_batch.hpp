@@ -18,6 +18,12 @@ struct MeshDesc {
     int64_t npairs[3];            // unordered pair counts per type
     int nT;
     int pad;
+    // the vertices of each tile of 64 consecutive panels, TILE_LIST entries: their
+    // number (0: more than TILE_VERTS), then their indices; and each panel's
+    // corners as numbers into its tile's list, eight bits each
+    const double* xyz;
+    const int32_t* tile_list;
+    const uint32_t* corners;
     // per-pair outputs (per type, 2*npairs entries, reference task order)
     double4* fin[3];
     double4* prev[3];
@@ -47,6 +53,8 @@ constexpr int MAX_BATCH_MESHES = 256;
 constexpr int MASK_WORDS = MAX_BATCH_MESHES / 64;
 
 constexpr int N_COUNTERS = 2 + MAX_LEVELS * 3;
+
+constexpr int TILE_VERTS = 96, TILE_LIST = TILE_VERTS + 1;
 
 struct BatchArgs {
     const MeshDesc* meshes;

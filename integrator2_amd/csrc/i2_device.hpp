@@ -268,11 +268,9 @@ I2_HD __forceinline__ FarGeom far_geom(const FarFrame& F, const JGeom& J) {
             dot(c, c), 2.0 * dot(F.U, c), 2.0 * dot(F.V, c), dot(a, N), dot(F.U, N), dot(F.V, N),
             J.Lc * J.Lc, J.La * J.La, J.Lb * J.Lb};
 }
+// from the three distances
 template <bool DISTANT>
-I2_HD __forceinline__ q4 theta_terms_far(double b0, double b1, double pp, const FarGeom& G) {
-    const double la = i2m::sqrt_cubic(fma(b0, G.ua, fma(b1, G.va, G.ka + pp))),
-                 lb = i2m::sqrt_cubic(fma(b0, G.ub, fma(b1, G.vb, G.kb + pp))),
-                 lc = i2m::sqrt_cubic(fma(b0, G.uc, fma(b1, G.vc, G.kc + pp)));
+I2_HD __forceinline__ q4 theta_terms_of(double la, double lb, double lc, double b0, double b1, const FarGeom& G) {
     const double y = fma(b0, G.uy, fma(b1, G.vy, G.ky));           // 2 y
     const double S1 = la + lb, S2 = lb + lc, S3 = lc + la;
     const double s12 = S1 * S2, s123 = s12 * S3;
@@ -282,6 +280,20 @@ I2_HD __forceinline__ q4 theta_terms_far(double b0, double b1, double pp, const 
     const double r1 = i3 * S2, r2 = i3 * S1, r3 = i * s12, u = y * (inv * s123);
     return {r1 * i2m::atanh_over<DISTANT>(G.q1 * (r1 * r1)), r2 * i2m::atanh_over<DISTANT>(G.q2 * (r2 * r2)),
             r3 * i2m::atanh_over<DISTANT>(G.q3 * (r3 * r3)), u * i2m::atan_over<DISTANT>(u * u)};
+}
+// one vertex's distance polynomial
+struct VertexPoly { double k, u, v; };
+I2_HD __forceinline__ VertexPoly vertex_poly(const FarFrame& F, d3 x) {
+    const d3 a = F.m - x;
+    return {dot(a, a), 2.0 * dot(F.U, a), 2.0 * dot(F.V, a)};
+}
+I2_HD __forceinline__ double vertex_distance(const VertexPoly& x, double b0, double b1, double pp) {
+    return i2m::sqrt_cubic(fma(b0, x.u, fma(b1, x.v, x.k + pp)));
+}
+template <bool DISTANT>
+I2_HD __forceinline__ q4 theta_terms_far(double b0, double b1, double pp, const FarGeom& G) {
+    return theta_terms_of<DISTANT>(vertex_distance({G.ka, G.ua, G.va}, b0, b1, pp), vertex_distance({G.kb, G.ub, G.vb}, b0, b1, pp),
+                                   vertex_distance({G.kc, G.uc, G.vc}, b0, b1, pp), b0, b1, G);
 }
 // sums of theta_terms_far to sums of theta_terms
 I2_HD __forceinline__ q4 far_scale(q4 T, const JGeom& J) { return {2.0 * J.Lc * T.x, 2.0 * J.La * T.y, 2.0 * J.Lb * T.z, T.w}; }
