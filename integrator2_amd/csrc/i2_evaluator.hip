@@ -91,6 +91,16 @@ __device__ __forceinline__ q4 quad_far(const Rule& R, int level, int sub, int G,
     return acc;
 }
 
+__device__ __forceinline__ q4 lanes_sum(q4 v, int lanes) {
+    for (int m = 1; m < lanes; m <<= 1) {
+        v.x += __shfl_xor(v.x, m);
+        v.y += __shfl_xor(v.y, m);
+        v.z += __shfl_xor(v.z, m);
+        v.w += __shfl_xor(v.w, m);
+    }
+    return v;
+}
+
 // Level-`level` value of tasks: lanes per task = 1 << lanes_log2, of which
 // 1 << per_log2 share a sub-panel's points; the groups walk the sub-panels
 // < 4^level; butterfly reduction.
@@ -136,13 +146,83 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_
         }
         if (TYPE == I2_NOT_NEIGHBORS) acc = psi_of_terms(acc, JG);
     }
-    for (int m = 1; m < lanes; m <<= 1) {
-        acc.x += __shfl_xor(acc.x, m);
-        acc.y += __shfl_xor(acc.y, m);
-        acc.z += __shfl_xor(acc.z, m);
-        acc.w += __shfl_xor(acc.w, m);
-    }
+    acc = lanes_sum(acc, lanes);
     if (active && sub == 0) out[z] = make_double4(acc.x, acc.y, acc.z, acc.w);
+}
+
+// Appends the wavefront's unconverged tasks to a rest list, one atomic per wavefront.
+__device__ __forceinline__ void append_rest(bool unconv, int64_t z, int32_t* __restrict__ rest, unsigned long long* __restrict__ counter) {
+    const unsigned long long mask = __ballot(unconv);
+    const int lane = threadIdx.x & 63;
+    const int before = __popcll(mask & ((1ull << lane) - 1ull));
+    unsigned long long base = 0;
+    if (lane == 0 && mask) base = atomicAdd(counter, (unsigned long long)__popcll(mask));
+    base = __shfl(base, 0);
+    if (unconv) rest[base + before] = (int32_t)z;
+}
+
+// Levels 0 and 1 of all tasks and their comparison (k_level for the two levels,
+// then k_compare) in one launch: every task needs both, and the pair's
+// geometry and the tasks' decoding serve both.  1 << lanes_log2 lanes per task
+// share each level's points.  Plain run of 1,330 panels 1,250 -> 1,154 us, of 80
+// panels 183 -> 134 (with one launch for the closed forms of all types).
+template <int TYPE, bool IMPLICIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_NOT_NEIGHBORS ? 3 : 2))) void k_first_levels(
+    int64_t nitems, TaskSource src, const Panel* __restrict__ panels, Rule R, int lanes_log2, double tol, int keep_converged,
+    double4* __restrict__ out0, double4* __restrict__ out1, int8_t* __restrict__ conv, int32_t* __restrict__ rest_out,
+    unsigned long long* __restrict__ counter) {
+    __shared__ i2m::MathTable lt;
+    i2m::fill_mathtab(lt);
+    __syncthreads();
+    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int lanes = 1 << lanes_log2, s = (int)(gid & (lanes - 1));
+    const int per = max(1, lanes >> 2), subs = min(4, lanes), sub = s / per, k0 = s % per;   // level 1: per lanes a sub-panel
+    const int64_t z = gid >> lanes_log2;
+    const bool active = z < nitems;
+    q4 v0 = q4zero(), v1 = q4zero();
+    if (active) {
+        int i, j;
+        task_ij<IMPLICIT>(src, z, &i, &j);
+        const Panel I = panels[i];
+        const Panel J = panels[j];
+        const JGeom JG = make_jgeom(J.a, J.b, J.c, J.ta, J.tb, J.tc);
+        PairCtx<TYPE> ctx;
+        ctx.init(I, J);
+        const double area = I.area;
+        const int form = TYPE == I2_NOT_NEIGHBORS ? wave_form(true, panel_ball(I.a, I.b, I.c, R.reach), JG) : 0;
+        if (form != 0) {
+            const FarFrame F = far_frame(I.a, I.b, I.c);
+            const FarGeom FG = far_geom(F, JG);
+            if (form == 1) {
+                v0 = quad_far<false>(R, 0, 0, 1, s, lanes, F, FG);
+                v1 = quad_far<false>(R, 1, sub, subs, k0, per, F, FG);
+            } else {
+                v0 = quad_far<true>(R, 0, 0, 1, s, lanes, F, FG);
+                v1 = quad_far<true>(R, 1, sub, subs, k0, per, F, FG);
+            }
+            v0 = area * far_scale(v0, JG);
+            v1 = (0.25 * area) * far_scale(v1, JG);
+        } else {
+            v0 = quad_sub<TYPE>(R, &lt, I.a, I.b, I.c, area, JG, ctx, s, lanes);
+            for (uint32_t c = sub; c < 4; c += subs) {
+                d3 a = I.a, b = I.b, cc = I.c;
+                sub_panel(a, b, cc, 1, c);
+                v1 = v1 + quad_sub<TYPE>(R, &lt, a, b, cc, 0.25 * area, JG, ctx, k0, per);
+            }
+        }
+        if (TYPE == I2_NOT_NEIGHBORS) { v0 = psi_of_terms(v0, JG); v1 = psi_of_terms(v1, JG); }
+    }
+    v0 = lanes_sum(v0, lanes);
+    v1 = lanes_sum(v1, lanes);
+    bool unconv = false;
+    if (active && s == 0) {
+        unconv = runge_criterion(v1, v0, R.pow2p) > tol;
+        conv[z] = 1;
+        out1[z] = make_double4(v1.x, v1.y, v1.z, v1.w);
+        const q4 p = !unconv && keep_converged ? v1 : v0;
+        out0[z] = make_double4(p.x, p.y, p.z, p.w);
+    }
+    append_rest(unconv, z, rest_out, counter);
 }
 
 // Runge comparison of iteration `it` (evaluator3d.cu:76-99): items are all
@@ -166,22 +246,14 @@ __global__ __launch_bounds__(256) void k_compare(int64_t nitems, const int32_t* 
         conv[z] = (int8_t)it;
         if (!unconv && keep_converged) prev[z] = c4;
     }
-    const unsigned long long mask = __ballot(unconv);
-    const int lane = threadIdx.x & 63;
-    const int before = __popcll(mask & ((1ull << lane) - 1ull));
-    unsigned long long base = 0;
-    if (lane == 0 && mask) base = atomicAdd(counter, (unsigned long long)__popcll(mask));
-    base = __shfl(base, 0);
-    if (unconv) rest_out[base + before] = (int32_t)z;
+    append_rest(unconv, z, rest_out, counter);
 }
 
 // Analytic singular part (vertex/edge-sharing) and conversion to J
 // (evaluatorJ3DK.cu:22-56, 224-264).  The final integrals stay in `ints`.
 template <int TYPE, bool IMPLICIT>
-__global__ __launch_bounds__(256) void k_finalize(int64_t n, TaskSource src, const Panel* __restrict__ panels,
-                                                  double4* __restrict__ ints, double* __restrict__ results) {
-    const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (z >= n) return;
+__device__ __forceinline__ void finalize_one(int64_t z, const TaskSource& src, const Panel* __restrict__ panels,
+                                             double4* __restrict__ ints, double* __restrict__ results) {
     int i, j;
     task_ij<IMPLICIT>(src, z, &i, &j);
     const Panel I = panels[i];
@@ -206,6 +278,23 @@ __global__ __launch_bounds__(256) void k_finalize(int64_t n, TaskSource src, con
     }
     ints[z] = make_double4(v.x, v.y, v.z, v.w);
     results[3 * z] = res.x; results[3 * z + 1] = res.y; results[3 * z + 2] = res.z;
+}
+
+// All types in one launch, a range of workgroups each, the closed forms first:
+// one after another their 17 and 12 us on few tasks are latency.
+struct FinalizeType { int64_t n; unsigned blocks; TaskSource src; double4* ints; double* results; };
+struct FinalizeArgs { FinalizeType t[3]; bool implicit; };
+__global__ __launch_bounds__(256) void k_finalize(FinalizeArgs A, const Panel* __restrict__ panels) {
+    unsigned b = blockIdx.x;
+    int t = 0;
+    while (t < 2 && b >= A.t[t].blocks) b -= A.t[t++].blocks;
+    const FinalizeType& T = A.t[t];
+    const int64_t z = (int64_t)b * blockDim.x + threadIdx.x;
+    if (z >= T.n) return;
+    if (t == I2_SIMPLE_NEIGHBORS) finalize_one<I2_SIMPLE_NEIGHBORS, false>(z, T.src, panels, T.ints, T.results);
+    else if (t == I2_ATTACHED_NEIGHBORS) finalize_one<I2_ATTACHED_NEIGHBORS, false>(z, T.src, panels, T.ints, T.results);
+    else if (A.implicit) finalize_one<I2_NOT_NEIGHBORS, true>(z, T.src, panels, T.ints, T.results);
+    else finalize_one<I2_NOT_NEIGHBORS, false>(z, T.src, panels, T.ints, T.results);
 }
 
 // (i,j)/(j,i) symmetry error (evaluator3d.cu:45-57)
@@ -259,6 +348,18 @@ static int launch_level(i2_evaluator* ev, int64_t nitems, const int32_t* list, c
     return I2_OK;
 }
 
+// Lanes per task of k_first_levels, by the same rule: one to 64, disjoint pairs at
+// most 16 (their points cost less than the geometry each lane repeats: 80 panels
+// took 34 us with 64 lanes)
+template <int TYPE, bool IMPLICIT>
+static int launch_first_levels(hipStream_t st, const Panel* panels, const i2_integrator& it, int64_t n, const TaskSource& src,
+                               double4* out0, double4* out1, int8_t* conv, int32_t* rest, unsigned long long* counter) {
+    const int ll = std::min(lanes_log2_for(1, n), TYPE == I2_NOT_NEIGHBORS ? 4 : 6);
+    hipLaunchKernelGGL((k_first_levels<TYPE, IMPLICIT>), dim3(blocks_for(n << ll, 256)), dim3(256), 0, st, n, src, panels, it.rule, ll,
+                       it.tol, it.quirk ? 0 : 1, out0, out1, conv, rest, counter);
+    return check_launch("k_first_levels");
+}
+
 static void clear_launches(i2_evaluator* ev) {
     for (auto& r : ev->launches) {
         if (r.e0) (void)hipEventDestroy(r.e0);
@@ -274,16 +375,19 @@ static int launch_level_of(i2_evaluator* ev, int type, bool implicit, int64_t ni
     return implicit ? launch_level<I2_NOT_NEIGHBORS, true>(ev, nitems, list, src, level, out)
                     : launch_level<I2_NOT_NEIGHBORS, false>(ev, nitems, list, src, level, out);
 }
-static int launch_finalize(i2_evaluator* ev, int type, TypeState& ts, const TaskSource& src) {
-    const dim3 grid(blocks_for(ts.n, 256)), block(256);
+static int launch_first_levels_of(i2_evaluator* ev, int type, TypeState& ts, const TaskSource& src, unsigned long long* counter) {
     const Panel* panels = ev->mesh->d_panels.p;
-    double4* ints = ts.buf[ts.final_buf].p;
-#define I2_FINALIZE(T, I) hipLaunchKernelGGL((k_finalize<T, I>), grid, block, 0, ev->stream, ts.n, src, panels, ints, ts.results.p)
-    if (type == I2_SIMPLE_NEIGHBORS) I2_FINALIZE(I2_SIMPLE_NEIGHBORS, false);
-    else if (type == I2_ATTACHED_NEIGHBORS) I2_FINALIZE(I2_ATTACHED_NEIGHBORS, false);
-    else if (ts.implicit) I2_FINALIZE(I2_NOT_NEIGHBORS, true);
-    else I2_FINALIZE(I2_NOT_NEIGHBORS, false);
-#undef I2_FINALIZE
+#define I2_FIRST(T, I) launch_first_levels<T, I>(ev->stream, panels, *ev->integ, ts.n, src, ts.buf[0].p, ts.buf[1].p, ts.conv.p, ts.rest[1].p, counter)
+    if (type == I2_SIMPLE_NEIGHBORS) return I2_FIRST(I2_SIMPLE_NEIGHBORS, false);
+    if (type == I2_ATTACHED_NEIGHBORS) return I2_FIRST(I2_ATTACHED_NEIGHBORS, false);
+    return ts.implicit ? I2_FIRST(I2_NOT_NEIGHBORS, true) : I2_FIRST(I2_NOT_NEIGHBORS, false);
+#undef I2_FIRST
+}
+static int launch_finalize(hipStream_t st, const Panel* panels, FinalizeArgs A) {
+    unsigned blocks = 0;
+    for (FinalizeType& T : A.t) { T.blocks = blocks_for(T.n, 256); blocks += T.blocks; }
+    if (blocks == 0) return I2_OK;
+    hipLaunchKernelGGL(k_finalize, dim3(blocks), dim3(256), 0, st, A, panels);
     return check_launch("k_finalize");
 }
 
@@ -358,7 +462,6 @@ static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
             I2_TRY(launch_level_of(ev, t, ts.implicit, ts.n, nullptr, src[t], it.fixed_level, ts.buf[0].p));
             ts.refined_tasks = ts.n << (2 * it.fixed_level);
             ts.K = it.fixed_level;
-            I2_TRY(launch_finalize(ev, t, ts, src[t]));
             I2_TRY(marks.mark(t));
         }
     } else {
@@ -372,7 +475,9 @@ static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
         int64_t remaining[3];
         int cur_rest[3] = {0, 0, 0};
         for (int t = 0; t < 3; ++t) remaining[t] = ev->type[t].n;
-        for (int iter = 0; iter <= it.max_level && (remaining[0] > 0 || remaining[1] > 0 || remaining[2] > 0); ++iter) {
+        // levels 0 and 1 in one launch per type, but for profiled runs, which list each level's
+        const bool first = it.max_level > 0 && !ev->profile;
+        for (int iter = first ? 1 : 0; iter <= it.max_level && (remaining[0] > 0 || remaining[1] > 0 || remaining[2] > 0); ++iter) {
             if (iter > 1) I2_TRY(marks.mark(-1));
             for (int t = 0; t < 3; ++t) {
                 TypeState& ts = ev->type[t];
@@ -380,10 +485,16 @@ static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
                 if (n == 0) continue;
                 const int32_t* list = iter <= 1 ? nullptr : ts.rest[cur_rest[t]].p;
                 double4* cur = ts.buf[iter % 2].p;
-                I2_TRY(launch_level_of(ev, t, ts.implicit, n, list, src[t], iter, cur));
-                ts.refined_tasks += n << (2 * iter);
                 ts.K = iter;
                 ts.final_buf = iter % 2;
+                if (first && iter == 1) {
+                    I2_TRY(launch_first_levels_of(ev, t, ts, src[t], ev->d_counter.p + 3 + t));
+                    ts.refined_tasks = n + (n << 2);
+                    I2_TRY(marks.mark(t));
+                    continue;
+                }
+                I2_TRY(launch_level_of(ev, t, ts.implicit, n, list, src[t], iter, cur));
+                ts.refined_tasks += n << (2 * iter);
                 if (iter > 0) {
                     hipLaunchKernelGGL(k_compare, dim3(blocks_for(n, 256)), dim3(256), 0, ev->stream, n, list, cur, ts.buf[1 - iter % 2].p,
                                        it.rule.pow2p, it.tol, it.quirk ? 0 : 1, iter, ts.conv.p, ts.rest[1 - cur_rest[t]].p,
@@ -402,16 +513,23 @@ static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
                 remaining[t] = (int64_t)ev->h_counter[t];
             }
         }
-        I2_TRY(marks.mark(-1));
         for (int t = 0; t < 3; ++t) {
             TypeState& ts = ev->type[t];
-            if (ts.n == 0) continue;
-            if (remaining[t] > 0)   // still unconverged after the comparison at maxLevel (all tasks when maxLevel = 0)
+            if (ts.n > 0 && remaining[t] > 0)   // still unconverged after the comparison at maxLevel (all tasks when maxLevel = 0)
                 I2_TRY(mark_unconverged(ev, ts.implicit, src[t], remaining[t], it.max_level == 0 ? nullptr : ts.rest[cur_rest[t]].p, ts.unconv.p));
-            I2_TRY(launch_finalize(ev, t, ts, src[t]));
-            I2_TRY(marks.mark(t));
         }
     }
+    I2_TRY(marks.mark(-1));
+    FinalizeArgs F{};
+    F.implicit = ev->type[I2_NOT_NEIGHBORS].implicit;
+    int last = 0;
+    for (int t = 0; t < 3; ++t) {
+        TypeState& ts = ev->type[t];
+        F.t[t] = {ts.n, 0, src[t], ts.buf[ts.final_buf].p, ts.results.p};
+        if (ts.n > 0) last = t;
+    }
+    I2_TRY(launch_finalize(ev->stream, ev->mesh->d_panels.p, F));
+    I2_TRY(marks.mark(last));     // of all types, counted with the last
     I2_HIP(hipStreamSynchronize(ev->stream));
     return marks.times();
 }
@@ -700,16 +818,22 @@ static int run_tasks_noalloc(i2_evaluator* ev, const int32_t* d_tasks3, int64_t 
         I2_TRY(level(n, nullptr, it.fixed_level, buf[0]));
         K = it.fixed_level;
     } else {
-        I2_HIP(hipMemsetAsync(conv, 0, (size_t)n, st));
-        I2_TRY(level(n, nullptr, 0, buf[0]));
+        const bool first = it.max_level > 0 && !ev->profile;
+        if (!first) {
+            I2_HIP(hipMemsetAsync(conv, 0, (size_t)n, st));
+            I2_TRY(level(n, nullptr, 0, buf[0]));
+        }
         int64_t remaining = n;
         int iter = 0, cur_rest = 0;
         while (remaining > 0 && iter < it.max_level) {
             ++iter;
             const int32_t* list = (iter == 1) ? nullptr : rest[cur_rest];
-            I2_TRY(level(remaining, list, iter, buf[iter % 2]));
             I2_HIP(hipMemsetAsync(counter, 0, sizeof(unsigned long long), st));
-            hipLaunchKernelGGL(k_compare, dim3(blocks_for(remaining, 256)), dim3(256), 0, st, remaining, list, buf[iter % 2],
+            if (first && iter == 1)
+                I2_TRY((launch_first_levels<TYPE, false>(st, panels, it, n, src, buf[0], buf[1], conv, rest[1], counter)));
+            else
+                I2_TRY(level(remaining, list, iter, buf[iter % 2]));
+            if (!(first && iter == 1)) hipLaunchKernelGGL(k_compare, dim3(blocks_for(remaining, 256)), dim3(256), 0, st, remaining, list, buf[iter % 2],
                                buf[(iter - 1) % 2], it.rule.pow2p, it.tol, it.quirk ? 0 : 1, iter, conv, rest[1 - cur_rest],
                                counter);
             I2_TRY(check_launch("k_compare"));
@@ -722,8 +846,9 @@ static int run_tasks_noalloc(i2_evaluator* ev, const int32_t* d_tasks3, int64_t 
         final_buf = iter % 2;
     }
     if (final_buf == 1) I2_HIP(hipMemcpyAsync(buf[0], buf[1], sizeof(double4) * (size_t)n, hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL((k_finalize<TYPE, false>), dim3(blocks_for(n, 256)), dim3(256), 0, st, n, src, panels, buf[0], results);
-    I2_TRY(check_launch("k_finalize"));
+    FinalizeArgs F{};
+    F.t[TYPE] = {n, 0, src, buf[0], results};
+    I2_TRY(launch_finalize(st, panels, F));
     I2_HIP(hipStreamSynchronize(st));
     *Kout = K;
     return I2_OK;
