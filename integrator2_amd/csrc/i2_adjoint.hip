@@ -966,21 +966,28 @@ __global__ void k_adj_zero(unsigned long long* c, int nc, double* kj, int64_t nk
 int adjoint_launch(AdjState& S, hipStream_t st) {
     hipLaunchKernelGGL(k_adj_zero, dim3(4 * S.grid), dim3(256), 0, st, S.d_counters.p, N_ADJ_COUNTERS, S.d_kj.p, S.kj_total);
     I2_TRY(check_launch("k_adj_zero"));
+    // two streams, as in the forward pass
+    const bool two = S.args.singular_tasks > 0;
+    if (two) {
+        I2_TRY(S.side->fork(st));
+    }
     hipLaunchKernelGGL(k_adj_disjoint, dim3(4 * S.grid), dim3(64), 0, st, S.args);
     I2_TRY(check_launch("k_adj_disjoint"));
+    if (two) {
+        const hipStream_t sst = S.side->stream;
+        const int64_t blocks = std::min<int64_t>((S.args.singular_tasks + 15) / 16, 4 * (int64_t)S.grid);
+        hipLaunchKernelGGL(k_adj_singular<0>, dim3((unsigned)blocks), dim3(ADJ_BLOCK), 0, sst, S.args);
+        hipLaunchKernelGGL(k_adj_singular<1>, dim3((unsigned)blocks), dim3(ADJ_BLOCK), 0, sst, S.args);
+        hipLaunchKernelGGL(k_adj_singular<2>, dim3((unsigned)std::min<int64_t>(4 * blocks, 4 * (int64_t)S.grid)), dim3(ADJ_BLOCK), 0, sst, S.args);
+        I2_TRY(check_launch("k_adj_singular"));
+        hipLaunchKernelGGL(k_adj_singular_dual, dim3(S.grid), dim3(ADJ_BLOCK), 0, sst, S.args);
+        I2_TRY(check_launch("k_adj_singular_dual"));
+    }
     hipLaunchKernelGGL(k_adj_deep, dim3(16 * S.grid), dim3(256), 0, st, S.args);
     I2_TRY(check_launch("k_adj_deep"));
     hipLaunchKernelGGL(k_adj_deep_sum, dim3(4 * S.grid), dim3(64), 0, st, S.args);
     I2_TRY(check_launch("k_adj_deep_sum"));
-    if (S.args.singular_tasks > 0) {
-        const int64_t blocks = std::min<int64_t>((S.args.singular_tasks + 15) / 16, 4 * (int64_t)S.grid);
-        hipLaunchKernelGGL(k_adj_singular<0>, dim3((unsigned)blocks), dim3(ADJ_BLOCK), 0, st, S.args);
-        hipLaunchKernelGGL(k_adj_singular<1>, dim3((unsigned)blocks), dim3(ADJ_BLOCK), 0, st, S.args);
-        hipLaunchKernelGGL(k_adj_singular<2>, dim3((unsigned)std::min<int64_t>(4 * blocks, 4 * (int64_t)S.grid)), dim3(ADJ_BLOCK), 0, st, S.args);
-        I2_TRY(check_launch("k_adj_singular"));
-        hipLaunchKernelGGL(k_adj_singular_dual, dim3(S.grid), dim3(ADJ_BLOCK), 0, st, S.args);
-        I2_TRY(check_launch("k_adj_singular_dual"));
-    }
+    if (two) I2_TRY(S.side->join(st));
     if (S.args.npanels > 0) {
         const int64_t blocks = std::min<int64_t>((9 * S.args.npanels + 15) / 16, 16 * (int64_t)S.grid);
         hipLaunchKernelGGL(k_adj_panel_sum, dim3((unsigned)blocks), dim3(256), 0, st, S.args);
@@ -1097,6 +1104,7 @@ int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::ve
     A.seed = seed;
     A.disjoint_items = item_base[M];
     A.singular_tasks = sing_base[2 * M];
+    if (A.singular_tasks > 0) I2_TRY(S.side->ensure());
     I2_TRY(S.d_sing_rec.ensure(A.singular_tasks));
     A.sing_rec = S.d_sing_rec.p;
     I2_TRY(S.d_sing_deep.ensure(A.singular_tasks));
@@ -1187,6 +1195,7 @@ int i2_evaluator_loss_and_grad(i2_evaluator* ev, uint64_t seed, double* loss, do
             set_error("event creation failed");
             return I2_ERR_HIP;
         }
+        ev->adj->side = &ev->side;
     }
     const int8_t* conv[3];
     int K[3];

@@ -114,6 +114,7 @@ struct AdjState {
     DBuf<unsigned long long> d_counters;
     DBuf<SingRec> d_sing_rec;
     DBuf<int64_t> d_sing_deep;
+    SideStream* side = nullptr;   // the singular pairs' kernels beside the disjoint pairs' (of the batch or evaluator)
     hipEvent_t e0 = nullptr, e1 = nullptr;
 };
 

@@ -93,6 +93,7 @@ struct Engine {
     int out = OUT_PER_PAIR;
     int pairs_per_wg = 64;
     int ppl = 13;                 // quadrature points per lane (13 = whole rule per lane)
+    SideStream* side = nullptr;   // the singular pairs' kernels beside the disjoint pairs' (of the batch or evaluator)
     int sweep_grid = 0, deep_grid = 0, fin_grid = 0, levels_grid = 0;
     BatchArgs args{};
     std::vector<MeshDesc> h_meshes;

@@ -77,6 +77,41 @@ inline int check_launch(const char* what) {
     return I2_OK;
 }
 
+// A second stream beside a caller's, for kernels that do not depend on each
+// other.  Forks and joins are events, so that a graph captured from the caller's
+// stream gets two branches.
+struct SideStream {
+    hipStream_t stream = nullptr;
+    hipEvent_t forked = nullptr, joined = nullptr;
+    SideStream() = default;
+    SideStream(const SideStream&) = delete;
+    SideStream& operator=(const SideStream&) = delete;
+    ~SideStream() { reset(); }
+    int ensure() {
+        if (!stream) I2_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        if (!forked) I2_HIP(hipEventCreateWithFlags(&forked, hipEventDisableTiming));
+        if (!joined) I2_HIP(hipEventCreateWithFlags(&joined, hipEventDisableTiming));
+        return I2_OK;
+    }
+    int fork(hipStream_t from) {
+        I2_HIP(hipEventRecord(forked, from));
+        I2_HIP(hipStreamWaitEvent(stream, forked, 0));
+        return I2_OK;
+    }
+    int join(hipStream_t to) {
+        I2_HIP(hipEventRecord(joined, stream));
+        I2_HIP(hipStreamWaitEvent(to, joined, 0));
+        return I2_OK;
+    }
+    void reset() {
+        if (stream) (void)hipStreamDestroy(stream);
+        if (forked) (void)hipEventDestroy(forked);
+        if (joined) (void)hipEventDestroy(joined);
+        stream = nullptr;
+        forked = joined = nullptr;
+    }
+};
+
 // ------------------------------------------------------------ mesh
 }  // namespace i2
 
@@ -231,6 +266,7 @@ struct i2_evaluator {
     i2::DBuf<unsigned long long> d_counter;
     unsigned long long* h_counter = nullptr;   // pinned, one per type
     std::vector<hipEvent_t> marks;              // of the plain path's timing
+    i2::SideStream side;           // of the batched path and the adjoint
     i2::AdjState* adj = nullptr;   // adjoint buffers (created by the first loss-and-gradient call)
 };
 
