@@ -1025,7 +1025,7 @@ static int adjoint_tile(int nT) {
 // loss (one block of 3 nV + 1 doubles per mesh), and the vertex gather's
 // lists from each mesh's cells and vertex- and edge-sharing pair lists.
 int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::vector<const i2_mesh*>& meshes,
-                  const i2_integrator* it, uint64_t seed) {
+                  const i2_integrator* it, uint64_t seed, const int* K) {
     int cus = 0;
     I2_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     S.grid = std::max(1, cus) * 4;
@@ -1078,14 +1078,17 @@ int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::ve
         D[m].inc = x.d_inc.p;
     }
     // all tables in one upload
-    const int64_t words = (int64_t)(sizeof(AdjMesh) * M + 7) / 8;
+    const int64_t words = (int64_t)(sizeof(AdjMesh) * M + 7) / 8, kwords = K ? (3 * M + 1) / 2 : 0;
     std::vector<int64_t> table;
-    table.reserve(5 * M + 4 + words);
     for (const auto* v : {&pbase, &vbase, &item_base, &sing_base}) table.insert(table.end(), v->begin(), v->end());
     const int64_t at = (int64_t)table.size();
-    table.resize(at + words);
-    memcpy(table.data() + at, D.data(), sizeof(AdjMesh) * M);
+    table.resize(at + words + kwords);
     I2_TRY(S.d_base.ensure((int64_t)table.size()));
+    if (K) {
+        memcpy(table.data() + at + words, K, sizeof(int) * 3 * M);
+        for (int m = 0; m < M; ++m) D[m].K = reinterpret_cast<const int*>(S.d_base.p + at + words) + 3 * m;
+    }
+    memcpy(table.data() + at, D.data(), sizeof(AdjMesh) * M);
     I2_HIP(hipMemcpy(S.d_base.p, table.data(), sizeof(int64_t) * table.size(), hipMemcpyHostToDevice));
     I2_TRY(S.d_psum.ensure(9 * pbase[M]));
     A.psum = S.d_psum.p;
@@ -1150,8 +1153,11 @@ AdjMesh adjoint_mesh(const i2_mesh* mesh, const int8_t* const conv[3], const int
 int adjoint_copy_out(const AdjState& S, int mesh, double* loss, double* dLdX) {
     const double* base = S.d_grad.p + S.grad_off[mesh];
     const int64_t nV = S.nV[mesh];
-    if (dLdX) I2_HIP(hipMemcpy(dLdX, base, sizeof(double) * 3 * nV, hipMemcpyDeviceToHost));
-    if (loss) I2_HIP(hipMemcpy(loss, base + 3 * nV, sizeof(double), hipMemcpyDeviceToHost));
+    // dL/dX and L stand one after the other: one copy
+    std::vector<double> h((size_t)(3 * nV + 1));
+    I2_HIP(hipMemcpy(h.data(), base, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
+    if (dLdX) memcpy(dLdX, h.data(), sizeof(double) * 3 * (size_t)nV);
+    if (loss) *loss = h[(size_t)(3 * nV)];
     return I2_OK;
 }
 
@@ -1210,9 +1216,7 @@ int i2_evaluator_loss_and_grad(i2_evaluator* ev, uint64_t seed, double* loss, do
         }
     }
     AdjState& S = *ev->adj;
-    I2_TRY(S.d_K.ensure(3));
-    I2_HIP(hipMemcpy(S.d_K.p, K, 3 * sizeof(int), hipMemcpyHostToDevice));
-    I2_TRY(adjoint_setup(S, ev->mesh->device, {adjoint_mesh(ev->mesh, conv, S.d_K.p)}, {ev->mesh}, ev->integ, seed));
+    I2_TRY(adjoint_setup(S, ev->mesh->device, {adjoint_mesh(ev->mesh, conv, nullptr)}, {ev->mesh}, ev->integ, seed, K));
     return adjoint_run(S, ev->stream, loss, dLdX);
 }
 

@@ -102,7 +102,6 @@ struct AdjState {
     std::vector<int64_t> grad_off; // per mesh: dL/dX (3 nV) then L, in d_grad
     double ms = 0.0;              // device time of the last adjoint run
     int64_t kj_total = 0;         // doubles of K_j slots, all meshes
-    DBuf<int> d_K;
     DBuf<double> d_grad;          // dL/dX (3 nV) and L
     DBuf<double> d_ki, d_kj;      // partial panel cotangents (all meshes)
     DBuf<double> d_item_loss, d_sing_dl, d_psum, d_loss_part;
@@ -121,7 +120,7 @@ struct AdjState {
 void adjoint_release(AdjState*& S);
 AdjMesh adjoint_mesh(const i2_mesh* mesh, const int8_t* const conv[3], const int* dK);
 int adjoint_setup(AdjState& S, int device, std::vector<AdjMesh> D, const std::vector<const i2_mesh*>& meshes,
-                  const i2_integrator* it, uint64_t seed);
+                  const i2_integrator* it, uint64_t seed, const int* K = nullptr);
 // Enqueues the adjoint kernels (capturable: no host synchronisation, fills by kernels).
 int adjoint_launch(AdjState& S, hipStream_t st);
 int adjoint_copy_out(const AdjState& S, int mesh, double* loss, double* dLdX);

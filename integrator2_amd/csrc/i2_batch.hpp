@@ -97,11 +97,10 @@ struct Engine {
     int sweep_grid = 0, deep_grid = 0, fin_grid = 0, levels_grid = 0;
     BatchArgs args{};
     std::vector<MeshDesc> h_meshes;
-    std::vector<int64_t> h_item_base, h_sing_base, h_pair_base, h_row_base, h_qoff;
+    std::vector<int64_t> h_item_base, h_sing_base, h_pair_base, h_row_base, h_qoff, h_tables;
     std::vector<int64_t> nT;
     int64_t ordered[3] = {0, 0, 0};   // ordered tasks per type over the batch
-    DBuf<MeshDesc> d_meshes;
-    DBuf<int64_t> d_item_base, d_sing_base, d_pair_base, d_row_base, d_qoff;
+    DBuf<int64_t> d_tables;       // the tables of BatchArgs, then the mesh descriptors
     DBuf<unsigned long long> d_counters;
     DBuf<QEntry> d_queue;
     DBuf<unsigned long long> d_levelmask;
