@@ -42,17 +42,21 @@ __device__ __forceinline__ int64_t uniform64(int64_t x) {
     return ((int64_t)hi << 32) | (uint32_t)lo;
 }
 
-// position of the disjoint pair (i, j), i < j, in the lexicographic list
-__device__ __forceinline__ int64_t disjoint_rank(const MeshDesc& M, int i, int j) {
-    int64_t below = 0;
-    for (int64_t q = M.nbr_start[i]; q < M.nbr_start[i + 1]; ++q) {
-        if (M.nbr[q] < j) ++below; else break;
-    }
-    return M.row_start[i] + (j - i - 1) - below;
-}
-// task index of ordered disjoint pair (i, j) in [(i<j) list] ++ [reversed]
+// Task index of the ordered disjoint pair (i, j), i uniform over the workgroup,
+// in [(i<j) list] ++ [reversed]: the pair's place in the row of its smaller
+// panel, whose neighbours are no disjoint pairs.  Row i is the same for all
+// lanes; with the general loop over 64-bit positions a pair took 130
+// instructions for it.
 __device__ __forceinline__ int64_t disjoint_task(const MeshDesc& M, int i, int j) {
-    return (i < j) ? disjoint_rank(M, i, j) : M.npairs[I2_NOT_NEIGHBORS] + disjoint_rank(M, j, i);
+    int below = 0;
+    if (i < j) {
+        for (int64_t q = M.nbr_start[i]; q < M.nbr_start[i + 1]; ++q) below += M.nbr[q] < j;
+        return M.row_start[i] + (j - i - 1) - below;
+    }
+    const int64_t first = M.nbr_start[j];
+    const int32_t* nbr = M.nbr + first;
+    for (int n = (int)(M.nbr_start[j + 1] - first); below < n && nbr[below] < i; ++below) {}
+    return M.npairs[I2_NOT_NEIGHBORS] + M.row_start[j] + (i - j - 1) - below;
 }
 
 __device__ __forceinline__ int find_base(const int64_t* base, int n, int64_t x) {
@@ -487,7 +491,9 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
                 const bool in_range = p < P && j < M.nT;
                 const Panel J = M.panels[in_range ? j : i];
                 const bool valid = in_range && j != i && shared_count(I, J) == 0;
-                const int64_t z = valid ? disjoint_task(M, i, j) : 0;
+                // row sums alone need no place for the pair's own outputs
+                const bool numbered = OUT == OUT_PER_PAIR || M.conv[I2_NOT_NEIGHBORS] != nullptr;
+                const int64_t z = valid && numbered ? disjoint_task(M, i, j) : 0;
                 const int tile64 = __builtin_amdgcn_readfirstlane((tile * P + p) >> 6);
                 const StepOut o = sweep_task<LPP>(A, R, M, m, i, j, z, valid, s, I, J, pts, ball, F,
                                                   tables && 64 * tile64 < M.nT ? tables + (threadIdx.x >> 6) * TILE_POINTS * TILE_VERTS : nullptr,
