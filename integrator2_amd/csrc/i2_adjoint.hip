@@ -440,16 +440,33 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
     d3 X0 = {0.0, 0.0, 0.0}, X1 = X0;
     const uint32_t total = (uint32_t)npts << (2 * level);
     const uint32_t magic = (uint32_t)((0x100000000ull + npts - 1) / npts);   // q / npts for q <= 2^28
-    for (uint32_t q = s; q < total; q += G) {
-        const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
-        const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
-        const d3 p = beta.x * I.a + beta.y * I.b + beta.z * I.c;
-        const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
-        axpy(X0, beta.x, pb); axpy(X1, beta.y, pb);
+    // the pair's own form, whatever pairs share its wavefront (the list's order
+    // changes from run to run)
+    if (panel_far(panel_ball(I.a, I.b, I.c, A.rule.reach), JG) != 0) {
+        const FarFrame Fr = far_frame(I.a, I.b, I.c);
+        const FarGeom FG = far_geom(Fr, JG);
+        FarBar f = far_bar_zero();
+        for (uint32_t q = s; q < total; q += G) {
+            const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+            const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
+            theta_terms_far_rev<false>(far_point(beta.x - 1.0 / 3.0, beta.y - 1.0 / 3.0, R.w[k]), Fr, FG, JG, ct, f);
+        }
+        double* v = reinterpret_cast<double*>(&f);
+#pragma unroll
+        for (int k = 0; k < (int)(sizeof(FarBar) / sizeof(double)); ++k) v[k] = group_sum<G>(v[k]);
+        far_bar_expand(f, Fr, JG, g, X0, X1);
+    } else {
+        for (uint32_t q = s; q < total; q += G) {
+            const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+            const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
+            const d3 p = beta.x * I.a + beta.y * I.b + beta.z * I.c;
+            const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
+            axpy(X0, beta.x, pb); axpy(X1, beta.y, pb);
+        }
+        group_sum3<G>(g.a); group_sum3<G>(g.b); group_sum3<G>(g.c); group_sum3<G>(g.n); group_sum3<G>(X0); group_sum3<G>(X1);
+        g.T = {group_sum<G>(g.T.x), group_sum<G>(g.T.y), group_sum<G>(g.T.z), group_sum<G>(g.T.w)};
+        g.y = group_sum<G>(g.y); g.La = group_sum<G>(g.La); g.Lb = group_sum<G>(g.Lb); g.Lc = group_sum<G>(g.Lc);
     }
-    group_sum3<G>(g.a); group_sum3<G>(g.b); group_sum3<G>(g.c); group_sum3<G>(g.n); group_sum3<G>(X0); group_sum3<G>(X1);
-    g.T = {group_sum<G>(g.T.x), group_sum<G>(g.T.y), group_sum<G>(g.T.z), group_sum<G>(g.T.w)};
-    g.y = group_sum<G>(g.y); g.La = group_sum<G>(g.La); g.Lb = group_sum<G>(g.Lb); g.Lc = group_sum<G>(g.Lc);
     const q4 F = psi_of_terms(g.T, JG);
     const q4 Iv = fa * F;
     const d3 psi = {Iv.x, Iv.y, Iv.z};

@@ -816,4 +816,25 @@ I2_HD __forceinline__ d3 at_bary(const BaryPoint& Q, d3 a, d3 b, d3 c) {
     return p + Q.b2 * c;
 }
 
+// A disjoint pair's far terms (without far_scale) summed with the weights over
+// points k0, k0 + step, ... of the sub-panels sub, sub + G, ... of `level`, in
+// barycentric coordinates of K_i less 1/3.  R: the rule's arrays, n points.
+template <bool DISTANT, class R>
+__device__ __forceinline__ q4 quad_far(const R& rule, int n, int level, int sub, int G, int k0, int step, const FarFrame& F,
+                                       const FarGeom& J) {
+    q4 acc = q4zero();
+    const double h = 1.0 / 3.0;
+    for (uint32_t c = sub; c < (1u << (2 * level)); c += G) {
+        d3 a = {1.0 - h, -h, 0.0}, b = {-h, 1.0 - h, 0.0}, o = {-h, -h, 0.0};
+        sub_panel(a, b, o, level, c);
+        for (int k = k0; k < n; k += step) {
+            const double l1 = rule.L1[k], l2 = rule.L2[k], l3 = rule.L3[k], w = rule.w[k];
+            const FarPoint Q = far_point(l1 * a.x + l2 * b.x + l3 * o.x, l1 * a.y + l2 * b.y + l3 * o.y, w);
+            const q4 t = theta_terms_far<DISTANT>(Q.b0, Q.b1, far_pp(F, Q), J);
+            acc = {fma(w, t.x, acc.x), fma(w, t.y, acc.y), fma(w, t.z, acc.z), fma(w, t.w, acc.w)};
+        }
+    }
+    return acc;
+}
+
 }  // namespace i2d

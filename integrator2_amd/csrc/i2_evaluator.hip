@@ -71,26 +71,6 @@ __device__ __forceinline__ q4 quad_sub(const Rule& R, const i2m::MathTable* lt, 
     return area * acc;
 }
 
-// The same sum of a disjoint pair's far terms over the sub-panels sub, sub + G,
-// ... of `level`, in barycentric coordinates of K_i less 1/3.
-template <bool DISTANT>
-__device__ __forceinline__ q4 quad_far(const Rule& R, int level, int sub, int G, int k0, int step, const FarFrame& F,
-                                       const FarGeom& J) {
-    q4 acc = q4zero();
-    const double h = 1.0 / 3.0;
-    for (uint32_t c = sub; c < (1u << (2 * level)); c += G) {
-        d3 a = {1.0 - h, -h, 0.0}, b = {-h, 1.0 - h, 0.0}, o = {-h, -h, 0.0};
-        sub_panel(a, b, o, level, c);
-        for (int k = k0; k < R.n; k += step) {
-            const double l1 = R.L1[k], l2 = R.L2[k], l3 = R.L3[k], w = R.w[k];
-            const FarPoint Q = far_point(l1 * a.x + l2 * b.x + l3 * o.x, l1 * a.y + l2 * b.y + l3 * o.y, w);
-            const q4 t = theta_terms_far<DISTANT>(Q.b0, Q.b1, far_pp(F, Q), J);
-            acc = {fma(w, t.x, acc.x), fma(w, t.y, acc.y), fma(w, t.z, acc.z), fma(w, t.w, acc.w)};
-        }
-    }
-    return acc;
-}
-
 __device__ __forceinline__ q4 lanes_sum(q4 v, int lanes) {
     for (int m = 1; m < lanes; m <<= 1) {
         v.x += __shfl_xor(v.x, m);
@@ -135,8 +115,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_
         if (form != 0) {
             const FarFrame F = far_frame(I.a, I.b, I.c);
             const FarGeom FG = far_geom(F, JG);
-            acc = area * far_scale(form == 1 ? quad_far<false>(R, level, sub, G, k0, step, F, FG)
-                                               : quad_far<true>(R, level, sub, G, k0, step, F, FG), JG);
+            acc = area * far_scale(form == 1 ? quad_far<false>(R, R.n, level, sub, G, k0, step, F, FG)
+                                               : quad_far<true>(R, R.n, level, sub, G, k0, step, F, FG), JG);
         } else {
             for (uint32_t c = sub; c < nsub; c += G) {
                 d3 a = I.a, b = I.b, cc = I.c;
@@ -194,11 +174,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_
             const FarFrame F = far_frame(I.a, I.b, I.c);
             const FarGeom FG = far_geom(F, JG);
             if (form == 1) {
-                v0 = quad_far<false>(R, 0, 0, 1, s, lanes, F, FG);
-                v1 = quad_far<false>(R, 1, sub, subs, k0, per, F, FG);
+                v0 = quad_far<false>(R, R.n, 0, 0, 1, s, lanes, F, FG);
+                v1 = quad_far<false>(R, R.n, 1, sub, subs, k0, per, F, FG);
             } else {
-                v0 = quad_far<true>(R, 0, 0, 1, s, lanes, F, FG);
-                v1 = quad_far<true>(R, 1, sub, subs, k0, per, F, FG);
+                v0 = quad_far<true>(R, R.n, 0, 0, 1, s, lanes, F, FG);
+                v1 = quad_far<true>(R, R.n, 1, sub, subs, k0, per, F, FG);
             }
             v0 = area * far_scale(v0, JG);
             v1 = (0.25 * area) * far_scale(v1, JG);
