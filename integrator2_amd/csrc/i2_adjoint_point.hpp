@@ -1,7 +1,7 @@
 // i2_adjoint_point.hpp -- reverse mode of the per-point functions of the
-// quadrature loops, derived by hand: the inner integral thetaPsi (the
-// division-free form theta_psi_fast of i2_device.hpp) and the two singular
-// parts (evaluatorJ3DK.cu:315-350, 352-407).
+// quadrature loops, derived by hand: the inner integral thetaPsi
+// (theta_terms_rev and theta_terms_far_rev in the kernels; theta_psi_fast_rev,
+// with the tangents as parameters, for the host) and the two singular parts (evaluatorJ3DK.cu:315-350, 352-407).
 //
 // Each function recomputes the forward intermediates of one point, returns the
 // forward value f, and adds gb . df/dx to the cotangents of the point p and of
@@ -50,7 +50,7 @@ struct TPBar { d3 a, b, c, ta, tb, tc; };
 
 I2_HD __forceinline__ q4 theta_psi_fast_rev(d3 p, const JGeom& J, const i2m::MathTable* __restrict__ lt, q4 gb, d3* pbar,
                                             TPBar& g) {
-    // ---- forward, as theta_psi_fast
+    // ---- forward, from the l + d.tau of the reference formula
     const d3 da = p - J.a, db = p - J.b, dc = p - J.c;
     const double qa = dot(da, da), qb = dot(db, db), qc = dot(dc, dc);
     const double la = i2m::sqrt_pos(qa), lb = i2m::sqrt_pos(qb), lc = i2m::sqrt_pos(qc);
@@ -69,7 +69,7 @@ I2_HD __forceinline__ q4 theta_psi_fast_rev(d3 p, const JGeom& J, const i2m::Mat
     const double pab = dot(da, db), pbc = dot(db, dc), pca = dot(dc, da);
     const double y = dot(cross(da, db), dc);
     const double x = la * lb * lc + pab * lc + pbc * la + pca * lb;
-    // branch-free table paths, the rare lanes outside their ranges redone (theta_psi_fast)
+    // branch-free table paths, the rare lanes outside their ranges redone
     const bool o1 = i2m::pos_normal(a1), o2 = i2m::pos_normal(a2), o3 = i2m::pos_normal(a3);
     const bool o4 = i2m::atan2_in_range(y, x);
     double t1 = i2m::log_tab_any(a1, lt);

@@ -19,7 +19,7 @@
 // transcendental chains) needs the second wavefront to hide it.
 #define I2_TWO_WAVES __attribute__((amdgpu_waves_per_eu(2)))
 // The disjoint sweep fits three (168 registers, a few spills outside its
-// quadrature loop), which measured 7 % faster than two and than four.
+// quadrature loop): two measured the same time, four 15 % more (spills in it).
 #define I2_THREE_WAVES __attribute__((amdgpu_waves_per_eu(3)))
 
 #include "i2_math.hpp"
@@ -395,7 +395,7 @@ I2_HD __forceinline__ q4 sing_edge_fast(d3 p, const EdgeCtx& c, const i2m::MathT
     const double a1 = N * i2m::rcp_pos(D), a2 = P2 * c.ilvc, a3 = P3 * c.ilvc;
     const double y1 = dot(cross(va, c.taub), c.tauc), x1 = dot(c.taub - c.tauc, lva * c.taub + va);
     const double y2 = dot(cross(vb, c.taua), c.tauc), x2 = dot(c.taua - c.tauc, lvb * c.taua - vb);
-    // branch-free table paths, the rare lanes outside their ranges redone (theta_psi_fast)
+    // branch-free table paths, the rare lanes outside their ranges redone
     const bool o1 = i2m::pos_normal(a1), o2 = i2m::pos_normal(a2), o3 = i2m::pos_normal(a3);
     const bool o4 = i2m::atan2_in_range(y1, x1), o5 = i2m::atan2_in_range(y2, x2);
     double l1 = i2m::log_tab_any(a1, lt);
@@ -483,7 +483,7 @@ I2_HD __forceinline__ q4 sing_vertex_fast(d3 p, const VertexCtx& c, const i2m::M
     const d3 le = l * c.e;
     const double y1 = dot(cross(d, c.taua), c.e), x1 = dot(le - d, c.e - c.taua);
     const double y2 = dot(cross(d, c.taub), c.e), x2 = dot(le - d, c.e + c.taub);
-    // branch-free table paths, the rare lanes outside their ranges redone (theta_psi_fast)
+    // branch-free table paths, the rare lanes outside their ranges redone
     const bool o1 = i2m::pos_normal(a1), o2 = i2m::pos_normal(a2);
     const bool o3 = i2m::atan2_in_range(y1, x1), o4 = i2m::atan2_in_range(y2, x2);
     double la = i2m::log_tab_any(a1, lt);
