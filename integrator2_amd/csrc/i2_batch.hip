@@ -577,10 +577,14 @@ __global__ __launch_bounds__(256) I2_TWO_WAVES void k_sweep_singular(BatchArgs A
 }
 
 // Refinement level >= 2 of one queued task.
-// G lanes, Q of them per sub-panel.
-template <int TYPE, int OUT>
-__device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, int level, int G, int Q, int s, const QEntry& e,
-                                          bool valid) {
+// G lanes, Q of them per sub-panel.  LEAN: the panels and the previous value are
+// read again after the points instead of held across them (the index's empty
+// statement keeps the compiler from joining the reads), which leaves 14-20
+// registers to spill at three wavefronts per SIMD instead of 37-47.
+template <int TYPE, int OUT, bool LEAN>
+__device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, int level, int G, int Q, int s,
+                                          const QEntry* entry, bool valid) {
+    const QEntry e = *entry;
     const MeshDesc& M = A.meshes[e.m];
     const Panel I = M.panels[e.i];
     const Panel J = M.panels[e.j];
@@ -612,9 +616,13 @@ __device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, 
         }
     }
     acc = shfl_sum(acc, G);
-    if (TYPE == I2_NOT_NEIGHBORS) acc = psi_of_terms(acc, JG);
+    int again = 0;
+    if (LEAN) asm volatile("" : "+v"(again));
+    const Panel I1 = LEAN ? M.panels[e.i + again] : I, J1 = LEAN ? M.panels[e.j + again] : J;
+    if (TYPE == I2_NOT_NEIGHBORS) acc = psi_of_terms(acc, LEAN ? jgeom(J1) : JG);
     if (!valid || s != 0) return;
-    const q4 prev = {e.prev.x, e.prev.y, e.prev.z, e.prev.w};
+    const double4 pv = LEAN ? entry[again].prev : e.prev;
+    const q4 prev = {pv.x, pv.y, pv.z, pv.w};
     StepOut o{false, false, level, acc, acc};
     if (A.fixed) {
         o.finished = true;   // fixed mode queues tasks straight at the fixed level
@@ -625,7 +633,7 @@ __device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, 
     }
     if (o.finished) {
         q4 rp0, rp1;
-        finish_task<TYPE, OUT>(A, M, e.z, e.i, e.j, o, I, J, &rp0, &rp1);
+        finish_task<TYPE, OUT>(A, M, e.z, e.i, e.j, o, I1, J1, &rp0, &rp1);
         if (OUT == OUT_ROW_SUMS) add_row(M, TYPE, e.i, rp0, rp1);
     }
 }
@@ -635,9 +643,10 @@ __device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, 
 // 16 lanes per task, one sub-panel each, or a wavefront with four lanes per
 // sub-panel where 16 lanes each would leave SIMDs empty (4 rounds of points
 // instead of 13 in series, at 81 % of the lanes).  A workgroup without a task
-// ends before it loads the tables.
-template <int OUT, int T0, int T1>
-__global__ __launch_bounds__(256) I2_TWO_WAVES void k_deep(BatchArgs A, int level) {
+// ends before it loads the tables.  WAVES per SIMD: many disjoint tasks run with
+// three (DEEP_THREE_WAVES), the others with two and nothing spilled.
+template <int OUT, int T0, int T1, int WAVES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_deep(BatchArgs A, int level) {
     __shared__ RuleLDS R;
     bool loaded = false;
     for (int type = T0; type <= T1; ++type) {
@@ -658,10 +667,10 @@ __global__ __launch_bounds__(256) I2_TWO_WAVES void k_deep(BatchArgs A, int leve
              base += (unsigned long long)gridDim.x * per_block) {
             const unsigned long long t = base + slot;
             const bool valid = t < cnt;
-            QEntry e = q[valid ? t : base];
-            if (type == I2_NOT_NEIGHBORS) deep_task<I2_NOT_NEIGHBORS, OUT>(A, R, level, G, Q, s, e, valid);
-            else if (type == I2_SIMPLE_NEIGHBORS) deep_task<I2_SIMPLE_NEIGHBORS, OUT>(A, R, level, G, Q, s, e, valid);
-            else deep_task<I2_ATTACHED_NEIGHBORS, OUT>(A, R, level, G, Q, s, e, valid);
+            const QEntry* e = q + (valid ? t : base);
+            if (type == I2_NOT_NEIGHBORS) deep_task<I2_NOT_NEIGHBORS, OUT, WAVES == 3>(A, R, level, G, Q, s, e, valid);
+            else if (type == I2_SIMPLE_NEIGHBORS) deep_task<I2_SIMPLE_NEIGHBORS, OUT, WAVES == 3>(A, R, level, G, Q, s, e, valid);
+            else deep_task<I2_ATTACHED_NEIGHBORS, OUT, WAVES == 3>(A, R, level, G, Q, s, e, valid);
         }
     }
 }
@@ -927,6 +936,14 @@ static int compute_grids(Engine& E) {
     return I2_OK;
 }
 
+// Ordered disjoint pairs of a run from which k_deep takes three wavefronts per
+// SIMD.  Row sums, refinement to level 3 at 1e-8: 1,280 panels (1.6e6 pairs)
+// 1.052 ms with two, 1.004 with three, a 5,120-panel ellipsoid's outputs 7.81 and
+// 7.74; 320 panels (1e5 pairs), where each SIMD has a wavefront at most, 0.304 and
+// 0.315.  12 workgroups per CU with three: fixed level 2 on 5,120 panels 37.3 ms
+// with two, 37.1 so, 39.2 with 8 per CU, whose last round is a third full.
+constexpr int64_t DEEP_THREE_WAVES = 1 << 20;
+
 int batch_enqueue(Engine& E, hipStream_t st) {
     const BatchArgs& A = E.args;
     const unsigned row_blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>((A.total_rows + 255) / 256, E.fin_grid));
@@ -938,10 +955,15 @@ int batch_enqueue(Engine& E, hipStream_t st) {
     // first, so that its persistent workgroups start together: rows of 5,120
     // panels 6.26 ms in one stream, 6.30 with the singular kernels first, 5.87.
     // A profiled run, which times the disjoint sweep, keeps them apart.
+    const bool many = E.ordered[I2_NOT_NEIGHBORS] >= DEEP_THREE_WAVES;
     auto deep = [&](int L, bool singular, hipStream_t on) -> int {
-#define I2_DEEP(O, T0, T1) hipLaunchKernelGGL((k_deep<O, T0, T1>), dim3(E.deep_grid), dim3(256), 0, on, A, L)
-        if (E.out == OUT_PER_PAIR) { if (singular) I2_DEEP(OUT_PER_PAIR, 0, 1); else I2_DEEP(OUT_PER_PAIR, 2, 2); }
-        else { if (singular) I2_DEEP(OUT_ROW_SUMS, 0, 1); else I2_DEEP(OUT_ROW_SUMS, 2, 2); }
+        const dim3 grid(singular || !many ? E.deep_grid : E.deep_grid / 2 * 3);   // whole rounds of resident workgroups
+#define I2_DEEP(O, T0, T1, W) hipLaunchKernelGGL((k_deep<O, T0, T1, W>), grid, dim3(256), 0, on, A, L)
+        if (E.out == OUT_PER_PAIR) {
+            if (singular) I2_DEEP(OUT_PER_PAIR, 0, 1, 2); else if (many) I2_DEEP(OUT_PER_PAIR, 2, 2, 3); else I2_DEEP(OUT_PER_PAIR, 2, 2, 2);
+        } else {
+            if (singular) I2_DEEP(OUT_ROW_SUMS, 0, 1, 2); else if (many) I2_DEEP(OUT_ROW_SUMS, 2, 2, 3); else I2_DEEP(OUT_ROW_SUMS, 2, 2, 2);
+        }
 #undef I2_DEEP
         return check_launch("k_deep");
     };
