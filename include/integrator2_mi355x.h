@@ -72,6 +72,10 @@ int i2_device_math(int device, int fn, const double* x, const double* y, int64_t
  * the neighbour type).  For checking. */
 int i2_host_task_value(const double* I9, const double* J9, const int32_t* vid6, int level, const double* L12,
                        const double* w, int nPts, double* out4);
+/* Host-side evaluation of the adjoint kernels' numbering of a refined panel's
+ * points: point q of a rule of nPts on the sub-panels, in order, is the rule's
+ * point `point` on sub-panel `sub` (0 <= q <= 2^28).  For checking. */
+int i2_host_point_split(int nPts, const int64_t* q, int64_t n, int64_t* sub, int64_t* point);
 
 /* ======================================================================
  * Mesh3D (src/Mesh3d.cuh:55-126, src/Mesh3d.cu)

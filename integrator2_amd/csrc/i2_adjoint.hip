@@ -439,7 +439,7 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
     TermsBar g = terms_bar_zero();
     d3 X0 = {0.0, 0.0, 0.0}, X1 = X0;
     const uint32_t total = (uint32_t)npts << (2 * level);
-    const uint32_t magic = (uint32_t)((0x100000000ull + npts - 1) / npts);   // q / npts for q <= 2^28
+    const uint32_t factor = split_factor(npts);
     // the pair's own form, whatever pairs share its wavefront (the list's order
     // changes from run to run)
     if (panel_far(panel_ball(I.a, I.b, I.c, A.rule.reach), JG) != 0) {
@@ -447,7 +447,7 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
         const FarGeom FG = far_geom(Fr, JG);
         FarBar f = far_bar_zero();
         for (uint32_t q = s; q < total; q += G) {
-            const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+            const uint32_t sub = split_point(q, factor), k = q - sub * npts;
             const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
             theta_terms_far_rev<false>(far_point(beta.x - 1.0 / 3.0, beta.y - 1.0 / 3.0, R.w[k]), Fr, FG, JG, ct, f);
         }
@@ -457,7 +457,7 @@ __device__ __forceinline__ void deep_pair(const AdjArgs& A, const RuleSh& R, con
         far_bar_expand(f, Fr, JG, g, X0, X1);
     } else {
         for (uint32_t q = s; q < total; q += G) {
-            const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+            const uint32_t sub = split_point(q, factor), k = q - sub * npts;
             const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
             const d3 p = beta.x * I.a + beta.y * I.b + beta.z * I.c;
             const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
@@ -647,7 +647,7 @@ __device__ __forceinline__ void singular_task(const AdjArgs& A, const RuleSh& R,
     const Panel I = M.panels[i];
     const int npts = A.rule.n;
     const uint32_t total = (uint32_t)npts << (2 * level);
-    const uint32_t magic = (uint32_t)((0x100000000ull + npts - 1) / npts);   // q / npts for q <= 2^28
+    const uint32_t factor = split_factor(npts);
     double fa = I.area;
     for (int l = 0; l < level; ++l) fa *= 0.25;
     // one of the pair's four draws per lane of a quad
@@ -664,7 +664,7 @@ __device__ __forceinline__ void singular_task(const AdjArgs& A, const RuleSh& R,
         const q4 ct = {fa * dot(gP, J.tc), fa * dot(gP, J.ta), fa * dot(gP, J.tb), 2.0 * fa * gb.w};
         TermsBar g = terms_bar_zero();
         for (uint32_t q = s; q < total; q += G) {
-            const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+            const uint32_t sub = split_point(q, factor), k = q - sub * npts;
             const d3 beta = sub_point(d3{R.L1[k], R.L2[k], R.L3[k]}, level, sub);
             const d3 p = beta.x * I.a + beta.y * I.b + beta.z * I.c;
             const d3 pb = theta_terms_rev(p, JG, &R.lt, R.w[k], ct, g);
@@ -699,7 +699,7 @@ __device__ __forceinline__ void singular_task(const AdjArgs& A, const RuleSh& R,
     q4 Fs = q4zero();
     d3 Y0 = z3, Y1 = z3;
     for (uint32_t q = s; q < total; q += G) {
-        const uint32_t sub = __umulhi(q, magic), k = q - sub * npts;
+        const uint32_t sub = split_point(q, factor), k = q - sub * npts;
         // these derivatives amplify the point's rounding: it comes from the
         // sub-panel's vertices, as in the quadrature
         d3 a = I.a, b = I.b, c = I.c;

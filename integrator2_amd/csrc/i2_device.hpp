@@ -787,6 +787,15 @@ I2_HD __forceinline__ d3 sub_point(d3 b, int level, uint32_t path) {
     return b;
 }
 
+// Point q of the n 4^level points of a rule on a panel's sub-panels, in order:
+// the rule's point q - n s of sub-panel s = q / n.  The quotient by one
+// multiplication with ceil(2^32 / n), exact for n <= 16 and q <= 2^28 (level
+// 12).  For n = 1 that factor does not fit 32 bits; 0 stands for it, and s = q.
+I2_HD __forceinline__ uint32_t split_factor(uint32_t n) { return n > 1 ? (uint32_t)((0x100000000ull + n - 1) / n) : 0u; }
+I2_HD __forceinline__ uint32_t split_point(uint32_t q, uint32_t factor) {
+    return factor != 0u ? (uint32_t)(((uint64_t)q * factor) >> 32) : q;
+}
+
 // A rule's point on a sub-panel, barycentric on the original panel, with its
 // weight: 32-byte records that the kernels keep in LDS for levels 0 and 1
 // (the rule's points on the panel, then on its four level-1 children).

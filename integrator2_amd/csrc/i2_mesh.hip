@@ -459,6 +459,17 @@ int i2_host_task_value(const double* I9, const double* J9, const int32_t* vid6, 
     return I2_OK;
 }
 
+int i2_host_point_split(int nPts, const int64_t* q, int64_t n, int64_t* sub, int64_t* point) {
+    if (!q || !sub || !point || n < 0 || nPts < 1 || nPts > i2d::MAX_POINTS) { set_error("invalid argument"); return I2_ERR_INVALID; }
+    const uint32_t factor = i2d::split_factor(nPts);
+    for (int64_t k = 0; k < n; ++k) {
+        if (q[k] < 0 || q[k] > (int64_t)1 << 28) { set_error("point number %lld out of range", (long long)q[k]); return I2_ERR_RANGE; }
+        sub[k] = i2d::split_point((uint32_t)q[k], factor);
+        point[k] = q[k] - sub[k] * nPts;
+    }
+    return I2_OK;
+}
+
 int i2_device_count(int* n) {
     if (!n) { set_error("null pointer"); return I2_ERR_INVALID; }
     int c = 0;
