@@ -315,17 +315,10 @@ class EvaluatorJ3DK:
     def results(self, t, errors=False):
         """Dict with tasks (n,3), integrals (n,4), results (n,3), conv (n,), errors (n,) if requested."""
         n = self.taskCount(t)
-        # one allocation for all arrays: from 4 MB on numpy asks for huge pages,
-        # and the first touch of small ones costs more than the copy
-        sizes = dict(integrals=(np.float64, 4), results=(np.float64, 3), errors=(np.float64, errors), tasks=(np.int32, 3),
-                     conv=(np.int8, 1))
-        store, out, at = np.empty(n * sum(np.dtype(d).itemsize * c for d, c in sizes.values()), np.uint8), {}, 0
-        for k, (d, c) in sizes.items():
-            size = n * c * np.dtype(d).itemsize
-            out[k] = store[at:at + size].view(d).reshape((n, c) if c > 1 else n) if c else None
-            at += size
-        out = {k: out[k] for k in ("tasks", "integrals", "results", "conv", "errors")}
-        err = out.pop("errors")
+        # not zeroed: the call writes every element
+        out = dict(tasks=np.empty((n, 3), np.int32), integrals=np.empty((n, 4)), results=np.empty((n, 3)),
+                   conv=np.empty(n, np.int8))
+        err = np.empty(n) if errors else None
         _check(lib().i2_evaluator_get_results(self._h, ctypes.c_int(t), _ptr(out["tasks"]), _ptr(out["integrals"]),
                                               _ptr(out["results"]), _ptr(err), _ptr(out["conv"])))
         if errors:
