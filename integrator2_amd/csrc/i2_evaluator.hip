@@ -682,7 +682,10 @@ static int read_back(hipStream_t st, const PackArgs& P, int64_t n, double* ints,
         hipEvent_t e[2] = {nullptr, nullptr};
         ~Events() { for (hipEvent_t x : e) if (x) (void)hipEventDestroy(x); }
     } E;
-    if (chunks > 1) for (hipEvent_t& e : E.e) I2_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    // The slots are not coherent memory (Portable alone leaves that to
+    // HIP_HOST_COHERENT): the host sees a chunk after a release to the system, which
+    // a stream's synchronisation is and an event's record is only with the flag.
+    if (chunks > 1) for (hipEvent_t& e : E.e) I2_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem));
     auto launch = [&](int64_t c) -> int {
         const int64_t z0 = c * most, m = std::min(most, n - z0);
         hipLaunchKernelGGL(k_pack, dim3((unsigned)std::min<int64_t>((m + 255) / 256, 256)), dim3(256), 0, st, P, z0, m,
