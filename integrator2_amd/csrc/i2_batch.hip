@@ -536,9 +536,9 @@ __device__ __forceinline__ void singular_sweep_task(const BatchArgs& A, const Ru
         const BaryPoint Q = pts[k];
         const d3 p = at_bary(Q, I.a, I.b, I.c);
         const q4 f = theta_psi_fast(p, JG, &R.lt) - sg.at(p, &R.lt);
-        const double w0 = k < npts ? Q.w : 0.0, w1 = k < npts ? 0.0 : Q.w;
-        v0 = v0 + w0 * f;
-        v1 = v1 + w1 * f;
+        // not both with a weight of 0, which would carry one level's NaN into the other
+        if (k < npts) v0 = v0 + Q.w * f;
+        else v1 = v1 + Q.w * f;
     }
     v0 = I.area * shfl_sum(v0, G);
     v1 = (0.25 * I.area) * shfl_sum(v1, G);
