@@ -199,11 +199,18 @@ struct FarTerms {
 // against 192 corners.  Four points at a time, lane v writes the distance of
 // vertex v (and v + 64) to the wavefront's table in LDS, and each panel reads
 // its three: 65 FP64 instructions per evaluation instead of 83, and three LDS
-// reads.  One wavefront's LDS operations complete in order, so that no barrier
-// is needed between the writes and the reads.  Rows of 5,120 panels 6.75 -> 6.28
+// reads.  One wavefront's LDS operations complete in order, so that the writes
+// and the reads need no barrier, only wave_exchange.  Rows of 5,120 panels 6.75 -> 6.28
 // ms, at 84 % of the issue slots instead of 94; the chip's clock follows the
 // load (1.82 and 1.89 GHz), and two or three wavefronts per SIMD give the same.
 constexpr int TILE_POINTS = 4;
+// Orders a wavefront's LDS accesses before and after it, for the compiler as
+// well: the fences are of one wavefront's scope and emit no instruction.
+__device__ __forceinline__ void wave_exchange() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 template <bool DISTANT>
 struct SharedTerms {
     const PtsLDS& P;
@@ -228,7 +235,7 @@ struct SharedTerms {
                 table[p * TILE_VERTS + 64 + lane] = vertex_distance(v1, Q.b0, Q.b1, Q.pp);
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_exchange();
         const double *a = table + (corners & 255u), *b = table + ((corners >> 8) & 255u), *c = table + (corners >> 16);
 #pragma unroll
         for (int p = 0; p < N; ++p) {
@@ -236,7 +243,7 @@ struct SharedTerms {
             const q4 t = theta_terms_of<DISTANT>(a[p * TILE_VERTS], b[p * TILE_VERTS], c[p * TILE_VERTS], Q.b0, Q.b1, G);
             acc = {fma(Q.w, t.x, acc.x), fma(Q.w, t.y, acc.y), fma(Q.w, t.z, acc.z), fma(Q.w, t.w, acc.w)};
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_exchange();
         return acc;
     }
     __device__ __forceinline__ q4 sum(int k0, int k1, int, q4 acc) const {
