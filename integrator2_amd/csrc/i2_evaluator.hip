@@ -268,9 +268,11 @@ __device__ __forceinline__ void finalize_one(int64_t z, const TaskSource& src, c
 }
 
 // All types in one launch, a range of workgroups each, the closed forms first:
-// one after another their 17 and 12 us on few tasks are latency.
+// one after another their 17 and 12 us on few tasks are latency.  `clock`, in the
+// host's memory, receives when each type's first workgroup began and its last
+// one ended, by which the launch's time is divided among the types.
 struct FinalizeType { int64_t n; unsigned blocks; TaskSource src; double4* ints; double* results; };
-struct FinalizeArgs { FinalizeType t[3]; bool implicit; };
+struct FinalizeArgs { FinalizeType t[3]; bool implicit; long long* clock; };
 __global__ __launch_bounds__(256) void k_finalize(FinalizeArgs A, const Panel* __restrict__ panels) {
     unsigned b = blockIdx.x;
     int t = 0;
@@ -278,10 +280,15 @@ __global__ __launch_bounds__(256) void k_finalize(FinalizeArgs A, const Panel* _
     const FinalizeType& T = A.t[t];
     const int64_t z = (int64_t)b * blockDim.x + threadIdx.x;
     if (z >= T.n) return;
+    if (A.clock && b == 0 && threadIdx.x == 0) A.clock[2 * t] = wall_clock64();
     if (t == I2_SIMPLE_NEIGHBORS) finalize_one<I2_SIMPLE_NEIGHBORS, false>(z, T.src, panels, T.ints, T.results);
     else if (t == I2_ATTACHED_NEIGHBORS) finalize_one<I2_ATTACHED_NEIGHBORS, false>(z, T.src, panels, T.ints, T.results);
     else if (A.implicit) finalize_one<I2_NOT_NEIGHBORS, true>(z, T.src, panels, T.ints, T.results);
     else finalize_one<I2_NOT_NEIGHBORS, false>(z, T.src, panels, T.ints, T.results);
+    if (A.clock && b + 1 == T.blocks && threadIdx.x == 0) {
+        __threadfence();               // after the outputs
+        A.clock[2 * t + 1] = wall_clock64();
+    }
 }
 
 // (i,j)/(j,i) symmetry error (evaluator3d.cu:45-57)
@@ -391,9 +398,11 @@ __global__ void k_begin_run(unsigned long long* counters, int nc, uint8_t* f0, u
 
 // Device time of the launches between marks on the evaluator's stream, by type
 struct RunMarks {
+    static constexpr int NONE = -1, ALL = 3;
     i2_evaluator* ev;
     size_t used = 0;
-    std::vector<int> type;           // of the stretch that ends at the mark, -1: none
+    std::vector<int> type;           // of the stretch that ends at the mark; ALL: k_finalize's, by its clock
+    long long* clock() const { return reinterpret_cast<long long*>(ev->h_counter + 3); }
     int mark(int t) {
         if (used == ev->marks.size()) {
             hipEvent_t e;
@@ -405,12 +414,18 @@ struct RunMarks {
         return I2_OK;
     }
     int times() {
-        for (int t = 0; t < 3; ++t) ev->type[t].ms = 0.0;
+        double share[3], sum = 0.0;
+        for (int t = 0; t < 3; ++t) {
+            ev->type[t].ms = 0.0;
+            share[t] = ev->type[t].n > 0 ? (double)std::max(clock()[2 * t + 1] - clock()[2 * t], 1ll) : 0.0;
+            sum += share[t];
+        }
         for (size_t q = 1; q < used; ++q) {
-            if (type[q] < 0) continue;
+            if (type[q] == NONE) continue;
             float ms = 0.f;
             I2_HIP(hipEventElapsedTime(&ms, ev->marks[q - 1], ev->marks[q]));
-            ev->type[type[q]].ms += ms;
+            if (type[q] != ALL) ev->type[type[q]].ms += ms;
+            else for (int t = 0; t < 3; ++t) if (share[t] > 0.0) ev->type[t].ms += ms * share[t] / sum;
         }
         return I2_OK;
     }
@@ -440,7 +455,7 @@ static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
         I2_TRY(ts.rest[1].ensure(n));
         I2_TRY(ts.unconv.ensure(nT));
     }
-    I2_TRY(marks.mark(-1));
+    I2_TRY(marks.mark(RunMarks::NONE));
     if (it.fixed) {
         for (int t = 0; t < 3; ++t) {
             TypeState& ts = ev->type[t];
@@ -465,7 +480,7 @@ static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
         // levels 0 and 1 in one launch per type, but for profiled runs, which list each level's
         const bool first = it.max_level > 0 && !ev->profile;
         for (int iter = first ? 1 : 0; iter <= it.max_level && (remaining[0] > 0 || remaining[1] > 0 || remaining[2] > 0); ++iter) {
-            if (iter > 1) I2_TRY(marks.mark(-1));
+            if (iter > 1) I2_TRY(marks.mark(RunMarks::NONE));
             for (int t = 0; t < 3; ++t) {
                 TypeState& ts = ev->type[t];
                 const int64_t n = remaining[t];
@@ -506,17 +521,17 @@ static int run_types(i2_evaluator* ev, const TaskSource (&src)[3]) {
                 I2_TRY(mark_unconverged(ev, ts.implicit, src[t], remaining[t], it.max_level == 0 ? nullptr : ts.rest[cur_rest[t]].p, ts.unconv.p));
         }
     }
-    I2_TRY(marks.mark(-1));
+    I2_TRY(marks.mark(RunMarks::NONE));
     FinalizeArgs F{};
     F.implicit = ev->type[I2_NOT_NEIGHBORS].implicit;
-    int last = 0;
+    F.clock = marks.clock();
     for (int t = 0; t < 3; ++t) {
         TypeState& ts = ev->type[t];
         F.t[t] = {ts.n, 0, src[t], ts.buf[ts.final_buf].p, ts.results.p};
-        if (ts.n > 0) last = t;
+        F.clock[2 * t] = F.clock[2 * t + 1] = 0;
     }
     I2_TRY(launch_finalize(ev->stream, ev->mesh->d_panels.p, F));
-    I2_TRY(marks.mark(last));     // of all types, counted with the last
+    I2_TRY(marks.mark(RunMarks::ALL));
     I2_HIP(hipStreamSynchronize(ev->stream));
     return marks.times();
 }
@@ -922,7 +937,7 @@ int i2_evaluator_create(i2_evaluator** out, const i2_mesh* m, i2_integrator* it)
     ev->mesh = m;
     ev->integ = it;
     if (hipStreamCreateWithFlags(&ev->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc((void**)&ev->h_counter, 3 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&ev->h_counter, 9 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         set_error("failed to create evaluator stream/events");
         i2_evaluator_destroy(ev);

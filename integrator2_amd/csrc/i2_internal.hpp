@@ -264,7 +264,7 @@ struct i2_evaluator {
     uint64_t all_pairs_generation = 0;
     i2::TypeState type[3];
     i2::DBuf<unsigned long long> d_counter;
-    unsigned long long* h_counter = nullptr;   // pinned, one per type
+    unsigned long long* h_counter = nullptr;   // pinned, one per type, then k_finalize's six clocks
     std::vector<hipEvent_t> marks;              // of the plain path's timing
     i2::SideStream side;           // of the batched path and the adjoint
     i2::AdjState* adj = nullptr;   // adjoint buffers (created by the first loss-and-gradient call)
