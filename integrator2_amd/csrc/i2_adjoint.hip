@@ -131,8 +131,6 @@ __device__ __forceinline__ double wsum(double x) {
     for (int m = 1; m < 64; m <<= 1) x += __shfl_xor(x, m);
     return x;
 }
-__device__ __forceinline__ void wsum3(d3& v) { v.x = wsum(v.x); v.y = wsum(v.y); v.z = wsum(v.z); }
-__device__ __forceinline__ void wsum4(q4& v) { v.x = wsum(v.x); v.y = wsum(v.y); v.z = wsum(v.z); v.w = wsum(v.w); }
 __device__ __forceinline__ void store3(double* dst, d3 v) { dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; }
 __device__ __forceinline__ void add_to3(double* dst, d3 v) { dst[0] += v.x; dst[1] += v.y; dst[2] += v.z; }
 __device__ __forceinline__ double dot4(q4 a, q4 b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }

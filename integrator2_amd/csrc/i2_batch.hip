@@ -13,13 +13,15 @@
 // each task's last two level values in the finalize kernel.
 //
 // Kernels (one graph):
-//   k_sweep    levels 0 and 1 of every task.  Disjoint pairs are enumerated
-//              implicitly: a workgroup item is one control panel i and P
-//              consecutive panels j (i is uniform, its panel record is read
-//              with scalar loads); lane groups of LPP lanes share a pair and
-//              split its quadrature points.  Vertex- and edge-sharing tasks
-//              come from the mesh's lists, P per item.  Items are claimed from
-//              an atomic counter by persistent workgroups.
+//   k_sweep_disjoint  levels 0 and 1 of the disjoint pairs, enumerated implicitly:
+//              an item is one control panel i and P consecutive panels j (i is
+//              uniform, its panel record is read with scalar loads); lane
+//              groups of LPP lanes share a pair and split its quadrature
+//              points.  Persistent workgroups take runs of consecutive items,
+//              the first by their number and the next from an atomic counter.
+//   k_singular_closed, k_sweep_singular  closed forms, then levels 0 and 1, of the
+//              vertex- and edge-sharing tasks from the meshes' lists, on a
+//              second stream beside the disjoint pairs' kernels.
 //   k_deep     refinement level L >= 2 of the tasks queued by level L-1: 16 or
 //              64 lanes per task, fixed-order reduction.
 //   k_levels / k_compute_K   K per (mesh, type) from queue membership.
@@ -1035,10 +1037,9 @@ int engine_setup(Engine& E, const i2_integrator& it) {
     if (A.last_level >= MAX_LEVELS) { set_error("refinement level above %d", MAX_LEVELS - 1); return I2_ERR_RANGE; }
     I2_TRY(compute_grids(E));
     const int P = E.pairs_per_wg;
-    // sweep items (disjoint per mesh; singular per (type, mesh), 256 tasks each) and per-pair ranges
+    // sweep items (disjoint per mesh; singular per (type, mesh), 256 tasks each)
     E.h_item_base.assign(M + 1, 0);
     E.h_sing_base.assign(2 * M + 1, 0);
-    E.h_pair_base.assign(3 * M + 1, 0);
     E.nT.resize(M);
     int64_t acc = 0;
     for (int m = 0; m < M; ++m) {
@@ -1066,12 +1067,10 @@ int engine_setup(Engine& E, const i2_integrator& it) {
     for (int m = 0; m < M; ++m) {
         E.nT[m] = E.h_meshes[m].nT;
         for (int t = 0; t < 3; ++t) {
-            E.h_pair_base[3 * m + t] = pb;
             pb += 2 * E.h_meshes[m].npairs[t];
             E.ordered[t] += 2 * E.h_meshes[m].npairs[t];
         }
     }
-    E.h_pair_base[3 * M] = pb;
     E.total_tasks = pb;
     E.h_row_base.assign(M + 1, 0);
     for (int m = 0; m < M; ++m) E.h_row_base[m + 1] = E.h_row_base[m] + E.h_meshes[m].nT;
@@ -1100,8 +1099,7 @@ int engine_setup(Engine& E, const i2_integrator& it) {
         E.h_tables.insert(E.h_tables.end(), v.begin(), v.end());
         return at;
     };
-    const size_t qoff = table(E.h_qoff), items = table(E.h_item_base), sing = table(E.h_sing_base), pairs = table(E.h_pair_base),
-                 rows = table(E.h_row_base), meshes = E.h_tables.size();
+    const size_t qoff = table(E.h_qoff), items = table(E.h_item_base), sing = table(E.h_sing_base), rows = table(E.h_row_base), meshes = E.h_tables.size();
     static_assert(sizeof(MeshDesc) % sizeof(int64_t) == 0, "descriptors behind the tables");
     E.h_tables.resize(meshes + M * sizeof(MeshDesc) / sizeof(int64_t));
     memcpy(E.h_tables.data() + meshes, E.h_meshes.data(), M * sizeof(MeshDesc));
@@ -1111,7 +1109,6 @@ int engine_setup(Engine& E, const i2_integrator& it) {
     A.meshes = reinterpret_cast<const MeshDesc*>(d + meshes);
     A.item_base = d + items;
     A.sing_base = d + sing;
-    A.pair_base = d + pairs;
     A.row_base = d + rows;
     A.qoff = d + qoff;
     A.counters = E.d_counters.p;

@@ -72,9 +72,7 @@ struct BatchArgs {
     int64_t disjoint_items;
     int64_t sweep_chunk;          // consecutive disjoint items per claim
     int64_t singular_items;
-    // per-pair finalize ranges: pair_base[3 * m + type]; disjoint rows of all
-    // meshes: row_base[m] (nmeshes + 1)
-    const int64_t* pair_base;
+    // disjoint rows of all meshes: row_base[m] (nmeshes + 1)
     const int64_t* row_base;
     int64_t total_rows;
     // counters: [0] disjoint chunk counter, [1 + level*3 + type] queue counts
@@ -97,7 +95,7 @@ struct Engine {
     int sweep_grid = 0, deep_grid = 0, fin_grid = 0, levels_grid = 0;
     BatchArgs args{};
     std::vector<MeshDesc> h_meshes;
-    std::vector<int64_t> h_item_base, h_sing_base, h_pair_base, h_row_base, h_qoff, h_tables;
+    std::vector<int64_t> h_item_base, h_sing_base, h_row_base, h_qoff, h_tables;
     std::vector<int64_t> nT;
     int64_t ordered[3] = {0, 0, 0};   // ordered tasks per type over the batch
     DBuf<int64_t> d_tables;       // the tables of BatchArgs, then the mesh descriptors
