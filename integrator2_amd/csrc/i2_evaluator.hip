@@ -110,14 +110,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TYPE == I2_
         double area = I.area;
         for (int l = 0; l < level; ++l) area *= 0.25;
         const uint32_t nsub = 1u << (2 * level);
-        // Disjoint pairs at levels 0 and 1: one loop per wavefront, in the form that
-        // holds for all its pairs, which stand side by side in the task list.  Refined
-        // pairs: each in its own form, because a rest list's order changes from run
-        // to run (a wavefront holds four of them at level 2 above 8,192 tasks).
+        // Disjoint pairs: one loop per wavefront, in the form that holds for all its
+        // pairs.  Those of a rest list each in its own form, because the list's
+        // order changes from run to run (a wavefront holds four of them at level 2
+        // above 8,192 tasks); a task list's pairs stand as the caller put them, and
+        // four forms in turn cost 19 % there (1,280 panels at fixed level 2).
         int form = 0;
         if (TYPE == I2_NOT_NEIGHBORS) {
             const Ball ball = panel_ball(I.a, I.b, I.c, R.reach);
-            form = level >= 2 ? panel_far(ball, JG) : wave_form(true, ball, JG);
+            form = list ? panel_far(ball, JG) : wave_form(true, ball, JG);
         }
         if (form != 0) {
             const FarFrame F = far_frame(I.a, I.b, I.c);
