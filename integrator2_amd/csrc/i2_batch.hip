@@ -651,7 +651,10 @@ __device__ __forceinline__ void deep_task(const BatchArgs& A, const RuleLDS& R, 
 // wavefront per task from level 3 (a sub-panel per lane at level 3), at level 2
 // 16 lanes per task, one sub-panel each, or a wavefront with four lanes per
 // sub-panel where 16 lanes each would leave SIMDs empty (4 rounds of points
-// instead of 13 in series, at 81 % of the lanes).  A workgroup without a task
+// instead of 13 in series, at 81 % of the lanes) and the rule has more than four
+// points: with fewer there is no series to shorten, and a wavefront's tasks enter
+// the next queue with one atomic, 26 ns each on its counter (320 panels' 3,780
+// singular tasks with one point, all refined: 43 us with 16 lanes, 100 with 64).  A workgroup without a task
 // ends before it loads the tables.  WAVES per SIMD: many disjoint tasks run with
 // three (DEEP_THREE_WAVES), the others with two and nothing spilled.
 template <int OUT, int T0, int T1, int WAVES>
@@ -661,7 +664,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
     for (int type = T0; type <= T1; ++type) {
         const int qi = level * 3 + type;
         const unsigned long long cnt = min(A.counters[1 + qi], (unsigned long long)A.qcap[type]);
-        const bool wide = level >= 3 || cnt <= 8192;
+        const bool wide = level >= 3 || (cnt <= 8192 && A.rule.n > 4);
         const int G = wide ? 64 : 16, Q = level == 2 && wide ? 4 : 1;
         const int per_block = blockDim.x / G;
         if ((unsigned long long)blockIdx.x * per_block >= cnt) continue;   // uniform
