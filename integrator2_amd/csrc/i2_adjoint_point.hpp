@@ -252,7 +252,7 @@ I2_HD __forceinline__ void theta_terms_far_rev(const FarPoint& Q, const FarFrame
 // The vector sums: g as theta_terms_rev leaves it, and added to X0 and X1 the
 // points' cotangents times their first two barycentric coordinates.
 I2_HD __forceinline__ void far_bar_expand(const FarBar& f, const FarFrame& F, const JGeom& J, TermsBar& g, d3& X0, d3& X1) {
-    const d3 a = F.m - J.a, b = F.m - J.b, c = F.m - J.c;
+    const d3 a = from_vertex(F, J.a), b = from_vertex(F, J.b), c = from_vertex(F, J.c);
     g.a = f.a * a; axpy(g.a, f.a0, F.U); axpy(g.a, f.a1, F.V);
     g.b = f.b * b; axpy(g.b, f.b0, F.U); axpy(g.b, f.b1, F.V);
     g.c = f.c * c; axpy(g.c, f.c0, F.U); axpy(g.c, f.c1, F.V);

@@ -147,7 +147,18 @@ __device__ __forceinline__ q4 quad_part(const RuleLDS& R, int npts, int s, int s
 // point is a 32-byte record, two 128-bit LDS reads: |b0 U + b1 V|^2, (b0, b1)
 // and the rule weight.
 struct alignas(32) QPoint { double pp, b0, b1, w; };
-struct PtsLDS { QPoint f[5 * MAX_POINTS]; };
+// The panel's frame stands beside them: read where it is used (the index's empty
+// statement keeps the reads there) it is not held in registers across the loops,
+// which left 27 of them to spill, four so.  Rows of 5,120 panels 6.15 -> 6.09 ms.
+struct PtsLDS {
+    QPoint f[5 * MAX_POINTS];
+    FarFrame F;
+    __device__ __forceinline__ FarFrame frame() const {
+        int again = 0;
+        asm volatile("" : "+v"(again));
+        return (&F)[again];
+    }
+};
 
 // Levels 0 and 1 in one pass with a rule whose point 0 is the centroid: the
 // centroid of K_i is also the centroid of its central level-1 child (child 4),
@@ -157,12 +168,14 @@ __device__ __forceinline__ bool share_centroid(const BatchArgs& A) {
     return A.rule.centroid == 0 && !A.fixed && A.last_level >= 1;
 }
 
-__device__ __forceinline__ void load_points(PtsLDS& P, const RuleLDS& R, int npts, const FarFrame& F) {
+__device__ __forceinline__ void load_points(PtsLDS& P, const Rule& R, const FarFrame& F) {
+    const int npts = R.n;
     for (int t = threadIdx.x; t < 5 * npts; t += blockDim.x) {
         const BaryPoint Q = bary_point(R.L1, R.L2, R.L3, R.w, npts, t);
         const FarPoint x = far_point(Q.b0 - 1.0 / 3.0, Q.b1 - 1.0 / 3.0, Q.w);
         P.f[t] = {far_pp(F, x), x.b0, x.b1, x.w};
     }
+    if (threadIdx.x == 0) P.F = F;
 }
 
 // The ways a wavefront evaluates the terms (forms of wave_form).  General: at
@@ -171,14 +184,14 @@ __device__ __forceinline__ void load_points(PtsLDS& P, const RuleLDS& R, int npt
 // instead of once per panel corner.  sum() adds w times the terms of points k =
 // k0, k0 + step, ... < k1 to acc, in that order.
 struct GeneralTerms {
-    const RuleLDS& R;
+    const i2m::MathTable& lt;
     const PtsLDS& P;
-    const FarFrame& F;
     const JGeom& J;
     __device__ __forceinline__ q4 sum(int k0, int k1, int step, q4 acc) const {
         for (int k = k0; k < k1; k += step) {
             const QPoint Q = P.f[k];
-            const q4 t = theta_terms(F.m + Q.b0 * F.U + Q.b1 * F.V, J, &R.lt);
+            const FarFrame F = P.frame();
+            const q4 t = theta_terms(F.o + (F.g + Q.b0 * F.U + Q.b1 * F.V), J, &lt);
             acc = {fma(Q.w, t.x, acc.x), fma(Q.w, t.y, acc.y), fma(Q.w, t.z, acc.z), fma(Q.w, t.w, acc.w)};
         }
         return acc;
@@ -394,10 +407,11 @@ __device__ __forceinline__ void flush_row(const MeshDesc& M, int type, int i, q4
 // take part.
 template <bool DISTANT>
 __device__ __forceinline__ void shared_sums(const BatchArgs& A, const PtsLDS& pts, const MeshDesc& M, int tile, uint32_t corners,
-                                            double* table, const FarFrame& F, const JGeom& JG, bool need0, bool need1, q4& T0,
+                                            double* table, const JGeom& JG, bool need0, bool need1, q4& T0,
                                             q4& T1) {
     const int32_t* list = M.tile_list + (int64_t)tile * TILE_LIST;
     const int lane = threadIdx.x & 63, n = list[0];
+    const FarFrame F = pts.frame();
     auto vertex = [&](int k) {
         const double* x = M.xyz + 3 * (int64_t)list[1 + (k < n ? k : 0)];
         return vertex_poly(F, d3{x[0], x[1], x[2]});
@@ -413,9 +427,9 @@ __device__ __forceinline__ void shared_sums(const BatchArgs& A, const PtsLDS& pt
 // check.  table: of the wavefront, whose pairs are with tile `tile` of the mesh
 // (null: their panels are not one tile).
 template <int LPP>
-__device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS& R, const MeshDesc& M, int m, int i, int j, int64_t z,
+__device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const i2m::MathTable& lt, const MeshDesc& M, int m, int i, int j, int64_t z,
                                               bool valid, int s, const Panel& I, const Panel& J, const PtsLDS& pts, const Ball& ball,
-                                              const FarFrame& F, double* table, int tile) {
+                                              double* table, int tile) {
     const JGeom JG = jgeom(J);
     const int npts = A.rule.n;
     const bool need0 = !A.fixed || A.last_level == 0;
@@ -426,13 +440,13 @@ __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS&
     q4 T0 = q4zero(), T1 = q4zero();
     if (LPP == 1 && form != 0 && table && M.tile_list[(int64_t)tile * TILE_LIST] > 0) {
         const uint32_t corners = M.corners[min(j, M.nT - 1)];
-        if (form == 1) shared_sums<false>(A, pts, M, tile, corners, table, F, JG, need0, need1, T0, T1);
-        else shared_sums<true>(A, pts, M, tile, corners, table, F, JG, need0, need1, T0, T1);
+        if (form == 1) shared_sums<false>(A, pts, M, tile, corners, table, JG, need0, need1, T0, T1);
+        else shared_sums<true>(A, pts, M, tile, corners, table, JG, need0, need1, T0, T1);
     } else if (valid) {
         if (form == 0) {
-            sweep_terms<LPP>(GeneralTerms{R, pts, F, JG}, npts, share_centroid(A), need0, need1, s, T0, T1);
+            sweep_terms<LPP>(GeneralTerms{lt, pts, JG}, npts, share_centroid(A), need0, need1, s, T0, T1);
         } else {
-            const FarGeom G = far_geom(F, JG);
+            const FarGeom G = far_geom(pts.frame(), JG);
             if (form == 1) sweep_terms<LPP>(FarTerms<false>{pts, G}, npts, share_centroid(A), need0, need1, s, T0, T1);
             else sweep_terms<LPP>(FarTerms<true>{pts, G}, npts, share_centroid(A), need0, need1, s, T0, T1);
             T0 = far_scale(T0, JG);
@@ -460,12 +474,11 @@ __device__ __forceinline__ StepOut sweep_task(const BatchArgs& A, const RuleLDS&
 // one to the next.
 template <int OUT, int LPP>
 __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs A) {
-    __shared__ struct { PtsLDS pts; RuleLDS R; } S;
-    RuleLDS& R = S.R;
+    __shared__ struct { PtsLDS pts; i2m::MathTable lt; } S;
     PtsLDS& pts = S.pts;
     __shared__ long long chunk_sh;
     extern __shared__ double wave_tables[];   // one table per wavefront, where each has a tile (tile_table_bytes)
-    load_rule(R, A.rule);
+    i2m::fill_mathtab(S.lt);
     const int P = A.pairs_per_item;
     double* const tables = LPP == 1 && P % 64 == 0 ? wave_tables : nullptr;
     const int per_round = blockDim.x / LPP;
@@ -489,11 +502,10 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
                 i = row;
                 i_mesh = m;
                 __syncthreads();
-                load_points(pts, R, A.rule.n, far_frame(I.a, I.b, I.c));
+                load_points(pts, A.rule, far_frame(I.a, I.b, I.c));
                 __syncthreads();
             }
             const Ball ball = panel_ball(I.a, I.b, I.c, A.rule.reach);
-            const FarFrame F = far_frame(I.a, I.b, I.c);
             for (int round = 0; round < P; round += per_round) {
                 const int p = round + p0;
                 const int j = tile * P + p;
@@ -504,7 +516,7 @@ __global__ __launch_bounds__(256) I2_THREE_WAVES void k_sweep_disjoint(BatchArgs
                 const bool numbered = OUT == OUT_PER_PAIR || M.conv[I2_NOT_NEIGHBORS] != nullptr;
                 const int64_t z = valid && numbered ? disjoint_task(M, i, j) : 0;
                 const int tile64 = __builtin_amdgcn_readfirstlane((tile * P + p) >> 6);
-                const StepOut o = sweep_task<LPP>(A, R, M, m, i, j, z, valid, s, I, J, pts, ball, F,
+                const StepOut o = sweep_task<LPP>(A, S.lt, M, m, i, j, z, valid, s, I, J, pts, ball,
                                                   tables && 64 * tile64 < M.nT ? tables + (threadIdx.x >> 6) * TILE_POINTS * TILE_VERTS : nullptr,
                                                   tile64);
                 q4 rp0 = q4zero(), rp1 = q4zero();

@@ -238,7 +238,10 @@ I2_HD __forceinline__ q4 theta_terms(d3 p, const JGeom& J, const i2m::MathTable*
 //
 // The point is p = m + b0 U + b1 V, with m the centroid of K_i, U = A_i - C_i,
 // V = B_i - C_i and (b0, b1) its first two barycentric coordinates less 1/3
-// (FarFrame, FarPoint).  A squared distance to a vertex is then |m - a|^2 +
+// (FarFrame, FarPoint).  m itself, rounded, would shift all of the panel's points
+// by some 2^-53 |m| together: with m = C_i + (U + V)/3 kept in two parts, m - a is
+// (C_i - a) + (U + V)/3 and only differences of coordinates enter (pairs of a
+// mesh 500 radii from the origin: median error 2.2e-14 instead of 8.3e-14).  A squared distance to a vertex is then |m - a|^2 +
 // 2 b0 U.(m - a) + 2 b1 V.(m - a) + |b0 U + b1 V|^2: three instructions with
 // the last term, common to all vertices, in `pp`; and da.N2 is affine in (b0,
 // b1).  It loses no more than the plain difference because K_i's points lie
@@ -250,11 +253,13 @@ I2_HD __forceinline__ q4 theta_terms(d3 p, const JGeom& J, const i2m::MathTable*
 // evaluated it before that (six dot products, table logs and atan2) 212.  Rows
 // of 5,120 panels, where 81 % of the wavefronts are distant and 6 % general:
 // 7.31 -> 6.77 ms.
-struct FarFrame { d3 m, U, V; double uu, uv, vv; };
+struct FarFrame { d3 o, g, U, V; double uu, uv, vv; };   // m = o + g
 I2_HD __forceinline__ FarFrame far_frame(d3 a, d3 b, d3 c) {
     const d3 U = a - c, V = b - c;
-    return {(1.0 / 3.0) * (a + b + c), U, V, dot(U, U), 2.0 * dot(U, V), dot(V, V)};
+    return {c, (1.0 / 3.0) * (U + V), U, V, dot(U, U), 2.0 * dot(U, V), dot(V, V)};
 }
+// m - x
+I2_HD __forceinline__ d3 from_vertex(const FarFrame& F, d3 x) { return (F.o - x) + F.g; }
 // A quadrature point in that frame, with the products the kernels need of it
 struct alignas(16) FarPoint { double b0, b1, b00, b01, b11, w; };
 I2_HD __forceinline__ FarPoint far_point(double b0, double b1, double w) { return {b0, b1, b0 * b0, b0 * b1, b1 * b1, w}; }
@@ -263,7 +268,7 @@ I2_HD __forceinline__ double far_pp(const FarFrame& F, const FarPoint& Q) { retu
 // and the squared edge lengths
 struct FarGeom { double ka, ua, va, kb, ub, vb, kc, uc, vc, ky, uy, vy, q1, q2, q3; };
 I2_HD __forceinline__ FarGeom far_geom(const FarFrame& F, const JGeom& J) {
-    const d3 a = F.m - J.a, b = F.m - J.b, c = F.m - J.c, N = 2.0 * J.N2;
+    const d3 a = from_vertex(F, J.a), b = from_vertex(F, J.b), c = from_vertex(F, J.c), N = 2.0 * J.N2;
     return {dot(a, a), 2.0 * dot(F.U, a), 2.0 * dot(F.V, a), dot(b, b), 2.0 * dot(F.U, b), 2.0 * dot(F.V, b),
             dot(c, c), 2.0 * dot(F.U, c), 2.0 * dot(F.V, c), dot(a, N), dot(F.U, N), dot(F.V, N),
             J.Lc * J.Lc, J.La * J.La, J.Lb * J.Lb};
@@ -284,7 +289,7 @@ I2_HD __forceinline__ q4 theta_terms_of(double la, double lb, double lc, double 
 // one vertex's distance polynomial
 struct VertexPoly { double k, u, v; };
 I2_HD __forceinline__ VertexPoly vertex_poly(const FarFrame& F, d3 x) {
-    const d3 a = F.m - x;
+    const d3 a = from_vertex(F, x);
     return {dot(a, a), 2.0 * dot(F.U, a), 2.0 * dot(F.V, a)};
 }
 I2_HD __forceinline__ double vertex_distance(const VertexPoly& x, double b0, double b1, double pp) {
