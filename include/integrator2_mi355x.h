@@ -50,8 +50,9 @@ int i2_device_count(int* n);
 /* Host-side evaluation of the inner integral (Psi, Theta) of triangle tri9 at
  * n points, with the device formulas compiled for the CPU: fast = 0 is the
  * reference's expression (thetaPsi, src/evaluators/evaluatorJ3DK.cu:266-313),
- * fast = 1 the form the kernels use at any point, fast = 2 the form they use
- * for points at least twice K_j's longest edge away from it.  For checking. */
+ * fast = 1 the form the kernels use at any point, fast = 2 and 3 the forms they
+ * use for points at least two and six of K_j's longest edges away from it.  For
+ * checking. */
 int i2_host_theta_psi(int fast, const double* pts, int64_t n, const double* tri9, double* out4);
 /* Host-side evaluation of the kernels' FP64 logarithm (fn = 0, of x),
  * two-argument arctangent (fn = 1, atan2(y, x)), square root (fn = 2, of x;
@@ -68,7 +69,7 @@ int i2_host_math(int fn, const double* x, const double* y, int64_t n, double* ou
 int i2_device_math(int device, int fn, const double* x, const double* y, int64_t n, double* out);
 /* Host-side evaluation of one ordered task's integrals (Psi, Theta) at
  * refinement level `level` with the kernels' device code compiled for the
- * host: I9, J9 the two panels' vertices, vid6 their vertex ids (which decide
+ * host (the inner integral in its general form): I9, J9 the two panels' vertices, vid6 their vertex ids (which decide
  * the neighbour type).  For checking. */
 int i2_host_task_value(const double* I9, const double* J9, const int32_t* vid6, int level, const double* L12,
                        const double* w, int nPts, double* out4);
@@ -257,9 +258,10 @@ int i2_host_loss_weights(uint64_t seed, const int32_t* ij, int64_t n, int nT, do
 /* Host-side reverse mode of one per-point function, for checking: kind 0
  * thetaPsi (params: A, B, C, tau_a, tau_b, tau_c; 18), 1 edge-sharing singular
  * part (JB, JC, tau_a, tau_b, tau_c, 1/|JC-JB|; 16), 2 vertex-sharing singular
- * part (JA, tau_a, tau_b, e, 1/sqrt(S_i); 13), 3 and 4 the terms of thetaPsi
- * (line integrals of 1/r along AB, BC, CA and Theta/2) in the general and in
- * the far form (A, B, C; 9).  Returns f(p) and gbar4 . df
+ * part (JA, tau_a, tau_b, e, 1/sqrt(S_i); 13), 3, 4 and 5 the terms of thetaPsi
+ * (line integrals of 1/r along AB, BC, CA and Theta/2) in the general form and
+ * in the far ones from two and six longest edges (A, B, C; 9).  The kernels run
+ * kinds 1 to 5; kind 0 is the formula with free tangents.  Returns f(p) and gbar4 . df
  * with respect to p (pbar3) and to every parameter (parbar). */
 int i2_host_point_adjoint(int kind, const double* p3, const double* params, const double* gbar4, double* f4,
                           double* pbar3, double* parbar);

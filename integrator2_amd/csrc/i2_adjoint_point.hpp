@@ -1,7 +1,7 @@
 // i2_adjoint_point.hpp -- reverse mode of the per-point functions of the
 // quadrature loops, derived by hand: the inner integral thetaPsi
 // (theta_terms_rev and theta_terms_far_rev in the kernels; theta_psi_fast_rev,
-// with the tangents as parameters, for the host) and the two singular parts (evaluatorJ3DK.cu:315-350, 352-407).
+// with the tangents as free parameters, which no kernel runs, for the host) and the two singular parts (evaluatorJ3DK.cu:315-350, 352-407).
 //
 // Each function recomputes the forward intermediates of one point, returns the
 // forward value f, and adds gb . df/dx to the cotangents of the point p and of

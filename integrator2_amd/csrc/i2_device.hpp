@@ -241,12 +241,14 @@ I2_HD __forceinline__ q4 theta_terms(d3 p, const JGeom& J, const i2m::MathTable*
 // (FarFrame, FarPoint).  m itself, rounded, would shift all of the panel's points
 // by some 2^-53 |m| together: with m = C_i + (U + V)/3 kept in two parts, m - a is
 // (C_i - a) + (U + V)/3 and only differences of coordinates enter (pairs of a
-// mesh 500 radii from the origin: median error 2.2e-14 instead of 8.3e-14).  A squared distance to a vertex is then |m - a|^2 +
-// 2 b0 U.(m - a) + 2 b1 V.(m - a) + |b0 U + b1 V|^2: three instructions with
-// the last term, common to all vertices, in `pp`; and da.N2 is affine in (b0,
-// b1).  It loses no more than the plain difference because K_i's points lie
-// nearer to m than to K_j (panel_far).  From S1 S2 S3 = la^2 (lb + lc) + lb^2 (lc +
-// la) + lc^2 (la + lb) + 2 la lb lc, 2 x = S1 S2 S3 - (L_c^2 lc + L_a^2 la + L_b^2 lb).
+// mesh 500 radii from the origin: median error 2.2e-14 instead of 8.3e-14).
+//
+// A squared distance to a vertex is then |m - a|^2 + 2 b0 U.(m - a) + 2 b1
+// V.(m - a) + |b0 U + b1 V|^2: three instructions with the last term, common to
+// all vertices, in `pp`; and da.N2 is affine in (b0, b1).  It loses no more than
+// the plain difference because K_i's points lie nearer to m than to K_j
+// (panel_far).  From S1 S2 S3 = la^2 (lb + lc) + lb^2 (lc + la) + lc^2 (la + lb) +
+// 2 la lb lc, 2 x = S1 S2 S3 - (L_c^2 lc + L_a^2 la + L_b^2 lb).
 //
 // 94 FP64 instructions, DISTANT 83; from vertex differences and the three P it
 // was 110, theta_terms takes 184, and the reference's formula as the kernels

@@ -9,7 +9,8 @@
 // reproduces the reference's swapped result buffers exactly.  Unlike the
 // reference, child tasks are never materialised: a task at level k is one
 // group of lanes that walks its 4^k sub-panels by path digits and reduces in
-// a fixed order, so results are bitwise reproducible.
+// a fixed order, and nothing in a refined task depends on the order in which
+// the lists of unconverged tasks were filled, so results are bitwise reproducible.
 #include "i2_internal.hpp"
 #include "i2_batch.hpp"
 #include "i2_adjoint.hpp"

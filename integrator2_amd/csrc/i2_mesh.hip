@@ -373,12 +373,6 @@ __global__ void k_math(int fn, int64_t n, const double* __restrict__ x, const do
     else out[q] = i2m::atan2_any(y[q], x[q], &lt);
 }
 
-// Host evaluation of one ordered task's integrals with the kernels' device
-// code compiled for the host: level-`level` quadrature of (thetaPsi -
-// singular part) over K_i's sub-panels (the batched path's point and
-// sub-panel arithmetic, the division-free inner integral) plus the closed-form
-// singular part.  tri9 are the two panels' vertices, vid6 their vertex ids
-// (they decide the neighbour type and the rotations).  For checking.
 int i2_device_math(int device, int fn, const double* x, const double* y, int64_t n, double* out) {
     if (!x || !out || n <= 0 || fn < 0 || fn > 11 || ((fn == 1 || fn == 4 || fn == 11) && !y)) { set_error("invalid argument"); return I2_ERR_INVALID; }
     DeviceGuard g(device);
@@ -393,6 +387,14 @@ int i2_device_math(int device, int fn, const double* x, const double* y, int64_t
     return I2_OK;
 }
 
+// Host evaluation of one ordered task's integrals with the kernels' device
+// code compiled for the host: level-`level` quadrature of (thetaPsi -
+// singular part) over K_i's sub-panels, points from the sub-panels' vertices
+// and the inner integral's general form, plus the closed-form singular part.
+// The kernels evaluate disjoint pairs by the terms and far ones by polynomials;
+// this value agrees with theirs to rounding.  I9 and J9 are the two panels'
+// vertices, vid6 their vertex ids (they decide the neighbour type and the
+// rotations).  For checking.
 int i2_host_task_value(const double* I9, const double* J9, const int32_t* vid6, int level, const double* L12,
                        const double* w, int nPts, double* out4) {
     if (!I9 || !J9 || !vid6 || !L12 || !w || !out4 || nPts < 1 || nPts > i2d::MAX_POINTS || level < 0 || level > 12) {
