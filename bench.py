@@ -65,13 +65,13 @@ EVALS_PER_PAIR = 5 * POINTS - 1
 # lanes / evaluations.  roofline.achieved = this x evaluations / the kernel's
 # live HIP-event time.  VALU_ISSUE is the share of the VALU issue capacity the
 # same dispatch used (SQ_INSTS_VALU x 4 cycles / (SIMDs x busy cycles)).
-COUNTER_FLOPS_PER_EVAL = 125.7
-COUNTER_VALU_PER_EVAL = 95.7
-VALU_ISSUE = 0.79
+COUNTER_FLOPS_PER_EVAL = 126.2
+COUNTER_VALU_PER_EVAL = 97.2
+VALU_ISSUE = 0.82
 # HBM bytes per sweep dispatch on this workload, measured with rocprofv3
 # FETCH_SIZE and WRITE_SIZE and scaled by a 1 GiB copy's readings
-# (0.86 GB read + 3.37 GB written; the algorithmic figure is 2.33 GB)
-SWEEP_HBM_BYTES = 4.23e9
+# (0.62 GB read + 3.09 GB written; the algorithmic figure is 2.33 GB)
+SWEEP_HBM_BYTES = 3.71e9
 
 
 def flops_per_point():

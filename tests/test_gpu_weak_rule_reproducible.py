@@ -1,16 +1,17 @@
-"""The plain path's refined values with a rule that refines pairs at all
-distances: a task's value is its own, whichever tasks share its wavefront."""
+"""Refined values with a rule that refines pairs at all distances: a task's
+value is its own, whichever tasks share its wavefront."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-def test_weak_rule_bitwise_reproducible(gpu):
-    """3-point rule at a tight tolerance on 1,280 panels: with K = 2, so that tasks
-    report their level-2 value: many times the 8,192
-    disjoint tasks from which four share a wavefront at level 2, near and far
-    ones in the order in which they were found, which changes from run to run."""
+@pytest.mark.parametrize("path", [0, 1])
+def test_weak_rule_bitwise_reproducible(gpu, path):
+    """3-point rule at a tight tolerance on 1,280 panels, with K = 2, so that tasks
+    report their level-2 value: many times the 8,192 disjoint tasks from which
+    four share a wavefront at level 2, near and far ones in the order in which
+    they were found, which changes from run to run."""
     xyz, tri = gpu.icosphere(3, (1.4, 1.0, 0.8), 0.05, 7)
     L12, W, order = gpu.quadrature_rule(3)
     m = gpu.Mesh3D()
@@ -19,9 +20,10 @@ def test_weak_rule_bitwise_reproducible(gpu):
     it = gpu.NumericalIntegrator3D(m, L12.ravel(), W, order)
     it.setErrorControl(2, 1e-6, True)
     ev = gpu.EvaluatorJ3DK(m, it)
+    ev.setPath(path)
     first = None
     for rep in range(4):
-        print(f"run {rep}", flush=True)
+        print(f"path {path}, run {rep}", flush=True)
         ev.runAllPairs(False)
         r = ev.results(gpu.NOT_NEIGHBORS)
         if first is None:
