@@ -70,8 +70,8 @@ COUNTER_VALU_PER_EVAL = 97.2
 VALU_ISSUE = 0.82
 # HBM bytes per sweep dispatch on this workload, measured with rocprofv3
 # FETCH_SIZE and WRITE_SIZE and scaled by a 1 GiB copy's readings
-# (0.62 GB read + 3.09 GB written; the algorithmic figure is 2.33 GB)
-SWEEP_HBM_BYTES = 3.71e9
+# (0.61 GB read + 3.09 GB written; the algorithmic figure is 2.33 GB)
+SWEEP_HBM_BYTES = 3.70e9
 
 
 def flops_per_point():
